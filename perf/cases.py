@@ -75,7 +75,7 @@ def listed():
               tuned=True, forces=True),
         # The six-equation model, on the launch shapes a program gets without
         # tuning.
-        _case(name="sst_257x65", viscous=True, turb="sst", wall_k=300.0, cfl=2.0, passes=60),
+        _case(name="sst_257x65", viscous=True, turb="sst", wall_k=300.0, cfl=0.5, passes=40),
         # The reference's own multigrid: Runge-Kutta smoothing on three levels.
         _case(name="rk3_vcycle_257x65", levels=3, method="rk3", cfl=0.5, passes=50, tuned=True),
         # Time-accurate stepping: every inner iteration's norms go to the host.
@@ -126,9 +126,12 @@ def draw(rng):
     if kind == "rk3":
         return _case(nx=coarse, ny=4 * rng.randint(4, 20) + 1, levels=rng.randint(1, 3), method="rk3", cfl=0.5,
                      passes=rng.randint(20, 60), tuned=True)
-    if kind in ("sst", "bl"):
-        return _case(nx=odd, ny=ny, viscous=True, turb=kind, wall_k=300.0, cfl=2.0, passes=rng.randint(20, 60),
+    if kind == "sst":
+        return _case(nx=odd, ny=ny, viscous=True, turb="sst", wall_k=300.0, cfl=0.5, passes=rng.randint(15, 40),
                      tuned=rng.random() < 0.5)
+    if kind == "bl":
+        return _case(family="monitor", nx=odd, ny=ny, viscous=True, turb="bl", wall_k=300.0, cfl=0.2,
+                     passes=rng.randint(4, 10))
     if kind == "dual":
         return _case(nx=2 * (_log(rng, 49, 161) // 2) + 1, ny=_log(rng, 14, 49), viscous=True, turb="sa",
                      method="dual", cfl=0.2, passes=rng.randint(2, 4), inner=rng.randint(8, 20))
@@ -195,7 +198,11 @@ def _solver_cases(case, key):
     if case["grid"] == "blocks":
         return [solver.Case(_control(case, aoa=0.0), meshes[0])]
     if len(meshes) == 1 and case["sections"] * case["conditions"] == 1 and case["family"] != "drop":
-        re, ma = (6.5e6, 0.73) if case["fdm"] else (1.0e5, 0.5) if case["viscous"] else (1.0e6, 0.5)
+        re, ma = 1.0e6, 0.5
+        if case["fdm"]:
+            re, ma = 6.5e6, 0.73
+        elif case["viscous"] and case["turb"] != "sst":
+            re = 1.0e5
         return [solver.Case(_control(case, Ma=ma, aoa=2.0 if case["fdm"] else 1.25, Re=re), meshes[0])]
     free = _section_params(case)[1]
     per = case["conditions"]
