@@ -305,7 +305,7 @@ int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false)
     // slot per step (npad <= S + 7) and double, all sentinel
     int max_S = 1;
     for (auto& d : L.hb) max_S = std::max(max_S, d.sk_S);
-    L.gstride = ((int64_t)(max_S + 8) * 2 * L.o.nvar + 31) / 32 * 32;
+    L.gstride = ((int64_t)(max_S + 8) * L.o.nvar + 31) / 32 * 32;
     const int64_t n = (int64_t)L.hb.size() * (split - 1) * 2 * L.gstride;
     HIPCHK(hipMalloc(&L.dgring, sizeof(unsigned long long) * n));
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, R.s, L.dgring, n, GSENT);

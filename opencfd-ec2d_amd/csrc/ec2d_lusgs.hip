@@ -1,39 +1,61 @@
 // LU-SGS implicit update: du_LU_SGS_2D (sub_LU_SGS.f90:4-108), optionally
 // followed by U = U + dU (sub_NS_singlegrid.f90:203-211), for all blocks of
-// one mesh level.  Three launches:
+// one mesh level.  Two paths, chosen per level (ec2d_autotune):
 //
-//   k_lusgs_prep     every cell in parallel: writes, for each of the two
-//                    sweeps, a record of all the cell's update needs that does
-//                    not depend on dU - Res, U, the diagonal, the neighbours'
-//                    face coefficients and F(U_nb).n, which is the half of
-//                    comput_DFn that depends on the old state only;
-//   k_lusgs_sweep    one workgroup per block: the two dependent sweeps;
-//   k_lusgs_scatter  every cell in parallel: dU into the block planes and,
-//                    when asked, U = U + dU.
+//   split   k_lusgs_prep (every cell in parallel) writes, for each of the two
+//           sweeps, a record of all the cell's update needs that does not
+//           depend on dU; k_lusgs_sweep runs the two dependent sweeps;
+//           k_lusgs_scatter puts dU into the block planes (and U = U + dU);
+//   fused   k_lusgs_fused makes the records in the sweep's own workgroup and
+//           writes the planes itself (blocks of at most 64 rows).
 //
 // Sweep order.  The forward sweep needs dU(i-1,j) and dU(i,j-1), the backward
 // sweep dU(i+1,j) and dU(i,j+1).  Any order that respects these dependencies
-// gives the reference's result bit for bit.  Two lanes own one row of cells
-// and step s handles hyperplane s (sub_LU_SGS.f90:25-29, 70-75): row t takes
-// its cell at column offset c = s - t.  Of the pair, lane 2t evaluates the
-// j-neighbour's flux difference and lane 2t+1 the i-neighbour's; they swap
-// the two halves with a DPP quad permute and both finish the cell with the
-// same bits.  Every lane then finds its neighbour one lane down (DPP wave
-// shift): lane 2t the result of row t-1 (the j-neighbour), lane 2t+1 the
-// result of its own row at the step before (the i-neighbour); the first lane
-// of a wave gets row t-1 through LDS.
+// gives the reference's result bit for bit.  Step s handles hyperplane s
+// (sub_LU_SGS.f90:25-29, 70-75): row t takes its cell at column offset
+// c = s - t.
 //
-// The pair never selects by lane.  The backward sum dui + duj is one addition
-// and commutes.  The forward sum (Res + dui) + duj becomes pre + swap(pre)
-// with pre = X_k + (own term): lane 2t+1 loads Res as X_k, lane 2t loads -0.0
-// (the unwritten trash pad of the forward set's X fields holds it), and
-// -0.0 + x == x for every x, so both lanes add (Res + dui) and duj.
+// The sender's side of a cell.  Of the sums dui and duj of a cell, the part
+// that comes from one neighbour (sub_LU_SGS.f90:42-58, 85-100) needs that
+// neighbour's dU and U + dU, the face's normal and area, and the neighbour's
+// spectral radii: nothing of the receiving cell's own solution.  So the lane
+// that has just finished a cell forms both of the terms that its cell hands
+// on (to the next cell of its row, and to the cell of the next row) and
+// passes on these, NV doubles each, instead of dU and U + dU:
+//  - p and 1/rho of U + dU are formed once per cell, not once per user;
+//  - a neighbour's term crosses lanes in 2 NV register moves instead of 4 NV
+//    (and waves and workgroups in NV doubles instead of 2 NV);
+//  - F(U).n of a record is the cell's own, so a record is made from the
+//    cell's planes and the metrics of its two outgoing faces;
+//  - no lane selects: a cell without a neighbour adds the zero that an
+//    untouched lane holds (a row's lane before its first cell computes with
+//    a neutral record - U = (1, 0, 0, ...), everything else zero - whose
+//    outgoing terms are zero).
+// A sweep wave issues one instruction at a time, so its step takes as long
+// as its instruction count (4 cycles each in FP64); with the neighbour's side
+// a step of SA's one-lane form took about 290 vector instructions.
 //
-// Division by the diagonal.  The prep stores y = 1/alfa (correctly rounded);
-// the sweep forms q = a*y and refines it twice with FMA residuals (Markstein):
-// the first refinement makes q faithful, the second, with y = RN(1/alfa),
-// returns RN(a/alfa) - the quotient the reference's division gives, in five
-// dependent operations instead of the eleven of a full division.
+// Lanes.  One lane per row (LPC = 1), or two (LPC = 2): lane 2t forms the
+// term for the next cell of the row, lane 2t+1 the one for the next row.  The
+// terms move one lane up (DPP wave shift): lane 2t then holds its own term
+// and row t-1's, forms the sum and hands it to lane 2t+1 (DPP quad permute),
+// and both finish the cell with the same bits; with one lane per row, lane t
+// receives row t-1's.  The first lane of a wave gets row t-1 through LDS.
+//
+// Divisions.  Every quotient of a sweep has a divisor known before its
+// numerator (the diagonal) or shared by three quotients (rho of U + dU).  The
+// record holds y = RN(1/alfa), the sweep forms y = RN(1/rho) once per cell
+// (rcp_rn); a/b is q = a*y refined twice with FMA residuals (div_rcp,
+// Markstein): the first refinement makes q faithful, the second, with y
+// correctly rounded, returns RN(a/b) - the quotient the reference's division
+// gives, in five dependent operations instead of eleven.  (A quotient from 1/b
+// held to 2^-104 in two doubles takes two operations, but is not RN(a/b) where
+// rho is within a few units in the last place of 1, as it is in a cell the
+// flow has not reached: the quotients there lie next to rounding boundaries.)
+//
+// Scaling.  0.5*(DF*a + Lc*dU) is formed as DF*(0.5 a) + (0.5 Lc)*dU, and
+// -0.5*(DF*a - Lc*dU) as DF*(-0.5 a) + (0.5 Lc)*dU, with the factors in the
+// record: scaling by a power of two commutes with rounding.
 //
 // Record layout ("skewed").  A block's records are stored hyperplane by
 // hyperplane: the record of the cell that row t handles at step s sits at
@@ -46,8 +68,7 @@
 // waves.  Every load of a step is one contiguous run per wave (buffer loads
 // with one lane offset and a scalar offset per pair).  The forward record of
 // (s, t) belongs to cell (c+1, t+1), the backward record to cell
-// (ncol-c, nrow-t): both sweeps use the same neighbour tests (c != 0 for the
-// i-neighbour, t != 0 for the j-neighbour) and the same index arithmetic.
+// (ncol-c, nrow-t): both sweeps use the same index arithmetic.
 //
 // Per block the records occupy (2*NREC + 2*XP) * n doubles: the forward set,
 // the backward set (whose X pairs receive the forward dU from the forward
@@ -74,7 +95,7 @@ struct LusgsArgs {
   int split;              // sweep: workgroups per block (1, 2 or 4: a block's rows split between CUs)
   int dir;                // sweep: 0 both sweeps, 1 forward only, 2 backward only (split launches)
   unsigned long long* gring;  // sweep, split: one ring per boundary between workgroups and direction
-  int64_t gstride;        // sweep, split: slots of one ring (at least npad * 2 * NV)
+  int64_t gstride;        // sweep, split: slots of one ring (at least npad * NV)
   int* err;               // sweep, split: set when a cross-workgroup wait ran out of its budget
   int spin_max;           // the budget of a bounded wait, in polls
   int nblk;               // skew: blocks of this launch
@@ -82,26 +103,26 @@ struct LusgsArgs {
 };
 
 // Field layout of one record set (one sweep direction) of a block.  A
-// record has a part shared by the two lanes of a cell and a part per side
-// (k = 0: the j-neighbour, k = 1: the i-neighbour).  Both are sequences of
-// doubles stored in pairs; in doubles from the set's start:
-//   shared double d of position pos:   (d/2)*2n + 2*pos + d%2
+// record has a part of the cell and a part per side (k = 0: the term for the
+// next cell of the row, k = 1: the term for the next row).  Both are
+// sequences of doubles stored in pairs; in doubles from the set's start:
+//   cell's double d of position pos:   (d/2)*2n + 2*pos + d%2
 //   side double e of (pos, k):         NSH*n + (e/2)*4n + 2*(2*pos + k) + e%2
 // so that a wave's pair loads are contiguous and the two lanes of a cell
 // read adjacent pairs of their sides.
 template <int NV, bool VISC>
 struct RecF {
-  // shared: X = Res (forward) or the forward dU (backward), in whole pairs
-  // of their own (the forward pair lanes read them from another position);
-  // then U, the diagonal and its correctly rounded reciprocal (a separate one
-  // for the SA equation)
+  // cell: X = Res (forward) or the forward dU (backward), in whole pairs
+  // of their own; then U, the diagonal and its correctly rounded reciprocal (a
+  // separate one for the SA equation)
   static constexpr int XP = (NV + 1) / 2;
   static constexpr int U = 2 * XP, AL0 = U + NV, Y0 = AL0 + 1, AL4 = AL0 + 2, Y4 = AL0 + 3;
   static constexpr int NSH = 2 * XP + (NV + 2 + (NV == 5 ? 2 : 0) + 1) / 2 * 2;
-  // per side: F(U_nb).n, the normal, the face area, the neighbour's inviscid
-  // and viscous spectral radius (padded to whole pairs)
+  // per side: F(U).n, the normal, half the face area (negated: backward), half the
+  // inviscid and the viscous spectral radius (padded to whole pairs)
   static constexpr int F = 0, N1 = NV, N2 = NV + 1, A = NV + 2, LC = NV + 3, LV = NV + 4;
-  static constexpr int NSD = (NV + 4 + (VISC ? 1 : 0) + 1) / 2 * 2;
+  static constexpr int NSDU = NV + 4 + (VISC ? 1 : 0);  // without the padding
+  static constexpr int NSD = (NSDU + 1) / 2 * 2;
   static constexpr int NREC = NSH + 2 * NSD;  // doubles per position
 };
 
@@ -132,19 +153,20 @@ inline int lusgs_rec_doubles(int nv, bool visc) {
 }
 inline int lusgs_out_doubles(int nv) { return 2 * ((nv + 1) / 2); }
 
-// operands of one lane for one cell: the shared part and NS sides (NS = 1:
-// the lane's own side k, NS = 2: side 0 (j) and side 1 (i))
+// operands of one lane for one cell: the cell's part and NS sides (NS = 1:
+// the lane's own side k, NS = 2: both)
 template <int NV, int NS>
 struct Rec {
   double X[NV], U[NV];
   double F[NS][NV], n1[NS], n2[NS], a[NS], Lc[NS], Lv[NS];
-  double al0, al4, y0, y4;
+  double al0, y0, al4, y4;
 };
 
-// one cell as its neighbours need it: dU and U + dU
-template <int NV>
-struct Out {
-  double du[NV], W[NV];
+// what a cell hands on: the term of the next cell of its row and that of the
+// next row; with two lanes per cell each lane holds its own side's in j
+template <int NV, int LPC>
+struct Terms {
+  double i[LPC == 1 ? NV : 1], j[NV];
 };
 
 // lane l-1 -> lane l (lane 0 receives 0: bound_ctrl)
@@ -154,10 +176,10 @@ __device__ __forceinline__ double shr1(double v) {
   return __hiloint2double(hi, lo);
 }
 
-// lane l <-> lane l^1 (quad_perm [1,0,3,2])
-__device__ __forceinline__ double swap_pair(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+// lane 2t -> lanes 2t, 2t+1 (quad_perm [0,0,2,2])
+__device__ __forceinline__ double even_lane(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xA0, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xA0, 0xF, 0xF, true);
   return __hiloint2double(hi, lo);
 }
 
@@ -186,18 +208,18 @@ __device__ __forceinline__ void bstore1(double x, __amdgpu_buffer_rsrc_t r, uint
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), r, voff, soff, 0);
 }
 
-// v16: byte offset 16*pos of the lane's position, vx16 that of its X pairs
-// (its own, or a trash-pad slot); the field offsets are scalar and fixed.
-// base: byte offset of the record set in the block's record region, n16 =
-// 16n (bytes of one pair field); NS = 1 loads side k, NS = 2 both sides.
+// v16: byte offset 16*pos of the lane's position; the field offsets are
+// scalar and fixed.  base: byte offset of the record set in the block's
+// record region, n16 = 16n (bytes of one pair field); NS = 1 loads side k,
+// NS = 2 both sides.
 template <int NV, bool VISC, int NS>
 __device__ __forceinline__ void load_rec(Rec<NV, NS>& p, __amdgpu_buffer_rsrc_t r, uint32_t base, uint32_t n16,
-                                         uint32_t v16, uint32_t vx16, int k) {
+                                         uint32_t v16, int k) {
   using F = RecF<NV, VISC>;
   double sh[F::NSH];
 #pragma unroll
   for (int j = 0; j < F::NSH / 2; j++) {
-    const D2 v = bload2(r, j < F::XP ? vx16 : v16, base + (uint32_t)j * n16);
+    const D2 v = bload2(r, v16, base + (uint32_t)j * n16);
     sh[2 * j] = v.x;
     sh[2 * j + 1] = v.y;
   }
@@ -238,49 +260,54 @@ __device__ __forceinline__ void load_rec(Rec<NV, NS>& p, __amdgpu_buffer_rsrc_t 
 }
 
 // ----------------------------------------------------------------- prep
-// The arithmetic of one record (sub_LU_SGS.f90:31-58 forward, :76-100
-// backward) from a loader LD of its inputs; SH(d) and SD(k, e) give the
-// destination of shared double d and of side double e of side k (the global
-// skewed records of k_lusgs_prep, or an LDS slot of k_lusgs_fused).
-template <int NV, bool VISC, bool FWD, class SHF, class SDF, class LDF>
-__device__ __forceinline__ void rec_body(SHF SH, SDF SD, LDF LD, bool has_j, bool has_i, double g, double alfa1) {
+// The inputs of one record, loaded ahead of its arithmetic: the cell's own
+// planes and the metrics of its two outgoing faces.  Forward: the faces to
+// (i+1, j) and (i, j+1), whose normals and areas are those of the receiving
+// cells (sub_LU_SGS.f90:43-56).  Backward: the receiving cells' normals
+// (i-1, j), (i, j-1) with the cell's own areas (sub_LU_SGS.f90:86-99).  The
+// defaults are those of the neutral record.
+template <int NV>
+struct RecSrc {
+  double U[NV] = {1.0}, Res[NV] = {};
+  double vol = 1.0, dt = 1.0;
+  double Lc[2] = {}, Lv[2] = {}, n1[2] = {}, n2[2] = {}, s[2] = {};  // side 0: i, side 1: j
+};
+
+// The arithmetic of one record.  SH(d) and SD(k, e) give the destination of
+// the cell's double d and of side k's double e (the global skewed records of
+// k_lusgs_prep, or an LDS slot of k_lusgs_fused).
+// CF: the field numbers of the cell's part.
+template <int NV, bool VISC, bool FWD, class CF, class SHF, class SDF>
+__device__ __forceinline__ void rec_body(SHF SH, SDF SD, const RecSrc<NV>& q, double g, double alfa1) {
   using F = RecF<NV, VISC>;
-  using I = RecIn;
-  // LD(plane, who): who 0 the cell, 1 its j-neighbour, 2 its i-neighbour
 #pragma unroll
   for (int m = 0; m < NV; m++) {
-    SH(F::U + m) = LD(I::U + m, 0);
-    if (FWD) SH(m) = LD(I::RES<NV> + m, 0);
+    SH(CF::U + m) = q.U[m];
+    if (FWD) SH(m) = q.Res[m];
   }
   // diagonal (sub_LU_SGS.f90:31-39, 76-83)
-  const double vol = LD(I::VOL<NV>, 0), dt = LD(I::DT<NV>, 0);
-  double alfa = vol / dt + 1.0 * (LD(I::LCI<NV>, 0) + LD(I::LCJ<NV>, 0)) + vol * alfa1;
-  if constexpr (VISC) alfa = alfa + 2.0 * (LD(I::LVI<NV>, 0) + LD(I::LVJ<NV>, 0));
-  SH(F::AL0) = alfa;
-  SH(F::Y0) = 1.0 / alfa;
+  double alfa = q.vol / q.dt + 1.0 * (q.Lc[0] + q.Lc[1]) + q.vol * alfa1;
+  if constexpr (VISC) alfa = alfa + 2.0 * (q.Lv[0] + q.Lv[1]);
+  SH(CF::AL0) = alfa;
+  SH(CF::Y0) = rcp_rn(alfa);
   if constexpr (NV == 5) {
-    const double alfa4 = alfa + LD(I::LVI<NV>, 0) + LD(I::LVJ<NV>, 0);
-    SH(F::AL4) = alfa4;
-    SH(F::Y4) = 1.0 / alfa4;
+    const double alfa4 = alfa + q.Lv[0] + q.Lv[1];
+    SH(CF::AL4) = alfa4;
+    SH(CF::Y4) = rcp_rn(alfa4);
   }
-  // sides: k = 0 the j-neighbour, k = 1 the i-neighbour
+  const double y = rcp_rn(q.U[0]);
+  const double p = pressure_y(q.U, y, g);
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const bool has = k == 0 ? has_j : has_i;
-    if (!has) continue;
-    const int who = 1 + k;
-    const double n1 = LD(k == 0 ? I::NJ1<NV> : I::NI1<NV>, 0), n2 = LD(k == 0 ? I::NJ2<NV> : I::NI2<NV>, 0);
-    double Un[NV], Fo[NV];
-#pragma unroll
-    for (int m = 0; m < NV; m++) Un[m] = LD(I::U + m, who);
-    flux_n_old<NV>(Fo, Un, n1, n2, g);
+    double Fo[NV];
+    flux_n<NV>(Fo, q.U, y, p, q.n1[k], q.n2[k]);
 #pragma unroll
     for (int m = 0; m < NV; m++) SD(k, F::F + m) = Fo[m];
-    SD(k, F::N1) = n1;
-    SD(k, F::N2) = n2;
-    SD(k, F::A) = LD(k == 0 ? I::SJ<NV> : I::SI<NV>, FWD ? 0 : who);
-    SD(k, F::LC) = LD(k == 0 ? I::LCJ<NV> : I::LCI<NV>, who);
-    if constexpr (VISC) SD(k, F::LV) = LD(k == 0 ? I::LVJ<NV> : I::LVI<NV>, who);
+    SD(k, F::N1) = q.n1[k];
+    SD(k, F::N2) = q.n2[k];
+    SD(k, F::A) = (FWD ? 0.5 : -0.5) * q.s[k];
+    SD(k, F::LC) = 0.5 * q.Lc[k];
+    if constexpr (VISC) SD(k, F::LV) = q.Lv[k];
   }
 }
 
@@ -304,84 +331,85 @@ __device__ __forceinline__ int rec_in_slot(const PlaneMap& pm, int plane) {
     case 10: return pm.si;
     default: return pm.sj;
   }
-  (void)sizeof(I);
 }
 
-// One record set at position (c, r) from the block planes.  Forward: cell
-// (c+1, r+1), neighbours (i-1,j) and (i,j-1); the face areas are the cell's
-// own (sub_LU_SGS.f90:43-56).  Backward: cell (ncol-c, nrow-r), neighbours
-// (i+1,j) and (i,j+1), areas of the neighbour, normals of the cell itself
-// (sub_LU_SGS.f90:86-99).  SH(d) and SD(k, e) give the destination of shared
-// double d and of side double e of side k.
-template <int NV, bool VISC, bool FWD, class SHF, class SDF>
-__device__ __forceinline__ void make_rec(SHF SH, SDF SD, const BlockDesc& B, const double* base, const PlaneMap& pm,
-                                         int c, int r, double g, double alfa1) {
+// The inputs of position (c, r) from the block planes: forward cell
+// (c+1, r+1), backward cell (ncol-c, nrow-r).  The planes hold the metrics of
+// (i+1, j) and (i, j+1) for every cell (1:nx, 1:ny), and of the ghost layer
+// (unused values) before the first.
+template <int NV, bool VISC, bool FWD>
+__device__ __forceinline__ void load_src(RecSrc<NV>& o, const BlockDesc& B, const double* base, const PlaneMap& pm,
+                                         int c, int r) {
   const int ncol = B.nx - 1, nrow = B.ny - 1;
-  // A padding position is never active in a sweep, and a side without a
-  // neighbour is never used (the sweep selects 0 for it): neither is
-  // written.  They keep the zeros the record arena starts with, which no
-  // sweep overwrites (sweep stores go to the X pairs of cells and the trash
-  // pad), so an inactive lane only ever reads finite values.
-  if (r >= nrow || c < 0 || c >= ncol) return;
   const int i = FWD ? c + 1 : ncol - c;
   const int j = FWD ? r + 1 : nrow - r;
-  const int d = FWD ? -1 : 1;
-  const int64_t qw[3] = {pidx(B, i, j), pidx(B, i, j + d), pidx(B, i + d, j)};
-  auto LD = [&](int plane, int who) { return base[(int64_t)rec_in_slot<NV>(pm, plane) * B.plane + qw[who]]; };
-  rec_body<NV, VISC, FWD>(SH, SD, LD, r != 0, c != 0, g, alfa1);
+  const int d = FWD ? 1 : -1;
+  const int64_t q = pidx(B, i, j), qi = pidx(B, i + d, j), qj = pidx(B, i, j + d);
+  auto LD = [&](int slot, int64_t at) { return base[(int64_t)slot * B.plane + at]; };
+#pragma unroll
+  for (int m = 0; m < NV; m++) {
+    o.U[m] = LD(pm.U + m, q);
+    if constexpr (FWD) o.Res[m] = LD(pm.Res + m, q);
+  }
+  o.vol = LD(pm.vol, q);
+  o.dt = LD(pm.dt, q);
+  o.Lc[0] = LD(pm.Lci, q);
+  o.Lc[1] = LD(pm.Lcj, q);
+  if constexpr (VISC) {
+    o.Lv[0] = LD(pm.Lvi, q);
+    o.Lv[1] = LD(pm.Lvj, q);
+  }
+  o.n1[0] = LD(pm.ni1, qi);
+  o.n2[0] = LD(pm.ni2, qi);
+  o.s[0] = LD(pm.si, FWD ? qi : q);
+  o.n1[1] = LD(pm.nj1, qj);
+  o.n2[1] = LD(pm.nj2, qj);
+  o.s[1] = LD(pm.sj, FWD ? qj : q);
 }
 
-// The same record from the skewed copy of the inputs (k_lusgs_skew: logical
-// plane k of the block at sk + k n, a cell at its forward position
-// (i-1 + j-1) R + j-1).  Backward position (c, r) is the cell whose forward
-// position is (ncol-1-c + nrow-1-r) R + nrow-1-r; its neighbours (i+1, j),
-// (i, j+1) sit R and R + 1 further, the forward neighbours (i-1, j), (i, j-1)
-// R and R + 1 before.  Lanes of consecutive rows read consecutive positions.
-// Every input is loaded (one batch of independent loads) before the
-// arithmetic starts: a producer of the fused launch then waits for memory
-// once per record.
-template <int NV, bool VISC, bool FWD, class SHF, class SDF>
-__device__ __forceinline__ void make_rec_sk(SHF SH, SDF SD, const BlockDesc& B, const double* sk, int c, int r,
-                                            double g, double alfa1) {
+// The same inputs from the skewed copy (k_lusgs_skew: logical plane k of the
+// block at sk + k n, a cell at its forward position (i-1 + j-1) R + j-1).
+// Backward position (c, r) is the cell whose forward position is
+// (ncol-1-c + nrow-1-r) R + nrow-1-r; the cells (i+1, j), (i, j+1) sit R and
+// R + 1 further, (i-1, j), (i, j-1) R and R + 1 before.  Lanes of consecutive
+// rows read consecutive positions.  A position without a cell keeps the
+// neutral record, a face without a receiving cell zero metrics.
+template <int NV, bool VISC, bool FWD>
+__device__ __forceinline__ void load_src_sk(RecSrc<NV>& o, const BlockDesc& B, const double* __restrict__ sk, int c,
+                                            int r) {
   using I = RecIn;
   const int ncol = B.nx - 1, nrow = B.ny - 1;
+  o = RecSrc<NV>();
   if (r >= nrow || c < 0 || c >= ncol) return;
   const int64_t R = B.sk_R, n = B.sk_n;
   const int cf = FWD ? c : ncol - 1 - c, rf = FWD ? r : nrow - 1 - r;
   const int64_t p = (int64_t)(cf + rf) * R + rf;
-  const int64_t pw[3] = {p, FWD ? p - R - 1 : p + R + 1, FWD ? p - R : p + R};
-  const bool has[2] = {r != 0, c != 0};
-  // the cell's planes; per side the neighbour's U, Lc, Lv and face area
-  constexpr int NK = I::COUNT<NV>, NB = NV + 3;
-  double own[NK], nb[2][NB];
+  auto LD = [&](int plane, int64_t at) { return sk[(int64_t)plane * n + at]; };
 #pragma unroll
-  for (int k = 0; k < NK; k++) {
-    const bool need = (FWD || k < I::RES<NV> || k >= I::VOL<NV>) &&
-                      (VISC || (k != I::LVI<NV> && k != I::LVJ<NV>));
-    own[k] = need ? sk[(int64_t)k * n + p] : 0.0;
+  for (int m = 0; m < NV; m++) {
+    o.U[m] = LD(I::U + m, p);
+    if constexpr (FWD) o.Res[m] = LD(I::RES<NV> + m, p);
   }
-#pragma unroll
-  for (int kk = 0; kk < 2; kk++) {
-    const int64_t q = pw[1 + kk];
-#pragma unroll
-    for (int m = 0; m < NB; m++) nb[kk][m] = 0.0;
-    if (has[kk]) {
-#pragma unroll
-      for (int m = 0; m < NV; m++) nb[kk][m] = sk[(int64_t)(I::U + m) * n + q];
-      nb[kk][NV] = sk[(int64_t)(kk == 0 ? I::LCJ<NV> : I::LCI<NV>) * n + q];
-      if constexpr (VISC) nb[kk][NV + 1] = sk[(int64_t)(kk == 0 ? I::LVJ<NV> : I::LVI<NV>) * n + q];
-      if constexpr (!FWD) nb[kk][NV + 2] = sk[(int64_t)(kk == 0 ? I::SJ<NV> : I::SI<NV>) * n + q];
-    }
+  o.vol = LD(I::VOL<NV>, p);
+  o.dt = LD(I::DT<NV>, p);
+  o.Lc[0] = LD(I::LCI<NV>, p);
+  o.Lc[1] = LD(I::LCJ<NV>, p);
+  if constexpr (VISC) {
+    o.Lv[0] = LD(I::LVI<NV>, p);
+    o.Lv[1] = LD(I::LVJ<NV>, p);
   }
-  auto LD = [&](int plane, int who) -> double {
-    if (who == 0) return own[plane];
-    const double* v = nb[who - 1];
-    if (plane < NV) return v[plane];
-    if (plane == I::LCI<NV> || plane == I::LCJ<NV>) return v[NV];
-    if (plane == I::LVI<NV> || plane == I::LVJ<NV>) return v[NV + 1];
-    return v[NV + 2];  // the face area
-  };
-  rec_body<NV, VISC, FWD>(SH, SD, LD, has[0], has[1], g, alfa1);
+  if (c + 1 < ncol) {
+    const int64_t q = FWD ? p + R : p - R;
+    o.n1[0] = LD(I::NI1<NV>, q);
+    o.n2[0] = LD(I::NI2<NV>, q);
+    o.s[0] = LD(I::SI<NV>, FWD ? q : p);
+  }
+  if (r + 1 < nrow) {
+    const int64_t q = FWD ? p + R + 1 : p - R - 1;
+    o.n1[1] = LD(I::NJ1<NV>, q);
+    o.n2[1] = LD(I::NJ2<NV>, q);
+    o.s[1] = LD(I::SJ<NV>, FWD ? q : p);
+  }
 }
 
 template <int NV, bool VISC, bool FWD>
@@ -389,12 +417,14 @@ __device__ __forceinline__ void write_rec(double* __restrict__ rb, int64_t n, in
                                           const double* base, const PlaneMap& pm, int c, int r, double g,
                                           double alfa1) {
   using F = RecF<NV, VISC>;
-  // shared double d, side double e of side k (layout of RecF)
+  // the cell's double d, side double e of side k (layout of RecF)
   auto SH = [&](int d) -> double& { return rb[(int64_t)(d / 2) * 2 * n + 2 * pos + (d & 1)]; };
   auto SD = [&](int k, int e) -> double& {
     return rb[(int64_t)F::NSH * n + (int64_t)(e / 2) * 4 * n + 2 * (2 * pos + k) + (e & 1)];
   };
-  make_rec<NV, VISC, FWD>(SH, SD, B, base, pm, c, r, g, alfa1);
+  RecSrc<NV> q;
+  load_src<NV, VISC, FWD>(q, B, base, pm, c, r);
+  rec_body<NV, VISC, FWD, F>(SH, SD, q, g, alfa1);
 }
 
 // One thread per cell, a wave per 8 x 8 tile of cells (a workgroup per 32
@@ -424,14 +454,14 @@ __global__ __launch_bounds__(256) void k_lusgs_prep(LusgsArgs a) {
   const double* base = a.arena + B.base;
   double* fw = a.sk + B.sk_base;
   const int64_t R = B.sk_R;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    // -0.0 in the first trash-pad slot of the forward X pairs: the X operand
-    // of the j-neighbour lane of a pair (no sweep stores there)
-    const int64_t pad = (int64_t)B.sk_S * R;
-#pragma unroll
-    for (int d = 0; d < 2 * F::XP; d++) fw[(int64_t)(d / 2) * 2 * n + 2 * pad + (d & 1)] = -0.0;
+  if (s < S && r < nrow && c < 0) {
+    // a row's lane before its first cell: the neutral record of both sets
+    // (the rest of the position keeps the zeros the record arena starts with)
+    const int64_t at = (int64_t)(F::U / 2) * 2 * n + 2 * ((int64_t)s * R + r) + (F::U & 1);
+    fw[at] = 1.0;
+    fw[F::NREC * n + at] = 1.0;
   }
-  if (s >= S || r >= nrow || c < 0 || c >= ncol) return;  // padding positions stay unwritten
+  if (s >= S || r >= nrow || c < 0 || c >= ncol) return;  // other padding positions stay unwritten
   // the cell's forward record at (c, r), its backward record at (ncol-1-c, nrow-1-r)
   const int cb = ncol - 1 - c, rb = nrow - 1 - r;
   write_rec<NV, VISC, true>(fw, n, (int64_t)(c + r) * R + r, B, base, a.pm, c, r, g, a.alfa1);
@@ -565,21 +595,18 @@ __global__ __launch_bounds__(256) void k_lusgs_unskew(LusgsArgs a) {
 }
 
 // ----------------------------------------------------------------- sweeps
-// One side's share of a cell, dui (the i-neighbour) or duj (the
-// j-neighbour), of sub_LU_SGS.f90:42-58 (forward) or :85-100 (backward);
-// h selects the side held in the record.
-template <int NV, bool VISC, bool FWD, int NS>
-__device__ __forceinline__ void side_term(double* d, const Rec<NV, NS>& p, int h, const Out<NV>& nb, bool has,
-                                          double g) {
+// The term that a finished cell (dU, W = U + dU, the reciprocal of its density
+// and its pressure) hands on through side h of its record: dui or duj of
+// sub_LU_SGS.f90:42-58 (forward) or :85-100 (backward) for the receiving cell.
+template <int NV, bool VISC, int NS>
+__device__ __forceinline__ void side_term(double* v, const Rec<NV, NS>& p, int h, const double* W, const double* du,
+                                          double y, double pr) {
   double DF[NV];
-  dfn_from_old<NV>(DF, nb.W, p.F[h], p.n1[h], p.n2[h], g);
+  dfn<NV>(DF, W, p.F[h], y, pr, p.n1[h], p.n2[h]);
 #pragma unroll
   for (int m = 0; m < NV; m++) {
-    double v;
-    if (FWD) v = 0.5 * (DF[m] * p.a[h] + 1.0 * p.Lc[h] * nb.du[m]);
-    else v = -0.5 * (DF[m] * p.a[h] - 1.0 * p.Lc[h] * nb.du[m]);
-    if constexpr (VISC) v = v + p.Lv[h] * nb.du[m];
-    d[m] = has ? v : 0.0;
+    v[m] = DF[m] * p.a[h] + p.Lc[h] * du[m];
+    if constexpr (VISC) v[m] = v[m] + p.Lv[h] * du[m];
   }
 }
 
@@ -610,10 +637,10 @@ __device__ __forceinline__ void side_term(double* d, const Rec<NV, NS>& p, int h
 // ring[w] is the input of wave w: its producer is wave w-1 (or, in the upper
 // workgroup of a split block, the communication wave), prog[w] that
 // producer's progress and cons[w] wave w's consumption.
-constexpr int RING = 8;
+constexpr int RING = 16;
 template <int NV>
 struct Chain {
-  double ring[17][RING][2 * NV];  // input of wave w: (dU, U + dU) of the row below it
+  double ring[17][RING][NV];  // input of wave w: the terms of the row below it
   int prog[17];                   // steps finished by the producer of ring[w]
   int cons[17];                   // steps whose input wave w has read
 };
@@ -622,7 +649,7 @@ struct Chain {
 // seen when it was read
 template <int NV>
 struct Ahead {
-  double du[NV], W[NV];
+  double v[NV];
   int prog, cons;
 };
 
@@ -638,25 +665,27 @@ __device__ __forceinline__ void wait_at_least(const int* p, int v) {
 }
 
 // One step of a sweep: the cell of row t at column offset c = s - t.
-// LPC = 2: lanes 2t (k = 0, the j-neighbour's term) and 2t+1 (k = 1, the
-// i-neighbour's term) share the cell and swap their halves; LPC = 1: lane t
-// computes both.
+// LPC = 2: lanes 2t (k = 0, the term for the next cell of the row) and 2t+1
+// (k = 1, the term for the next row) share the cell; LPC = 1: lane t forms both.
 // ODD1 (the fused launch's layout): with an odd equation count the last X
 // field holds single doubles, not a pair padded with zero, and lanes without
-// a cell store nothing (no trash-pad slot)
+// a cell store nothing (no trash-pad slot).  out: the cell's dU and U + dU.
+template <int NV>
+struct Out {
+  double du[NV], W[NV];
+};
+
 template <int NV, bool VISC, bool FWD, int LPC, bool STORE = true, bool ODD1 = false>
-__device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Out<NV>& own, __amdgpu_buffer_rsrc_t rs,
-                                           uint32_t dst, uint32_t n16, int s, int S, int R, int ncol, int nrow, int t,
-                                           int k, int lane, int wave, bool cin, bool cout, double g,
-                                           Chain<NV>& ch, Ahead<NV>& ah) {
-  // the j-neighbour's result: row t-1's, one lane down (the last lane of the
-  // previous wave through the LDS ring); the i-neighbour's is the own row's
-  Out<NV> up;
+__device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Terms<NV, LPC>& tm, Out<NV>& o,
+                                           __amdgpu_buffer_rsrc_t rs, uint32_t dst, uint32_t n16, int s, int S, int R,
+                                           int ncol, int nrow, int t, int k, int lane, int wave, bool cin, bool cout,
+                                           double g, Chain<NV>& ch, Ahead<NV>& ah) {
+  // the term of row t-1 (LPC = 2: lane 2t receives it, lane 2t+1 the term of
+  // its own row, which it does not use), one lane down; the first lane's
+  // from the last lane of the previous wave through the LDS ring
+  double jin[NV];
 #pragma unroll
-  for (int m = 0; m < NV; m++) {
-    up.du[m] = shr1(own.du[m]);
-    up.W[m] = shr1(own.W[m]);
-  }
+  for (int m = 0; m < NV; m++) jin[m] = shr1(tm.j[m]);
   if (cin) {
     // the row below this wave at step s-1 (an LDS broadcast), lane 0 keeps
     // it; read one step ahead unless the producer was not there yet
@@ -664,16 +693,10 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Out<NV>& o
       wait_at_least(&ch.prog[wave], s);
       const double* x = ch.ring[wave][(s - 1) & (RING - 1)];
 #pragma unroll
-      for (int m = 0; m < NV; m++) {
-        ah.du[m] = x[m];
-        ah.W[m] = x[NV + m];
-      }
+      for (int m = 0; m < NV; m++) ah.v[m] = x[m];
     }
 #pragma unroll
-    for (int m = 0; m < NV; m++) {
-      up.du[m] = lane == 0 ? ah.du[m] : up.du[m];
-      up.W[m] = lane == 0 ? ah.W[m] : up.W[m];
-    }
+    for (int m = 0; m < NV; m++) jin[m] = lane == 0 ? ah.v[m] : jin[m];
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.cons[wave], s);
     // the input of step s+1: prog first, the slot behind it
@@ -681,52 +704,39 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Out<NV>& o
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     const double* x = ch.ring[wave][s & (RING - 1)];
 #pragma unroll
-    for (int m = 0; m < NV; m++) {
-      ah.du[m] = x[m];
-      ah.W[m] = x[NV + m];
-    }
+    for (int m = 0; m < NV; m++) ah.v[m] = x[m];
   }
-  const int c = s - t;
-  const bool act = t < nrow && c >= 0 && c < ncol;
-  // sum: (Res + dui) + duj forward, dui + duj backward
-  double sum[NV];
-  if constexpr (LPC == 2) {
-    // the neighbour one lane down is the j-neighbour for lane 2t and the
-    // i-neighbour for lane 2t+1
-    double mine[NV];
-    side_term<NV, VISC, FWD, 1>(mine, p, 0, up, k == 0 ? t != 0 : c != 0, g);
-#pragma unroll
-    for (int m = 0; m < NV; m++) {
-      const double pre = FWD ? p.X[m] + mine[m] : mine[m];  // forward: X = Res (lane 2t+1), -0.0 (lane 2t)
-      sum[m] = pre + swap_pair(pre);
-    }
-  } else {
-    double dui[NV], duj[NV];
-    side_term<NV, VISC, FWD, 2>(duj, p, 0, up, t != 0, g);
-    side_term<NV, VISC, FWD, 2>(dui, p, 1, own, c != 0, g);
-#pragma unroll
-    for (int m = 0; m < NV; m++) sum[m] = FWD ? p.X[m] + dui[m] + duj[m] : dui[m] + duj[m];
-  }
-  Out<NV> o;
+  // (Res + dui) + duj forward, X + (dui + duj) / alfa backward
 #pragma unroll
   for (int m = 0; m < NV; m++) {
+    const double iin = LPC == 1 ? tm.i[LPC == 1 ? m : 0] : tm.j[m];
+    double sum = FWD ? (p.X[m] + iin) + jin[m] : iin + jin[m];
+    if constexpr (LPC == 2) sum = even_lane(sum);
     const bool sa = NV == 5 && m == 4;
-    const double q = div_rcp(sum[m], sa ? p.al4 : p.al0, sa ? p.y4 : p.y0);
-    const double du = FWD ? q : p.X[m] + q;
-    o.du[m] = du;
-    o.W[m] = p.U[m] + du;
+    const double q = div_rcp(sum, sa ? p.al4 : p.al0, sa ? p.y4 : p.y0);
+    o.du[m] = FWD ? q : p.X[m] + q;
+    o.W[m] = p.U[m] + o.du[m];
   }
-  // Every lane keeps its result, active or not: an inactive lane's value
-  // never reaches an active cell.  Row t's first cell (c = 0) ignores its
-  // i-neighbour; row t+1 at step s+1 sits at the same column offset as row t
-  // at step s, so it is inactive whenever row t was.
-  own = o;
+  // Every lane keeps its terms, active or not: an inactive lane's never
+  // reach an active cell.  Before its first cell a row holds the neutral
+  // record's zeros; row t+1 at step s+1 sits at the same column offset as
+  // row t at step s, so it is inactive whenever row t was.
+  const double y = rcp_rn(o.W[0]);
+  const double pr = pressure_y(o.W, y, g);
+  if constexpr (LPC == 1) {
+    side_term<NV, VISC>(tm.i, p, 0, o.W, o.du, y, pr);
+    side_term<NV, VISC>(tm.j, p, 1, o.W, o.du, y, pr);
+  } else {
+    side_term<NV, VISC>(tm.j, p, 0, o.W, o.du, y, pr);
+  }
   if constexpr (STORE) {
     // one lane of an active cell stores; every other lane writes its own
     // slot of the trash pad (positions S*R .. S*R+63)
-    const uint32_t w = (act && k == 0) ? (FWD ? (uint32_t)((S - 1 - s) * R + (nrow - 1 - t)) : (uint32_t)(s * R + t))
-                                       : (uint32_t)(S * R + lane);
-    if (!ODD1 || (act && k == 0)) {
+    const int c = s - t;
+    const bool act = t < nrow && c >= 0 && c < ncol && k == 0;
+    const uint32_t w = act ? (FWD ? (uint32_t)((S - 1 - s) * R + (nrow - 1 - t)) : (uint32_t)(s * R + t))
+                           : (uint32_t)(S * R + lane);
+    if (!ODD1 || act) {
 #pragma unroll
       for (int j = 0; j < (NV + 1) / 2; j++) {
         if (ODD1 && 2 * j + 1 == NV) bstore1(o.du[2 * j], rs, w * 8u, dst + (uint32_t)j * n16);
@@ -740,7 +750,7 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Out<NV>& o
     if (lane == 63) {
       double* x = ch.ring[wave + 1][s & (RING - 1)];
 #pragma unroll
-      for (int m = 0; m < NV; m++) { x[m] = own.du[m]; x[NV + m] = own.W[m]; }
+      for (int m = 0; m < NV; m++) x[m] = tm.j[m];
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.prog[wave + 1], s + 1);
@@ -748,12 +758,7 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Out<NV>& o
   }
 }
 
-// One sweep.  With LPC = 2 lanes 2t and 2t+1 own row t: lane 2t computes
-// the j-neighbour's term, lane 2t+1 the i-neighbour's, the pair swaps them
-// (DPP) and both finish the cell, so both hold the cell's result.  With
-// LPC = 1 lane t owns row t alone.  The i-neighbour of a cell is the own
-// row's previous result (registers); the j-neighbour is the previous result
-// of row t-1, which the next lane down holds: one DPP shift up.
+// One sweep (lanes: the head of this file).
 // The records come in two register sets of U steps each, loaded one phase
 // ahead: [load B] [steps of A] [load A] [steps of B] ...  Whenever the code
 // waits for a set, the only loads still in flight are the other set's, issued
@@ -771,23 +776,22 @@ __device__ __forceinline__ void sweep(__amdgpu_buffer_rsrc_t rs, uint32_t rec, u
   // results never reach a cell)
   const int tl = min(t, nrow - 1);
   constexpr int NS = 3 - LPC;
-  Out<NV> own = {};
+  Terms<NV, LPC> tm = {};
   Rec<NV, NS> A[U], B[U];
-  // forward pairs: lane 2t reads X (-0.0) from the first trash-pad slot
-  const bool xpad = FWD && LPC == 2 && k == 0;
-  const uint32_t pad16 = (uint32_t)(S * R) * 16u;
   auto load_set = [&](Rec<NV, NS>* set, int s_first) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const uint32_t v16 = (uint32_t)(min(s_first + u, S - 1) * R + tl) * 16u;
-      load_rec<NV, VISC, NS>(set[u], rs, rec, n16, v16, xpad ? pad16 : v16, k);
+      load_rec<NV, VISC, NS>(set[u], rs, rec, n16, v16, k);
     }
   };
   auto run_set = [&](const Rec<NV, NS>* set, int s_first) {
 #pragma unroll
-    for (int u = 0; u < U; u++)
-      sweep_step<NV, VISC, FWD, LPC>(set[u], own, rs, dst, n16, s_first + u, S, R, ncol, nrow, t, k, lane, wave,
-                                     cin, cout, g, ch, ah);
+    for (int u = 0; u < U; u++) {
+      Out<NV> o;
+      sweep_step<NV, VISC, FWD, LPC>(set[u], tm, o, rs, dst, n16, s_first + u, S, R, ncol, nrow, t, k, lane, wave, cin,
+                                     cout, g, ch, ah);
+    }
   };
   load_set(A, 0);
   for (int s0 = 0; s0 < npad; s0 += 2 * U) {
@@ -837,14 +841,14 @@ __global__ void k_fill_u64(unsigned long long* p, int64_t n, unsigned long long 
   if (i < n) p[i] = v;
 }
 
-// The communication waves move CK = 64 / (2 NV) steps at a time, one double
-// per lane, so that one round trip to global memory covers CK steps.
+// The communication waves move CK steps at a time (64 / NV, at most half the
+// LDS ring), one double per lane, so that one round trip to global memory covers CK steps.
 template <int NV>
 struct CommLane {
-  static constexpr int CK = 64 / (2 * NV);
+  static constexpr int CK = 64 / NV < RING / 2 ? 64 / NV : RING / 2;
   int kk, f;
   bool on;  // this lane carries double f of step kk of the batch
-  __device__ CommLane() : kk((int)(threadIdx.x & 63) / (2 * NV)), f((int)(threadIdx.x & 63) % (2 * NV)), on(kk < CK) {}
+  __device__ CommLane() : kk((int)(threadIdx.x & 63) / NV), f((int)(threadIdx.x & 63) % NV), on(kk < CK) {}
 };
 
 // sending side: take ring[nw] (the last compute wave's row) and store it
@@ -858,7 +862,7 @@ __device__ void comm_forward(Chain<NV>& ch, int nw, unsigned long long* gr, int 
     const double v = on ? ch.ring[nw][(s0 + c.kk) & (RING - 1)][c.f] : 0.0;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.cons[nw], s0 + nst);
-    if (on) gstore(gr + (s0 + c.kk) * (2 * NV) + c.f, __builtin_bit_cast(unsigned long long, v));
+    if (on) gstore(gr + (s0 + c.kk) * NV + c.f, __builtin_bit_cast(unsigned long long, v));
   }
 }
 
@@ -873,7 +877,7 @@ __device__ void comm_receive(Chain<NV>& ch, unsigned long long* gr, int npad, in
     const bool on = c.on && c.kk < nst;
     double v = 0.0;
     if (on && !gone) {
-      unsigned long long* slot = gr + (s0 + c.kk) * (2 * NV) + c.f;
+      unsigned long long* slot = gr + (s0 + c.kk) * NV + c.f;
       unsigned long long x;
       int n = 0;
       while ((x = gload(slot)) == GSENT && ++n < spin_max) __builtin_amdgcn_s_sleep(1);
@@ -890,7 +894,7 @@ __device__ void comm_receive(Chain<NV>& ch, unsigned long long* gr, int npad, in
     lds_put(&ch.prog[0], s0 + nst);
   }
   // every value of this launch has been read: back to the sentinel
-  for (int i = (int)(threadIdx.x & 63); i < (npad - 1) * 2 * NV; i += 64) gstore(gr + i, GSENT);
+  for (int i = (int)(threadIdx.x & 63); i < (npad - 1) * NV; i += 64) gstore(gr + i, GSENT);
 }
 
 // LPC lanes per cell (1 or 2), U steps per register set, MAXT threads at most.
@@ -935,10 +939,9 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
     else if (rcv) comm_receive<NV>(ch[0], gr(half - 1, 0), npad, a.err, a.spin_max);
     else if (snd) comm_forward<NV>(ch[0], nw, gr(half, 0), npad);
   }
-  if (a.dir == 0) {
-    __threadfence();
-    __syncthreads();
-  }
+  // the forward sweep's X before the backward sweep reads it: in one launch
+  // only when the block has one workgroup, so a barrier (workgroup scope) does
+  if (a.dir == 0) __syncthreads();
   if (a.dir != 1) {
     if (wave < nw) sweep<NV, VISC, false, U, LPC>(rs, bw, out, n16, S, R, ncol, nrow, t, k, lane, wave, cin, cout, g, ch[1]);
     else if (rcv) comm_receive<NV>(ch[1], gr(half - 1, 1), npad, a.err, a.spin_max);
@@ -954,8 +957,9 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
 // highest issue priority of its SIMD; waves 1..NP produce the records, each
 // every NP-th step of the sequence (forward steps 0..npad-1, then backward
 // steps 0..npad-1), lane t the cell of row t, from the skewed copy of the
-// inputs that k_lusgs_skew made (make_rec_sk, the arithmetic of
-// k_lusgs_prep), into a ring of LDS slots (6 for NP = 3, 7 for NP = 6).  The
+// inputs that k_lusgs_skew (or the residual) made, into a ring of LDS slots.
+// A producer loads the inputs of its next record before it waits for a slot,
+// so that memory latency is off the records' path.  The
 // forward dU goes to the backward records' X pairs in global memory (the
 // backward sweep reads it there, after a fence).  The sweep wave puts the
 // backward U + dU (with update; dU without) of eight steps into an LDS
@@ -963,30 +967,43 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
 // the writer, takes each chunk and stores it to the block planes eight
 // consecutive cells of a row at a time: this replaces k_lusgs_scatter
 // (stores along a hyperplane, one cache line per lane, hold up whichever
-// wave issues them).  NP = 3 or 6 (5 or 8 waves; with 6 the ring and the
-// buffer of a six-equation record take 157 KB of the CU's 160 KB).
+// wave issues them).  NP = 3 or 6 (5 or 8 waves).
+//
+// The slots hold the records without RecF's padding: 34 doubles of SA, eight
+// slots and the buffer take 156 KB of the CU's 160 KB (a six-equation record
+// has six slots).  The slot count is a multiple of the steps per turn of the
+// sweep's loop, so that a step's slot is a constant of the unrolled loop plus
+// the turn's first.
 //
 // The writer waits for ob_ready > chunk, reads the chunk, then sets
 // ob_taken = chunk + 1; the sweep wave waits for ob_taken >= chunk before
 // it writes the chunk's first step, and sets ob_ready after its last.
-// Protocol: produced[p] counts the steps producer p has written, consumed
-// the steps whose slot the sweep wave has finished with (it releases slot g
-// after computing step g).  The sweep wave waits, before reading step g,
-// for produced[g % NP] > g / NP; producer p waits, before writing step g
-// into slot g % NRING, for consumed >= g - NRING + 1.  A producer waits only
+// Protocol: ready[slot] is one more than the step whose record the slot holds,
+// consumed the steps whose slot the sweep wave has finished with (it releases
+// slot g after computing step g).  The sweep wave waits, before reading step
+// g, for ready[g % NRING] > g; a producer waits, before writing step
+// g into slot g % NRING, for consumed >= g - NRING + 1.  A producer waits only
 // for the sweep wave and the sweep wave only for producers that are never
 // more than NRING steps ahead, so every wait ends; waits are also bounded
 // (a.spin_max polls, then err is set and the wave stops waiting).
-template <int NV, bool VISC, int NP>
-struct FusedLds {
+template <int NV, bool VISC>
+struct FusedSlot {
   using F = RecF<NV, VISC>;
-  static constexpr int NRING = NP == 3 ? 6 : 7;  // LDS record slots
-  double sh[NRING][F::NSH][64];     // shared doubles of slot, lane
-  double sd[NRING][2][F::NSD][64];  // side doubles
-  double ob[8][NV][64];             // the sweep's backward U + dU (update) or dU of eight steps
-  int produced[NP];
+  // the cell's doubles (X without its padding) and a side's
+  static constexpr int U = NV, AL0 = 2 * NV, Y0 = AL0 + 1, AL4 = AL0 + 2, Y4 = AL0 + 3;
+  static constexpr int NSH = 2 * NV + 2 + (NV == 5 ? 2 : 0), NSD = F::NSDU;
+  static constexpr int XD = NV >= 6 ? 2 : 4;     // sweep steps per turn of its loop
+  static constexpr int NRING = NV >= 6 ? 6 : 8;  // record slots
+};
+template <int NV, bool VISC>
+struct FusedLds {
+  using F = FusedSlot<NV, VISC>;
+  double sh[F::NRING][F::NSH][64];     // the cells' doubles of slot, lane
+  double sd[F::NRING][2][F::NSD][64];  // the sides'
+  double ob[8][NV][64];                // the sweep's backward U + dU (update) or dU of eight steps
+  int ready[8];
   int consumed;
-  int ob_ready, ob_taken;           // chunks of eight backward steps put into / taken from ob
+  int ob_ready, ob_taken;              // chunks of eight backward steps put into / taken from ob
 };
 
 __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int spin_max) {
@@ -1005,8 +1022,9 @@ __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int 
 template <int NV, bool VISC, int NP>
 __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
   using F = RecF<NV, VISC>;
-  using LDS = FusedLds<NV, VISC, NP>;
-  constexpr int FPROD = NP, FRING = LDS::NRING;
+  using LDS = FusedLds<NV, VISC>;
+    constexpr int FPROD = NP, FRING = FusedSlot<NV, VISC>::NRING, XD = FusedSlot<NV, VISC>::XD;
+  static_assert(FRING % XD == 0 && FRING <= 8, "slots per turn");
   __shared__ LDS L;
   const BlockDesc B = a.blocks[a.block_list[blockIdx.x]];
   if (case_frozen(B.case_id)) return;
@@ -1014,7 +1032,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
   const int ncol = B.nx - 1, nrow = B.ny - 1;
   const int S = B.sk_S, R = B.sk_R;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid < FPROD) L.produced[tid] = 0;
+  if (tid < 8) L.ready[tid] = 0;
   if (tid == 0) L.consumed = L.ob_ready = L.ob_taken = 0;
   __syncthreads();
   constexpr int U = 2;  // the sweep's step padding (npad) of k_lusgs_sweep<..., 2, ..., 1>
@@ -1088,37 +1106,47 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
     // ---- producer: the inputs from their skewed copy (k_lusgs_skew), so
     // that the lanes (rows) of a step read consecutive positions
     const double* skin = a.sk + B.sk_base;
-    const int p = wave - 1;
-    for (int gs = p, k = 0; gs < ntot && ok; gs += FPROD, k++) {
-      ok = wait_bounded(&L.consumed, gs - FRING + 1, a.err, a.spin_max);
-      const int slot = gs % FRING;
-      const bool fwd = gs < npad;
-      const int st = fwd ? gs : gs - npad;
-      auto SH = [&](int d) -> double& { return L.sh[slot][d][lane]; };
-      auto SD = [&](int kk, int e) -> double& { return L.sd[slot][kk][e][lane]; };
-      if (fwd) make_rec_sk<NV, VISC, true>(SH, SD, B, skin, st - lane, lane, g, a.alfa1);
-      else make_rec_sk<NV, VISC, false>(SH, SD, B, skin, st - lane, lane, g, a.alfa1);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // the slot's LDS writes done (lgkmcnt 0) before publishing
-      lds_put(&L.produced[p], k + 1);
-    }
+    auto produce = [&](auto fwd_c, int first) {
+      constexpr bool fwd = decltype(fwd_c)::value;
+      const int gs0 = fwd ? 0 : npad;
+      RecSrc<NV> nx;
+      load_src_sk<NV, VISC, fwd>(nx, B, skin, first - gs0 - lane, lane);
+      int gs = first;
+      for (; gs < gs0 + npad && ok; gs += FPROD) {
+        const RecSrc<NV> q = nx;
+        // the next record's inputs (past the last step: clamped to it)
+        load_src_sk<NV, VISC, fwd>(nx, B, skin, min(gs + FPROD - gs0, npad - 1) - lane, lane);
+        ok = wait_bounded(&L.consumed, gs - FRING + 1, a.err, a.spin_max);
+        const int slot = gs % FRING;
+        auto SH = [&](int d) -> double& { return L.sh[slot][d][lane]; };
+        auto SD = [&](int kk, int e) -> double& { return L.sd[slot][kk][e][lane]; };
+        rec_body<NV, VISC, fwd, FusedSlot<NV, VISC>>(SH, SD, q, g, a.alfa1);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // the slot's LDS writes done (lgkmcnt 0) before publishing
+        lds_put(&L.ready[slot], gs + 1);
+      }
+      return gs;
+    };
+    const int g1 = produce(std::true_type{}, wave - 1);
+    if (ok) produce(std::false_type{}, g1);
     return;
   }
   // ---- the sweep wave: lane t = row t; it issues first on its SIMD
   __builtin_amdgcn_s_setprio(3);
   const int t = lane;
   Chain<NV>& ch = *reinterpret_cast<Chain<NV>*>(&L);  // no other compute wave: never touched
+  using FS = FusedSlot<NV, VISC>;
   auto load_lds = [&](Rec<NV, 2>& r, int slot, bool fwd) {
 #pragma unroll
     for (int m = 0; m < NV; m++) {
       if (fwd) r.X[m] = L.sh[slot][m][t];
-      r.U[m] = L.sh[slot][F::U + m][t];
+      r.U[m] = L.sh[slot][FS::U + m][t];
     }
-    r.al0 = L.sh[slot][F::AL0][t];
-    r.y0 = L.sh[slot][F::Y0][t];
+    r.al0 = L.sh[slot][FS::AL0][t];
+    r.y0 = L.sh[slot][FS::Y0][t];
     if constexpr (NV == 5) {
-      r.al4 = L.sh[slot][F::AL4][t];
-      r.y4 = L.sh[slot][F::Y4][t];
+      r.al4 = L.sh[slot][FS::AL4][t];
+      r.y4 = L.sh[slot][FS::Y4][t];
     } else {
       r.al4 = r.al0;
       r.y4 = r.y0;
@@ -1161,25 +1189,26 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
   // is read from its slot while this step computes; in the backward sweep
   // each step's X (the forward dU) is loaded XD steps ahead, into one of XD
   // register sets (the loop runs XD steps per turn; npad is a multiple of 4).
+  int slot0 = 0;  // the slot of the turn's first step
   auto run_dir = [&](auto fwd_c) {
     constexpr bool fwd = decltype(fwd_c)::value;
-    constexpr int dir = fwd ? 0 : 1;
-    const int gs0 = dir * npad;
+    const int gs0 = fwd ? 0 : npad;
     Ahead<NV> ah = {};
-    Out<NV> own = {};
-    constexpr int XD = NV >= 6 ? 2 : 4;  // six-equation records leave no registers for four sets
+    Terms<NV, 1> tm = {};
     double xs[XD][2 * F::XP] = {};
     if (!fwd) {
-      // the forward sweep's stores to the X pairs before these loads
-      __threadfence();
+      // the forward sweep's stores to the X pairs before these loads, which
+      // the same wave issues: workgroup scope.  A device-scope fence also
+      // writes back the whole L2 (a launch of one block took 0.11 ms longer).
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
 #pragma unroll
       for (int k = 0; k < XD; k++) load_x(xs[k], k);
     }
     Rec<NV, 2> rn;
-    if (ok) ok = wait_bounded(&L.produced[gs0 % FPROD], gs0 / FPROD + 1, a.err, a.spin_max);
-    load_lds(rn, gs0 % FRING, fwd);
-    int pv = -1;  // the count of the next step's producer, read one step earlier (-1: not read)
-    auto one_step = [&](int st, double* x) {
+    if (ok) ok = wait_bounded(&L.ready[slot0], gs0 + 1, a.err, a.spin_max);
+    load_lds(rn, slot0, fwd);
+    int pv = 0;  // the next slot's ready word, read one step earlier (0: not read)
+    auto one_step = [&](int st, int slot, int next, int after, double* x) {
       const int gs = gs0 + st;
       Rec<NV, 2> r = rn;
       // The next step's record.  pv was read a step ago, so the wait (an LDS
@@ -1190,11 +1219,11 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
       // After the direction's last step the slot read is not waited for and
       // its values are never used (the next direction reloads after its own
       // wait), and load_x clamps the step to S - 1.
-      if (st + 1 < npad && ok && pv <= (gs + 1) / FPROD)
-        ok = wait_bounded(&L.produced[(gs + 1) % FPROD], (gs + 1) / FPROD + 1, a.err, a.spin_max);
+      if (st + 1 < npad && ok && pv < gs + 2)
+        ok = wait_bounded(&L.ready[next], gs + 2, a.err, a.spin_max);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      load_lds(rn, (gs + 1) % FRING, fwd);
-      pv = lds_get(&L.produced[(gs + 2) % FPROD]);
+      load_lds(rn, next, fwd);
+      pv = lds_get(&L.ready[after]);
       if constexpr (!fwd) {
 #pragma unroll
         for (int m = 0; m < NV; m++) r.X[m] = x[m];
@@ -1203,8 +1232,9 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
       // forward: dU to the backward records' X pairs; backward: U + dU (the
       // record's U is the plane's value; with update) or dU into the output
       // buffer, which the writer wave stores eight steps at a time
-      sweep_step<NV, VISC, fwd, 1, fwd, true>(r, own, rs, bw, n16, st, S, R, ncol, nrow, t, 0, lane, 0, false, false, g, ch,
-                                        ah);
+      Out<NV> o;
+      sweep_step<NV, VISC, fwd, 1, fwd, true>(r, tm, o, rs, bw, n16, st, S, R, ncol, nrow, t, 0, lane, 0, false, false,
+                                              g, ch, ah);
       // Slot gs is released after the step: its reads were issued a step ago
       // and the next slot's at this step's start, so the wait costs nothing
       // here, and it comes before the output buffer's writes so that it does
@@ -1219,10 +1249,10 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
         if (b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
         if (a.update) {
 #pragma unroll
-          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = own.W[m];
+          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.W[m];
         } else {
 #pragma unroll
-          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = own.du[m];
+          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.du[m];
         }
         if (b8 == 7 || st == npad - 1) {
           __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -1232,8 +1262,12 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
       }
     };
     for (int st = 0; st < npad; st += XD) {
+      const int turn = slot0 + XD == FRING ? 0 : slot0 + XD;  // the next turn's first slot
 #pragma unroll
-      for (int k = 0; k < XD; k++) one_step(st + k, xs[k]);
+      for (int k = 0; k < XD; k++)
+        one_step(st + k, slot0 + k, k + 1 < XD ? slot0 + k + 1 : turn,
+                 k + 2 < XD ? slot0 + k + 2 : turn + (k + 2 - XD), xs[k]);
+      slot0 = turn;
     }
   };
   run_dir(std::true_type{});

@@ -26,6 +26,20 @@ __device__ __forceinline__ double div_rcp(double a, double b, double y) {
   return __builtin_fma(r, y, q);
 }
 
+// RN(1/b) for a normal b away from the ends of the exponent range: the steps
+// of a correctly rounded division of 1 by b (two Newton steps on the hardware's
+// estimate, then the residual step) without its operand scaling, which only
+// other exponents need: seven operations instead of eleven.
+__device__ __forceinline__ double rcp_rn(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const double e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(e, y, y);
+  }
+  return y;
+}
+
 // sub_Residual.f90:477-487
 __device__ __forceinline__ double minmod(double a, double b) {
   if (a * b <= 0.0) return 0.0;
@@ -321,33 +335,32 @@ __device__ __forceinline__ void face_flux(int iflux, const double* QL, const dou
 }
 
 // comput_DFn (sub_LU_SGS.f90:111-138), F(U+dU).n - F(U).n of the Euler normal
-// flux, split in two: flux_n_old gives F(U).n, which depends on the old state
-// only, and dfn_from_old the difference for U2 = U + dU.  Both halves evaluate
-// the reference's expressions unchanged, so the difference is bit-identical
-// to the undivided routine.
-template <int NV>
-__device__ __forceinline__ void flux_n_old(double* F, const double* U, double n1, double n2, double g) {
-  double un1 = (U[1] * n1 + U[2] * n2) / U[0];
-  double p1 = (g - 1.0) * (U[3] - 0.5 * (U[1] * U[1] + U[2] * U[2]) / U[0]);
-  F[0] = U[0] * un1;
-  F[1] = U[1] * un1 + p1 * n1;
-  F[2] = U[2] * un1 + p1 * n2;
-  F[3] = (U[3] + p1) * un1;
-#pragma unroll
-  for (int m = 4; m < NV; m++) F[m] = U[m] * un1;
+// flux, in pieces that two faces of a cell share: pressure_y gives the
+// cell's p from y = RN(1/density), flux_n F(U).n, dfn the difference for
+// U2 = U + dU.  Every expression is the reference's, so the difference is
+// bit-identical to the undivided routine's; U(4) - 0.5*K/U(1) is one fma of
+// K/U(1), whose product with 0.5 is exact.
+__device__ __forceinline__ double pressure_y(const double* U, double y, double g) {
+  return (g - 1.0) * __builtin_fma(-0.5, div_rcp(U[1] * U[1] + U[2] * U[2], U[0], y), U[3]);
 }
 
 template <int NV>
-__device__ __forceinline__ void dfn_from_old(double* DF, const double* U2, const double* F, double n1, double n2,
-                                             double g) {
-  double un2 = (U2[1] * n1 + U2[2] * n2) / U2[0];
-  double p2 = (g - 1.0) * (U2[3] - 0.5 * (U2[1] * U2[1] + U2[2] * U2[2]) / U2[0]);
-  DF[0] = U2[0] * un2 - F[0];
-  DF[1] = (U2[1] * un2 + p2 * n1) - F[1];
-  DF[2] = (U2[2] * un2 + p2 * n2) - F[2];
-  DF[3] = (U2[3] + p2) * un2 - F[3];
+__device__ __forceinline__ void flux_n(double* F, const double* U, double y, double p, double n1, double n2) {
+  const double un = div_rcp(U[1] * n1 + U[2] * n2, U[0], y);
+  F[0] = U[0] * un;
+  F[1] = U[1] * un + p * n1;
+  F[2] = U[2] * un + p * n2;
+  F[3] = (U[3] + p) * un;
 #pragma unroll
-  for (int m = 4; m < NV; m++) DF[m] = U2[m] * un2 - F[m];
+  for (int m = 4; m < NV; m++) F[m] = U[m] * un;
+}
+
+template <int NV>
+__device__ __forceinline__ void dfn(double* DF, const double* U2, const double* F, double y, double p, double n1,
+                                    double n2) {
+  flux_n<NV>(DF, U2, y, p, n1, n2);
+#pragma unroll
+  for (int m = 0; m < NV; m++) DF[m] = DF[m] - F[m];
 }
 
 }  // namespace ec2d
