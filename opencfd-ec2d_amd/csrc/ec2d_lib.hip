@@ -80,11 +80,9 @@ struct DLevel {
   int lusgs_threads = 64;
   int lusgs_lpc = 1;          // LU-SGS lanes per cell: 2 when every block has at most 32 rows
   int lusgs_split = 1;        // LU-SGS sweep workgroups per block (2 or 4: a block's rows split between CUs)
-  int lusgs_u = 2;            // LU-SGS sweep steps per register set (record prefetch depth), up to 4 waves
   bool lusgs_fused = false;   // LU-SGS records made inside the sweep workgroup (k_lusgs_fused)
   bool planar_stale = false;  // Res, dt, Lc, Lv are current only in the hyperplane copy (planar_refresh)
   bool skew_static = false;   // the record arena holds the skewed copy of the mesh planes
-  int fused_np = 6;           // its producer waves (3 or 6)
   unsigned long long* dgring = nullptr;  // split sweeps: one ring per boundary between workgroups and direction
   int64_t gstride = 0;                   // slots of one ring
   int4* dwall = nullptr;      // wall faces (block, face, i, j), cases in order
@@ -719,8 +717,8 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
   dim3 gskew((unsigned)(8 * (((int64_t)a.sk_tiles * nblk + 7) / 8)));
   int nv = L.o.nvar;
   // the instantiation is chosen by thread count (its launch bound): up to 4
-  // waves one wave per SIMD and two steps per register set; more waves (up
-  // to 16) one step per set
+  // waves one wave per SIMD and four record sets in registers; more waves (up
+  // to 16) two
   const int nth = L.lusgs_threads;
   const bool pair = L.lusgs_lpc == 2;
   // every instantiation below is compiled for at most its MAXT threads
@@ -740,10 +738,7 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
       hipLaunchKernelGGL((k_lusgs_skew<NV, V, false>), gskew, dim3(256), 0, R.s, a);        \
     prof_mark(-(4 + pk));                                                                   \
     prof_mark(5 + pk);                                                                      \
-    if (L.fused_np == 3)                                                                    \
-      hipLaunchKernelGGL((k_lusgs_fused<NV, V, 3>), dim3(nblk), dim3(320), 0, R.s, a);      \
-    else                                                                                    \
-      hipLaunchKernelGGL((k_lusgs_fused<NV, V, 6>), dim3(nblk), dim3(512), 0, R.s, a);      \
+    hipLaunchKernelGGL((k_lusgs_fused<NV, V>), dim3(nblk), dim3(FUSED_THREADS), 0, R.s, a); \
     prof_mark(-(5 + pk));                                                                   \
   } else {                                                                                  \
   prof_mark(4 + pk);                                                                        \
@@ -753,17 +748,14 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
   for (int d = (a.split > 1 ? 1 : 0); d <= (a.split > 1 ? 2 : 0); d++) {                  \
   a.dir = d;                                                                                \
   if (pair) {                                                                                \
-    if (nth <= 64 && L.lusgs_u == 4) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 4, 64, 2>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 64) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 64, 2>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 256 && L.lusgs_u == 4) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 4, 256, 2>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 256 && L.lusgs_u == 3) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 3, 256, 2>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 256) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 256, 2>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 512) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 1, 512, 2>), gsweep, blk, 0, R.s, a); \
-    else hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 1, 1024, 2>), gsweep, blk, 0, R.s, a);       \
+    if (nth <= 64) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 4, 64, 2>), gsweep, blk, 0, R.s, a); \
+    else if (nth <= 256) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 4, 256, 2>), gsweep, blk, 0, R.s, a); \
+    else if (nth <= 512) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 512, 2>), gsweep, blk, 0, R.s, a); \
+    else hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 1024, 2>), gsweep, blk, 0, R.s, a);       \
   } else {                                                                                  \
-    if (nth <= 256) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 256, 1>), gsweep, blk, 0, R.s, a); \
-    else if (nth <= 512) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 1, 512, 1>), gsweep, blk, 0, R.s, a); \
-    else hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 1, 1024, 1>), gsweep, blk, 0, R.s, a);       \
+    if (nth <= 256) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 4, 256, 1>), gsweep, blk, 0, R.s, a); \
+    else if (nth <= 512) hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 512, 1>), gsweep, blk, 0, R.s, a); \
+    else hipLaunchKernelGGL((k_lusgs_sweep<NV, V, 2, 1024, 1>), gsweep, blk, 0, R.s, a);       \
   }                                                                                         \
   }                                                                                         \
   prof_mark(-(5 + pk));                                                                     \
@@ -1318,9 +1310,9 @@ struct Lcg {
 };
 
 // autotune report text of an LU-SGS shape (0: the fused launch)
-std::string shape_text(int sp, int u) {
-  if (sp == 0) return "fused preparation and sweeps, " + std::to_string(u == 3 ? 3 : 6) + " producer waves";
-  return "workgroups per block " + std::to_string(sp) + ", steps per set " + std::to_string(u);
+std::string shape_text(int sp) {
+  if (sp == 0) return "fused preparation and sweeps";
+  return "workgroups per block " + std::to_string(sp);
 }
 
 extern "C" {
@@ -2367,7 +2359,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
   if (lanes_per_cell != 1 && lanes_per_cell != 2) return fail("lanes per cell must be 1 or 2");
   HIPCHK(hipStreamSynchronize(R.s));
   DLevel& L = R.lv[nMesh - 1];
-  // 0: fused with 6 producer waves, -3: fused with 3
+  // 0 (or -3, once a launch with fewer producer waves): fused
   const bool fused = workgroups_per_block == 0 || workgroups_per_block == -3;
   if (workgroups_per_block < 0 && !fused) return fail("workgroups per block 1, 2, 4, or 0 / -3 (fused)");
   if (fused) {
@@ -2376,9 +2368,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
       if (b.ny - 1 > 64) return fail("the fused LU-SGS launch needs blocks of at most 64 rows of cells");
   }
   if (lusgs_layout(L, lanes_per_cell, fused ? 1 : workgroups_per_block, true, fused)) return 1;
-  L.lusgs_u = 2;
   L.lusgs_fused = fused;
-  L.fused_np = workgroups_per_block == -3 ? 3 : 6;
   if (R.graph) {  // a captured graph holds the old launch shape
     HIPCHK(hipGraphExecDestroy(R.graph));
     R.graph = nullptr;
@@ -2391,7 +2381,8 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
   if (R.profile) return fail("autotune needs the profile mode off");
   if (reps < 1) reps = 5;
   HIPCHK(hipStreamSynchronize(R.s));  // the layouts below are rewritten with null-stream copies
-  // cache: one line per level configuration, "key tile_rows lpc split steps"
+  // cache: one line per level configuration, "key tile_rows lpc split u"; the
+  // last field held a launch option that no longer exists (kept, so that older files still load)
   struct Choice { int tr, lp, sp, u; };
   std::vector<std::pair<std::string, Choice>> cache;
   if (cache_path && cache_path[0]) {
@@ -2421,9 +2412,9 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
       std::snprintf(hx, sizeof(hx), "_b%zu_%016llx", L.hb.size(), (unsigned long long)h);
       key += hx;
     }
-    int best_tr = -1, best_lp = -1, best_sp = 1, best_u = 2;
+    int best_tr = -1, best_lp = -1, best_sp = 1;
     for (auto& e : cache)
-      if (e.first == key) { best_tr = e.second.tr; best_lp = e.second.lp; best_sp = e.second.sp; best_u = e.second.u; }
+      if (e.first == key) { best_tr = e.second.tr; best_lp = e.second.lp; best_sp = e.second.sp; }
     char line[1024];
     if (best_tr < 0) {
       // the timed launches write the level's state (with a learned closure,
@@ -2443,6 +2434,10 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
         if (time_launches(reps, [&] { return launch_residual(l, 0); }, &ms)) return 1;
         if (ms < best) { best = ms; best_tr = tr; }
       }
+      const double res_ms = best;
+      L.tile_cols = best_tr >= 100 ? 32 : 64;
+      L.tile_rows = best_tr % 100;
+      if (build_tiles(L)) return 1;
       // LU-SGS lanes per cell and workgroups per block (the state after a
       // residual; dU only is written)
       best = 1e30;
@@ -2459,35 +2454,32 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
             R.err.clear();
             continue;  // layout not possible for these blocks
           }
-          // record prefetch depth: steps per register set (deeper sets for
-          // up to four waves with two lanes per cell)
-          for (int u : {2, 3, 4}) {
-            if (u != 2 && !(lp == 2 && L.lusgs_threads <= 256 && (u == 4 || L.lusgs_threads > 64))) continue;
-            L.lusgs_u = u;
-            double ms;
-            if (time_launches(reps, [&] { return launch_lusgs(l, L.dblocks_all, (int)L.hb.size(), 0.0, 0); }, &ms))
-              return 1;
-            char tag[32];
-            std::snprintf(tag, sizeof(tag), "w%dl%du%d", sp, lp, u);
-            note(tag, ms);
-            if (ms < best) { best = ms; best_lp = lp; best_sp = sp; best_u = u; }
-          }
-          L.lusgs_u = 2;
+          double ms;
+          if (time_launches(reps, [&] { return launch_lusgs(l, L.dblocks_all, (int)L.hb.size(), 0.0, 0); }, &ms))
+            return 1;
+          char tag[32];
+          std::snprintf(tag, sizeof(tag), "w%dl%d", sp, lp);
+          note(tag, ms);
+          if (ms < best) { best = ms; best_lp = lp; best_sp = sp; }
         }
       // the fused variant: records made in the sweep workgroup (rows <= 64)
       bool fits = true;
       for (auto& b : L.hb) fits = fits && b.ny - 1 <= 64;
       if (fits && !lusgs_layout(L, 1, 1, true, true)) {
+        // timed with the residual before it, which writes its inputs in a
+        // main-loop pass (advance_lusgs), less the plain residual: the copy
+        // kernel that a lone update needs is no part of a pass
         L.lusgs_fused = true;
-        for (int np : {3, 6}) {
-          L.fused_np = np;
-          double ms;
-          if (time_launches(reps, [&] { return launch_lusgs(l, L.dblocks_all, (int)L.hb.size(), 0.0, 0); }, &ms))
-            return 1;
-          note(np == 3 ? "fused3" : "fused6", ms);
-          // the cache's fourth field holds the producer waves of a fused choice
-          if (ms < best) { best = ms; best_lp = 1; best_sp = 0; best_u = np; }
-        }
+        const bool rskew = !L.fdm;
+        double ms;
+        if (time_launches(reps, [&] {
+              return launch_residual(l, 0, 0, 0, rskew ? L.sk : nullptr, rskew && R.num_mesh == 1) ||
+                     launch_lusgs(l, L.dblocks_all, (int)L.hb.size(), 0.0, 0, nullptr, nullptr, rskew);
+            }, &ms))
+          return 1;
+        ms -= res_ms;
+        note("fused", ms);
+        if (ms < best) { best = ms; best_lp = 1; best_sp = 0; }
         L.lusgs_fused = false;
       }
       R.err.clear();
@@ -2495,15 +2487,15 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
       HIPCHK(hipStreamSynchronize(R.s));
       HIPCHK(hipFree(keep));
       if (best_lp < 0) return fail("no LU-SGS layout fits this level");
-      added.push_back({key, {best_tr, best_lp, best_sp, best_u}});
+      added.push_back({key, {best_tr, best_lp, best_sp, 2}});
       std::snprintf(line, sizeof(line), "level %d: measured tile %dx%d, lanes per cell %d, %s;", l + 1,
-                    best_tr >= 100 ? 32 : 64, best_tr % 100, best_lp, shape_text(best_sp, best_u).c_str());
+                    best_tr >= 100 ? 32 : 64, best_tr % 100, best_lp, shape_text(best_sp).c_str());
       rep_txt += line;
-      // LU-SGS times of every shape (w: workgroups per block, l: lanes per cell, u: steps per set)
+      // LU-SGS times of every shape (w: workgroups per block, l: lanes per cell)
       std::snprintf(line, sizeof(line), " LU-SGS ms:%s\n", cand.c_str());
     } else {
       std::snprintf(line, sizeof(line), "level %d: cached tile %dx%d, lanes per cell %d, %s\n", l + 1,
-                    best_tr >= 100 ? 32 : 64, best_tr % 100, best_lp, shape_text(best_sp, best_u).c_str());
+                    best_tr >= 100 ? 32 : 64, best_tr % 100, best_lp, shape_text(best_sp).c_str());
     }
     rep_txt += line;
     L.tile_cols = best_tr >= 100 ? 32 : 64;
@@ -2511,8 +2503,6 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
     if (build_tiles(L)) return 1;
     if (lusgs_layout(L, best_lp, best_sp == 0 ? 1 : best_sp, true, best_sp == 0)) return 1;
     L.lusgs_fused = best_sp == 0;
-    L.lusgs_u = L.lusgs_fused ? 2 : best_u;
-    if (L.lusgs_fused) L.fused_np = best_u == 3 ? 3 : 6;
   }
   if (!added.empty() && cache_path && cache_path[0]) {
     if (FILE* f = std::fopen(cache_path, "a")) {

@@ -43,15 +43,18 @@
 // receives row t-1's.  The first lane of a wave gets row t-1 through LDS.
 //
 // Divisions.  Every quotient of a sweep has a divisor known before its
-// numerator (the diagonal) or shared by three quotients (rho of U + dU).  The
-// record holds y = RN(1/alfa), the sweep forms y = RN(1/rho) once per cell
-// (rcp_rn); a/b is q = a*y refined twice with FMA residuals (div_rcp,
-// Markstein): the first refinement makes q faithful, the second, with y
-// correctly rounded, returns RN(a/b) - the quotient the reference's division
-// gives, in five dependent operations instead of eleven.  (A quotient from 1/b
-// held to 2^-104 in two doubles takes two operations, but is not RN(a/b) where
-// rho is within a few units in the last place of 1, as it is in a cell the
-// flow has not reached: the quotients there lie next to rounding boundaries.)
+// numerator (the diagonal) or shared by three quotients (rho of U + dU).
+//   The record holds 1/alfa as yh + yl, good to 2^-104, and a/alfa is
+// fma(a, yh, a*yl): one rounding of a value within 2^-104 of the quotient,
+// RN(a/alfa) - the value of the reference's division - unless the quotient
+// lies that close to a rounding boundary (one in 2^50 of unrelated operands);
+// two operations instead of the eleven of a division.
+//   rho of a cell that the flow has not reached is within a few units in the
+// last place of 1, where quotients do lie next to rounding boundaries.  Its
+// three quotients take y = RN(1/rho), formed once per cell (rcp_rn), and
+// q = a*y refined twice with FMA residuals (div_rcp, Markstein): the first
+// refinement makes q faithful, the second, with y correctly rounded, returns
+// RN(a/rho).
 //
 // Scaling.  0.5*(DF*a + Lc*dU) is formed as DF*(0.5 a) + (0.5 Lc)*dU, and
 // -0.5*(DF*a - Lc*dU) as DF*(-0.5 a) + (0.5 Lc)*dU, with the factors in the
@@ -113,10 +116,10 @@ struct LusgsArgs {
 template <int NV, bool VISC>
 struct RecF {
   // cell: X = Res (forward) or the forward dU (backward), in whole pairs
-  // of their own; then U, the diagonal and its correctly rounded reciprocal (a
+  // of their own; then U and the reciprocal of the diagonal as yh + yl (a
   // separate one for the SA equation)
   static constexpr int XP = (NV + 1) / 2;
-  static constexpr int U = 2 * XP, AL0 = U + NV, Y0 = AL0 + 1, AL4 = AL0 + 2, Y4 = AL0 + 3;
+  static constexpr int U = 2 * XP, YH0 = U + NV, YL0 = YH0 + 1, YH4 = YH0 + 2, YL4 = YH0 + 3;
   static constexpr int NSH = 2 * XP + (NV + 2 + (NV == 5 ? 2 : 0) + 1) / 2 * 2;
   // per side: F(U).n, the normal, half the face area (negated: backward), half the
   // inviscid and the viscous spectral radius (padded to whole pairs)
@@ -159,7 +162,7 @@ template <int NV, int NS>
 struct Rec {
   double X[NV], U[NV];
   double F[NS][NV], n1[NS], n2[NS], a[NS], Lc[NS], Lv[NS];
-  double al0, y0, al4, y4;
+  double yh0, yl0, yh4, yl4;  // 1/alfa (SA: and of the SA equation) as yh + yl
 };
 
 // what a cell hands on: the term of the next cell of its row and that of the
@@ -173,6 +176,13 @@ struct Terms {
 __device__ __forceinline__ double shr1(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x138, 0xF, 0xF, true);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x138, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// lane l-1 -> lane l; lane 0 receives in
+__device__ __forceinline__ double shr1_in(double in, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(in), __double2loint(v), 0x138, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(in), __double2hiint(v), 0x138, 0xF, 0xF, false);
   return __hiloint2double(hi, lo);
 }
 
@@ -228,14 +238,14 @@ __device__ __forceinline__ void load_rec(Rec<NV, NS>& p, __amdgpu_buffer_rsrc_t 
     p.X[m] = sh[m];
     p.U[m] = sh[F::U + m];
   }
-  p.al0 = sh[F::AL0];
-  p.y0 = sh[F::Y0];
+  p.yh0 = sh[F::YH0];
+  p.yl0 = sh[F::YL0];
   if constexpr (NV == 5) {
-    p.al4 = sh[F::AL4];
-    p.y4 = sh[F::Y4];
+    p.yh4 = sh[F::YH4];
+    p.yl4 = sh[F::YL4];
   } else {
-    p.al4 = p.al0;
-    p.y4 = p.y0;
+    p.yh4 = p.yh0;
+    p.yl4 = p.yl0;
   }
   const uint32_t sb = base + (uint32_t)(F::NSH / 2) * n16;  // side part, at 2*pos + k
 #pragma unroll
@@ -276,25 +286,26 @@ struct RecSrc {
 // The arithmetic of one record.  SH(d) and SD(k, e) give the destination of
 // the cell's double d and of side k's double e (the global skewed records of
 // k_lusgs_prep, or an LDS slot of k_lusgs_fused).
-// CF: the field numbers of the cell's part.
-template <int NV, bool VISC, bool FWD, class CF, class SHF, class SDF>
+// CF: the field numbers of the cell's part.  XB: also write a backward record's
+// X (q.Res; the split path's X is where the forward sweep stored it).
+template <int NV, bool VISC, bool FWD, bool XB, class CF, class SHF, class SDF>
 __device__ __forceinline__ void rec_body(SHF SH, SDF SD, const RecSrc<NV>& q, double g, double alfa1) {
   using F = RecF<NV, VISC>;
 #pragma unroll
   for (int m = 0; m < NV; m++) {
     SH(CF::U + m) = q.U[m];
-    if (FWD) SH(m) = q.Res[m];
+    if constexpr (FWD || XB) SH(m) = q.Res[m];
   }
   // diagonal (sub_LU_SGS.f90:31-39, 76-83)
   double alfa = q.vol / q.dt + 1.0 * (q.Lc[0] + q.Lc[1]) + q.vol * alfa1;
   if constexpr (VISC) alfa = alfa + 2.0 * (q.Lv[0] + q.Lv[1]);
-  SH(CF::AL0) = alfa;
-  SH(CF::Y0) = rcp_rn(alfa);
-  if constexpr (NV == 5) {
-    const double alfa4 = alfa + q.Lv[0] + q.Lv[1];
-    SH(CF::AL4) = alfa4;
-    SH(CF::Y4) = rcp_rn(alfa4);
-  }
+  auto recip = [&](int d, double al) {  // 1/al as yh + yl
+    const double y = rcp_rn(al);
+    SH(d) = y;
+    SH(d + 1) = __builtin_fma(-al, y, 1.0) * y;
+  };
+  recip(CF::YH0, alfa);
+  if constexpr (NV == 5) recip(CF::YH4, alfa + q.Lv[0] + q.Lv[1]);
   const double y = rcp_rn(q.U[0]);
   const double p = pressure_y(q.U, y, g);
 #pragma unroll
@@ -424,7 +435,7 @@ __device__ __forceinline__ void write_rec(double* __restrict__ rb, int64_t n, in
   };
   RecSrc<NV> q;
   load_src<NV, VISC, FWD>(q, B, base, pm, c, r);
-  rec_body<NV, VISC, FWD, F>(SH, SD, q, g, alfa1);
+  rec_body<NV, VISC, FWD, false, F>(SH, SD, q, g, alfa1);
 }
 
 // One thread per cell, a wave per 8 x 8 tile of cells (a workgroup per 32
@@ -610,47 +621,43 @@ __device__ __forceinline__ void side_term(double* v, const Rec<NV, NS>& p, int h
   }
 }
 
-// The waves of a block as a pipeline.  Wave w needs, at step s, the result
+// The waves of a block as a pipeline.  Wave w needs, at step s, the terms
 // of the last row of wave w-1 at step s-1 and nothing else from other waves,
 // so waves do not meet at a barrier per step: wave w-1 puts its last row's
-// result of step s into slot s % RING of an LDS ring and then publishes
-// prog = s + 1; wave w waits for prog >= s, reads slot (s-1) % RING and
-// publishes cons = s (the input of step s taken).  Before wave w-1 reuses a
-// slot it waits for cons >= s - RING + 1.  Neither wait can block forever:
-// wave w-1 waits only while wave w is RING steps behind, and then wave w does
-// not wait (prog is ahead of it), so wave w advances; wave 0 never waits for
-// input.  Every wave runs the same fixed number of steps, so all waits end.
+// terms of step s into slot s % RING of an LDS ring and then publishes
+// prog = s + 1; wave w reads slot (s-1) % RING.  A sweep wave runs turns of
+// D steps and looks at the other waves' counters
+// once a turn: before a turn that starts at s0 it waits for prog >= s0+D-1
+// (its inputs) and for cons >= s0+D-RING (the slots it will write), and
+// after the turn it publishes cons = s0+D-1 (the inputs of these steps
+// taken).  Checked at every step, the counters, the branches around them and
+// the selects of the first lane cost each linked wave about 50 instructions a
+// step, a quarter of the step.
+//   Neither wait can block forever: a wave at s0 has published s0-1, the wave
+// below stops at a turn of at most s0+D-2 when that turn needs more than
+// s0-1, that is when 2D > RING+1; D <= 4 and RING = 16.  The communication
+// waves move at most RING/2 steps at a time, under the same rules.  Wave 0
+// without an input below it reads a ring of zeros whose prog is at its end,
+// the last wave without a consumer writes a ring whose cons is, so that no
+// step branches on its place in the block.  Every wave runs the same fixed
+// number of steps, so all waits end.
 // LDS operations of one wave execute in issue order, so a published counter
 // is never seen before the ring data written ahead of it, and a slot is never
 // rewritten before the read that cons acknowledges; compiler fences keep
 // that order in the instruction stream.  The spins read LDS only and never
 // wait for the global-load prefetch.
 //
-// Both sides read ahead, so that no LDS latency sits on a step's dependent
-// path: during step s the consumer reads prog and then, behind it, the slot
-// holding its input of step s+1; at step s+1 the data is used if that prog
-// showed the producer past step s (the data read executed after the prog
-// read, so it saw the slot written), and read again after a wait otherwise.
-// The producer likewise reads cons one step ahead; a stale value only makes
-// it wait longer.
-//
 // ring[w] is the input of wave w: its producer is wave w-1 (or, in the upper
 // workgroup of a split block, the communication wave), prog[w] that
 // producer's progress and cons[w] wave w's consumption.
 constexpr int RING = 16;
+constexpr int CHAIN_END = 0x7fffffff;
 template <int NV>
 struct Chain {
+  double dump[RING][NV];      // where the lanes below a wave's last one write
   double ring[17][RING][NV];  // input of wave w: the terms of the row below it
-  int prog[17];                   // steps finished by the producer of ring[w]
-  int cons[17];                   // steps whose input wave w has read
-};
-
-// per-wave read-ahead state: the next input (lane 0's) and the counters
-// seen when it was read
-template <int NV>
-struct Ahead {
-  double v[NV];
-  int prog, cons;
+  int prog[17];               // steps finished by the producer of ring[w]
+  int cons[17];               // steps whose input wave w has read
 };
 
 __device__ __forceinline__ int lds_get(const int* p) {
@@ -664,48 +671,24 @@ __device__ __forceinline__ void wait_at_least(const int* p, int v) {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// One step of a sweep: the cell of row t at column offset c = s - t.
-// LPC = 2: lanes 2t (k = 0, the term for the next cell of the row) and 2t+1
-// (k = 1, the term for the next row) share the cell; LPC = 1: lane t forms both.
-// ODD1 (the fused launch's layout): with an odd equation count the last X
-// field holds single doubles, not a pair padded with zero, and lanes without
-// a cell store nothing (no trash-pad slot).  out: the cell's dU and U + dU.
+// one cell's result
 template <int NV>
 struct Out {
   double du[NV], W[NV];
 };
 
-template <int NV, bool VISC, bool FWD, int LPC, bool STORE = true, bool ODD1 = false>
-__device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Terms<NV, LPC>& tm, Out<NV>& o,
-                                           __amdgpu_buffer_rsrc_t rs, uint32_t dst, uint32_t n16, int s, int S, int R,
-                                           int ncol, int nrow, int t, int k, int lane, int wave, bool cin, bool cout,
-                                           double g, Chain<NV>& ch, Ahead<NV>& ah) {
-  // the term of row t-1 (LPC = 2: lane 2t receives it, lane 2t+1 the term of
-  // its own row, which it does not use), one lane down; the first lane's
-  // from the last lane of the previous wave through the LDS ring
-  double jin[NV];
-#pragma unroll
-  for (int m = 0; m < NV; m++) jin[m] = shr1(tm.j[m]);
-  if (cin) {
-    // the row below this wave at step s-1 (an LDS broadcast), lane 0 keeps
-    // it; read one step ahead unless the producer was not there yet
-    if (ah.prog < s) {
-      wait_at_least(&ch.prog[wave], s);
-      const double* x = ch.ring[wave][(s - 1) & (RING - 1)];
-#pragma unroll
-      for (int m = 0; m < NV; m++) ah.v[m] = x[m];
-    }
-#pragma unroll
-    for (int m = 0; m < NV; m++) jin[m] = lane == 0 ? ah.v[m] : jin[m];
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    lds_put(&ch.cons[wave], s);
-    // the input of step s+1: prog first, the slot behind it
-    ah.prog = lds_get(&ch.prog[wave]);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    const double* x = ch.ring[wave][s & (RING - 1)];
-#pragma unroll
-    for (int m = 0; m < NV; m++) ah.v[m] = x[m];
-  }
+// One cell of a sweep from its record p, the terms tm of its row's last cell
+// and those of the row below (jin; LPC = 2: lane 2t holds them): its dU and
+// U + dU, and in tm the terms it hands on.  LPC = 2: lanes 2t (the term for
+// the next cell of the row) and 2t+1 (the term for the next row) share the
+// cell; LPC = 1: lane t forms both.
+//   Every lane keeps its terms, active or not: an inactive lane's never
+// reach an active cell.  Before its first cell a row holds the neutral
+// record's zeros; row t+1 at step s+1 sits at the same column offset as
+// row t at step s, so it is inactive whenever row t was.
+template <int NV, bool VISC, bool FWD, int LPC>
+__device__ __forceinline__ void cell_step(const Rec<NV, 3 - LPC>& p, Terms<NV, LPC>& tm, const double* jin, Out<NV>& o,
+                                          double g) {
   // (Res + dui) + duj forward, X + (dui + duj) / alfa backward
 #pragma unroll
   for (int m = 0; m < NV; m++) {
@@ -713,14 +696,10 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Terms<NV, 
     double sum = FWD ? (p.X[m] + iin) + jin[m] : iin + jin[m];
     if constexpr (LPC == 2) sum = even_lane(sum);
     const bool sa = NV == 5 && m == 4;
-    const double q = div_rcp(sum, sa ? p.al4 : p.al0, sa ? p.y4 : p.y0);
+    const double q = div_hl(sum, sa ? p.yh4 : p.yh0, sa ? p.yl4 : p.yl0);
     o.du[m] = FWD ? q : p.X[m] + q;
     o.W[m] = p.U[m] + o.du[m];
   }
-  // Every lane keeps its terms, active or not: an inactive lane's never
-  // reach an active cell.  Before its first cell a row holds the neutral
-  // record's zeros; row t+1 at step s+1 sits at the same column offset as
-  // row t at step s, so it is inactive whenever row t was.
   const double y = rcp_rn(o.W[0]);
   const double pr = pressure_y(o.W, y, g);
   if constexpr (LPC == 1) {
@@ -729,80 +708,108 @@ __device__ __forceinline__ void sweep_step(const Rec<NV, 3 - LPC>& p, Terms<NV, 
   } else {
     side_term<NV, VISC>(tm.j, p, 0, o.W, o.du, y, pr);
   }
-  if constexpr (STORE) {
-    // one lane of an active cell stores; every other lane writes its own
-    // slot of the trash pad (positions S*R .. S*R+63)
-    const int c = s - t;
-    const bool act = t < nrow && c >= 0 && c < ncol && k == 0;
-    const uint32_t w = act ? (FWD ? (uint32_t)((S - 1 - s) * R + (nrow - 1 - t)) : (uint32_t)(s * R + t))
-                           : (uint32_t)(S * R + lane);
-    if (!ODD1 || act) {
+}
+
+// Scheduling of the block so far: N times one instruction of the kind MASK
+// (0x20: memory loads, 0x100: LDS reads), then V vector instructions.  A wave
+// that issues a step's loads in one burst waits for the address unit (16
+// cycles a load) or the LDS (8) to take them.
+template <int MASK, int N, int V>
+__device__ __forceinline__ void interleave() {
 #pragma unroll
-      for (int j = 0; j < (NV + 1) / 2; j++) {
-        if (ODD1 && 2 * j + 1 == NV) bstore1(o.du[2 * j], rs, w * 8u, dst + (uint32_t)j * n16);
-        else bstore2(o.du[2 * j], 2 * j + 1 < NV ? o.du[2 * j + 1] : 0.0, rs, w * 16u, dst + (uint32_t)j * n16);
-      }
-    }
-  }
-  if (cout) {
-    // slot s % RING is free once the next wave has read step s - RING's result
-    if (ah.cons < s - RING + 1) wait_at_least(&ch.cons[wave + 1], s - RING + 1);
-    if (lane == 63) {
-      double* x = ch.ring[wave + 1][s & (RING - 1)];
-#pragma unroll
-      for (int m = 0; m < NV; m++) x[m] = tm.j[m];
-    }
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    lds_put(&ch.prog[wave + 1], s + 1);
-    ah.cons = lds_get(&ch.cons[wave + 1]);
+  for (int k = 0; k < N; k++) {
+    __builtin_amdgcn_sched_group_barrier(MASK, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
   }
 }
 
 // One sweep (lanes: the head of this file).
-// The records come in two register sets of U steps each, loaded one phase
-// ahead: [load B] [steps of A] [load A] [steps of B] ...  Whenever the code
-// waits for a set, the only loads still in flight are the other set's, issued
-// after it, so the waits the compiler places never drain a prefetch that is
-// not yet needed.  Loads past the last step are clamped to it.  The cell's dU goes to dst: for the forward sweep the X field of the
+// The records come through a ring of D register sets: step s works on set
+// s % D while the loads of step s + D - 1 go into the set that step s - 1 has
+// finished with, spread over the step's arithmetic (interleave).  Loads past
+// the last step are clamped to it.  The cell's dU
+// goes to dst: for the forward sweep the X field of the
 // backward record of the same cell, for the backward sweep the output fields.
-template <int NV, bool VISC, bool FWD, int U, int LPC>
+// LINK: the wave has others to exchange with (not a block of one wave).
+template <int NV, bool VISC, bool FWD, int D, int LPC, bool LINK>
 __device__ __forceinline__ void sweep(__amdgpu_buffer_rsrc_t rs, uint32_t rec, uint32_t dst, uint32_t n16, int S, int R,
-                                      int ncol, int nrow, int t, int k, int lane, int wave, bool cin, bool cout,
-                                      double g, Chain<NV>& ch) {
-  Ahead<NV> ah = {};  // prog = 0: step 0 needs nothing (its input is never used)
-  const int npad = (S + 2 * U - 1) / (2 * U) * (2 * U);
+                                      int ncol, int nrow, int t, int k, int lane, int wave, double g, Chain<NV>& ch) {
+  using F = RecF<NV, VISC>;
+  static_assert(2 * D <= RING + 1 && RING % D == 0, "the turns of linked waves must fit the ring");
+  const int npad = (S + D - 1) / D * D;
   // lanes past the block's last row load that row's records: the same cache
   // lines as its own lane, so padding rows cost no memory traffic (their
   // results never reach a cell)
   const int tl = min(t, nrow - 1);
   constexpr int NS = 3 - LPC;
   Terms<NV, LPC> tm = {};
-  Rec<NV, NS> A[U], B[U];
-  auto load_set = [&](Rec<NV, NS>* set, int s_first) {
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const uint32_t v16 = (uint32_t)(min(s_first + u, S - 1) * R + tl) * 16u;
-      load_rec<NV, VISC, NS>(set[u], rs, rec, n16, v16, k);
-    }
+  Rec<NV, NS> set[D];
+  auto load_step = [&](Rec<NV, NS>& r, int s) {
+    load_rec<NV, VISC, NS>(r, rs, rec, n16, (uint32_t)(min(s, S - 1) * R + tl) * 16u, k);
   };
-  auto run_set = [&](const Rec<NV, NS>* set, int s_first) {
+  // One lane of an active cell stores; every other lane writes its own slot
+  // of the trash pad (positions S*R .. S*R+63).  A lane that never stores has
+  // a row number that no step reaches.
+  const int ts = t < nrow && k == 0 ? t : 0x40000000;
+  const uint32_t trash = (uint32_t)(S * R + lane) * 16u;
+  const uint32_t dw = FWD ? (uint32_t)(-R * 16) : (uint32_t)(R * 16);
+  uint32_t w16 = (uint32_t)(FWD ? (S - 1) * R + (nrow - 1 - t) : t) * 16u;
+  // The input of the next step: an LDS broadcast, lane 0 uses it.  The last
+  // lane's terms go to the next wave's ring, the other lanes' to the dump (a
+  // store without a branch).
+  double in[NV];
+  const double(*rin)[NV] = ch.ring[wave];
+  double(*rout)[NV] = lane == 63 ? ch.ring[wave + 1] : ch.dump;
+  int prog = 0, cons = 0;
+  auto look = [&] {
+    prog = lds_get(&ch.prog[wave]);
+    cons = lds_get(&ch.cons[wave + 1]);
+  };
+  auto read_in = [&](int slot) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
+    for (int m = 0; m < NV; m++) in[m] = rin[slot][m];
+  };
+#pragma unroll
+  for (int u = 0; u < D - 1; u++) load_step(set[u], u);
+  if constexpr (LINK) look();
+  for (int s0 = 0; s0 < npad; s0 += D) {
+    const int slot0 = s0 & (RING - 1);
+    if constexpr (LINK) {
+      if (prog < s0 + D - 1) wait_at_least(&ch.prog[wave], s0 + D - 1);
+      if (cons < s0 + D - RING) wait_at_least(&ch.cons[wave + 1], s0 + D - RING);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      read_in((s0 - 1) & (RING - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < D; u++) {
+      const int s = s0 + u;
+      load_step(set[(u + D - 1) % D], s + D - 1);
+      double jin[NV];
+#pragma unroll
+      for (int m = 0; m < NV; m++) jin[m] = LINK ? shr1_in(in[m], tm.j[m]) : shr1(tm.j[m]);
+      if (LINK && u + 1 < D) read_in(slot0 + u);  // the turn's next step's (its first one's follows the wait)
       Out<NV> o;
-      sweep_step<NV, VISC, FWD, LPC>(set[u], tm, o, rs, dst, n16, s_first + u, S, R, ncol, nrow, t, k, lane, wave, cin,
-                                     cout, g, ch, ah);
+      cell_step<NV, VISC, FWD, LPC>(set[u], tm, jin, o, g);
+      const uint32_t w = (uint32_t)(s - ts) < (uint32_t)ncol ? w16 : trash;
+      w16 += dw;
+#pragma unroll
+      for (int j = 0; j < (NV + 1) / 2; j++)
+        bstore2(o.du[2 * j], 2 * j + 1 < NV ? o.du[2 * j + 1] : 0.0, rs, w, dst + (uint32_t)j * n16);
+      if constexpr (LINK) {
+#pragma unroll
+        for (int m = 0; m < NV; m++) rout[slot0 + u][m] = tm.j[m];
+      }
+      interleave<0x20, (F::NSH + NS * F::NSD) / 2, LPC == 2 ? 8 : 10>();
+      if constexpr (LINK) {
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        lds_put(&ch.prog[wave + 1], s + 1);
+        // the counters of the next turn, read early (a stale value only makes
+        // it look again)
+        if (u == D - 2) look();
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  load_set(A, 0);
-  for (int s0 = 0; s0 < npad; s0 += 2 * U) {
-    load_set(B, s0 + U);
-    __builtin_amdgcn_sched_barrier(0);
-    run_set(A, s0);
-    __builtin_amdgcn_sched_barrier(0);
-    load_set(A, s0 + 2 * U);
-    __builtin_amdgcn_sched_barrier(0);
-    run_set(B, s0 + U);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (LINK) lds_put(&ch.cons[wave], s0 + D - 1);
   }
 }
 
@@ -897,15 +904,16 @@ __device__ void comm_receive(Chain<NV>& ch, unsigned long long* gr, int npad, in
   for (int i = (int)(threadIdx.x & 63); i < (npad - 1) * NV; i += 64) gstore(gr + i, GSENT);
 }
 
-// LPC lanes per cell (1 or 2), U steps per register set, MAXT threads at most.
+// LPC lanes per cell (1 or 2), D register sets of records, MAXT threads at most.
 // a.split workgroups per block (blockIdx.x = block * split + part); with a
 // split each part has its compute waves, then a receiving communication wave
 // (all parts but the first), then a sending one (all parts but the last), and
 // the two sweeps are separate launches (a.dir), since the backward sweep of
 // one part needs forward results of the others.
-template <int NV, bool VISC, int U, int MAXT, int LPC>
+template <int NV, bool VISC, int D, int MAXT, int LPC>
 __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   using F = RecF<NV, VISC>;
+  constexpr bool LINK = MAXT > 64;
   __shared__ Chain<NV> ch[2];  // one per sweep
   const int G = a.split, bi = blockIdx.x / G, half = blockIdx.x % G;  // half: the part of the block
   const BlockDesc B = a.blocks[a.block_list[bi]];
@@ -920,9 +928,11 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   const int nw = R * LPC / (64 * G);
   const int t = half * (R / G) + (LPC == 2 ? tid >> 1 : tid), k = LPC == 2 ? tid & 1 : 0;
   const bool has_in = half > 0, has_out = half < G - 1;
-  const bool cin = wave > 0 || has_in, cout = wave < nw - 1 || has_out;
-  if (tid < 17) {
-    ch[0].prog[tid] = ch[0].cons[tid] = ch[1].prog[tid] = ch[1].cons[tid] = 0;
+  for (int q = tid; q < 2 * (int)(sizeof(Chain<NV>) / 8); q += blockDim.x) reinterpret_cast<double*>(ch)[q] = 0.0;
+  __syncthreads();
+  if (tid < 2) {
+    if (!has_in) ch[tid].prog[0] = CHAIN_END;
+    if (!has_out) ch[tid].cons[nw] = CHAIN_END;
   }
   __syncthreads();
   // the block's record region: forward set, backward set (its X pairs first),
@@ -930,12 +940,12 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   const uint32_t bytes = (uint32_t)((2 * F::NREC + 2 * F::XP) * B.sk_n * 8);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.sk + B.sk_base, 0, bytes, 0x00020000);
   const uint32_t fw = 0, bw = F::NREC * n8, out = 2 * F::NREC * n8;
-  const int npad = (S + 2 * U - 1) / (2 * U) * (2 * U);
+  const int npad = (S + D - 1) / D * D;
   // global ring of boundary b (between parts b and b+1) for sweep direction d
   auto gr = [&](int b, int d) { return a.gring + (((int64_t)bi * (G - 1) + b) * 2 + d) * a.gstride; };
   const bool rcv = has_in && wave == nw, snd = has_out && wave == nw + (has_in ? 1 : 0);
   if (a.dir != 2) {
-    if (wave < nw) sweep<NV, VISC, true, U, LPC>(rs, fw, bw, n16, S, R, ncol, nrow, t, k, lane, wave, cin, cout, g, ch[0]);
+    if (wave < nw) sweep<NV, VISC, true, D, LPC, LINK>(rs, fw, bw, n16, S, R, ncol, nrow, t, k, lane, wave, g, ch[0]);
     else if (rcv) comm_receive<NV>(ch[0], gr(half - 1, 0), npad, a.err, a.spin_max);
     else if (snd) comm_forward<NV>(ch[0], nw, gr(half, 0), npad);
   }
@@ -943,7 +953,7 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   // only when the block has one workgroup, so a barrier (workgroup scope) does
   if (a.dir == 0) __syncthreads();
   if (a.dir != 1) {
-    if (wave < nw) sweep<NV, VISC, false, U, LPC>(rs, bw, out, n16, S, R, ncol, nrow, t, k, lane, wave, cin, cout, g, ch[1]);
+    if (wave < nw) sweep<NV, VISC, false, D, LPC, LINK>(rs, bw, out, n16, S, R, ncol, nrow, t, k, lane, wave, g, ch[1]);
     else if (rcv) comm_receive<NV>(ch[1], gr(half - 1, 1), npad, a.err, a.spin_max);
     else if (snd) comm_forward<NV>(ch[1], nw, gr(half, 1), npad);
   }
@@ -953,57 +963,59 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
 // For levels whose blocks have at most 64 rows (one wave per block, one lane
 // per row): k_lusgs_fused does the work of k_lusgs_prep inside the sweep's
 // workgroup, so the records never go through HBM.  Wave 0 runs both sweeps
-// exactly as k_lusgs_sweep<..., LPC = 1> does (the same sweep_step), at the
-// highest issue priority of its SIMD; waves 1..NP produce the records, each
-// every NP-th step of the sequence (forward steps 0..npad-1, then backward
+// exactly as k_lusgs_sweep<..., LPC = 1> does (the same cell_step), at the
+// highest issue priority of its SIMD; FPROD waves produce the records, each
+// every FPROD-th step of the sequence (forward steps 0..npad-1, then backward
 // steps 0..npad-1), lane t the cell of row t, from the skewed copy of the
 // inputs that k_lusgs_skew (or the residual) made, into a ring of LDS slots.
 // A producer loads the inputs of its next record before it waits for a slot,
 // so that memory latency is off the records' path.  The
-// forward dU goes to the backward records' X pairs in global memory (the
-// backward sweep reads it there, after a fence).  The sweep wave puts the
+// forward dU goes to the backward records' X in global memory, from where the
+// producers take it into the backward records once the sweep wave has turned
+// (turned, set behind a fence).  The sweep wave puts the
 // backward U + dU (with update; dU without) of eight steps into an LDS
-// buffer; wave NP + 1,
-// the writer, takes each chunk and stores it to the block planes eight
+// buffer; the writer wave takes each chunk and stores it to the block planes eight
 // consecutive cells of a row at a time: this replaces k_lusgs_scatter
 // (stores along a hyperplane, one cache line per lane, hold up whichever
-// wave issues them).  NP = 3 or 6 (5 or 8 waves).
+// wave issues them).
 //
 // The slots hold the records without RecF's padding: 34 doubles of SA, eight
 // slots and the buffer take 156 KB of the CU's 160 KB (a six-equation record
-// has six slots).  The slot count is a multiple of the steps per turn of the
-// sweep's loop, so that a step's slot is a constant of the unrolled loop plus
-// the turn's first.
+// has six slots).  They are filled and released in groups of XD steps, one
+// turn of the sweep's loop: it looks at the producers' counters once a turn,
+// and a record's LDS offsets are constants of the unrolled loop from one
+// address per group.
 //
 // The writer waits for ob_ready > chunk, reads the chunk, then sets
 // ob_taken = chunk + 1; the sweep wave waits for ob_taken >= chunk before
 // it writes the chunk's first step, and sets ob_ready after its last.
-// Protocol: ready[slot] is one more than the step whose record the slot holds,
-// consumed the steps whose slot the sweep wave has finished with (it releases
-// slot g after computing step g).  The sweep wave waits, before reading step
-// g, for ready[g % NRING] > g; a producer waits, before writing step
-// g into slot g % NRING, for consumed >= g - NRING + 1.  A producer waits only
-// for the sweep wave and the sweep wave only for producers that are never
-// more than NRING steps ahead, so every wait ends; waits are also bounded
+// Protocol: filled[q] counts the records written into group slot q, consumed
+// the steps of the groups that the sweep wave has finished with.  The sweep
+// wave waits, before it reads the first record of group G (slot G % NGRP), for
+// filled >= XD (G / NGRP + 1); a producer waits, before it writes step g's
+// record, for consumed >= XD (g / XD + 1) - NRING.  A producer waits only
+// for the sweep wave and the sweep wave only for producers of groups whose
+// slots are free, so every wait ends; waits are also bounded
 // (a.spin_max polls, then err is set and the wave stops waiting).
 template <int NV, bool VISC>
 struct FusedSlot {
   using F = RecF<NV, VISC>;
-  // the cell's doubles (X without its padding) and a side's
-  static constexpr int U = NV, AL0 = 2 * NV, Y0 = AL0 + 1, AL4 = AL0 + 2, Y4 = AL0 + 3;
-  static constexpr int NSH = 2 * NV + 2 + (NV == 5 ? 2 : 0), NSD = F::NSDU;
-  static constexpr int XD = NV >= 6 ? 2 : 4;     // sweep steps per turn of its loop
+  // the cell's doubles (X without its padding), then side k's from side(k)
+  static constexpr int U = NV, YH0 = 2 * NV, YL0 = YH0 + 1, YH4 = YH0 + 2, YL4 = YH0 + 3;
+  static constexpr int NSH = 2 * NV + 2 + (NV == 5 ? 2 : 0), NSD = F::NSDU, N = NSH + 2 * NSD;
+  static constexpr int side(int k) { return NSH + k * NSD; }
+  static constexpr int XD = NV >= 6 ? 2 : 4;     // sweep steps per turn of its loop: one group of slots
   static constexpr int NRING = NV >= 6 ? 6 : 8;  // record slots
+  static constexpr int NGRP = NRING / XD;
 };
 template <int NV, bool VISC>
 struct FusedLds {
   using F = FusedSlot<NV, VISC>;
-  double sh[F::NRING][F::NSH][64];     // the cells' doubles of slot, lane
-  double sd[F::NRING][2][F::NSD][64];  // the sides'
-  double ob[8][NV][64];                // the sweep's backward U + dU (update) or dU of eight steps
-  int ready[8];
-  int consumed;
-  int ob_ready, ob_taken;              // chunks of eight backward steps put into / taken from ob
+  double rec[F::NRING][F::N][64];  // slot, field, lane
+  double ob[8][NV][64];            // the sweep's backward U + dU (update) or dU of eight steps
+  int filled[F::NGRP];
+  int consumed, turned;
+  int ob_ready, ob_taken;          // chunks of eight backward steps put into / taken from ob
 };
 
 __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int spin_max) {
@@ -1019,30 +1031,59 @@ __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int 
   return true;
 }
 
-template <int NV, bool VISC, int NP>
-__global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
+// The waves of the fused launch: the sweep wave, FPROD producers, the writer,
+// and wave 4, which ends at once: a workgroup's waves go to the CU's four SIMDs
+// in turn, so waves 0 and 4 share one, and the sweep wave has its SIMD for
+// itself (256 SA blocks of 48-64 rows: 0.380 -> 0.368 ms).  A record takes its
+// producer about 2 us, most of it memory latency: five producers keep up with
+// the sweep, three did not (0.43 ms).
+constexpr int FPROD = 5;
+constexpr int FUSED_THREADS = 64 * (FPROD + 3);
+template <int NV, bool VISC>
+__global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
   using F = RecF<NV, VISC>;
-  using LDS = FusedLds<NV, VISC>;
-    constexpr int FPROD = NP, FRING = FusedSlot<NV, VISC>::NRING, XD = FusedSlot<NV, VISC>::XD;
-  static_assert(FRING % XD == 0 && FRING <= 8, "slots per turn");
-  __shared__ LDS L;
+  using FS = FusedSlot<NV, VISC>;
+  constexpr int FRING = FS::NRING, XD = FS::XD, NGRP = FS::NGRP;
+  __shared__ FusedLds<NV, VISC> L;
   const BlockDesc B = a.blocks[a.block_list[blockIdx.x]];
   if (case_frozen(B.case_id)) return;
   const double g = a.cps[B.case_id].gamma;
   const int ncol = B.nx - 1, nrow = B.ny - 1;
   const int S = B.sk_S, R = B.sk_R;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid < 8) L.ready[tid] = 0;
-  if (tid == 0) L.consumed = L.ob_ready = L.ob_taken = 0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = tid < 320 ? tid >> 6 : (tid >> 6) - 1;  // without the idle one
+  if (tid < NGRP) L.filled[tid] = 0;
+  if (tid == 0) L.consumed = L.turned = L.ob_ready = L.ob_taken = 0;
   __syncthreads();
-  constexpr int U = 2;  // the sweep's step padding (npad) of k_lusgs_sweep<..., 2, ..., 1>
-  const int npad = (S + 2 * U - 1) / (2 * U) * (2 * U);
+  if (tid >= 256 && tid < 320) return;  // the sweep wave's SIMD stays free
+  const int npad = (S + 3) / 4 * 4;  // whole turns of the sweep
   const int ntot = 2 * npad;
   const uint32_t n8 = (uint32_t)B.sk_n * 8u, n16 = 2u * n8;
   const uint32_t bytes = (uint32_t)((2 * F::NREC + 2 * F::XP) * B.sk_n * 8);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.sk + B.sk_base, 0, bytes, 0x00020000);
   const uint32_t bw = F::NREC * n8;
   double* planes = a.arena + B.base;
+  // The forward dU at a step's backward positions (the backward sweep's X),
+  // pairs and, with an odd equation count, a last field of single doubles.
+  // A lane whose row has no cell at this step reads the nearest row that has
+  // one: positions without a cell (about (nrow-1)/ncol of the field) are
+  // never written, and a wave reading them would fetch lines nobody needs;
+  // such a lane's value never reaches a cell.
+  auto load_x = [&](double* x, int st) {
+    const int sc = min(st, S - 1);
+    const int tr = min(max(lane, sc - (ncol - 1)), min(sc, nrow - 1));
+    const uint32_t pos = (uint32_t)(sc * R + tr);
+#pragma unroll
+    for (int j = 0; j < F::XP; j++) {
+      if (2 * j + 1 == NV) {
+        x[2 * j] = bload1(rs, pos * 8u, bw + (uint32_t)j * n16);
+      } else {
+        const D2 v = bload2(rs, pos * 16u, bw + (uint32_t)j * n16);
+        x[2 * j] = v.x;
+        x[2 * j + 1] = v.y;
+      }
+    }
+  };
   bool ok = true;
   if (wave == FPROD + 1) {
     // ---- writer: each chunk of eight backward steps from ob to the block
@@ -1109,21 +1150,43 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
     auto produce = [&](auto fwd_c, int first) {
       constexpr bool fwd = decltype(fwd_c)::value;
       const int gs0 = fwd ? 0 : npad;
-      RecSrc<NV> nx;
-      load_src_sk<NV, VISC, fwd>(nx, B, skin, first - gs0 - lane, lane);
-      int gs = first;
-      for (; gs < gs0 + npad && ok; gs += FPROD) {
-        const RecSrc<NV> q = nx;
-        // the next record's inputs (past the last step: clamped to it)
-        load_src_sk<NV, VISC, fwd>(nx, B, skin, min(gs + FPROD - gs0, npad - 1) - lane, lane);
-        ok = wait_bounded(&L.consumed, gs - FRING + 1, a.err, a.spin_max);
-        const int slot = gs % FRING;
-        auto SH = [&](int d) -> double& { return L.sh[slot][d][lane]; };
-        auto SD = [&](int kk, int e) -> double& { return L.sd[slot][kk][e][lane]; };
-        rec_body<NV, VISC, fwd, FusedSlot<NV, VISC>>(SH, SD, q, g, a.alfa1);
+      // the inputs of the producer's next two records are in flight while it
+      // makes one: a load takes up to 2 us, a sweep step about 0.45
+      RecSrc<NV> nx[2];
+      auto fetch = [&](RecSrc<NV>& q, int gs, bool x) {
+        const int sn = min(gs - gs0, npad - 1);  // past the last step: clamped to it
+        load_src_sk<NV, VISC, fwd>(q, B, skin, sn - lane, lane);
+        if (!fwd && x) load_x(q.Res, sn);
+      };
+      fetch(nx[0], first, false);
+      fetch(nx[1], first + FPROD, false);
+      if constexpr (!fwd) {
+        // the forward dU, from here on in memory
+        ok = wait_bounded(&L.turned, 1, a.err, a.spin_max);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        load_x(nx[0].Res, min(first - gs0, npad - 1));
+        load_x(nx[1].Res, min(first + FPROD - gs0, npad - 1));
+      }
+      auto record = [&](RecSrc<NV>& n, int gs) {
+        const RecSrc<NV> q = n;
+        fetch(n, gs + 2 * FPROD, true);
+        ok = wait_bounded(&L.consumed, (gs / XD + 1) * XD - FRING, a.err, a.spin_max);
+        double* rec = &L.rec[gs % FRING][0][lane];
+        auto SH = [&](int d) -> double& { return rec[d * 64]; };
+        auto SD = [&](int kk, int e) -> double& { return rec[(FS::side(kk) + e) * 64]; };
+        rec_body<NV, VISC, fwd, true, FS>(SH, SD, q, g, a.alfa1);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // the slot's LDS writes done (lgkmcnt 0) before publishing
-        lds_put(&L.ready[slot], gs + 1);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // the slot's LDS writes done (lgkmcnt 0) before counting it
+        if (lane == 0)
+          __hip_atomic_fetch_add(&L.filled[(gs / XD) % NGRP], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      };
+      int gs = first;
+      while (gs < gs0 + npad && ok) {
+        record(nx[0], gs);
+        gs += FPROD;
+        if (gs >= gs0 + npad || !ok) break;
+        record(nx[1], gs);
+        gs += FPROD;
       }
       return gs;
     };
@@ -1134,143 +1197,129 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lusgs_fused(LusgsArgs a) {
   // ---- the sweep wave: lane t = row t; it issues first on its SIMD
   __builtin_amdgcn_s_setprio(3);
   const int t = lane;
-  Chain<NV>& ch = *reinterpret_cast<Chain<NV>*>(&L);  // no other compute wave: never touched
-  using FS = FusedSlot<NV, VISC>;
-  auto load_lds = [&](Rec<NV, 2>& r, int slot, bool fwd) {
+  auto load_lds = [&](Rec<NV, 2>& r, const double* rec) {  // rec: the slot's first field of the lane
 #pragma unroll
     for (int m = 0; m < NV; m++) {
-      if (fwd) r.X[m] = L.sh[slot][m][t];
-      r.U[m] = L.sh[slot][FS::U + m][t];
+      r.X[m] = rec[m * 64];
+      r.U[m] = rec[(FS::U + m) * 64];
     }
-    r.al0 = L.sh[slot][FS::AL0][t];
-    r.y0 = L.sh[slot][FS::Y0][t];
+    r.yh0 = rec[FS::YH0 * 64];
+    r.yl0 = rec[FS::YL0 * 64];
     if constexpr (NV == 5) {
-      r.al4 = L.sh[slot][FS::AL4][t];
-      r.y4 = L.sh[slot][FS::Y4][t];
+      r.yh4 = rec[FS::YH4 * 64];
+      r.yl4 = rec[FS::YL4 * 64];
     } else {
-      r.al4 = r.al0;
-      r.y4 = r.y0;
+      r.yh4 = r.yh0;
+      r.yl4 = r.yl0;
     }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
+      const double* sd = rec + FS::side(h) * 64;
 #pragma unroll
-      for (int m = 0; m < NV; m++) r.F[h][m] = L.sd[slot][h][F::F + m][t];
-      r.n1[h] = L.sd[slot][h][F::N1][t];
-      r.n2[h] = L.sd[slot][h][F::N2][t];
-      r.a[h] = L.sd[slot][h][F::A][t];
-      r.Lc[h] = L.sd[slot][h][F::LC][t];
-      if constexpr (VISC) r.Lv[h] = L.sd[slot][h][F::LV][t];
+      for (int m = 0; m < NV; m++) r.F[h][m] = sd[(F::F + m) * 64];
+      r.n1[h] = sd[F::N1 * 64];
+      r.n2[h] = sd[F::N2 * 64];
+      r.a[h] = sd[F::A * 64];
+      r.Lc[h] = sd[F::LC * 64];
+      if constexpr (VISC) r.Lv[h] = sd[F::LV * 64];
       else r.Lv[h] = 0.0;
     }
   };
-  // the backward sweep's X (the forward dU) from the backward records' X pairs
-  // (pairs, and with an odd equation count the last field as single doubles).
-  // A lane whose row has no cell at this step reads the nearest row that has
-  // one: positions without a cell (about (nrow-1)/ncol of the field) are
-  // never written, and a wave reading them would fetch lines nobody needs;
-  // such a lane's value never reaches a cell.
-  auto load_x = [&](double* x, int st) {
-    const int sc = min(st, S - 1);
-    const int tr = min(max(t, sc - (ncol - 1)), min(sc, nrow - 1));
-    const uint32_t pos = (uint32_t)(sc * R + tr);
-#pragma unroll
-    for (int j = 0; j < F::XP; j++) {
-      if (2 * j + 1 == NV) {
-        x[2 * j] = bload1(rs, pos * 8u, bw + (uint32_t)j * n16);
-      } else {
-        const D2 v = bload2(rs, pos * 16u, bw + (uint32_t)j * n16);
-        x[2 * j] = v.x;
-        x[2 * j + 1] = v.y;
-      }
-    }
-  };
-  // one direction of the sweep; the direction is a compile-time constant so
+  // One direction of the sweep; the direction is a compile-time constant so
   // that every register array keeps fixed indices.  The next step's record
-  // is read from its slot while this step computes; in the backward sweep
-  // each step's X (the forward dU) is loaded XD steps ahead, into one of XD
-  // register sets (the loop runs XD steps per turn; npad is a multiple of 4).
-  int slot0 = 0;  // the slot of the turn's first step
+  // is read from its slot while this step computes.
+  int grp = 0, round = 1;  // the group slot of the turn and its use
   auto run_dir = [&](auto fwd_c) {
     constexpr bool fwd = decltype(fwd_c)::value;
     const int gs0 = fwd ? 0 : npad;
-    Ahead<NV> ah = {};
     Terms<NV, 1> tm = {};
-    double xs[XD][2 * F::XP] = {};
-    if (!fwd) {
-      // the forward sweep's stores to the X pairs before these loads, which
-      // the same wave issues: workgroup scope.  A device-scope fence also
-      // writes back the whole L2 (a launch of one block took 0.11 ms longer).
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-#pragma unroll
-      for (int k = 0; k < XD; k++) load_x(xs[k], k);
-    }
+    // a lane without a cell at a step sends its stores out of the buffer's
+    // range, where they are dropped; a row past the block never has a cell
+    constexpr uint32_t NOWHERE = 0x80000000u;
+    const int ts = t < nrow ? t : 0x40000000;
+    uint32_t w8 = (uint32_t)((S - 1) * R + (nrow - 1 - t)) * 8u;  // forward: the cell's X position, falling by R a step
     Rec<NV, 2> rn;
-    if (ok) ok = wait_bounded(&L.ready[slot0], gs0 + 1, a.err, a.spin_max);
-    load_lds(rn, slot0, fwd);
-    int pv = 0;  // the next slot's ready word, read one step earlier (0: not read)
-    auto one_step = [&](int st, int slot, int next, int after, double* x) {
-      const int gs = gs0 + st;
-      Rec<NV, 2> r = rn;
-      // The next step's record.  pv was read a step ago, so the wait (an LDS
-      // round trip on the chain) is taken only when that read found the
-      // record missing.  Both loads below are unconditional: a load under a
-      // branch makes its registers a phi, which the compiler resolves with
-      // copies that wait for the load in flight and so undo the prefetch.
-      // After the direction's last step the slot read is not waited for and
-      // its values are never used (the next direction reloads after its own
-      // wait), and load_x clamps the step to S - 1.
-      if (st + 1 < npad && ok && pv < gs + 2)
-        ok = wait_bounded(&L.ready[next], gs + 2, a.err, a.spin_max);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      load_lds(rn, next, fwd);
-      pv = lds_get(&L.ready[after]);
-      if constexpr (!fwd) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) r.X[m] = x[m];
-        load_x(x, st + XD);
-      }
-      // forward: dU to the backward records' X pairs; backward: U + dU (the
-      // record's U is the plane's value; with update) or dU into the output
-      // buffer, which the writer wave stores eight steps at a time
-      Out<NV> o;
-      sweep_step<NV, VISC, fwd, 1, fwd, true>(r, tm, o, rs, bw, n16, st, S, R, ncol, nrow, t, 0, lane, 0, false, false,
-                                              g, ch, ah);
-      // Slot gs is released after the step: its reads were issued a step ago
-      // and the next slot's at this step's start, so the wait costs nothing
-      // here, and it comes before the output buffer's writes so that it does
-      // not wait for them.
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0xc07f);
-      lds_put(&L.consumed, gs + 1);
-      if constexpr (!fwd) {
-        // chunks of eight steps; npad is a multiple of four, so the last
-        // chunk may end after four
-        const int b8 = st & 7, ck = st >> 3;
-        if (b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
-        if (a.update) {
-#pragma unroll
-          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.W[m];
-        } else {
-#pragma unroll
-          for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.du[m];
-        }
-        if (b8 == 7 || st == npad - 1) {
-          __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          __builtin_amdgcn_s_waitcnt(0xc07f);  // the chunk's writes done before it is handed over
-          lds_put(&L.ob_ready, ck + 1);
-        }
-      }
-    };
+    if (ok) ok = wait_bounded(&L.filled[grp], XD * round, a.err, a.spin_max);
+    load_lds(rn, &L.rec[grp * XD][0][t]);
     for (int st = 0; st < npad; st += XD) {
-      const int turn = slot0 + XD == FRING ? 0 : slot0 + XD;  // the next turn's first slot
+      const double* rec = &L.rec[grp * XD][0][t];
+      const int grp1 = grp + 1 == NGRP ? 0 : grp + 1, round1 = grp + 1 == NGRP ? round + 1 : round;
+      int pv = 0;  // the next group's count, read a step before it is needed
 #pragma unroll
-      for (int k = 0; k < XD; k++)
-        one_step(st + k, slot0 + k, k + 1 < XD ? slot0 + k + 1 : turn,
-                 k + 2 < XD ? slot0 + k + 2 : turn + (k + 2 - XD), xs[k]);
-      slot0 = turn;
+      for (int k = 0; k < XD; k++) {
+        const int s = st + k;
+        Rec<NV, 2> r = rn;
+        // The next step's record.  Its loads are unconditional: a load under
+        // a branch makes its registers a phi, which the compiler resolves
+        // with copies that wait for the load in flight and so undo the
+        // prefetch.  After the direction's last step the slot read is not
+        // waited for and its values are never used (the next direction
+        // reloads after its own wait).
+        if (k == XD - 1) {
+          if (s + 1 < npad && ok && pv < XD * round1)
+            ok = wait_bounded(&L.filled[grp1], XD * round1, a.err, a.spin_max);
+          __atomic_signal_fence(__ATOMIC_SEQ_CST);
+          load_lds(rn, &L.rec[grp1 * XD][0][t]);
+        } else {
+          load_lds(rn, rec + (k + 1) * FS::N * 64);
+          if (k == XD - 2) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            pv = lds_get(&L.filled[grp1]);
+          }
+        }
+        Out<NV> o;
+        double jin[NV];
+#pragma unroll
+        for (int m = 0; m < NV; m++) jin[m] = shr1(tm.j[m]);
+        cell_step<NV, VISC, fwd, 1>(r, tm, jin, o, g);
+        interleave<0x100, FS::N / 2, 7>();
+        if constexpr (fwd) {
+          // dU to the backward records' X (with an odd equation count the
+          // last field holds single doubles)
+          const bool act = (uint32_t)(s - ts) < (uint32_t)ncol;
+          const uint32_t w = act ? 2 * w8 : NOWHERE, wo = act ? w8 : NOWHERE;
+          w8 -= (uint32_t)R * 8u;
+#pragma unroll
+          for (int j = 0; j < F::XP; j++) {
+            if (2 * j + 1 == NV) bstore1(o.du[2 * j], rs, wo, bw + (uint32_t)j * n16);
+            else bstore2(o.du[2 * j], o.du[2 * j + 1], rs, w, bw + (uint32_t)j * n16);
+          }
+        } else {
+          // U + dU (the record's U is the plane's value; with update) or dU
+          // into the output buffer, which the writer wave stores eight steps
+          // at a time; npad is a multiple of four, so the last chunk may end
+          // after four
+          const int b8 = s & 7, ck = s >> 3;
+          if (k == 0 || XD < 4)
+            if (b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
+          if (a.update) {
+#pragma unroll
+            for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.W[m];
+          } else {
+#pragma unroll
+            for (int m = 0; m < NV; m++) L.ob[b8][m][t] = o.du[m];
+          }
+          if ((k == XD - 1) && (b8 == 7 || s == npad - 1)) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // the chunk's writes done before it is handed over
+            lds_put(&L.ob_ready, ck + 1);
+          }
+        }
+      }
+      // the group's records have all been read (the last one's values were
+      // used by its step)
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      lds_put(&L.consumed, gs0 + st + XD);
+      grp = grp1;
+      round = round1;
     }
   };
   run_dir(std::true_type{});
+  // The forward sweep's stores before the producers' loads: waves of one
+  // workgroup, so workgroup scope.  (A device-scope fence also writes back the
+  // whole L2.)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  lds_put(&L.turned, 1);
   run_dir(std::false_type{});
 }
 

@@ -40,6 +40,10 @@ __device__ __forceinline__ double rcp_rn(double b) {
   return y;
 }
 
+// a / b from 1/b held as h + l to 2^-104: two operations, one rounding of a
+// value within 2^-104 of the quotient.
+__device__ __forceinline__ double div_hl(double a, double h, double l) { return __builtin_fma(a, h, a * l); }
+
 // sub_Residual.f90:477-487
 __device__ __forceinline__ double minmod(double a, double b) {
   if (a * b <= 0.0) return 0.0;
