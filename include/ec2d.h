@@ -311,21 +311,21 @@ int ec2d_set_profile(int on);
 int ec2d_set_wait_budget(int polls);
 
 /* No reference counterpart: the LU-SGS launch shape of one level, chosen by
- * hand (ec2d_autotune chooses it by timing otherwise): lanes per cell 1 or 2,
+ * hand (a rule on the block sizes chooses it at ec2d_commit, ec2d_autotune by
+ * timing): lanes per cell 1 or 2,
  * workgroups per block 1, 2 or 4 (each block's rows split between that many
  * CUs, for levels of at most 256/split blocks taller than split/2 waves), or
- * 0 with one lane per cell: the fused launch, whose workgroups make each
- * block's records themselves (blocks of at most 64 rows of cells), so that
- * they never go through device memory, with 6 producer waves and a writer
- * wave beside the sweep wave (-3: with 3 producers).  Results do not depend
- * on it. */
+ * 0 with one lane per cell, for blocks of at most 64 rows: the fused launches,
+ * whose workgroups make each block's records themselves, so that they never go
+ * through device memory - in parts of 32 rows where every part finds a CU of
+ * its own, one workgroup per block otherwise (-3: one workgroup per block in
+ * any case).  Results do not depend on it. */
 int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block);
 
 /* Autotune the launch shapes of every mesh level on the committed batch:
  * residual tile rows (1, 2, 4, 8 x 64 cells), LU-SGS lanes per cell (1 or 2),
- * workgroups per block (1, 2 or 4, see ec2d_lusgs_shape) and sweep steps per
- * prefetched register set (2, 3 or 4 with two lanes per cell and at most four
- * waves), each timed with HIP events over `reps` launches on the current
+ * workgroups per block (1, 2 or 4, see ec2d_lusgs_shape) and the fused LU-SGS
+ * launches, each timed with HIP events over `reps` launches on the current
  * state; the fastest is kept.  Results are cached per level configuration
  * (equations, scheme, flux, reconstruction, turbulence model, viscosity,
  * block shapes) in the text file cache_path (NULL or "": no cache).  report

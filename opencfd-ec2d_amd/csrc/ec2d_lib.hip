@@ -80,7 +80,8 @@ struct DLevel {
   int lusgs_threads = 64;
   int lusgs_lpc = 1;          // LU-SGS lanes per cell: 2 when every block has at most 32 rows
   int lusgs_split = 1;        // LU-SGS sweep workgroups per block (2 or 4: a block's rows split between CUs)
-  bool lusgs_fused = false;   // LU-SGS records made inside the sweep workgroup (k_lusgs_fused)
+  bool lusgs_fused = false;   // LU-SGS records made inside the sweep workgroup (k_lusgs_fused, k_lusgs_parts)
+  bool lusgs_parts = false;   // with lusgs_fused: workgroups of 32 rows (k_lusgs_parts), lusgs_split per block
   bool planar_stale = false;  // Res, dt, Lc, Lv are current only in the hyperplane copy (planar_refresh)
   bool skew_static = false;   // the record arena holds the skewed copy of the mesh planes
   unsigned long long* dgring = nullptr;  // split sweeps: one ring per boundary between workgroups and direction
@@ -102,6 +103,7 @@ struct DLevel {
 
 struct Runtime {
   bool inited = false, committed = false;
+  int ncu = 256;  // compute units of the device
   std::vector<HCase> cases;
   std::vector<DLevel> lv;
   CaseParams* dcps = nullptr;
@@ -247,23 +249,41 @@ void ghost_phases(const BlockDesc& B, SubfaceDesc* s, int* units) {
   }
 }
 
+// k_lusgs_parts waits between the workgroups of a block: all of them must be
+// resident at once, one per CU.  A block of one part has nothing to wait for.
+bool parts_fit(const DLevel& L) {
+  int max_rows = 1;
+  for (auto& d : L.hb) max_rows = std::max(max_rows, d.ny - 1);
+  const int G = (max_rows + PART_ROWS - 1) / PART_ROWS;
+  return G == 1 || (int64_t)G * (int64_t)L.hb.size() <= R.ncu;
+}
+
 // LU-SGS record layout of a level for lpc lanes per cell (see ec2d_lusgs.hip);
 // upload: also refresh the device block table (after ec2d_commit).  fused:
 // the layout of k_lusgs_fused, whose single sweep wave needs no whole waves
 // of rows, so a step holds exactly the block's rows (R = nrow): the rows of
 // consecutive steps share cache lines instead of padding each step to 64.
-int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false) {
+// parts: that of k_lusgs_parts (also R = nrow), with `split` set here to the
+// parts of 32 rows of the tallest block.
+int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false, bool parts = false) {
   L.skew_static = false;  // the arena is cleared below
   int max_rows = 1;
   for (auto& d : L.hb) max_rows = std::max(max_rows, d.ny - 1);
   const int rq = 64 / lpc;  // rows per wave
-  if (split != 1 && split != 2 && split != 4) return fail("LU-SGS split must be 1, 2 or 4");
+  if (parts) {
+    fused = true;
+    split = (max_rows + PART_ROWS - 1) / PART_ROWS;
+    if (!parts_fit(L)) return fail("too many blocks for an LU-SGS launch in parts of 32 rows");
+    if (max_rows > 1024) return fail("blocks with more than 1024 rows of cells are not supported by the LU-SGS kernel");
+  } else if (split != 1 && split != 2 && split != 4) {
+    return fail("LU-SGS split must be 1, 2 or 4");
+  }
   // every workgroup of a split launch must be resident at once: one per CU at most
-  if (split > 1 && (max_rows <= rq * (split / 2) || split * (int)L.hb.size() > 256))
+  if (!parts && split > 1 && (max_rows <= rq * (split / 2) || split * (int)L.hb.size() > 256))
     return fail("a split LU-SGS sweep needs blocks taller than split/2 waves and at most 256/split blocks");
   // rows rounded to whole waves per workgroup; split: one communication wave
   // more, two for the middle parts of a split into four
-  const int waves = (max_rows + rq * split - 1) / (rq * split) + (split > 2 ? 2 : split - 1);
+  const int waves = parts ? PART_THREADS / 64 : (max_rows + rq * split - 1) / (rq * split) + (split > 2 ? 2 : split - 1);
   const int threads = 64 * waves;
   if (threads > 1024) return fail("blocks with more than 1024 rows of cells are not supported by the LU-SGS kernel");
   const int nv = L.o.nvar;
@@ -738,7 +758,13 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
       hipLaunchKernelGGL((k_lusgs_skew<NV, V, false>), gskew, dim3(256), 0, R.s, a);        \
     prof_mark(-(4 + pk));                                                                   \
     prof_mark(5 + pk);                                                                      \
-    hipLaunchKernelGGL((k_lusgs_fused<NV, V>), dim3(nblk), dim3(FUSED_THREADS), 0, R.s, a); \
+    if (L.lusgs_parts) {                                                                    \
+      for (int d = (a.split > 1 ? 1 : 0); d <= (a.split > 1 ? 2 : 0); d++) {                \
+        a.dir = d;                                                                          \
+        hipLaunchKernelGGL((k_lusgs_parts<NV, V>), dim3(nblk * a.split), dim3(PART_THREADS), 0, R.s, a); \
+      }                                                                                     \
+    } else                                                                                  \
+      hipLaunchKernelGGL((k_lusgs_fused<NV, V>), dim3(nblk), dim3(FUSED_THREADS), 0, R.s, a); \
     prof_mark(-(5 + pk));                                                                   \
   } else {                                                                                  \
   prof_mark(4 + pk);                                                                        \
@@ -1309,9 +1335,10 @@ struct Lcg {
   double uniform() { return (next() + 0.5) / 2147483648.0; }  // (0, 1)
 };
 
-// autotune report text of an LU-SGS shape (0: the fused launch)
+// autotune report text of an LU-SGS shape (0, -1: the fused launches)
 std::string shape_text(int sp) {
   if (sp == 0) return "fused preparation and sweeps";
+  if (sp == -1) return "fused preparation and sweeps in parts of 32 rows";
   return "workgroups per block " + std::to_string(sp);
 }
 
@@ -1334,6 +1361,12 @@ int ec2d_init(void) {
       if (e != hipSuccess || !p) return fail(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
       scratch_addr[dev] = p;
     }
+  }
+  {
+    int dev = 0, n_cu = 0;
+    HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+    if (n_cu > 0) R.ncu = n_cu;
   }
   HIPCHK(hipStreamCreateWithFlags(&R.s, hipStreamNonBlocking));
   HIPCHK(hipEventCreate(&R.ev0));
@@ -1782,9 +1815,18 @@ int ec2d_commit(void) {
     }
     L.case_first_block.push_back((int)L.hb.size());
     L.arena_n = off;
-    // two lanes per cell when one wave holds every block's rows that way;
-    // otherwise one lane per row (fewer waves, fewer barriers per step)
-    if (lusgs_layout(L, max_rows <= 32 ? 2 : 1, 1, false)) return 1;
+    // The LU-SGS shape until ec2d_autotune times them.  In parts of 32 rows
+    // where all parts fit the device: 257 x 65 cells of six equations 0.31 ms an
+    // update (0.38 with one lane per row and the records in memory), 64 blocks
+    // of up to 257 x 129 cells 0.28 ms (0.40).  Blocks of one part have no chain
+    // between workgroups to shorten: the records in memory are as fast up to
+    // about 16 blocks of 129 x 33 cells (0.148 against 0.146 ms a pass; one
+    // block 0.136 against 0.144, 64 blocks 0.183 against 0.168).  Else the fused
+    // launch for blocks of at most 64 rows (256 SA blocks: 0.36 against 1.35 ms);
+    // else the records in memory.
+    L.lusgs_parts = parts_fit(L) && (max_rows > PART_ROWS || L.hb.size() >= 16);
+    L.lusgs_fused = L.lusgs_parts || (max_rows > PART_ROWS && max_rows <= 64);
+    if (lusgs_layout(L, !L.lusgs_fused && max_rows <= 32 ? 2 : 1, 1, false, L.lusgs_fused, L.lusgs_parts)) return 1;
     // host image of the arena
     std::vector<double> img((size_t)off, 0.0);
     init_default_state(L, l, img);
@@ -2359,7 +2401,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
   if (lanes_per_cell != 1 && lanes_per_cell != 2) return fail("lanes per cell must be 1 or 2");
   HIPCHK(hipStreamSynchronize(R.s));
   DLevel& L = R.lv[nMesh - 1];
-  // 0 (or -3, once a launch with fewer producer waves): fused
+  // 0: fused, in parts of 32 rows where they fit; -3: fused, a workgroup per block
   const bool fused = workgroups_per_block == 0 || workgroups_per_block == -3;
   if (workgroups_per_block < 0 && !fused) return fail("workgroups per block 1, 2, 4, or 0 / -3 (fused)");
   if (fused) {
@@ -2367,8 +2409,10 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
     for (auto& b : L.hb)
       if (b.ny - 1 > 64) return fail("the fused LU-SGS launch needs blocks of at most 64 rows of cells");
   }
-  if (lusgs_layout(L, lanes_per_cell, fused ? 1 : workgroups_per_block, true, fused)) return 1;
+  const bool parts = workgroups_per_block == 0 && parts_fit(L);
+  if (lusgs_layout(L, lanes_per_cell, fused ? 1 : workgroups_per_block, true, fused, parts)) return 1;
   L.lusgs_fused = fused;
+  L.lusgs_parts = parts;
   if (R.graph) {  // a captured graph holds the old launch shape
     HIPCHK(hipGraphExecDestroy(R.graph));
     R.graph = nullptr;
@@ -2441,7 +2485,7 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
       // LU-SGS lanes per cell and workgroups per block (the state after a
       // residual; dU only is written)
       best = 1e30;
-      L.lusgs_fused = false;
+      L.lusgs_fused = L.lusgs_parts = false;
       std::string cand;  // every timed LU-SGS shape, for the report
       auto note = [&](const char* tag, double ms) {
         char t[64];
@@ -2462,14 +2506,17 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
           note(tag, ms);
           if (ms < best) { best = ms; best_lp = lp; best_sp = sp; }
         }
-      // the fused variant: records made in the sweep workgroup (rows <= 64)
+      // the fused variants: records made in the sweep workgroup, a workgroup
+      // per block (0; rows <= 64) or per part of 32 rows (-1).  Timed with the
+      // residual before them, which writes their inputs in a main-loop pass
+      // (advance_lusgs), less the plain residual: the copy kernel that a lone
+      // update needs is no part of a pass.
       bool fits = true;
       for (auto& b : L.hb) fits = fits && b.ny - 1 <= 64;
-      if (fits && !lusgs_layout(L, 1, 1, true, true)) {
-        // timed with the residual before it, which writes its inputs in a
-        // main-loop pass (advance_lusgs), less the plain residual: the copy
-        // kernel that a lone update needs is no part of a pass
+      for (int sp : {0, -1}) {
+        if (!(sp == 0 ? fits : parts_fit(L)) || lusgs_layout(L, 1, 1, true, true, sp == -1)) continue;
         L.lusgs_fused = true;
+        L.lusgs_parts = sp == -1;
         const bool rskew = !L.fdm;
         double ms;
         if (time_launches(reps, [&] {
@@ -2478,10 +2525,10 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
             }, &ms))
           return 1;
         ms -= res_ms;
-        note("fused", ms);
-        if (ms < best) { best = ms; best_lp = 1; best_sp = 0; }
-        L.lusgs_fused = false;
+        note(sp == 0 ? "fused" : "parts", ms);
+        if (ms < best) { best = ms; best_lp = 1; best_sp = sp; }
       }
+      L.lusgs_fused = L.lusgs_parts = false;
       R.err.clear();
       HIPCHK(hipMemcpyAsync(L.arena, keep, sizeof(double) * (size_t)L.arena_n, hipMemcpyDeviceToDevice, R.s));
       HIPCHK(hipStreamSynchronize(R.s));
@@ -2501,8 +2548,10 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
     L.tile_cols = best_tr >= 100 ? 32 : 64;
     L.tile_rows = best_tr % 100;
     if (build_tiles(L)) return 1;
-    if (lusgs_layout(L, best_lp, best_sp == 0 ? 1 : best_sp, true, best_sp == 0)) return 1;
-    L.lusgs_fused = best_sp == 0;
+    if (best_sp == -1 && !parts_fit(L)) best_sp = 1;  // a cache file of a device with more compute units
+    if (lusgs_layout(L, best_lp, best_sp <= 0 ? 1 : best_sp, true, best_sp <= 0, best_sp == -1)) return 1;
+    L.lusgs_fused = best_sp <= 0;
+    L.lusgs_parts = best_sp == -1;
   }
   if (!added.empty() && cache_path && cache_path[0]) {
     if (FILE* f = std::fopen(cache_path, "a")) {

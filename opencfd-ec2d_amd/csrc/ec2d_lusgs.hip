@@ -1,13 +1,16 @@
 // LU-SGS implicit update: du_LU_SGS_2D (sub_LU_SGS.f90:4-108), optionally
 // followed by U = U + dU (sub_NS_singlegrid.f90:203-211), for all blocks of
-// one mesh level.  Two paths, chosen per level (ec2d_autotune):
+// one mesh level.  Three paths, chosen per level (ec2d_commit's rule, or
+// ec2d_autotune):
 //
 //   split   k_lusgs_prep (every cell in parallel) writes, for each of the two
 //           sweeps, a record of all the cell's update needs that does not
 //           depend on dU; k_lusgs_sweep runs the two dependent sweeps;
 //           k_lusgs_scatter puts dU into the block planes (and U = U + dU);
 //   fused   k_lusgs_fused makes the records in the sweep's own workgroup and
-//           writes the planes itself (blocks of at most 64 rows).
+//           writes the planes itself (blocks of at most 64 rows);
+//   parts   k_lusgs_parts does the same by workgroups of 32 rows, linked as
+//           the split sweeps are (few blocks, any number of rows).
 //
 // Sweep order.  The forward sweep needs dU(i-1,j) and dU(i,j-1), the backward
 // sweep dU(i+1,j) and dU(i,j+1).  Any order that respects these dependencies
@@ -195,6 +198,9 @@ __device__ __forceinline__ double even_lane(double v) {
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 struct D2 {
+  double x, y;
+};
+struct alignas(16) D2a {  // in LDS: one 16-byte read
   double x, y;
 };
 
@@ -652,12 +658,12 @@ __device__ __forceinline__ void side_term(double* v, const Rec<NV, NS>& p, int h
 // producer's progress and cons[w] wave w's consumption.
 constexpr int RING = 16;
 constexpr int CHAIN_END = 0x7fffffff;
-template <int NV>
+template <int NV, int NW>  // NW: rings (waves and one more)
 struct Chain {
   double dump[RING][NV];      // where the lanes below a wave's last one write
-  double ring[17][RING][NV];  // input of wave w: the terms of the row below it
-  int prog[17];               // steps finished by the producer of ring[w]
-  int cons[17];               // steps whose input wave w has read
+  double ring[NW][RING][NV];  // input of wave w: the terms of the row below it
+  int prog[NW];               // steps finished by the producer of ring[w]
+  int cons[NW];               // steps whose input wave w has read
 };
 
 __device__ __forceinline__ int lds_get(const int* p) {
@@ -733,7 +739,7 @@ __device__ __forceinline__ void interleave() {
 // LINK: the wave has others to exchange with (not a block of one wave).
 template <int NV, bool VISC, bool FWD, int D, int LPC, bool LINK>
 __device__ __forceinline__ void sweep(__amdgpu_buffer_rsrc_t rs, uint32_t rec, uint32_t dst, uint32_t n16, int S, int R,
-                                      int ncol, int nrow, int t, int k, int lane, int wave, double g, Chain<NV>& ch) {
+                                      int ncol, int nrow, int t, int k, int lane, int wave, double g, Chain<NV, 17>& ch) {
   using F = RecF<NV, VISC>;
   static_assert(2 * D <= RING + 1 && RING % D == 0, "the turns of linked waves must fit the ring");
   const int npad = (S + D - 1) / D * D;
@@ -859,8 +865,8 @@ struct CommLane {
 };
 
 // sending side: take ring[nw] (the last compute wave's row) and store it
-template <int NV>
-__device__ void comm_forward(Chain<NV>& ch, int nw, unsigned long long* gr, int npad) {
+template <int NV, int NW>
+__device__ void comm_forward(Chain<NV, NW>& ch, int nw, unsigned long long* gr, int npad) {
   const CommLane<NV> c;
   for (int s0 = 0; s0 < npad - 1; s0 += c.CK) {
     const int nst = min(c.CK, npad - 1 - s0);
@@ -874,8 +880,8 @@ __device__ void comm_forward(Chain<NV>& ch, int nw, unsigned long long* gr, int 
 }
 
 // receiving side: take each batch of rows and feed ring[0]; then reset
-template <int NV>
-__device__ void comm_receive(Chain<NV>& ch, unsigned long long* gr, int npad, int* err, int spin_max) {
+template <int NV, int NW>
+__device__ void comm_receive(Chain<NV, NW>& ch, unsigned long long* gr, int npad, int* err, int spin_max) {
   const CommLane<NV> c;
   static_assert(CommLane<NV>::CK <= RING, "a batch must fit the LDS ring");
   bool gone = false;  // the other workgroup stopped answering: wait no more
@@ -914,7 +920,7 @@ template <int NV, bool VISC, int D, int MAXT, int LPC>
 __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   using F = RecF<NV, VISC>;
   constexpr bool LINK = MAXT > 64;
-  __shared__ Chain<NV> ch[2];  // one per sweep
+  __shared__ Chain<NV, 17> ch[2];  // one per sweep
   const int G = a.split, bi = blockIdx.x / G, half = blockIdx.x % G;  // half: the part of the block
   const BlockDesc B = a.blocks[a.block_list[bi]];
   if (case_frozen(B.case_id)) return;  // every part of the block returns: no part waits on another
@@ -928,7 +934,7 @@ __global__ __launch_bounds__(MAXT) void k_lusgs_sweep(LusgsArgs a) {
   const int nw = R * LPC / (64 * G);
   const int t = half * (R / G) + (LPC == 2 ? tid >> 1 : tid), k = LPC == 2 ? tid & 1 : 0;
   const bool has_in = half > 0, has_out = half < G - 1;
-  for (int q = tid; q < 2 * (int)(sizeof(Chain<NV>) / 8); q += blockDim.x) reinterpret_cast<double*>(ch)[q] = 0.0;
+  for (int q = tid; q < 2 * (int)(sizeof(Chain<NV, 17>) / 8); q += blockDim.x) reinterpret_cast<double*>(ch)[q] = 0.0;
   __syncthreads();
   if (tid < 2) {
     if (!has_in) ch[tid].prog[0] = CHAIN_END;
@@ -1031,6 +1037,93 @@ __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int 
   return true;
 }
 
+// The forward dU at a step's backward positions (the backward sweep's X) for
+// row r, pairs and, with an odd equation count, a last field of single doubles.
+// A lane whose row has no cell at this step reads the nearest row that has
+// one: positions without a cell (about (nrow-1)/ncol of the field) are
+// never written, and a wave reading them would fetch lines nobody needs;
+// such a lane's value never reaches a cell.
+template <int NV, bool VISC>
+__device__ __forceinline__ void load_x(double* x, __amdgpu_buffer_rsrc_t rs, uint32_t bw, uint32_t n16, int st, int r,
+                                       int S, int R, int ncol, int nrow) {
+  const int sc = min(st, S - 1);
+  const int tr = min(max(r, sc - (ncol - 1)), min(sc, nrow - 1));
+  const uint32_t pos = (uint32_t)(sc * R + tr);
+#pragma unroll
+  for (int j = 0; j < (NV + 1) / 2; j++) {
+    if (2 * j + 1 == NV) {
+      x[2 * j] = bload1(rs, pos * 8u, bw + (uint32_t)j * n16);
+    } else {
+      const D2 v = bload2(rs, pos * 16u, bw + (uint32_t)j * n16);
+      x[2 * j] = v.x;
+      x[2 * j + 1] = v.y;
+    }
+  }
+}
+
+// The writer: each chunk of eight backward steps of ROWS rows (from row0 of
+// the backward order) from ob to the block
+// planes, every store one aligned 64-byte run (8 cells) of each of 8
+// rows.  Row r's cells of a chunk (steps 8ck .. 8ck+7, columns c = step
+// - r, plane offset ncol + 1 - c in the row, whose start is 128-byte
+// aligned: the pitch is a multiple of 16) straddle two aligned runs.
+// Lane = 8 rows x position p of the run (offset mod 8): it reads the one
+// step whose cell sits at position p, always the same slot sub of the
+// chunk.  Positions 0..q (q = (ncol + 1 + r) mod 8) complete the run they
+// fall in and are stored at once; positions q+1..7 start the next run and
+// are held one chunk, while the value held from the previous chunk
+// completes this one.  A last turn stores the runs held after the final
+// chunk.  Every cell is stored exactly once, cells outside the block
+// (columns < 0 or >= ncol, rows >= nrow) are skipped.  With update the
+// planes are U (U + dU, the update of k_lusgs_scatter; nothing reads the
+// dU planes after a main-loop pass, so they are not rewritten), without
+// it dU.
+template <int NV, int ROWS>
+__device__ __forceinline__ void write_planes(double (*ob)[NV][ROWS], int& ob_ready, int& ob_taken, const LusgsArgs& a,
+                                             const BlockDesc& B, int row0, int npad, int lane) {
+  constexpr int RG = ROWS / 8;
+  const int ncol = B.nx - 1, nrow = B.ny - 1;
+  double* planes = a.arena + B.base;
+  const int p = lane & 7, rl = lane >> 3;
+  const int q = (ncol + 1 + rl) & 7;   // rows rl + 8k share it: the pitch and row0 are multiples of 8
+  const int sub = (q - p) & 7;
+  const bool held = p > q;             // this lane's cell starts the next run
+  const int dst = a.update ? a.pm.U : a.pm.dU;
+  const int nck = (npad + 7) / 8;
+  double keep[RG][NV] = {};
+  for (int ck = 0; ck <= nck; ck++) {
+    double v[RG][NV];
+    if (ck < nck) {
+      if (!wait_bounded(&ob_ready, ck + 1, a.err, a.spin_max)) break;
+#pragma unroll
+      for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+        for (int m = 0; m < NV; m++) v[rg][m] = ob[sub][m][rg * 8 + rl];
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // the buffer read before it is handed back
+      lds_put(&ob_taken, ck + 1);
+    } else {
+#pragma unroll
+      for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+        for (int m = 0; m < NV; m++) v[rg][m] = 0.0;
+    }
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++) {
+      const int r = row0 + rg * 8 + rl;
+      // the run's offset in the row: 8 * floor((ncol + 1 + r) / 8) - 8ck + p
+      const int off = ((ncol + 1 + r) & ~7) - 8 * ck + p, c = ncol + 1 - off;
+      if (r < nrow && c >= 0 && c < ncol) {
+        const int64_t qi = (int64_t)(nrow - r + 1) * B.P + off;  // pidx(B, ncol - c, nrow - r)
+#pragma unroll
+        for (int m = 0; m < NV; m++) planes[(int64_t)(dst + m) * B.plane + qi] = held ? keep[rg][m] : v[rg][m];
+      }
+#pragma unroll
+      for (int m = 0; m < NV; m++) keep[rg][m] = v[rg][m];
+    }
+  }
+}
+
 // The waves of the fused launch: the sweep wave, FPROD producers, the writer,
 // and wave 4, which ends at once: a workgroup's waves go to the CU's four SIMDs
 // in turn, so waves 0 and 4 share one, and the sweep wave has its SIMD for
@@ -1062,85 +1155,9 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
   const uint32_t bytes = (uint32_t)((2 * F::NREC + 2 * F::XP) * B.sk_n * 8);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.sk + B.sk_base, 0, bytes, 0x00020000);
   const uint32_t bw = F::NREC * n8;
-  double* planes = a.arena + B.base;
-  // The forward dU at a step's backward positions (the backward sweep's X),
-  // pairs and, with an odd equation count, a last field of single doubles.
-  // A lane whose row has no cell at this step reads the nearest row that has
-  // one: positions without a cell (about (nrow-1)/ncol of the field) are
-  // never written, and a wave reading them would fetch lines nobody needs;
-  // such a lane's value never reaches a cell.
-  auto load_x = [&](double* x, int st) {
-    const int sc = min(st, S - 1);
-    const int tr = min(max(lane, sc - (ncol - 1)), min(sc, nrow - 1));
-    const uint32_t pos = (uint32_t)(sc * R + tr);
-#pragma unroll
-    for (int j = 0; j < F::XP; j++) {
-      if (2 * j + 1 == NV) {
-        x[2 * j] = bload1(rs, pos * 8u, bw + (uint32_t)j * n16);
-      } else {
-        const D2 v = bload2(rs, pos * 16u, bw + (uint32_t)j * n16);
-        x[2 * j] = v.x;
-        x[2 * j + 1] = v.y;
-      }
-    }
-  };
   bool ok = true;
   if (wave == FPROD + 1) {
-    // ---- writer: each chunk of eight backward steps from ob to the block
-    // planes, every store one aligned 64-byte run (8 cells) of each of 8
-    // rows.  Row r's cells of a chunk (steps 8ck .. 8ck+7, columns c = step
-    // - r, plane offset ncol + 1 - c in the row, whose start is 128-byte
-    // aligned: the pitch is a multiple of 16) straddle two aligned runs.
-    // Lane = 8 rows x position p of the run (offset mod 8): it reads the one
-    // step whose cell sits at position p, always the same slot sub of the
-    // chunk.  Positions 0..q (q = (ncol + 1 + r) mod 8) complete the run they
-    // fall in and are stored at once; positions q+1..7 start the next run and
-    // are held one chunk, while the value held from the previous chunk
-    // completes this one.  A last turn stores the runs held after the final
-    // chunk.  Every cell is stored exactly once, cells outside the block
-    // (columns < 0 or >= ncol, rows >= nrow) are skipped.  With update the
-    // planes are U (U + dU, the update of k_lusgs_scatter; nothing reads the
-    // dU planes after a main-loop pass, so they are not rewritten), without
-    // it dU.
-    const int p = lane & 7, rl = lane >> 3;
-    const int q = (ncol + 1 + rl) & 7;   // rows rl + 8k share it: the pitch is a multiple of 8
-    const int sub = (q - p) & 7;
-    const bool held = p > q;             // this lane's cell starts the next run
-    const int dst = a.update ? a.pm.U : a.pm.dU;
-    const int nck = (npad + 7) / 8;
-    double keep[8][NV] = {};
-    for (int ck = 0; ck <= nck && ok; ck++) {
-      double v[8][NV];
-      if (ck < nck) {
-        ok = wait_bounded(&L.ob_ready, ck + 1, a.err, a.spin_max);
-        if (!ok) break;
-#pragma unroll
-        for (int rg = 0; rg < 8; rg++)
-#pragma unroll
-          for (int m = 0; m < NV; m++) v[rg][m] = L.ob[sub][m][rg * 8 + rl];
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // the buffer read before it is handed back
-        lds_put(&L.ob_taken, ck + 1);
-      } else {
-#pragma unroll
-        for (int rg = 0; rg < 8; rg++)
-#pragma unroll
-          for (int m = 0; m < NV; m++) v[rg][m] = 0.0;
-      }
-#pragma unroll
-      for (int rg = 0; rg < 8; rg++) {
-        const int r = rg * 8 + rl;
-        // the run's offset in the row: 8 * floor((ncol + 1 + r) / 8) - 8ck + p
-        const int off = ((ncol + 1 + r) & ~7) - 8 * ck + p, c = ncol + 1 - off;
-        if (r < nrow && c >= 0 && c < ncol) {
-          const int64_t qi = (int64_t)(nrow - r + 1) * B.P + off;  // pidx(B, ncol - c, nrow - r)
-#pragma unroll
-          for (int m = 0; m < NV; m++) planes[(int64_t)(dst + m) * B.plane + qi] = held ? keep[rg][m] : v[rg][m];
-        }
-#pragma unroll
-        for (int m = 0; m < NV; m++) keep[rg][m] = v[rg][m];
-      }
-    }
+    write_planes<NV, 64>(L.ob, L.ob_ready, L.ob_taken, a, B, 0, npad, lane);
     return;
   }
   if (wave > 0) {
@@ -1156,7 +1173,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
       auto fetch = [&](RecSrc<NV>& q, int gs, bool x) {
         const int sn = min(gs - gs0, npad - 1);  // past the last step: clamped to it
         load_src_sk<NV, VISC, fwd>(q, B, skin, sn - lane, lane);
-        if (!fwd && x) load_x(q.Res, sn);
+        if (!fwd && x) load_x<NV, VISC>(q.Res, rs, bw, n16, sn, lane, S, R, ncol, nrow);
       };
       fetch(nx[0], first, false);
       fetch(nx[1], first + FPROD, false);
@@ -1164,8 +1181,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
         // the forward dU, from here on in memory
         ok = wait_bounded(&L.turned, 1, a.err, a.spin_max);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        load_x(nx[0].Res, min(first - gs0, npad - 1));
-        load_x(nx[1].Res, min(first + FPROD - gs0, npad - 1));
+        load_x<NV, VISC>(nx[0].Res, rs, bw, n16, min(first - gs0, npad - 1), lane, S, R, ncol, nrow);
+        load_x<NV, VISC>(nx[1].Res, rs, bw, n16, min(first + FPROD - gs0, npad - 1), lane, S, R, ncol, nrow);
       }
       auto record = [&](RecSrc<NV>& n, int gs) {
         const RecSrc<NV> q = n;
@@ -1321,6 +1338,278 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   lds_put(&L.turned, 1);
   run_dir(std::false_type{});
+}
+
+// ------------------------------------- the same, in parts of 32 rows of a block
+// For levels of few blocks (k parts each, at most one workgroup per CU): each
+// part of 32 rows is a workgroup of its own, linked to the next through
+// global memory as the split sweeps' workgroups are, and makes its records in
+// LDS as k_lusgs_fused does.  The sweep wave has two lanes per cell: its step
+// is a quarter shorter than with one, and what bounds a single block is the
+// chain of steps (the split sweeps' wave reads its records by 13 memory loads a
+// step, which take it about 7 ns each to issue; the LDS reads here 3).
+//   A producer's 64 lanes make the records of two steps at a time.  LDS
+// records come in pairs of doubles: the cell's part by row, the sides' by lane,
+// so that the sweep wave's reads are 16 bytes a lane without bank conflicts.
+//   A block of one part runs both sweeps in one launch; with several the
+// sweeps are separate launches (a.dir), as in k_lusgs_sweep.
+template <int NV, bool VISC>
+struct PartSlot {
+  using F = RecF<NV, VISC>;
+  static constexpr int U = NV, YH0 = 2 * NV, YL0 = YH0 + 1, YH4 = YH0 + 2, YL4 = YH0 + 3;
+  static constexpr int NSH = 2 * NV + 2 + (NV == 5 ? 2 : 0), NSD = F::NSD;
+  static constexpr int SIDE = NSH / 2 * 64, N = SIDE + NSD / 2 * 128;  // doubles of a slot
+  static constexpr int XD = 4;                      // sweep steps per turn: one group of slots
+  static constexpr int NRING = NV >= 6 ? 12 : 16;   // record slots
+  static constexpr int NGRP = NRING / XD;
+  // the cell's double d of a row, side k's double e of a row
+  __device__ static constexpr int cell(int d, int row) { return d / 2 * 64 + 2 * row + (d & 1); }
+  __device__ static constexpr int side(int k, int e, int row) { return SIDE + e / 2 * 128 + 2 * (2 * row + k) + (e & 1); }
+};
+template <int NV, bool VISC>
+struct PartLds {
+  using F = PartSlot<NV, VISC>;
+  alignas(16) double rec[F::NRING][F::N];
+  double ob[8][NV][32];  // the backward U + dU (update) or dU of eight steps
+  Chain<NV, 2> ch[2];    // one per sweep
+  int filled[F::NGRP];
+  int consumed, turned, ob_ready, ob_taken;
+};
+constexpr int PART_ROWS = 32;
+constexpr int PART_PROD = 3;       // producers: waves 1 .. 3 (wave 4 ends at once, see FUSED_THREADS)
+constexpr int PART_THREADS = 512;  // then the writer, the receiving and the sending wave
+
+template <int NV, bool VISC>
+__global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
+  using F = RecF<NV, VISC>;
+  using PS = PartSlot<NV, VISC>;
+  constexpr int NRING = PS::NRING, XD = PS::XD, NGRP = PS::NGRP;
+  __shared__ PartLds<NV, VISC> L;
+  const int G = a.split, bi = blockIdx.x / G, part = blockIdx.x % G;
+  const BlockDesc B = a.blocks[a.block_list[bi]];
+  if (case_frozen(B.case_id)) return;  // every part of the block returns: no part waits on another
+  const double g = a.cps[B.case_id].gamma;
+  const int ncol = B.nx - 1, nrow = B.ny - 1;
+  const int nparts = (nrow + PART_ROWS - 1) / PART_ROWS;
+  if (part >= nparts) return;  // the launch fits the level's tallest block
+  const bool has_in = part > 0, has_out = part < nparts - 1;
+  const int S = B.sk_S, R = B.sk_R, row0 = part * PART_ROWS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int q = tid; q < 2 * (int)(sizeof(Chain<NV, 2>) / 8); q += PART_THREADS) reinterpret_cast<double*>(L.ch)[q] = 0.0;
+  if (tid < NGRP) L.filled[tid] = 0;
+  if (tid == 0) {
+    L.consumed = L.ob_ready = L.ob_taken = 0;
+    L.turned = a.dir == 2 ? 1 : 0;  // a backward launch finds the forward dU in memory
+  }
+  __syncthreads();
+  if (tid < 2) {
+    if (!has_in) L.ch[tid].prog[0] = CHAIN_END;
+    if (!has_out) L.ch[tid].cons[1] = CHAIN_END;
+  }
+  __syncthreads();
+  const int npad = (S + XD - 1) / XD * XD;
+  const bool do_f = a.dir != 2, do_b = a.dir != 1;
+  const uint32_t n8 = (uint32_t)B.sk_n * 8u, n16 = 2u * n8;
+  const uint32_t bytes = (uint32_t)((2 * F::NREC + 2 * F::XP) * B.sk_n * 8);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(a.sk + B.sk_base, 0, bytes, 0x00020000);
+  const uint32_t bw = F::NREC * n8;
+  auto gr = [&](int b, int d) { return a.gring + (((int64_t)bi * (G - 1) + b) * 2 + d) * a.gstride; };
+  bool ok = true;
+  if (wave == PART_PROD + 1) return;
+  if (wave == PART_PROD + 3) {
+    if (!has_in) return;
+    if (do_f) comm_receive<NV>(L.ch[0], gr(part - 1, 0), npad, a.err, a.spin_max);
+    if (do_b) comm_receive<NV>(L.ch[1], gr(part - 1, 1), npad, a.err, a.spin_max);
+    return;
+  }
+  if (wave == PART_PROD + 4) {
+    if (!has_out) return;
+    if (do_f) comm_forward<NV>(L.ch[0], 1, gr(part, 0), npad);
+    if (do_b) comm_forward<NV>(L.ch[1], 1, gr(part, 1), npad);
+    return;
+  }
+  if (wave == PART_PROD + 2) {
+    if (do_b) write_planes<NV, PART_ROWS>(L.ob, L.ob_ready, L.ob_taken, a, B, row0, npad, lane);
+    return;
+  }
+  if (wave > 0) {
+    // ---- producer: steps 2q (lanes 0-31) and 2q + 1 (lanes 32-63) of every
+    // PART_PROD-th q
+    const double* skin = a.sk + B.sk_base;
+    const int row = lane & 31, half = lane >> 5, r = row0 + row;
+    auto produce = [&](auto fwd_c, int q0) {
+      constexpr bool fwd = decltype(fwd_c)::value;
+      RecSrc<NV> nx[2];
+      auto fetch = [&](RecSrc<NV>& n, int q, bool x) {
+        const int sn = min(2 * q + half, npad - 1);  // past the last step: clamped to it
+        load_src_sk<NV, VISC, fwd>(n, B, skin, sn - r, r);
+        if (!fwd && x) load_x<NV, VISC>(n.Res, rs, bw, n16, sn, r, S, R, ncol, nrow);
+      };
+      int q = wave - 1;
+      fetch(nx[0], q, false);
+      fetch(nx[1], q + PART_PROD, false);
+      if constexpr (!fwd) {
+        // the forward dU, from here on in memory
+        ok = wait_bounded(&L.turned, 1, a.err, a.spin_max);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        load_x<NV, VISC>(nx[0].Res, rs, bw, n16, min(2 * q + half, npad - 1), r, S, R, ncol, nrow);
+        load_x<NV, VISC>(nx[1].Res, rs, bw, n16, min(2 * (q + PART_PROD) + half, npad - 1), r, S, R, ncol, nrow);
+      }
+      auto record = [&](RecSrc<NV>& n, int q) {
+        const RecSrc<NV> in = n;
+        fetch(n, q + 2 * PART_PROD, true);
+        const int gs = q0 + 2 * q;  // the first of the two steps in the sequence of both sweeps
+        ok = wait_bounded(&L.consumed, (gs / XD + 1) * XD - NRING, a.err, a.spin_max);
+        double* rec = L.rec[(gs + half) % NRING];
+        auto SH = [&](int d) -> double& { return rec[PS::cell(d, row)]; };
+        auto SD = [&](int k, int e) -> double& { return rec[PS::side(k, e, row)]; };
+        rec_body<NV, VISC, fwd, true, PS>(SH, SD, in, g, a.alfa1);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // the slots' LDS writes done (lgkmcnt 0) before counting them
+        if (lane == 0)
+          __hip_atomic_fetch_add(&L.filled[(gs / XD) % NGRP], 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      };
+      while (2 * q < npad && ok) {
+        record(nx[0], q);
+        q += PART_PROD;
+        if (2 * q >= npad || !ok) break;
+        record(nx[1], q);
+        q += PART_PROD;
+      }
+    };
+    if (do_f) produce(std::true_type{}, 0);
+    if (do_b && ok) produce(std::false_type{}, do_f ? npad : 0);
+    return;
+  }
+  // ---- the sweep wave: lanes 2t, 2t+1 = row row0 + t; it issues first on its SIMD
+  __builtin_amdgcn_s_setprio(3);
+  const int row = lane >> 1, t = row0 + row, k = lane & 1;
+  auto load_lds = [&](Rec<NV, 1>& r, const double* rec) {
+    const double* cp = rec + 2 * row;
+    double c[PS::NSH], e[PS::NSD];
+#pragma unroll
+    for (int j = 0; j < PS::NSH / 2; j++) {
+      const D2a v = *reinterpret_cast<const D2a*>(cp + j * 64);
+      c[2 * j] = v.x;
+      c[2 * j + 1] = v.y;
+    }
+    const double* sp = rec + PS::SIDE + 2 * lane;
+#pragma unroll
+    for (int j = 0; j < PS::NSD / 2; j++) {
+      const D2a v = *reinterpret_cast<const D2a*>(sp + j * 128);
+      e[2 * j] = v.x;
+      e[2 * j + 1] = v.y;
+    }
+#pragma unroll
+    for (int m = 0; m < NV; m++) {
+      r.X[m] = c[m];
+      r.U[m] = c[PS::U + m];
+      r.F[0][m] = e[F::F + m];
+    }
+    r.yh0 = c[PS::YH0];
+    r.yl0 = c[PS::YL0];
+    r.yh4 = NV == 5 ? c[NV == 5 ? PS::YH4 : 0] : r.yh0;
+    r.yl4 = NV == 5 ? c[NV == 5 ? PS::YL4 : 0] : r.yl0;
+    r.n1[0] = e[F::N1];
+    r.n2[0] = e[F::N2];
+    r.a[0] = e[F::A];
+    r.Lc[0] = e[F::LC];
+    r.Lv[0] = VISC ? e[VISC ? F::LV : 0] : 0.0;
+  };
+  int grp = 0, round = 1;  // the group slot of the turn and its use
+  auto run_dir = [&](auto fwd_c, int gs0) {
+    constexpr bool fwd = decltype(fwd_c)::value;
+    Chain<NV, 2>& ch = L.ch[fwd ? 0 : 1];
+    Terms<NV, 2> tm = {};
+    constexpr uint32_t NOWHERE = 0x80000000u;  // out of the buffer's range: the store is dropped
+    const int ts = t < nrow && k == 0 ? t : 0x40000000;
+    uint32_t w8 = (uint32_t)((S - 1) * R + (nrow - 1 - t)) * 8u;
+    double in[NV];
+    double(*rout)[NV] = lane == 63 ? ch.ring[1] : ch.dump;
+    auto read_in = [&](int slot) {
+#pragma unroll
+      for (int m = 0; m < NV; m++) in[m] = ch.ring[0][slot][m];
+    };
+    int prog = 0, cons = 0, pv = 0;
+    auto look = [&] {
+      prog = lds_get(&ch.prog[0]);
+      cons = lds_get(&ch.cons[1]);
+    };
+    look();
+    Rec<NV, 1> rn;
+    if (ok) ok = wait_bounded(&L.filled[grp], XD * round, a.err, a.spin_max);
+    load_lds(rn, L.rec[grp * XD]);
+    for (int st = 0; st < npad; st += XD) {
+      const double* rec = L.rec[grp * XD];
+      const int grp1 = grp + 1 == NGRP ? 0 : grp + 1, round1 = grp + 1 == NGRP ? round + 1 : round;
+      const int slot0 = st & (RING - 1);
+      if (prog < st + XD - 1) wait_at_least(&ch.prog[0], st + XD - 1);
+      if (cons < st + XD - RING) wait_at_least(&ch.cons[1], st + XD - RING);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      read_in((st - 1) & (RING - 1));
+#pragma unroll
+      for (int u = 0; u < XD; u++) {
+        const int s = st + u;
+        const Rec<NV, 1> r = rn;
+        // the next step's record (see k_lusgs_fused)
+        if (u == XD - 1) {
+          if (s + 1 < npad && ok && pv < XD * round1)
+            ok = wait_bounded(&L.filled[grp1], XD * round1, a.err, a.spin_max);
+          __atomic_signal_fence(__ATOMIC_SEQ_CST);
+          load_lds(rn, L.rec[grp1 * XD]);
+        } else {
+          load_lds(rn, rec + (u + 1) * PS::N);
+        }
+        double jin[NV];
+#pragma unroll
+        for (int m = 0; m < NV; m++) jin[m] = shr1_in(in[m], tm.j[m]);
+        if (u + 1 < XD) read_in(slot0 + u);
+        Out<NV> o;
+        cell_step<NV, VISC, fwd, 2>(r, tm, jin, o, g);
+#pragma unroll
+        for (int m = 0; m < NV; m++) rout[slot0 + u][m] = tm.j[m];
+        interleave<0x100, (PS::NSH + PS::NSD) / 2, 1>();
+        if constexpr (fwd) {
+          const bool act = (uint32_t)(s - ts) < (uint32_t)ncol;
+          const uint32_t w = act ? 2 * w8 : NOWHERE, wo = act ? w8 : NOWHERE;
+          w8 -= (uint32_t)R * 8u;
+#pragma unroll
+          for (int j = 0; j < F::XP; j++) {
+            if (2 * j + 1 == NV) bstore1(o.du[2 * j], rs, wo, bw + (uint32_t)j * n16);
+            else bstore2(o.du[2 * j], o.du[2 * j + 1], rs, w, bw + (uint32_t)j * n16);
+          }
+        } else {
+          const int b8 = s & 7, ck = s >> 3;
+          if (u == 0 && b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
+#pragma unroll
+          for (int m = 0; m < NV; m++) L.ob[b8][m][row] = a.update ? o.W[m] : o.du[m];
+          if (u == XD - 1 && (b8 == 7 || s == npad - 1)) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // the chunk's writes done before it is handed over
+            lds_put(&L.ob_ready, ck + 1);
+          }
+        }
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        lds_put(&ch.prog[1], s + 1);
+        if (u == XD - 2) {
+          look();
+          pv = lds_get(&L.filled[grp1]);
+        }
+      }
+      lds_put(&ch.cons[0], st + XD - 1);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      lds_put(&L.consumed, gs0 + st + XD);
+      grp = grp1;
+      round = round1;
+    }
+  };
+  if (do_f) run_dir(std::true_type{}, 0);
+  if (do_f && do_b) {
+    // the forward sweep's stores before the producers' loads (see k_lusgs_fused)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    lds_put(&L.turned, 1);
+  }
+  if (do_b) run_dir(std::false_type{}, do_f ? npad : 0);
 }
 
 // ----------------------------------------------------------------- scatter
