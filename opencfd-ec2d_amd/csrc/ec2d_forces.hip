@@ -9,7 +9,7 @@
 //               the face-centred gradient stencil of Residual_FVM
 //               (sub_Residual.f90:301-343, 408-450), mu = Amu + Amu_t of the
 //               adjacent interior cell (that routine's wall-face rule).
-// One workgroup per case; each thread sums every 256th face in order, then a
+// One workgroup; each thread sums every 256th face in order, then a
 // fixed tree combines the threads: the result depends only on the input.
 #include "ec2d_device.h"
 
@@ -23,12 +23,13 @@ struct ForceArgs {
   const double* arena;
   PlaneMap pm;
   int viscous;
-  double* out;            // 4 per case: pressure Fx, Fy, viscous Fx, Fy
+  int c;                  // the case
+  double* out;            // pressure Fx, Fy, viscous Fx, Fy (pinned host memory)
 };
 
 __global__ __launch_bounds__(256) void k_forces(ForceArgs a) {
   __shared__ double sh[4][256];
-  const int c = blockIdx.x;
+  const int c = a.c;
   const int f0 = a.case_face0[c], f1 = a.case_face0[c + 1];
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   for (int f = f0 + threadIdx.x; f < f1; f += 256) {
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(256) void k_forces(ForceArgs a) {
     }
     __syncthreads();
   }
-  if (threadIdx.x < 4) a.out[4 * c + threadIdx.x] = sh[threadIdx.x][0];
+  if (threadIdx.x < 4) a.out[threadIdx.x] = sh[threadIdx.x][0];
 }
 
 }  // namespace ec2d

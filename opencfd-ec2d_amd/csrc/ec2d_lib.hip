@@ -19,6 +19,7 @@
 #include "ec2d_ghost.hip"
 #include "ec2d_lusgs.hip"
 #include "ec2d_sst.hip"
+#include "ec2d_transfer.hip"
 #include "ec2d_forces.hip"
 #include "ec2d_closure.hip"
 #include "ec2d_pointwise.hip"
@@ -88,7 +89,6 @@ struct DLevel {
   int64_t gstride = 0;                   // slots of one ring
   int4* dwall = nullptr;      // wall faces (block, face, i, j), cases in order
   int* dcase_wall0 = nullptr;
-  double* dforces = nullptr;  // 4 per case
   double* sk = nullptr;       // LU-SGS records (skewed, see ec2d_lusgs.hip)
   int64_t sk_max_n = 0;       // largest record field of a block (doubles)
   int64_t sk_total = 0;       // doubles of the level's record arena
@@ -113,6 +113,9 @@ struct Runtime {
   long long sko_passes = 0;    // passes whose residual wrote the hyperplane copy alone (advance_lusgs)
   bool graph_sko = false;      // the captured loop body is such a pass
   hipStream_t s = nullptr;
+  Mail* mail = nullptr;             // pinned
+  double* stage[2] = {nullptr, nullptr};  // pinned, STAGE_N doubles each (move_array)
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
   std::string err;
   int num_mesh = 1;
   int tile_rows = 4;
@@ -157,6 +160,8 @@ struct Runtime {
 };
 
 Runtime R;
+
+constexpr int STAGE_N = 1 << 17;  // 1 MiB: a 257 x 65 block of six components in one chunk
 
 // Scratch of ec2d_du_lu_sgs_2d_noalloc: the LU-SGS records (and split-sweep
 // rings) of one level in a device array that exists as soon as the library
@@ -334,7 +339,8 @@ int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false,
   return 0;
 }
 
-int reduce_norms(DLevel& L);
+// mail_case: also put that case's norms and the error words into the mailbox
+int reduce_norms(DLevel& L, int mail_case = -1);
 
 // Residual tiles of a level (64 x L.tile_rows cells), their XCD-aware launch
 // order and the per-tile norm partials.
@@ -470,13 +476,19 @@ int check_ready(bool refresh = true) {
 //   derr: the first cell with T < 1e-5 (sub_Residual.f90:143-146), status 2
 //     with the reference's message; also kept until ec2d_init_flow.
 // cold: also report derr (the caller may read the arrays of a stopped run).
+int mailed_errors(bool cold);
+
 int device_errors(bool cold) {
-  unsigned long long e = ~0ull;
-  int se = 0;
-  HIPCHK(hipMemcpyAsync(&se, R.dsweep_err, sizeof(se), hipMemcpyDeviceToHost, R.s));
-  if (cold) HIPCHK(hipMemcpyAsync(&e, R.derr, sizeof(e), hipMemcpyDeviceToHost, R.s));
+  hipLaunchKernelGGL(k_mail, dim3(1), dim3(64), 0, R.s, R.mail, (const double*)nullptr, R.derr, R.dsweep_err);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(R.s));
-  if (se) {
+  return mailed_errors(cold);
+}
+
+// the same from a mailbox that is filled and waited for
+int mailed_errors(bool cold) {
+  const unsigned long long e = cold ? R.mail->derr : ~0ull;
+  if (R.mail->sweep_err) {
     for (auto& L : R.lv)
       if (L.dgring) {
         const int64_t n = (int64_t)L.hb.size() * (L.lusgs_split - 1) * 2 * L.gstride;
@@ -694,11 +706,15 @@ int launch_residual(int level, int clip, int force = 0, int set_un = 0, double* 
 
 // Res_max / Res_rms of every case of a level from the per-tile partials of
 // the level's last residual launch.
-int reduce_norms(DLevel& L) {
+int reduce_norms(DLevel& L, int mail_case) {
   const int nv = L.o.nvar, ncase = (int)R.cases.size();
-  if (nv == 4) hipLaunchKernelGGL(k_norms<4>, dim3(ncase), dim3(256), 0, R.s, L.dpartials, L.dcase_tile0, L.dncell, L.dnorms);
-  else if (nv == 5) hipLaunchKernelGGL(k_norms<5>, dim3(ncase), dim3(256), 0, R.s, L.dpartials, L.dcase_tile0, L.dncell, L.dnorms);
-  else hipLaunchKernelGGL(k_norms<6>, dim3(ncase), dim3(256), 0, R.s, L.dpartials, L.dcase_tile0, L.dncell, L.dnorms);
+  Mail* mail = mail_case >= 0 ? R.mail : nullptr;
+#define NORMS(NV) hipLaunchKernelGGL(k_norms<NV>, dim3(ncase), dim3(256), 0, R.s, L.dpartials, L.dcase_tile0, L.dncell, \
+                                     L.dnorms, mail, mail_case, R.derr, R.dsweep_err)
+  if (nv == 4) NORMS(4);
+  else if (nv == 5) NORMS(5);
+  else NORMS(6);
+#undef NORMS
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1164,34 +1180,53 @@ void to_plane(const BlockDesc& b, double* plane, const double* src, int kind, in
   }
 }
 
-void from_plane(const BlockDesc& b, const double* plane, double* dst, int kind, int nv, int m) {
-  int nx = b.nx, ny = b.ny;
-  switch (kind) {
-    case 0:
-      for (int j = -1; j <= ny + 1; j++)
-        for (int i = -1; i <= nx + 1; i++) dst[m + nv * gi(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
-    case 5:
-      for (int j = -1; j <= ny + 1; j++)
-        for (int i = -1; i <= nx + 1; i++) dst[gi(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
-    case 1:
-      for (int j = 1; j <= ny; j++)
-        for (int i = 1; i <= nx; i++) dst[pi_(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
-    case 4:
-      for (int j = 1; j <= ny; j++)
-        for (int i = 1; i <= nx; i++) dst[m + nv * pi_(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
-    case 2:
-      for (int j = 1; j <= ny - 1; j++)
-        for (int i = 1; i <= nx - 1; i++) dst[m + nv * ci_(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
-    case 3:
-      for (int j = 0; j <= ny; j++)
-        for (int i = 0; i <= nx; i++) dst[m + nv * wi_(nx, i, j)] = plane[pidx(b, i, j)];
-      break;
+// The caller's array `host` of kind `kind` (as to_plane) with nc components
+// into (PUT) or out of the planes of a block that start at dplane.  One chunk's
+// launch runs while the host copies the other's.  A get leaves the error
+// words in the mailbox.
+template <bool PUT>
+int move_array(const BlockDesc& b, double* dplane, double* host, int kind, int nc) {
+  MoveArgs a;
+  a.b = b;
+  a.planes = dplane;
+  a.nc = nc;
+  a.lo = kind == 0 || kind == 5 ? -1 : kind == 3 ? 0 : 1;
+  const int more = kind == 0 || kind == 5 ? 3 : kind == 3 ? 1 : kind == 2 ? -1 : 0;
+  a.ni = b.nx + more;
+  const int64_t n = (int64_t)a.ni * (b.ny + more) * nc;
+  const int64_t nchunk = (n + STAGE_N - 1) / STAGE_N;
+  auto len = [&](int64_t k) { return (int)std::min<int64_t>(STAGE_N, n - k * STAGE_N); };
+  auto launch = [&](int64_t k) {
+    a.host = R.stage[k & 1];
+    a.e0 = k * STAGE_N;
+    a.n = len(k);
+    hipLaunchKernelGGL(k_move<PUT>, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, R.s, a);
+  };
+  auto copy = [&](int64_t k) {
+    double *st = R.stage[k & 1], *h = host + k * STAGE_N;
+    std::memcpy(PUT ? st : h, PUT ? h : st, sizeof(double) * (size_t)len(k));
+  };
+  if (PUT) {
+    for (int64_t k = 0; k < nchunk; k++) {
+      if (k >= 2) HIPCHK(hipEventSynchronize(R.stage_ev[k & 1]));  // chunk k - 2 has been read
+      copy(k);
+      launch(k);
+      if (k + 2 < nchunk) HIPCHK(hipEventRecord(R.stage_ev[k & 1], R.s));
+    }
+  } else {
+    for (int64_t k = 0; k < nchunk; k++) {
+      launch(k);
+      if (k + 1 < nchunk) HIPCHK(hipEventRecord(R.stage_ev[k & 1], R.s));
+      if (k == 0) continue;
+      HIPCHK(hipEventSynchronize(R.stage_ev[(k - 1) & 1]));
+      copy(k - 1);
+    }
+    hipLaunchKernelGGL(k_mail, dim3(1), dim3(64), 0, R.s, R.mail, (const double*)nullptr, R.derr, R.dsweep_err);
   }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(R.s));
+  if (!PUT) copy(nchunk - 1);
+  return 0;
 }
 
 // which -> (first plane, components, layout kind)
@@ -1371,6 +1406,11 @@ int ec2d_init(void) {
   HIPCHK(hipStreamCreateWithFlags(&R.s, hipStreamNonBlocking));
   HIPCHK(hipEventCreate(&R.ev0));
   HIPCHK(hipEventCreate(&R.ev1));
+  HIPCHK(hipHostMalloc(&R.mail, sizeof(Mail)));
+  for (int k = 0; k < 2; k++) {
+    HIPCHK(hipHostMalloc(&R.stage[k], sizeof(double) * STAGE_N));
+    HIPCHK(hipEventCreateWithFlags(&R.stage_ev[k], hipEventDisableTiming));
+  }
   R.inited = true;
   return 0;
 }
@@ -1382,7 +1422,7 @@ int ec2d_finalize(void) {
   for (auto& L : R.lv) {
     hipFree(L.arena); hipFree(L.db); hipFree(L.ds); hipFree(L.dunits); hipFree(L.dnorm); hipFree(L.dt); hipFree(L.dperm);
     hipFree(L.dcase_tile0); hipFree(L.dncell); hipFree(L.dpartials); hipFree(L.dnorms); hipFree(L.drows);
-    hipFree(L.dblocks_all); hipFree(L.sk); hipFree(L.dwall); hipFree(L.dcase_wall0); hipFree(L.dforces);
+    hipFree(L.dblocks_all); hipFree(L.sk); hipFree(L.dwall); hipFree(L.dcase_wall0);
     hipFree(L.dgring);
     hipFree(L.d_ilines); hipFree(L.d_frows);
   }
@@ -1397,6 +1437,11 @@ int ec2d_finalize(void) {
   for (auto e : R.pev) hipEventDestroy(e);
   hipEventDestroy(R.ev0);
   hipEventDestroy(R.ev1);
+  hipHostFree(R.mail);
+  for (int k = 0; k < 2; k++) {
+    hipHostFree(R.stage[k]);
+    hipEventDestroy(R.stage_ev[k]);
+  }
   hipStreamDestroy(R.s);
   R = Runtime();
   return 0;
@@ -1960,7 +2005,6 @@ int ec2d_commit(void) {
       if (!wf.empty()) HIPCHK(hipMemcpy(L.dwall, wf.data(), sizeof(int4) * wf.size(), hipMemcpyHostToDevice));
       HIPCHK(hipMalloc(&L.dcase_wall0, sizeof(int) * w0.size()));
       HIPCHK(hipMemcpy(L.dcase_wall0, w0.data(), sizeof(int) * w0.size(), hipMemcpyHostToDevice));
-      HIPCHK(hipMalloc(&L.dforces, sizeof(double) * 4 * R.cases.size()));
     }
   }
   R.committed = true;
@@ -1978,15 +2022,7 @@ int ec2d_put_array(int case_id, int nMesh, int mBlock, int which, const double* 
   int slot, nc, kind;
   if (array_map(L, which, &slot, &nc, &kind)) return fail("bad array selector");
   const BlockDesc& bd = L.hb[gb];
-  std::vector<double> plane((size_t)bd.plane);
-  for (int m = 0; m < nc; m++) {
-    double* dptr = L.arena + bd.base + (int64_t)(slot + m) * bd.plane;
-    HIPCHK(hipMemcpyAsync(plane.data(), dptr, sizeof(double) * plane.size(), hipMemcpyDeviceToHost, R.s));
-    HIPCHK(hipStreamSynchronize(R.s));
-    to_plane(bd, plane.data(), src, kind == 5 ? 5 : kind, nc, m);
-    HIPCHK(hipMemcpyAsync(dptr, plane.data(), sizeof(double) * plane.size(), hipMemcpyHostToDevice, R.s));
-    HIPCHK(hipStreamSynchronize(R.s));
-  }
+  if (move_array<true>(bd, L.arena + bd.base + (int64_t)slot * bd.plane, const_cast<double*>(src), kind, nc)) return 1;
   if (which == EC2D_U) R.clip_pending[nMesh - 1] = false;
   return 0;
 }
@@ -2001,15 +2037,9 @@ int ec2d_get_array(int case_id, int nMesh, int mBlock, int which, double* dst) {
   int slot, nc, kind;
   if (array_map(L, which, &slot, &nc, &kind)) return fail("bad array selector");
   const BlockDesc& bd = L.hb[gb];
-  std::vector<double> plane((size_t)bd.plane);
-  for (int m = 0; m < nc; m++) {
-    const double* dptr = L.arena + bd.base + (int64_t)(slot + m) * bd.plane;
-    HIPCHK(hipMemcpyAsync(plane.data(), dptr, sizeof(double) * plane.size(), hipMemcpyDeviceToHost, R.s));
-    HIPCHK(hipStreamSynchronize(R.s));
-    from_plane(bd, plane.data(), dst, kind, nc, m);
-  }
+  if (move_array<false>(bd, L.arena + bd.base + (int64_t)slot * bd.plane, dst, kind, nc)) return 1;
   // the arrays of a run stopped by T < 1e-5 stay readable; a timed-out sweep fails
-  return device_errors(false);
+  return mailed_errors(false);
 }
 
 int ec2d_init_flow(void) {
@@ -2259,11 +2289,11 @@ int ec2d_run(int n_iter) {
     }
   }
   HIPCHK(hipEventRecord(R.ev1, R.s));
-  HIPCHK(hipEventSynchronize(R.ev1));
+  const int rc_dev = device_errors(true);  // waits for the stream
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, R.ev0, R.ev1));
   R.last_run_ms = ms;
-  if (int rc = device_errors(true)) return rc;
+  if (rc_dev) return rc_dev;
   if (R.profile) {
     // mean launch time per (kernel, level); ec2d_timing reports the finest level
     double acc[40] = {0};
@@ -2822,12 +2852,12 @@ int ec2d_force_coefficients(int case_id, double* cl, double* cd, double* forces)
   a.arena = L.arena;
   a.pm = L.pm;
   a.viscous = R.cases[0].cp.If_viscous == 1;
-  a.out = L.dforces;
-  hipLaunchKernelGGL(k_forces, dim3((unsigned)R.cases.size()), dim3(256), 0, R.s, a);
+  a.c = case_id;
+  a.out = R.mail->forces;
+  hipLaunchKernelGGL(k_forces, dim3(1), dim3(256), 0, R.s, a);
   HIPCHK(hipGetLastError());
-  double F[4];
-  HIPCHK(hipMemcpyAsync(F, L.dforces + 4 * case_id, sizeof(F), hipMemcpyDeviceToHost, R.s));
   HIPCHK(hipStreamSynchronize(R.s));
+  const double* F = R.mail->forces;
   const double al = R.cases[case_id].ctl.AoA;
   const double fx = F[0] + F[2], fy = F[1] + F[3];
   if (cl) *cl = (-fx * std::sin(al) + fy * std::cos(al)) / 0.5;
@@ -2870,18 +2900,19 @@ int ec2d_res_norms(int case_id, int nMesh, double* res_max, double* res_rms) {
   if (check_ready(false)) return 1;
   if (case_id < 0 || case_id >= (int)R.cases.size() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad case / mesh");
   DLevel& L = R.lv[nMesh - 1];
-  double buf[12];
-  if (L.residual_done && reduce_norms(L)) return 1;
-  HIPCHK(hipMemcpyAsync(buf, L.dnorms + 12 * case_id, sizeof(buf), hipMemcpyDeviceToHost, R.s));
-  HIPCHK(hipStreamSynchronize(R.s));
-  int se = 0;
-  HIPCHK(hipMemcpy(&se, R.dsweep_err, sizeof(se), hipMemcpyDeviceToHost));
-  if (se) return device_errors(true);
-  for (int m = 0; m < 6; m++) {
-    res_max[m] = buf[m];
-    res_rms[m] = buf[6 + m];
+  if (L.residual_done) {
+    if (reduce_norms(L, case_id)) return 1;
+  } else {
+    hipLaunchKernelGGL(k_mail, dim3(1), dim3(64), 0, R.s, R.mail, L.dnorms + 12 * case_id, R.derr, R.dsweep_err);
+    HIPCHK(hipGetLastError());
   }
-  return device_errors(true);
+  HIPCHK(hipStreamSynchronize(R.s));
+  if (R.mail->sweep_err) return mailed_errors(true);
+  for (int m = 0; m < 6; m++) {
+    res_max[m] = R.mail->norms[m];
+    res_rms[m] = R.mail->norms[6 + m];
+  }
+  return mailed_errors(true);
 }
 
 int ec2d_time(int case_id, int nMesh, int* kstep, double* tt) {

@@ -654,30 +654,41 @@ __global__ __launch_bounds__(TX* TY) void k_residual(ResArgs a) {
 // Deterministic second stage: one workgroup per case reduces its tiles in
 // logical order into Res_max(1:NV) and Res_rms(1:NV) = sqrt(sum/Num_Cell).
 template <int NV>
-__global__ void k_norms(const double* partials, const int* case_tile0, const double* ncell, double* norms) {
-  int c = blockIdx.x;
-  int t0 = case_tile0[c], t1 = case_tile0[c + 1];
-  __shared__ double sh[256];
-  for (int k = 0; k < 2 * NV; k++) {
-    double acc = 0.0;
-    bool is_sum = k & 1;
-    for (int t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-      double v = partials[(int64_t)t * 2 * NV + k];
-      acc = is_sum ? acc + v : fmax(acc, v);
+__global__ __launch_bounds__(256) void k_norms(const double* partials, const int* case_tile0, const double* ncell,
+                                               double* norms, Mail* mail, int mail_case,
+                                               const unsigned long long* derr, const int* sweep_err) {
+  const int c = blockIdx.x, t0 = case_tile0[c], t1 = case_tile0[c + 1];
+  __shared__ double sh[2 * NV][256];
+  double acc[2 * NV] = {};
+  for (int t = t0 + threadIdx.x; t < t1; t += 256) {
+#pragma unroll
+    for (int k = 0; k < 2 * NV; k++) {
+      const double v = partials[(int64_t)t * 2 * NV + k];
+      acc[k] = k & 1 ? acc[k] + v : fmax(acc[k], v);
     }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-      if (threadIdx.x < s) sh[threadIdx.x] = is_sum ? sh[threadIdx.x] + sh[threadIdx.x + s] : fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      int m = k >> 1;
-      if (is_sum) norms[c * 12 + 6 + m] = sqrt(sh[0] / ncell[c]);
-      else norms[c * 12 + m] = sh[0];
-    }
-    __syncthreads();
   }
+#pragma unroll
+  for (int k = 0; k < 2 * NV; k++) sh[k][threadIdx.x] = acc[k];
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  for (int k = threadIdx.x >> 6; k < 2 * NV; k += 4) {
+    const bool is_sum = k & 1;
+    auto op = [&](double a, double b) { return is_sum ? a + b : fmax(a, b); };
+    double v = op(op(sh[k][lane], sh[k][lane + 128]), op(sh[k][lane + 64], sh[k][lane + 192]));
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v = op(v, __shfl_down(v, s));
+    if (lane == 0) {
+      const int m = k >> 1;
+      v = is_sum ? sqrt(v / ncell[c]) : v;
+      const int at = is_sum ? 6 + m : m;
+      norms[c * 12 + at] = v;
+      if (mail && c == mail_case) mail->norms[at] = v;
+    }
+  }
+  if (!mail || c != mail_case) return;
+  const int m = threadIdx.x % 6;
+  if (threadIdx.x < 12 && m >= NV) mail->norms[threadIdx.x] = norms[c * 12 + threadIdx.x];
+  if (threadIdx.x == 0) mail_errors(mail, derr, sweep_err);
 }
 
 }  // namespace ec2d
