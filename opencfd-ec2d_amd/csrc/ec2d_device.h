@@ -23,6 +23,7 @@ enum {
 struct CaseParams {
   double gamma, Ma, Cv, Cp, Re, Pr, Tsb, CFL, dtmax, dtmin, dt_global, P_outlet;
   double u_inf, v_inf, p_inf, Twall, vt_inf, Kt_inf, Wt_inf, p00, inv_Re;
+  double c_am, yPr, yMa;  // (1 / Re) (1 + Tsb), 1 / Pr, 1 / Ma
   int If_viscous, Iflag_local_dt, Time_Method, pad;
 };
 

@@ -46,36 +46,101 @@ struct ResArgs {
                               // 3 (4 equations, Baldwin-Lomax): mu_t of every ring cell from Amu_t as k_bl left it
 };
 
-// FIX: the level's scheme, flux and reconstruction are MUSCL3 with the van
-// Albada limiter on both face directions, Roe and the original (primitive)
-// reconstruction, as compile-time constants, so that the compiler drops the
-// other branches of every face; the launch picks it when the options match.
-template <int TX, int TY, int NV, bool VISC, bool SA, bool FIX>
-__global__ __launch_bounds__(TX* TY) void k_residual(ResArgs a) {
+// Small quotients k / D of thread indices without the 32-bit high multiply.
+template <int D, int MAX>
+__device__ __forceinline__ int div_small(int k) {
+  constexpr int M = (65536 + D - 1) / D;
+  static_assert((int64_t)(MAX - 1) * M < ((int64_t)1 << 24) && (int64_t)(MAX - 1) * (M * D - 65536) < 65536,
+                "the quotient must be exact");
+  return __mul24(k, M) >> 16;
+}
+
+// One step of the norms' tree over a wave: the sum (maximum) over lanes l and
+// l ^ 32 (D = 32) or l ^ 16, of a in the lanes with that bit clear and of b in
+// those with it set.
+template <int D, class OP>
+__device__ __forceinline__ double fold(double a, double b, OP op) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  auto swap = [](uint32_t u, uint32_t v) {
+    if constexpr (D == 32) return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+    else return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+  };
+  const auto lo = swap((uint32_t)x, (uint32_t)y), hi = swap((uint32_t)(x >> 32), (uint32_t)(y >> 32));
+  return op(__builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]),
+            __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]));
+}
+// the same over lanes l and l ^ 8, 4, 2, 1 by a lane move (after the step of 8 the
+// values repeat every 8 lanes, so that a rotation by 4 is l ^ 4)
+template <int CTRL, class OP>
+__device__ __forceinline__ double fold_dpp(double a, OP op) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0u, (uint32_t)x, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0u, (uint32_t)(x >> 32), CTRL, 0xf, 0xf, true);
+  return op(a, __builtin_bit_cast(double, (uint64_t)hi << 32 | lo));
+}
+// N values over the wave in a butterfly's order (steps of 32, 16, ..., 1): value
+// m ends in lanes 32 (m & 1) + 16 (m >> 1 & 1) .. + 15 of v[m >> 2].  The first two
+// steps fold two values each, so that ten values take 80 instructions and no
+// LDS (with a shuffle per step and value: 60 operations and 120 LDS permutes).
+template <int N, class OP>
+__device__ __forceinline__ void wave_fold(double (&v)[N], OP op) {
+  constexpr int N2 = (N + 1) / 2, N4 = (N2 + 1) / 2;
+#pragma unroll
+  for (int m = 0; m < N2; m++) v[m] = fold<32>(v[2 * m], v[2 * m + 1 < N ? 2 * m + 1 : 2 * m], op);
+#pragma unroll
+  for (int m = 0; m < N4; m++) {
+    double x = fold<16>(v[2 * m], v[2 * m + 1 < N2 ? 2 * m + 1 : 2 * m], op);
+    x = fold_dpp<0x128>(x, op);  // row_ror:8
+    x = fold_dpp<0x124>(x, op);  // row_ror:4
+    x = fold_dpp<0x4e>(x, op);   // quad_perm [2, 3, 0, 1]
+    v[m] = fold_dpp<0xb1>(x, op);  // quad_perm [1, 0, 3, 2]
+  }
+}
+
+// One workgroup per tile of TX x TY cells, one thread per cell.  Instruction
+// issue bounds large batches: of 256 SA blocks (3.1e6 cells, 32 x 8 tiles) a
+// cell takes 2510 vector instructions, which keep the units busy 71% of 0.35
+// ms; its loads and stores alone would take 0.17 ms.  (3284 instructions and
+// 0.45 ms with the general divisions, square roots and pow, 64-bit addresses per
+// access, a division of each thread index by the halo's width, LDS
+// permutes in the norms, Amu / d formed by all users of a cell, and the faces beyond
+// one per thread in a pass of their own per direction.)  Tried without gain:
+// the next phase's loads ahead of the barrier (0.38 ms), the arguments by uniform
+// loads in each phase (0.37 ms: their waits hold up the LDS), wider LDS rows.
+//   waves_per_eu: 128 registers, so that the four workgroups that a CU's LDS
+// holds do run.
+//
+// FIX: the level's scheme and reconstruction are MUSCL3 with the van Albada
+// limiter on both face directions and the original (primitive) reconstruction,
+// and the flux is Roe's (1) or AUSM (2), as compile-time constants, so that the
+// compiler drops the other branches of every face; the launch picks it when
+// the options match.
+template <int TX, int TY, int NV, bool VISC, bool SA, int FIX>
+__global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) void k_residual(ResArgs a) {
   constexpr int RW = TX + 4, RH = TY + 4, NT = TX * TY;
+  constexpr int CW = TX + 2, CH = TY + 2;  // the viscous quantities are used one cell out
   const int o_scheme = FIX ? 5 : a.o.scheme, o_gscheme = FIX ? 5 : a.o.global_scheme;
-  const int o_flux = FIX ? 4 : a.o.flux, o_recon = FIX ? 0 : a.o.recon;
-  // correctly rounded reciprocals of the constant divisors; div_rcp with
-  // them gives the reference's quotients (x / Pr, x / Pr_t, x / sigma, x / k^2)
+  const int o_flux = FIX == 1 ? 4 : FIX == 2 ? 6 : a.o.flux, o_recon = FIX ? 0 : a.o.recon;
+  // reciprocals of the constant divisors; div_y with them gives the
+  // reference's quotients (x / Pr, x / Pr_t, x / sigma, x / k^2, x / Ma)
   constexpr double yPrt = 1.0 / EC2D_PRT, ySig = 1.0 / (2.0 / 3.0), yK2 = 1.0 / (0.41 * 0.41);
-  constexpr int NFI = (TX + 1) * TY, NFJ = TX * (TY + 1);
   // viscous cases stage T and rebuild p = p00 d T from it (the staging's own
   // expression, so the same value); the cell centres of the viscous
   // gradients are read from their planes, not staged
   __shared__ double sd[RH][RW], su[RH][RW], sv[RH][RW], sp[VISC ? 1 : RH][VISC ? 1 : RW];
   __shared__ double sT[VISC ? RH : 1][VISC ? RW : 1];
-  __shared__ double sAm[VISC ? RH : 1][VISC ? RW : 1], sAt[VISC ? RH : 1][VISC ? RW : 1];
-  __shared__ double svt[SA ? RH : 1][SA ? RW : 1];
-  // face fluxes: the i-faces' (sFi, SA: sFv) and, after every cell has taken
-  // its i-face difference, the j-faces' (sFj, sFw) in the same LDS, so that
-  // four workgroups of a 32 x 8 SA tile fit on a CU
-  constexpr int NIF = 4 * TY * (TX + 1) + (SA ? 2 * TY * (TX + 1) : 1);
-  constexpr int NJF = 4 * (TY + 1) * TX + (SA ? 2 * (TY + 1) * TX : 1);
-  __shared__ double sF[NIF > NJF ? NIF : NJF];
-  auto& sFi = *reinterpret_cast<double(*)[4][TY][TX + 1]>(sF);
-  auto& sFv = *reinterpret_cast<double(*)[SA ? 2 : 1][SA ? TY : 1][SA ? TX + 1 : 1]>(sF + 4 * TY * (TX + 1));
-  auto& sFj = *reinterpret_cast<double(*)[4][TY + 1][TX]>(sF);
-  auto& sFw = *reinterpret_cast<double(*)[SA ? 2 : 1][SA ? TY + 1 : 1][SA ? TX : 1]>(sF + 4 * (TY + 1) * TX);
+  __shared__ double sAm[VISC ? CH : 1][VISC ? CW : 1], sAt[VISC ? CH : 1][VISC ? CW : 1];
+  __shared__ double svt[SA ? CH : 1][SA ? CW : 1], snu[SA ? CH : 1][SA ? CW : 1];  // snu: Amu / d
+  // face fluxes (SA: two more each): the i-faces' sFi and, after every cell
+  // has taken its i-face difference, the j-faces' rows in the same LDS, so
+  // that four workgroups of a 32 x 8 SA tile fit on a CU.  The last row of
+  // j-faces lies behind sFi: it is made together with the last column of i-faces.
+  // (Row pitch TX + 2: the cells of a hyperplane, TY lanes one row and one column
+  // apart, read different banks.)
+  constexpr int NC = SA ? 6 : 4, NIF = NC * TY * (TX + 2);
+  __shared__ double sF[NIF + NC * TX];
+  auto& sFi = *reinterpret_cast<double(*)[NC][TY][TX + 2]>(sF);
+  auto& sFj = *reinterpret_cast<double(*)[TY + 1][NC][TX]>(sF + 2 * NC * TY);
   __shared__ double sred[2 * NV][NT / 64];
 
   const int lt = a.tile_perm[blockIdx.x];
@@ -83,40 +148,49 @@ __global__ __launch_bounds__(TX* TY) void k_residual(ResArgs a) {
   const BlockDesc B = a.blocks[t.block];
   if (case_frozen(B.case_id)) return;
   const CaseParams cp = a.cps[B.case_id];
-  const double yPr = 1.0 / cp.Pr;
   const PlaneMap pm = a.pm;
   const int nx = B.nx, ny = B.ny;
   const double g = cp.gamma;
   double* base = a.arena + B.base;
-  auto PL = [&](int slot) { return base + (int64_t)slot * B.plane; };
+  // a plane's base is uniform; the place in it is a 32-bit byte offset (a plane
+  // has less than 4 GiB), shared by all planes
+  int64_t plane = B.plane;
+  auto PL = [&](int slot) { return base + (int64_t)slot * plane; };
+  // planes' addresses are formed again in each phase: kept through all of them
+  // they fill the scalar registers, and each spill takes vector instructions
+  auto fresh = [&] { asm volatile("" : "+s"(plane)); };
+  auto off = [&](int i, int j) { return ((uint32_t)(j + 1) * (uint32_t)B.P + (uint32_t)(i + 1)) * 8u; };
+  auto at = [](double* plane, uint32_t q8) -> double& {
+    return *reinterpret_cast<double*>(reinterpret_cast<char*>(plane) + q8);
+  };
   const int tid = threadIdx.x;
   const int i0 = t.i0, j0 = t.j0;
-  const double* U[NV];
-#pragma unroll
-  for (int m = 0; m < NV; m++) U[m] = PL(pm.U + m);
-  // staged values of local cell (y, x): pressure, and the cell centres
-  const double* X1p = PL(pm.x1);
-  const double* Y1p = PL(pm.y1);
-  auto SX = [&](int y, int x) { return X1p[pidx(B, i0 - 2 + x, j0 - 2 + y)]; };
-  auto SY = [&](int y, int x) { return Y1p[pidx(B, i0 - 2 + x, j0 - 2 + y)]; };
-  auto SP = [&](int y, int x) -> double {
-    if constexpr (VISC) return cp.p00 * sd[y][x] * sT[y][x];
-    else return sp[y][x];
-  };
-  auto SD = [&](int y, int x) { return sd[y][x]; };
-  auto SU = [&](int y, int x) { return su[y][x]; };
-  auto SV = [&](int y, int x) { return sv[y][x]; };
 
   // ---- 1. stage tile + halo ------------------------------------------------
-  for (int idx = tid; idx < RW * RH; idx += NT) {
-    int li = idx % RW, lj = idx / RW;
-    int i = i0 - 2 + li, j = j0 - 2 + lj;
-    if (i < -1 || i > nx + 1 || j < -1 || j > ny + 1) continue;
-    int64_t q = pidx(B, i, j);
-    double d = U[0][q];
-    double uu = U[1][q] / d;
-    double vv = U[2][q] / d;
-    double T = (U[3][q] - 0.5 * d * (uu * uu + vv * vv)) / (cp.Cv * d);
+  struct Cell {
+    int li, lj, i, j;
+    uint32_t q8;
+    double u[4 + (SA ? 1 : 0)];
+  };
+  auto load = [&](Cell& c, int idx) {
+    c.lj = div_small<RW, 2 * RW * RH>(idx);
+    c.li = idx - __mul24(c.lj, RW);
+    c.i = i0 - 2 + c.li;
+    c.j = j0 - 2 + c.lj;
+    if (c.lj >= RH || c.i < -1 || c.i > nx + 1 || c.j < -1 || c.j > ny + 1) return false;
+    c.q8 = off(c.i, c.j);
+#pragma unroll
+    for (int m = 0; m < 4 + (SA ? 1 : 0); m++) c.u[m] = at(PL(pm.U + m), c.q8);
+    return true;
+  };
+  auto stage = [&](const Cell& c) {
+    const int li = c.li, lj = c.lj, i = c.i, j = c.j;
+    const uint32_t q8 = c.q8;
+    const double d = c.u[0], u1 = c.u[1], u2 = c.u[2], u3 = c.u[3];
+    const double yd = rcp_n(d);
+    double uu = div_y(u1, d, yd);
+    double vv = div_y(u2, d, yd);
+    double T = div_n(u3 - 0.5 * d * (uu * uu + vv * vv), cp.Cv * d);
     sd[lj][li] = d;
     su[lj][li] = uu;
     sv[lj][li] = vv;
@@ -132,56 +206,68 @@ __global__ __launch_bounds__(TX* TY) void k_residual(ResArgs a) {
     }
     if constexpr (VISC) {
       sT[lj][li] = T;
+      if (li < 1 || li > RW - 2 || lj < 1 || lj > RH - 2) return;
+      const int lc = lj - 1, lr = li - 1;
       bool ring = (i >= 0 && i <= nx && j >= 0 && j <= ny);
       double am = 0.0;
-      if (ring) am = 1.0 / cp.Re * (1.0 + cp.Tsb) * sqrt(T * T * T) / (cp.Tsb + T);
+      if (ring) am = div_n(cp.c_am * sqrt_n(T * T * T), cp.Tsb + T);
       // SST: the model scaled interior Amu by Re and back (sub_turbulence_SST.f90:85, 259)
       if constexpr (NV == 6) {
         if (interior) am = (am * cp.Re) / cp.Re;
       }
-      sAm[lj][li] = am;
-      double at = 0.0;
+      sAm[lc][lr] = am;
+      double at_ = 0.0;
       if constexpr (SA) {
-        double vt = U[4][q];
+        double vt = c.u[SA ? 4 : 0];
         if (a.clip && interior && vt < 0) {
           vt = 1.0e-10;
-          const_cast<double*>(U[4])[q] = vt;
+          at(PL(pm.U + 4), q8) = vt;
         }
-        svt[lj][li] = vt;
+        svt[lc][lr] = vt;
+        snu[lc][lr] = div_y(am, d, yd);
         if (ring) {
           const double Cv1_3 = 7.1 * 7.1 * 7.1;
-          double X = d * vt / am;
+          double X = div_n(d * vt, am);
           double X3 = X * X * X;
-          double fv1 = X3 / (X3 + Cv1_3);
-          at = fv1 * d * vt;
+          double fv1 = div_n(X3, X3 + Cv1_3);
+          at_ = fv1 * d * vt;
         }
-        if (a.closure && interior && PL(pm.clo + 1)[q] != 0.0) at = PL(pm.clo)[q];
+        if (a.closure && interior && at(PL(pm.clo + 1), q8) != 0.0) at_ = at(PL(pm.clo), q8);
       }
       // SST: mu_t as the model left it (interior and wall ghosts set by
       // k_sst_res, other ghosts untouched)
-      if constexpr (NV == 6) at = ring ? PL(pm.Amu_t)[q] : 0.0;
+      if constexpr (NV == 6) at_ = ring ? at(PL(pm.Amu_t), q8) : 0.0;
       // the learned closure as the eddy-viscosity model
       if constexpr (NV == 4) {
-        if (a.closure == 2 && ring) at = PL(pm.clo)[q];
+        if (a.closure == 2 && ring) at_ = at(PL(pm.clo), q8);
         // Baldwin-Lomax (k_bl wrote every cell, ghosts included, by its own rules)
-        if (a.closure == 3 && ring) at = PL(pm.Amu_t)[q];
+        if (a.closure == 3 && ring) at_ = at(PL(pm.Amu_t), q8);
       }
-      sAt[lj][li] = at;
+      sAt[lc][lr] = at_;
     }
+  };
+  // two cells' loads at a time
+  for (int idx = tid; idx < RW * RH; idx += 2 * NT) {
+    Cell c0, c1;
+    const bool in0 = load(c0, idx), in1 = load(c1, idx + NT);
+    if (in0) stage(c0);
+    if (in1) stage(c1);
   }
   __syncthreads();
-  if (SA || (NV == 4 && VISC && a.closure == 2)) {
+  // tiles with a ghost cell of the block in the ring
+  const bool rim = i0 == 1 || j0 == 1 || i0 + TX > nx - 1 || j0 + TY > ny - 1;
+  if (rim && (SA || (NV == 4 && VISC && a.closure == 2))) {
     // Amut_boundary: wall ghost cells of layer 0 take -Amu_t of the adjacent interior cell
     // (sub_turbulence_SA.f90:200-216; the closure's mu_t follows the same rule)
-    const double* flag = PL(pm.flag);
-    for (int idx = tid; idx < RW * RH; idx += NT) {
-      int li = idx % RW, lj = idx / RW;
-      int i = i0 - 2 + li, j = j0 - 2 + lj;
+    double* flag = PL(pm.flag);
+    for (int idx = tid; idx < CW * CH; idx += NT) {
+      const int lj = div_small<CW, CW * CH>(idx), li = idx - lj * CW;
+      int i = i0 - 1 + li, j = j0 - 1 + lj;
       if (i < 0 || i > nx || j < 0 || j > ny) continue;
       bool gi = (i == 0 || i == nx) && j >= 1 && j <= ny - 1;
       bool gj = (j == 0 || j == ny) && i >= 1 && i <= nx - 1;
       if (!(gi || gj)) continue;
-      if (flag[pidx(B, i, j)] == 0.0) continue;
+      if (at(flag, off(i, j)) == 0.0) continue;
       int ii = li, jj = lj;
       if (i == 0 && gi) ii = li + 1;
       else if (gi) ii = li - 1;
@@ -194,460 +280,418 @@ __global__ __launch_bounds__(TX* TY) void k_residual(ResArgs a) {
 
   const bool fdm = B.fdm != 0;
   const int LF = 4;
-  // ---- 2a. i-faces ---------------------------------------------------------
-  for (int f = tid; f < NFI; f += NT) {
-    int fi = f % (TX + 1), fj = f / (TX + 1);
-    int i = i0 + fi, j = j0 + fj;
-    if (i > nx || j > ny - 1) continue;
+  fresh();
+  // ---- 2. the flux through one face: the i-face (jd false) between cells
+  // (i-1, j) and (i, j) or the j-face between (i, j-1) and (i, j), (i, j) the
+  // tile's cell (fi, fj).  The reference's two loops (sub_Residual.f90:193-455) are
+  // the same expressions with the directions exchanged: `back` is the step to the
+  // face's other cell, `side` the step along the face.  Of the gradients,
+  // exchanging i and j turns the sign of both factors of each product with
+  // Ds, which leaves the same bits.  The one sum whose order differs picks it.
+  auto face = [&](auto jd, int fi, int fj, double* F) {
+    const bool J = jd;
+    const int i = i0 + fi, j = j0 + fj;
+    if (i > (J ? nx - 1 : nx) || j > (J ? ny : ny - 1)) return false;
     // faces of the finite-difference interior carry no FVM flux, but the SA
     // model's own face loops (sub_turbulence_SA.f90:43-73) cover every face
     const bool skip_fvm = fdm && (i >= LF + 2 && i <= nx - LF - 1) && (j >= LF + 2 && j <= ny - LF - 1);
-    if (skip_fvm && !SA) continue;
-    int64_t q = pidx(B, i, j);
-    double si = PL(pm.si)[q], ni1 = PL(pm.ni1)[q], ni2 = PL(pm.ni2)[q];
-    int lj = fj + 2, li = fi + 2;  // local index of cell (i, j); stencil li-2 .. li+1
+    if (skip_fvm && !SA) return false;
+    const uint32_t q8 = off(i, j);
+    const double sl = at(J ? PL(pm.sj) : PL(pm.si), q8), n1 = at(J ? PL(pm.nj1) : PL(pm.ni1), q8),
+                 n2 = at(J ? PL(pm.nj2) : PL(pm.ni2), q8);
+    // of the cell centres: the difference across the face, and along it that of the
+    // mean of its two cells
+    double Nx, Ny, Cx, Cy;
+    if constexpr (VISC) {
+      const uint32_t b8 = J ? (uint32_t)B.P * 8u : 8u, s8 = J ? 8u : (uint32_t)B.P * 8u;
+      double *X = PL(pm.x1), *Y = PL(pm.y1);
+      Nx = at(X, q8) - at(X, q8 - b8);
+      Ny = at(Y, q8) - at(Y, q8 - b8);
+      Cx = (at(X, q8 + s8 - b8) + at(X, q8 + s8) - at(X, q8 - b8 - s8) - at(X, q8 - s8)) * 0.25;
+      Cy = (at(Y, q8 + s8 - b8) + at(Y, q8 + s8) - at(Y, q8 - b8 - s8) - at(Y, q8 - s8)) * 0.25;
+    }
+    const int o = __mul24(fj + 2, RW) + fi + 2, back = J ? RW : 1, side = J ? 1 : RW;
+    const double *d_ = &sd[0][0] + o, *u_ = &su[0][0] + o, *v_ = &sv[0][0] + o;
     double UL[4], UR[4];
     double F1 = 0.0, F2 = 0.0, F3 = 0.0, F4 = 0.0;
     if (!skip_fvm) {
-    if (o_recon == 0) {
-#define RECON(ARR, m)                                                                                           \
-  UL[m] = scheme_fP(ARR(lj, li - 2), ARR(lj, li - 1), ARR(lj, li), ARR(lj, li + 1), o_scheme);              \
-  UR[m] = scheme_fm(ARR(lj, li - 2), ARR(lj, li - 1), ARR(lj, li), ARR(lj, li + 1), o_scheme);
-      RECON(SD, 0) RECON(SU, 1) RECON(SV, 2) RECON(SP, 3)
-#undef RECON
-    } else {
-      double U0[4][4];
-      for (int k = 0; k < 4; k++) {
-        int64_t qk = pidx(B, i - 2 + k, j);
-        for (int m = 0; m < 4; m++) U0[k][m] = U[m][qk];
-      }
-      if (o_recon == 1) {
-        double QL[4], QR[4];
-        for (int m = 0; m < 4; m++) {
-          QL[m] = scheme_fP(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
-          QR[m] = scheme_fm(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
+      // the j-direction original-variable reconstruction uses the global
+      // scheme option, not the mesh's own (sub_Residual.f90:367)
+      if (o_recon == 0) {
+        const int sch = J ? o_gscheme : o_scheme;
+        auto recon = [&](int m, double w0, double w1, double w2, double w3) {
+          UL[m] = scheme_fP(w0, w1, w2, w3, sch);
+          UR[m] = scheme_fm(w0, w1, w2, w3, sch);
+        };
+        recon(0, d_[-2 * back], d_[-back], d_[0], d_[back]);
+        recon(1, u_[-2 * back], u_[-back], u_[0], u_[back]);
+        recon(2, v_[-2 * back], v_[-back], v_[0], v_[back]);
+        if constexpr (VISC) {
+          const double* T_ = &sT[0][0] + o;
+          auto p = [&](int k) { return cp.p00 * d_[k] * T_[k]; };
+          recon(3, p(-2 * back), p(-back), p(0), p(back));
+        } else {
+          const double* p_ = &sp[0][0] + o;
+          recon(3, p_[-2 * back], p_[-back], p_[0], p_[back]);
         }
-        cons_to_prim(QL, UL, g);
-        cons_to_prim(QR, UR, g);
       } else {
-        recon_characteristic(U0, UL, UR, g, o_scheme);
+        double U0[4][4];
+        for (int k = 0; k < 4; k++) {
+          const uint32_t qk = J ? off(i, j - 2 + k) : off(i - 2 + k, j);
+          for (int m = 0; m < 4; m++) U0[k][m] = at(PL(pm.U + m), qk);
+        }
+        if (o_recon == 1) {
+          double QL[4], QR[4];
+          for (int m = 0; m < 4; m++) {
+            QL[m] = scheme_fP(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
+            QR[m] = scheme_fm(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
+          }
+          cons_to_prim(QL, UL, g);
+          cons_to_prim(QR, UR, g);
+        } else {
+          recon_characteristic(U0, UL, UR, g, o_scheme);
+        }
       }
-    }
-    double QL[4], QR[4], F0[4];
-    QL[0] = UL[0]; QL[1] = UL[1] * ni1 + UL[2] * ni2; QL[2] = -UL[1] * ni2 + UL[2] * ni1; QL[3] = UL[3];
-    QR[0] = UR[0]; QR[1] = UR[1] * ni1 + UR[2] * ni2; QR[2] = -UR[1] * ni2 + UR[2] * ni1; QR[3] = UR[3];
-    face_flux(o_flux, QL, QR, F0, g);
-    F1 = -F0[0] * si;
-    F2 = -(F0[1] * ni1 - F0[2] * ni2) * si;
-    F3 = -(F0[1] * ni2 + F0[2] * ni1) * si;
-    F4 = -F0[3] * si;
+      double QL[4], QR[4], F0[4];
+      QL[0] = UL[0]; QL[1] = UL[1] * n1 + UL[2] * n2; QL[2] = -UL[1] * n2 + UL[2] * n1; QL[3] = UL[3];
+      QR[0] = UR[0]; QR[1] = UR[1] * n1 + UR[2] * n2; QR[2] = -UR[1] * n2 + UR[2] * n1; QR[3] = UR[3];
+      face_flux(o_flux, QL, QR, F0, g);
+      F1 = -F0[0] * sl;
+      F2 = -(F0[1] * n1 - F0[2] * n2) * sl;
+      F3 = -(F0[1] * n2 + F0[2] * n1) * sl;
+      F4 = -F0[3] * sl;
     }
     if constexpr (VISC) {
+      const int oc = __mul24(fj + 1, CW) + fi + 1, cback = J ? CW : 1, cside = J ? 1 : CW;
+      const double *Am = &sAm[0][0] + oc, *At = &sAt[0][0] + oc, *T_ = &sT[0][0] + o;
+      const int e = J ? j : i, n = J ? ny : nx;
+      double am0 = Am[0], amb = Am[-cback], at0 = At[0], atb = At[-cback];
       double Amu1, Amk1;
-      if (i == 1) {
-        Amu1 = sAm[lj][li] + sAt[lj][li];
-        Amk1 = cp.Cp * (div_rcp(sAm[lj][li], cp.Pr, yPr) + div_rcp(sAt[lj][li], EC2D_PRT, yPrt));
-      } else if (i == nx) {
-        Amu1 = sAm[lj][li - 1] + sAt[lj][li - 1];
-        Amk1 = cp.Cp * (div_rcp(sAm[lj][li - 1], cp.Pr, yPr) + div_rcp(sAt[lj][li - 1], EC2D_PRT, yPrt));
+      if (e == 1 || e == n) {  // the inner cell's alone
+        const double am = e == 1 ? am0 : amb, at_ = e == 1 ? at0 : atb;
+        Amu1 = am + at_;
+        Amk1 = cp.Cp * (div_y(am, cp.Pr, cp.yPr) + div_y(at_, EC2D_PRT, yPrt));
       } else {
-        Amu1 = (sAm[lj][li - 1] + sAm[lj][li] + sAt[lj][li - 1] + sAt[lj][li]) * 0.5;
-        Amk1 = cp.Cp * (div_rcp(sAm[lj][li - 1] + sAm[lj][li], cp.Pr, yPr) + div_rcp(sAt[lj][li - 1] + sAt[lj][li], EC2D_PRT, yPrt)) * 0.5;
+        Amu1 = ((amb + am0) + (J ? at0 : atb) + (J ? atb : at0)) * 0.5;
+        Amk1 = cp.Cp * (div_y(amb + am0, cp.Pr, cp.yPr) + div_y(atb + at0, EC2D_PRT, yPrt)) * 0.5;
       }
-      double Dix = SX(lj, li) - SX(lj, li - 1);
-      double Diy = SY(lj, li) - SY(lj, li - 1);
-      double Djx = (SX(lj + 1, li - 1) + SX(lj + 1, li) - SX(lj - 1, li - 1) - SX(lj - 1, li)) * 0.25;
-      double Djy = (SY(lj + 1, li - 1) + SY(lj + 1, li) - SY(lj - 1, li - 1) - SY(lj - 1, li)) * 0.25;
-      double Ds = 1.0 / (Dix * Djy - Djx * Diy);
-      double Diu = su[lj][li] - su[lj][li - 1];
-      double Div = sv[lj][li] - sv[lj][li - 1];
-      double DiT = sT[lj][li] - sT[lj][li - 1];
-      double Dju = (su[lj + 1][li - 1] + su[lj + 1][li] - su[lj - 1][li - 1] - su[lj - 1][li]) * 0.25;
-      double Djv = (sv[lj + 1][li - 1] + sv[lj + 1][li] - sv[lj - 1][li - 1] - sv[lj - 1][li]) * 0.25;
-      double DjT = (sT[lj + 1][li - 1] + sT[lj + 1][li] - sT[lj - 1][li - 1] - sT[lj - 1][li]) * 0.25;
-      double ux = (Diu * Djy - Dju * Diy) * Ds, vx = (Div * Djy - Djv * Diy) * Ds, Tx = (DiT * Djy - DjT * Diy) * Ds;
-      double uy = (-Diu * Djx + Dju * Dix) * Ds, vy = (-Div * Djx + Djv * Dix) * Ds, Ty = (-DiT * Djx + DjT * Dix) * Ds;
-      double u1 = (su[lj][li] + su[lj][li - 1]) * 0.5;
-      double v1 = (sv[lj][li] + sv[lj][li - 1]) * 0.5;
+      auto across = [&](const double* w) { return w[0] - w[-back]; };
+      auto along = [&](const double* w) { return (w[side - back] + w[side] - w[-back - side] - w[-side]) * 0.25; };
+      const double Ds = rcp_rn(Nx * Cy - Cx * Ny);
+      const double Nu = across(u_), Nw = across(v_), NT_ = across(T_);
+      const double Cu = along(u_), Cw = along(v_), CT = along(T_);
+      double ux = (Nu * Cy - Cu * Ny) * Ds, vx = (Nw * Cy - Cw * Ny) * Ds, Tx = (NT_ * Cy - CT * Ny) * Ds;
+      double uy = (-Nu * Cx + Cu * Nx) * Ds, vy = (-Nw * Cx + Cw * Nx) * Ds, Ty = (-NT_ * Cx + CT * Nx) * Ds;
+      double u1 = (u_[0] + u_[-back]) * 0.5;
+      double v1 = (v_[0] + v_[-back]) * 0.5;
       double t11 = ((4.0 / 3.0) * ux - (2.0 / 3.0) * vy) * Amu1;
       double t22 = ((4.0 / 3.0) * vy - (2.0 / 3.0) * ux) * Amu1;
       double t12 = (uy + vx) * Amu1;
       double E1 = u1 * t11 + v1 * t12 + Amk1 * Tx;
       double E2 = u1 * t12 + v1 * t22 + Amk1 * Ty;
       if (!skip_fvm) {
-        F2 = F2 + (t11 * ni1 + t12 * ni2) * si;
-        F3 = F3 + (t12 * ni1 + t22 * ni2) * si;
-        F4 = F4 + (E1 * ni1 + E2 * ni2) * si;
+        F2 = F2 + (t11 * n1 + t12 * n2) * sl;
+        F3 = F3 + (t12 * n1 + t22 * n2) * sl;
+        F4 = F4 + (E1 * n1 + E2 * n2) * sl;
       }
       if constexpr (SA) {
         const double Cb2 = 0.622, SA_sigma = 2.0 / 3.0;
         const double c_diff = 0.5 * (1.0 + Cb2) / SA_sigma;
-        double vn1 = su[lj][li - 1] * ni1 + sv[lj][li - 1] * ni2;
-        double vn2 = su[lj][li] * ni1 + sv[lj][li] * ni2;
-        double vfi = -0.5 * ((vn1 + fabs(vn1)) * svt[lj][li - 1] + (vn2 - fabs(vn2)) * svt[lj][li]) * si;
-        double v0 = c_diff * (svt[lj][li] + sAm[lj][li] / sd[lj][li] + svt[lj][li - 1] + sAm[lj][li - 1] / sd[lj][li - 1]);
-        double Dv = svt[lj][li] - svt[lj][li - 1];
-        double Djvt = (svt[lj + 1][li - 1] + svt[lj + 1][li] - svt[lj - 1][li - 1] - svt[lj - 1][li]) * 0.25;
-        double vtx = (Dv * Djy - Djvt * Diy) * Ds;
-        double vty = (-Dv * Djx + Djvt * Dix) * Ds;
-        sFv[0][fj][fi] = vfi + v0 * (vtx * ni1 + vty * ni2) * si;
-        sFv[1][fj][fi] = (vtx * ni1 + vty * ni2) * si;
+        const double *vt = &svt[0][0] + oc, *nu = &snu[0][0] + oc;
+        double vn1 = u_[-back] * n1 + v_[-back] * n2;
+        double vn2 = u_[0] * n1 + v_[0] * n2;
+        double vfi = -0.5 * ((vn1 + fabs(vn1)) * vt[-cback] + (vn2 - fabs(vn2)) * vt[0]) * sl;
+        double v0 = c_diff * (vt[0] + nu[0] + vt[-cback] + nu[-cback]);
+        double Nv = vt[0] - vt[-cback];
+        double Cv = (vt[cside - cback] + vt[cside] - vt[-cback - cside] - vt[-cside]) * 0.25;
+        double vtx = (Nv * Cy - Cv * Ny) * Ds;
+        double vty = (-Nv * Cx + Cv * Nx) * Ds;
+        F[4] = vfi + v0 * (vtx * n1 + vty * n2) * sl;
+        F[5] = (vtx * n1 + vty * n2) * sl;
       }
     }
-    sFi[0][fj][fi] = F1;
-    sFi[1][fj][fi] = F2;
-    sFi[2][fj][fi] = F3;
-    sFi[3][fj][fi] = F4;
+    F[0] = F1;
+    F[1] = F2;
+    F[2] = F3;
+    F[3] = F4;
+    return true;
+  };
+  auto put_i = [&](int fi, int fj, const double* F) {
+#pragma unroll
+    for (int m = 0; m < NC; m++) sFi[m][fj][fi] = F[m];
+  };
+  auto put_j = [&](int fi, int fj, const double* F) {
+#pragma unroll
+    for (int m = 0; m < NC; m++) sFj[fj][m][fi] = F[m];
+  };
+  // ---- 2a. i-faces, one per thread; then the TY of the last column and, where
+  // one wave takes both in one pass (FIX: the same code for either direction),
+  // the TX j-faces of the last row
+  constexpr bool JOIN = FIX != 0;
+  constexpr int NX = JOIN ? TY + TX : TY;
+  for (int f = tid; f < NT + NX; f += NT) {
+    double F[6] = {};
+    const int x = f - NT;
+    if constexpr (JOIN) {
+      const bool J = x >= TY;
+      const int fi = x < 0 ? f % TX : J ? x - TY : TX, fj = x < 0 ? f / TX : J ? TY : x;
+      if (!face(J, fi, fj, F)) continue;
+      if (J) put_j(fi, fj, F);
+      else put_i(fi, fj, F);
+    } else {
+      const int fi = x < 0 ? f % TX : TX, fj = x < 0 ? f / TX : x;
+      if (face(std::false_type{}, fi, fj, F)) put_i(fi, fj, F);
+    }
   }
   __syncthreads();
 
+  fresh();
   // The cell of this thread in phases 3a and 3: row-major, or, when the
   // epilogue also writes the hyperplane-order copy (sk_out), along the
   // tile's hyperplanes: TY consecutive lanes take the TY rows of one
   // hyperplane, so that the copy's stores form runs of TY positions.
   const int kd = tid / TY, cjd = tid % TY;
-  const int cell_i = a.sk_out ? (kd - cjd + TX) % TX : tid % TX;
-  const int cell_j = a.sk_out ? cjd : tid / TX;
+  const int ci = a.sk_out ? (kd - cjd + TX) % TX : tid % TX;
+  const int cj = a.sk_out ? cjd : tid / TX;
+  const int i = i0 + ci, j = j0 + cj;
+  const bool mine = i <= nx - 1 && j <= ny - 1;
+  const bool fdm_cell = fdm && (i >= LF + 1 && i <= nx - LF - 1) && (j >= LF + 1 && j <= ny - LF - 1);
 
   // ---- 3a. each cell's i-face difference (the first terms of Res, in the
   // reference's order), before the j-faces take over the LDS --------------
   double R[NV];
   double r5 = 0.0, v0c = 0.0;  // SA: the cell's v0 of sub_turbulence_SA.f90, kept for phase 3
-  {
-    const int ci = cell_i, cj = cell_j;
-    const int i = i0 + ci, j = j0 + cj;
-    if (i <= nx - 1 && j <= ny - 1) {
-      const bool fdm_cell = fdm && (i >= LF + 1 && i <= nx - LF - 1) && (j >= LF + 1 && j <= ny - LF - 1);
-      if (!fdm_cell) {
+  if (mine) {
+    if (!fdm_cell) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) R[m] = sFi[m][cj][ci + 1] - sFi[m][cj][ci];
-      }
-      if constexpr (SA) {
-        const double SA_sigma = 2.0 / 3.0, Cb2 = 0.622;
-        const int li = ci + 2, lj = cj + 2;
-        v0c = div_rcp((svt[lj][li] + sAm[lj][li] / sd[lj][li]) * Cb2, SA_sigma, ySig);
-        r5 = sFv[0][cj][ci + 1] - sFv[0][cj][ci] - v0c * (sFv[1][cj][ci + 1] - sFv[1][cj][ci]);
-      }
+      for (int m = 0; m < 4; m++) R[m] = sFi[m][cj][ci + 1] - sFi[m][cj][ci];
+    }
+    if constexpr (SA) {
+      const double SA_sigma = 2.0 / 3.0, Cb2 = 0.622;
+      v0c = div_y((svt[cj + 1][ci + 1] + snu[cj + 1][ci + 1]) * Cb2, SA_sigma, ySig);
+      r5 = sFi[NC - 2][cj][ci + 1] - sFi[NC - 2][cj][ci] - v0c * (sFi[NC - 1][cj][ci + 1] - sFi[NC - 1][cj][ci]);
     }
   }
   __syncthreads();
-  // ---- 2b. j-faces ---------------------------------------------------------
-  // NFJ = NT + 64: the 64 faces beyond one per thread go to the last wave
-  // (the first wave already takes the TY i-faces beyond one per thread), so
-  // that no wave evaluates more than three faces
-  for (int f = (tid + 64) % NT; f < NFJ; f += NT) {
-    int fi = f % TX, fj = f / TX;
-    int i = i0 + fi, j = j0 + fj;
-    if (i > nx - 1 || j > ny) continue;
-    const bool skip_fvm = fdm && (i >= LF + 2 && i <= nx - LF - 1) && (j >= LF + 2 && j <= ny - LF - 1);
-    if (skip_fvm && !SA) continue;
-    int64_t q = pidx(B, i, j);
-    double sj = PL(pm.sj)[q], nj1 = PL(pm.nj1)[q], nj2 = PL(pm.nj2)[q];
-    int lj = fj + 2, li = fi + 2;
-    double UL[4], UR[4];
-    double F1 = 0.0, F2 = 0.0, F3 = 0.0, F4 = 0.0;
-    if (!skip_fvm) {
-    if (o_recon == 0) {
-      // the j-direction original-variable reconstruction uses the global
-      // scheme option, not the mesh's own (sub_Residual.f90:367)
-#define RECON(ARR, m)                                                                                              \
-  UL[m] = scheme_fP(ARR(lj - 2, li), ARR(lj - 1, li), ARR(lj, li), ARR(lj + 1, li), o_gscheme);          \
-  UR[m] = scheme_fm(ARR(lj - 2, li), ARR(lj - 1, li), ARR(lj, li), ARR(lj + 1, li), o_gscheme);
-      RECON(SD, 0) RECON(SU, 1) RECON(SV, 2) RECON(SP, 3)
-#undef RECON
-    } else {
-      double U0[4][4];
-      for (int k = 0; k < 4; k++) {
-        int64_t qk = pidx(B, i, j - 2 + k);
-        for (int m = 0; m < 4; m++) U0[k][m] = U[m][qk];
-      }
-      if (o_recon == 1) {
-        double QL[4], QR[4];
-        for (int m = 0; m < 4; m++) {
-          QL[m] = scheme_fP(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
-          QR[m] = scheme_fm(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
-        }
-        cons_to_prim(QL, UL, g);
-        cons_to_prim(QR, UR, g);
-      } else {
-        recon_characteristic(U0, UL, UR, g, o_scheme);
-      }
-    }
-    double QL[4], QR[4], F0[4];
-    QL[0] = UL[0]; QL[1] = UL[1] * nj1 + UL[2] * nj2; QL[2] = -UL[1] * nj2 + UL[2] * nj1; QL[3] = UL[3];
-    QR[0] = UR[0]; QR[1] = UR[1] * nj1 + UR[2] * nj2; QR[2] = -UR[1] * nj2 + UR[2] * nj1; QR[3] = UR[3];
-    face_flux(o_flux, QL, QR, F0, g);
-    F1 = -F0[0] * sj;
-    F2 = -(F0[1] * nj1 - F0[2] * nj2) * sj;
-    F3 = -(F0[1] * nj2 + F0[2] * nj1) * sj;
-    F4 = -F0[3] * sj;
-    }
-    if constexpr (VISC) {
-      double Amu1, Amk1;
-      if (j == 1) {
-        Amu1 = sAm[lj][li] + sAt[lj][li];
-        Amk1 = cp.Cp * (div_rcp(sAm[lj][li], cp.Pr, yPr) + div_rcp(sAt[lj][li], EC2D_PRT, yPrt));
-      } else if (j == ny) {
-        Amu1 = sAm[lj - 1][li] + sAt[lj - 1][li];
-        Amk1 = cp.Cp * (div_rcp(sAm[lj - 1][li], cp.Pr, yPr) + div_rcp(sAt[lj - 1][li], EC2D_PRT, yPrt));
-      } else {
-        Amu1 = (sAm[lj][li] + sAm[lj - 1][li] + sAt[lj][li] + sAt[lj - 1][li]) * 0.5;
-        Amk1 = cp.Cp * (div_rcp(sAm[lj - 1][li] + sAm[lj][li], cp.Pr, yPr) + div_rcp(sAt[lj - 1][li] + sAt[lj][li], EC2D_PRT, yPrt)) * 0.5;
-      }
-      double Dix = (SX(lj - 1, li + 1) + SX(lj, li + 1) - SX(lj - 1, li - 1) - SX(lj, li - 1)) * 0.25;
-      double Diy = (SY(lj - 1, li + 1) + SY(lj, li + 1) - SY(lj - 1, li - 1) - SY(lj, li - 1)) * 0.25;
-      double Djx = SX(lj, li) - SX(lj - 1, li);
-      double Djy = SY(lj, li) - SY(lj - 1, li);
-      double Ds = 1.0 / (Dix * Djy - Djx * Diy);
-      double Diu = (su[lj - 1][li + 1] + su[lj][li + 1] - su[lj - 1][li - 1] - su[lj][li - 1]) * 0.25;
-      double Div = (sv[lj - 1][li + 1] + sv[lj][li + 1] - sv[lj - 1][li - 1] - sv[lj][li - 1]) * 0.25;
-      double DiT = (sT[lj - 1][li + 1] + sT[lj][li + 1] - sT[lj - 1][li - 1] - sT[lj][li - 1]) * 0.25;
-      double Dju = su[lj][li] - su[lj - 1][li];
-      double Djv = sv[lj][li] - sv[lj - 1][li];
-      double DjT = sT[lj][li] - sT[lj - 1][li];
-      double ux = (Diu * Djy - Dju * Diy) * Ds, vx = (Div * Djy - Djv * Diy) * Ds, Tx = (DiT * Djy - DjT * Diy) * Ds;
-      double uy = (-Diu * Djx + Dju * Dix) * Ds, vy = (-Div * Djx + Djv * Dix) * Ds, Ty = (-DiT * Djx + DjT * Dix) * Ds;
-      double t11 = ((4.0 / 3.0) * ux - (2.0 / 3.0) * vy) * Amu1;
-      double t22 = ((4.0 / 3.0) * vy - (2.0 / 3.0) * ux) * Amu1;
-      double t12 = (uy + vx) * Amu1;
-      double u1 = (su[lj][li] + su[lj - 1][li]) * 0.5;
-      double v1 = (sv[lj][li] + sv[lj - 1][li]) * 0.5;
-      double E1 = u1 * t11 + v1 * t12 + Amk1 * Tx;
-      double E2 = u1 * t12 + v1 * t22 + Amk1 * Ty;
-      if (!skip_fvm) {
-        F2 = F2 + (t11 * nj1 + t12 * nj2) * sj;
-        F3 = F3 + (t12 * nj1 + t22 * nj2) * sj;
-        F4 = F4 + (E1 * nj1 + E2 * nj2) * sj;
-      }
-      if constexpr (SA) {
-        const double Cb2 = 0.622, SA_sigma = 2.0 / 3.0;
-        const double c_diff = 0.5 * (1.0 + Cb2) / SA_sigma;
-        double vn1 = su[lj - 1][li] * nj1 + sv[lj - 1][li] * nj2;
-        double vn2 = su[lj][li] * nj1 + sv[lj][li] * nj2;
-        double vfi = -0.5 * ((vn1 + fabs(vn1)) * svt[lj - 1][li] + (vn2 - fabs(vn2)) * svt[lj][li]) * sj;
-        double v0 = c_diff * (svt[lj][li] + sAm[lj][li] / sd[lj][li] + svt[lj - 1][li] + sAm[lj - 1][li] / sd[lj - 1][li]);
-        double Div2 = (svt[lj - 1][li + 1] + svt[lj][li + 1] - svt[lj - 1][li - 1] - svt[lj][li - 1]) * 0.25;
-        double Djv2 = svt[lj][li] - svt[lj - 1][li];
-        double vtx = (Div2 * Djy - Djv2 * Diy) * Ds;
-        double vty = (-Div2 * Djx + Djv2 * Dix) * Ds;
-        sFw[0][fj][fi] = vfi + v0 * (vtx * nj1 + vty * nj2) * sj;
-        sFw[1][fj][fi] = (vtx * nj1 + vty * nj2) * sj;
-      }
-    }
-    sFj[0][fj][fi] = F1;
-    sFj[1][fj][fi] = F2;
-    sFj[2][fj][fi] = F3;
-    sFj[3][fj][fi] = F4;
+  // ---- 2b. j-faces, one per thread (and the last row, without JOIN) ---------
+  for (int f = tid; f < (JOIN ? NT : NT + TX); f += NT) {
+    double F[6] = {};
+    if (face(std::true_type{}, f % TX, f / TX, F)) put_j(f % TX, f / TX, F);
   }
   __syncthreads();
 
+  fresh();
   // ---- 3. cells ------------------------------------------------------------
   double rmax[NV], rsum[NV];
 #pragma unroll
   for (int m = 0; m < NV; m++) { rmax[m] = 0.0; rsum[m] = 0.0; }
-  {
-    int ci = cell_i, cj = cell_j;
-    int i = i0 + ci, j = j0 + cj;
-    if (i <= nx - 1 && j <= ny - 1) {
-      int64_t q = pidx(B, i, j);
-      int li = ci + 2, lj = cj + 2;
-      bool fdm_cell = fdm && (i >= LF + 1 && i <= nx - LF - 1) && (j >= LF + 1 && j <= ny - LF - 1);
-      if (!fdm_cell) {
+  if (mine) {
+    const uint32_t q8 = off(i, j), P8 = (uint32_t)B.P * 8u;
+    const int li = ci + 2, lj = cj + 2, cr = ci + 1, cc_ = cj + 1;
+    const double d = sd[lj][li];
+    if (!fdm_cell) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) R[m] = R[m] + sFj[m][cj + 1][ci] - sFj[m][cj][ci];
-      }
-      if constexpr (SA) {
-        const double SA_sigma = 2.0 / 3.0, Cv1 = 7.1, Cb1 = 0.1355, Cb2 = 0.622, SA_k = 0.41;
-        const double Cw1 = Cb1 / (SA_k * SA_k) + (1.0 + Cb2) / SA_sigma, Cw2 = 0.3, Ct3 = 1.3, Ct4 = 0.5;
-        const double Cv1_3 = Cv1 * Cv1 * Cv1, Cw3_6 = 2.0 * 2.0 * 2.0 * 2.0 * 2.0 * 2.0;
-        double vtc = svt[lj][li];
-        const double v0 = v0c;
-        r5 = r5 + sFw[0][cj + 1][ci] - sFw[0][cj][ci] - v0 * (sFw[1][cj + 1][ci] - sFw[1][cj][ci]);
-        double Dix = (SX(lj, li + 1) - SX(lj, li - 1)) * 0.5;
-        double Diy = (SY(lj, li + 1) - SY(lj, li - 1)) * 0.5;
-        double Djx = (SX(lj + 1, li) - SX(lj - 1, li)) * 0.5;
-        double Djy = (SY(lj + 1, li) - SY(lj - 1, li)) * 0.5;
-        double Ds = 1.0 / (Dix * Djy - Djx * Diy);
-        double Diu = (su[lj][li + 1] - su[lj][li - 1]) * 0.5;
-        double Div = (sv[lj][li + 1] - sv[lj][li - 1]) * 0.5;
-        double Dju = (su[lj + 1][li] - su[lj - 1][li]) * 0.5;
-        double Djv = (sv[lj + 1][li] - sv[lj - 1][li]) * 0.5;
-        double vx = (Div * Djy - Djv * Diy) * Ds;
-        double uy = (-Diu * Djx + Dju * Dix) * Ds;
-        double S = fabs(vx - uy);
-        double dwc = PL(pm.dw)[q];
-        double X = sd[lj][li] * vtc / sAm[lj][li];
-        double X3 = X * X * X;
-        double fv1 = X3 / (X3 + Cv1_3);
-        double fv2 = 1.0 - X / (1.0 + X * fv1);
-        double kd = SA_k * dwc;
-        double S1 = fmax(S + fv2 * vtc / (kd * kd), EC2D_SP(0.3) * S);
-        double r = fmin(vtc / (S1 * SA_k * SA_k * dwc * dwc), 10.0);
-        double gg = r + Cw2 * (r * r * r * r * r * r - r);
-        double fw = gg * pow((1.0 + Cw3_6) / (gg * gg * gg * gg * gg * gg + Cw3_6), 1.0 / 6.0);
-        double ft2 = Ct3 * exp(-(Ct4 * X * X));
-        double qv = vtc / dwc;
-        double Q_SA = Cb1 * (1.0 - ft2) * S1 * vtc - (Cw1 * fw - div_rcp(Cb1 * ft2, SA_k * SA_k, yK2)) * (qv * qv);
-        r5 = r5 + Q_SA * PL(pm.vol)[q];
-        R[4] = r5;
-      }
-      double Rs[NV];  // Res as stored (with the forcing function on coarse levels)
-      if (!fdm_cell) {
+      for (int m = 0; m < 4; m++) R[m] = R[m] + sFj[cj + 1][m][ci] - sFj[cj][m][ci];
+    }
+    if constexpr (SA) {
+      const double SA_sigma = 2.0 / 3.0, Cv1 = 7.1, Cb1 = 0.1355, Cb2 = 0.622, SA_k = 0.41;
+      const double Cw1 = Cb1 / (SA_k * SA_k) + (1.0 + Cb2) / SA_sigma, Cw2 = 0.3, Ct3 = 1.3, Ct4 = 0.5;
+      const double Cv1_3 = Cv1 * Cv1 * Cv1, Cw3_6 = 2.0 * 2.0 * 2.0 * 2.0 * 2.0 * 2.0;
+      double vtc = svt[cc_][cr];
+      const double v0 = v0c;
+      r5 = r5 + sFj[cj + 1][NC - 2][ci] - sFj[cj][NC - 2][ci] - v0 * (sFj[cj + 1][NC - 1][ci] - sFj[cj][NC - 1][ci]);
+      double *X1 = PL(pm.x1), *Y1 = PL(pm.y1);
+      double Dix = (at(X1, q8 + 8u) - at(X1, q8 - 8u)) * 0.5;
+      double Diy = (at(Y1, q8 + 8u) - at(Y1, q8 - 8u)) * 0.5;
+      double Djx = (at(X1, q8 + P8) - at(X1, q8 - P8)) * 0.5;
+      double Djy = (at(Y1, q8 + P8) - at(Y1, q8 - P8)) * 0.5;
+      double Ds = rcp_rn(Dix * Djy - Djx * Diy);
+      double Diu = (su[lj][li + 1] - su[lj][li - 1]) * 0.5;
+      double Div = (sv[lj][li + 1] - sv[lj][li - 1]) * 0.5;
+      double Dju = (su[lj + 1][li] - su[lj - 1][li]) * 0.5;
+      double Djv = (sv[lj + 1][li] - sv[lj - 1][li]) * 0.5;
+      double vx = (Div * Djy - Djv * Diy) * Ds;
+      double uy = (-Diu * Djx + Dju * Dix) * Ds;
+      double S = fabs(vx - uy);
+      double dwc = at(PL(pm.dw), q8);
+      double X = div_n(d * vtc, sAm[cc_][cr]);
+      double X3 = X * X * X;
+      double fv1 = div_n(X3, X3 + Cv1_3);
+      double fv2 = 1.0 - div_n(X, 1.0 + X * fv1);
+      double kd_ = SA_k * dwc;
+      double S1 = fmax(S + div_n(fv2 * vtc, kd_ * kd_), EC2D_SP(0.3) * S);
+      // S1 is zero in a uniform stream: the full division, whose infinity becomes 10
+      double r = fmin(vtc / (S1 * SA_k * SA_k * dwc * dwc), 10.0);
+      double gg = r + Cw2 * (r * r * r * r * r * r - r);
+      // r has no lower bound (nu_t < 0 inside a Runge-Kutta pass): g^6 beyond
+      // pow_sixth's range, up to overflow, takes the general functions
+      const double g6 = gg * gg * gg * gg * gg * gg;
+      double fw;
+      if (g6 < 1.0e37) fw = gg * pow_sixth(div_n(1.0 + Cw3_6, g6 + Cw3_6));
+      else fw = gg * pow((1.0 + Cw3_6) / (g6 + Cw3_6), 1.0 / 6.0);
+      double ft2 = Ct3 * exp(-(Ct4 * X * X));
+      double qv = div_n(vtc, dwc);
+      double Q_SA = Cb1 * (1.0 - ft2) * S1 * vtc - (Cw1 * fw - div_y(Cb1 * ft2, SA_k * SA_k, yK2)) * (qv * qv);
+      r5 = r5 + Q_SA * at(PL(pm.vol), q8);
+      R[4] = r5;
+    }
+    double Rs[NV];  // Res as stored (with the forcing function on coarse levels)
+    if (!fdm_cell) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-          double r = R[m];
-          if (a.force == 1) PL(pm.QF + m)[q] = PL(pm.QF + m)[q] - r;
-          else if (a.force == 2) r = r + PL(pm.QF + m)[q];
-          if (!a.sk_only) PL(pm.Res + m)[q] = r;
-          Rs[m] = r;
-        }
+      for (int m = 0; m < 4; m++) {
+        double r = R[m];
+        if (a.force == 1) at(PL(pm.QF + m), q8) = at(PL(pm.QF + m), q8) - r;
+        else if (a.force == 2) r = r + at(PL(pm.QF + m), q8);
+        if (!a.sk_only) at(PL(pm.Res + m), q8) = r;
+        Rs[m] = r;
       }
-      if constexpr (SA) {
-        if (!a.sk_only) PL(pm.Res + 4)[q] = R[4];
-      }
-      if constexpr (NV == 6) {
-        // Res(5:6) came from k_sst_res; read for the norms
-        R[4] = PL(pm.Res + 4)[q];
-        R[5] = PL(pm.Res + 5)[q];
-      }
+    }
+    if constexpr (SA) {
+      if (!a.sk_only) at(PL(pm.Res + 4), q8) = R[4];
+    }
+    if constexpr (NV == 6) {
+      // Res(5:6) came from k_sst_res; read for the norms
+      R[4] = at(PL(pm.Res + 4), q8);
+      R[5] = at(PL(pm.Res + 5), q8);
+    }
 #pragma unroll
-      for (int m = 4; m < NV; m++) Rs[m] = R[m];
-      // comput_Lvc
-      int64_t qi1 = pidx(B, i + 1, j), qj1 = pidx(B, i, j + 1);
-      double s0 = PL(pm.vol)[q];
-      double si = 0.5 * (PL(pm.si)[q] + PL(pm.si)[qi1]);
-      double ni1 = 0.5 * (PL(pm.ni1)[q] + PL(pm.ni1)[qi1]);
-      double ni2 = 0.5 * (PL(pm.ni2)[q] + PL(pm.ni2)[qi1]);
-      double sj = 0.5 * (PL(pm.sj)[q] + PL(pm.sj)[qj1]);
-      double nj1 = 0.5 * (PL(pm.nj1)[q] + PL(pm.nj1)[qj1]);
-      double nj2 = 0.5 * (PL(pm.nj2)[q] + PL(pm.nj2)[qj1]);
-      double uni = su[lj][li] * ni1 + sv[lj][li] * ni2;
-      double unj = su[lj][li] * nj1 + sv[lj][li] * nj2;
-      double T = (U[3][q] - 0.5 * sd[lj][li] * (su[lj][li] * su[lj][li] + sv[lj][li] * sv[lj][li])) / (cp.Cv * sd[lj][li]);
-      double cc = sqrt(T) / cp.Ma;
-      double Lci = (fabs(uni) + cc) * si;
-      double Lcj = (fabs(unj) + cc) * sj;
-      double Lvi = 0.0, Lvj = 0.0;
+    for (int m = 4; m < NV; m++) Rs[m] = R[m];
+    // comput_Lvc
+    const uint32_t qi1 = q8 + 8u, qj1 = q8 + P8;
+    double s0 = at(PL(pm.vol), q8);
+    double si = 0.5 * (at(PL(pm.si), q8) + at(PL(pm.si), qi1));
+    double ni1 = 0.5 * (at(PL(pm.ni1), q8) + at(PL(pm.ni1), qi1));
+    double ni2 = 0.5 * (at(PL(pm.ni2), q8) + at(PL(pm.ni2), qi1));
+    double sj = 0.5 * (at(PL(pm.sj), q8) + at(PL(pm.sj), qj1));
+    double nj1 = 0.5 * (at(PL(pm.nj1), q8) + at(PL(pm.nj1), qj1));
+    double nj2 = 0.5 * (at(PL(pm.nj2), q8) + at(PL(pm.nj2), qj1));
+    double uni = su[lj][li] * ni1 + sv[lj][li] * ni2;
+    double unj = su[lj][li] * nj1 + sv[lj][li] * nj2;
+    double T;
+    if constexpr (VISC) T = sT[lj][li];
+    else T = div_n(at(PL(pm.U + 3), q8) - 0.5 * d * (su[lj][li] * su[lj][li] + sv[lj][li] * sv[lj][li]), cp.Cv * d);
+    double cc = div_y(sqrt_n(T), cp.Ma, cp.yMa);
+    double Lci = (fabs(uni) + cc) * si;
+    double Lcj = (fabs(unj) + cc) * sj;
+    double Lvi = 0.0, Lvj = 0.0;
+    if constexpr (VISC) {
+      double tmp1 = div_n(g, d) * (div_y(sAm[cc_][cr], cp.Pr, cp.yPr) + div_y(sAt[cc_][cr], EC2D_PRT, yPrt));
+      const double y0 = rcp_n(s0);
+      Lvi = div_y(tmp1 * si * si, s0, y0);
+      Lvj = div_y(tmp1 * sj * sj, s0, y0);
+    }
+    if (!a.sk_only) {
       if constexpr (VISC) {
-        double tmp1 = g / sd[lj][li] * (div_rcp(sAm[lj][li], cp.Pr, yPr) + div_rcp(sAt[lj][li], EC2D_PRT, yPrt));
-        Lvi = tmp1 * si * si / s0;
-        Lvj = tmp1 * sj * sj / s0;
+        at(PL(pm.Lvi), q8) = Lvi;
+        at(PL(pm.Lvj), q8) = Lvj;
       }
-      if (!a.sk_only) {
-        if constexpr (VISC) {
-          PL(pm.Lvi)[q] = Lvi;
-          PL(pm.Lvj)[q] = Lvj;
-        }
-        PL(pm.Lci)[q] = Lci;
-        PL(pm.Lcj)[q] = Lcj;
-      }
-      double dt;
-      if (cp.Iflag_local_dt == 0) {
-        dt = cp.dt_global;
-      } else {
-        dt = cp.CFL * s0 / (Lci + Lcj + 1.0 * (Lvi + Lvj));
-        if (dt > cp.dtmax) dt = cp.dtmax;
-        if (dt < cp.dtmin) dt = cp.dtmin;
-      }
-      if (!a.sk_only) PL(pm.dt)[q] = dt;
-      if (a.sk_out) {
-        // logical plane k of cell (i, j) at k n + (i-1 + j-1) R + j-1 (the
-        // layout of k_lusgs_skew): U (nu_t as clipped in the staging), Res,
-        // dt, Lci, Lcj and, viscous, Lvi, Lvj
-        using I = RecIn;
-        double* so = a.sk_out + B.sk_base + (int64_t)(i - 1 + j - 1) * B.sk_R + (j - 1);
-        const int64_t n = B.sk_n;
+      at(PL(pm.Lci), q8) = Lci;
+      at(PL(pm.Lcj), q8) = Lcj;
+    }
+    double dt;
+    if (cp.Iflag_local_dt == 0) {
+      dt = cp.dt_global;
+    } else {
+      dt = div_n(cp.CFL * s0, Lci + Lcj + 1.0 * (Lvi + Lvj));
+      if (dt > cp.dtmax) dt = cp.dtmax;
+      if (dt < cp.dtmin) dt = cp.dtmin;
+    }
+    if (!a.sk_only) at(PL(pm.dt), q8) = dt;
+    if (a.sk_out) {
+      // logical plane k of cell (i, j) at k n + (i-1 + j-1) R + j-1 (the
+      // layout of k_lusgs_skew): U (nu_t as clipped in the staging), Res,
+      // dt, Lci, Lcj and, viscous, Lvi, Lvj
+      using I = RecIn;
+      const int64_t n = B.sk_n;
+      double* so = a.sk_out + B.sk_base;
+      const uint32_t p8 = (uint32_t)((i - 1 + j - 1) * B.sk_R + (j - 1)) * 8u;
 #pragma unroll
-        for (int m = 0; m < NV; m++) {
-          double u = U[m][q];
-          if constexpr (SA) {
-            if (m == 4) u = svt[lj][li];
-          }
-          so[(I::U + m) * n] = u;
-          so[(I::RES<NV> + m) * n] = Rs[m];
-        }
-        so[I::DT<NV> * n] = dt;
-        so[I::LCI<NV> * n] = Lci;
-        so[I::LCJ<NV> * n] = Lcj;
-        if constexpr (VISC) {
-          so[I::LVI<NV> * n] = Lvi;
-          so[I::LVJ<NV> * n] = Lvj;
-        }
+      for (int m = 0; m < NV; m++) {
+        double u;
+        if (m == 0) u = d;
+        else if (SA && m == 4) u = svt[cc_][cr];
+        else u = at(PL(pm.U + m), q8);
+        at(so + (I::U + m) * n, p8) = u;
+        at(so + (I::RES<NV> + m) * n, p8) = Rs[m];
       }
-      if (!fdm_cell) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) {
-          rmax[m] = fabs(R[m]);
-          rsum[m] = R[m] * R[m];
-        }
-      } else {
-#pragma unroll
-        for (int m = 4; m < NV; m++) {
-          rmax[m] = fabs(R[m]);
-          rsum[m] = R[m] * R[m];
-        }
-      }
+      at(so + I::DT<NV> * n, p8) = dt;
+      at(so + I::LCI<NV> * n, p8) = Lci;
+      at(so + I::LCJ<NV> * n, p8) = Lcj;
       if constexpr (VISC) {
-        if (a.write_visc) {
-          PL(pm.Amu)[q] = sAm[lj][li];
-          PL(pm.Amu_t)[q] = sAt[lj][li];
-        }
+        at(so + I::LVI<NV> * n, p8) = Lvi;
+        at(so + I::LVJ<NV> * n, p8) = Lvj;
+      }
+    }
+    if (!fdm_cell) {
+#pragma unroll
+      for (int m = 0; m < NV; m++) {
+        rmax[m] = fabs(R[m]);
+        rsum[m] = R[m] * R[m];
+      }
+    } else {
+#pragma unroll
+      for (int m = 4; m < NV; m++) {
+        rmax[m] = fabs(R[m]);
+        rsum[m] = R[m] * R[m];
+      }
+    }
+    if constexpr (VISC) {
+      if (a.write_visc) {
+        at(PL(pm.Amu), q8) = sAm[cc_][cr];
+        at(PL(pm.Amu_t), q8) = sAt[cc_][cr];
       }
     }
   }
-  if constexpr (VISC) {
-    // mu_t of the first ghost layer (i = 0 or nx, j = 0 or ny, corners
-    // included), as the reference's array holds it after Amut_boundary; the
-    // output files carry it.  A ring cell belongs to the tile whose interior
-    // holds the cell next to it (its indices clamped to 1..nx-1, 1..ny-1).
-    // SST and Baldwin-Lomax read these cells from the plane above: the store
-    // writes back the value read.
-    if (a.write_visc) {
-      for (int idx = tid; idx < RW * RH; idx += NT) {
-        int li = idx % RW, lj = idx / RW;
-        int i = i0 - 2 + li, j = j0 - 2 + lj;
-        if (i < 0 || i > nx || j < 0 || j > ny) continue;
-        if (i != 0 && i != nx && j != 0 && j != ny) continue;
-        int ci = min(max(i, 1), nx - 1), cj = min(max(j, 1), ny - 1);
-        if (ci < i0 || ci >= i0 + TX || cj < j0 || cj >= j0 + TY) continue;
-        PL(pm.Amu_t)[pidx(B, i, j)] = sAt[lj][li];
-      }
-    }
-  }
-  if (a.set_un) {
-    // Set_Un over the cells and the first ghost layer; a ghost cell belongs
-    // to the tile that holds the interior cell next to it
-    for (int idx = tid; idx < RW * RH; idx += NT) {
-      int li = idx % RW, lj = idx / RW;
-      int i = i0 - 2 + li, j = j0 - 2 + lj;
+  // the cells (i, j) of the block and its first ghost layer (its corners
+  // included) that belong to this tile, a ghost cell to the tile that holds
+  // the interior cell next to it (its indices clamped to 1..nx-1, 1..ny-1)
+  auto each_own = [&](auto&& f) {
+    for (int idx = tid; idx < CW * CH; idx += NT) {
+      const int lj = div_small<CW, CW * CH>(idx), li = idx - lj * CW;
+      const int i = i0 - 1 + li, j = j0 - 1 + lj;
       if (i < 0 || i > nx || j < 0 || j > ny) continue;
       int ci = min(max(i, 1), nx - 1), cj = min(max(j, 1), ny - 1);
       if (ci < i0 || ci >= i0 + TX || cj < j0 || cj >= j0 + TY) continue;
-      int64_t q = pidx(B, i, j);
-#pragma unroll
-      for (int m = 0; m < 4; m++) PL(pm.Un + m)[q] = U[m][q];
+      f(i, j, lj, li);
     }
+  };
+  if constexpr (VISC) {
+    // mu_t of the first ghost layer (i = 0 or nx, j = 0 or ny, corners
+    // included), as the reference's array holds it after Amut_boundary; the
+    // output files carry it.  SST and Baldwin-Lomax read these cells from the
+    // plane above: the store writes back the value read.
+    if (a.write_visc && rim)
+      each_own([&](int i, int j, int lj, int li) {
+        if (i == 0 || i == nx || j == 0 || j == ny) at(PL(pm.Amu_t), off(i, j)) = sAt[lj][li];
+      });
+  }
+  if (a.set_un) {
+    // Set_Un over the cells and the first ghost layer
+    each_own([&](int i, int j, int, int) {
+      const uint32_t q8 = off(i, j);
+#pragma unroll
+      for (int m = 0; m < 4; m++) at(PL(pm.Un + m), q8) = at(PL(pm.U + m), q8);
+    });
   }
   // ---- tile reduction (fixed tree: wave butterfly, then waves in order) ----
+  wave_fold(rmax, [](double x, double y) { return fmax(x, y); });
+  wave_fold(rsum, [](double x, double y) { return x + y; });
+  const int lane = tid & 63;
+  if ((lane & 15) == 0) {
+    const int m0 = (lane >> 5) + (lane >> 4 & 1) * 2;  // lanes 0, 32, 16, 48: values 0, 1, 2, 3
 #pragma unroll
-  for (int m = 0; m < NV; m++) {
-    double mx = rmax[m], sm = rsum[m];
-    for (int off = 32; off > 0; off >>= 1) {
-      mx = fmax(mx, __shfl_xor(mx, off));
-      sm = sm + __shfl_xor(sm, off);
-    }
-    if ((tid & 63) == 0) {
-      sred[2 * m][tid >> 6] = mx;
-      sred[2 * m + 1][tid >> 6] = sm;
+    for (int k = 0; k < (NV + 3) / 4; k++) {
+      if (4 * k + m0 < NV) {
+        sred[2 * (4 * k + m0)][tid >> 6] = rmax[k];
+        sred[2 * (4 * k + m0) + 1][tid >> 6] = rsum[k];
+      }
     }
   }
   __syncthreads();
   if (tid < 2 * NV) {
-    int m = tid >> 1;
     double acc = sred[tid][0];
     for (int w = 1; w < NT / 64; w++) acc = (tid & 1) ? acc + sred[tid][w] : fmax(acc, sred[tid][w]);
     a.partials[(int64_t)lt * 2 * NV + tid] = acc;
-    (void)m;
   }
 }
 
