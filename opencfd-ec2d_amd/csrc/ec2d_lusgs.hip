@@ -54,10 +54,9 @@
 // two operations instead of the eleven of a division.
 //   rho of a cell that the flow has not reached is within a few units in the
 // last place of 1, where quotients do lie next to rounding boundaries.  Its
-// three quotients take y = RN(1/rho), formed once per cell (rcp_rn), and
-// q = a*y refined twice with FMA residuals (div_rcp, Markstein): the first
-// refinement makes q faithful, the second, with y correctly rounded, returns
-// RN(a/rho).
+// three quotients share rcp_n(rho) and take the steps of a division (div_y).
+// (RN(1/rho) and two refinements of each quotient: 257 x 65 Euler cells 1.03x a
+// pass.)
 //
 // Scaling.  0.5*(DF*a + Lc*dU) is formed as DF*(0.5 a) + (0.5 Lc)*dU, and
 // -0.5*(DF*a - Lc*dU) as DF*(-0.5 a) + (0.5 Lc)*dU, with the factors in the
@@ -312,7 +311,7 @@ __device__ __forceinline__ void rec_body(SHF SH, SDF SD, const RecSrc<NV>& q, do
   };
   recip(CF::YH0, alfa);
   if constexpr (NV == 5) recip(CF::YH4, alfa + q.Lv[0] + q.Lv[1]);
-  const double y = rcp_rn(q.U[0]);
+  const double y = rcp_n(q.U[0]);
   const double p = pressure_y(q.U, y, g);
 #pragma unroll
   for (int k = 0; k < 2; k++) {
@@ -706,7 +705,7 @@ __device__ __forceinline__ void cell_step(const Rec<NV, 3 - LPC>& p, Terms<NV, L
     o.du[m] = FWD ? q : p.X[m] + q;
     o.W[m] = p.U[m] + o.du[m];
   }
-  const double y = rcp_rn(o.W[0]);
+  const double y = rcp_n(o.W[0]);
   const double pr = pressure_y(o.W, y, g);
   if constexpr (LPC == 1) {
     side_term<NV, VISC>(tm.i, p, 0, o.W, o.du, y, pr);

@@ -13,19 +13,6 @@
 
 namespace ec2d {
 
-// a / b, correctly rounded, from y = RN(1/b) (Markstein): for b > 0 and
-// normal-range operands; q is faithful after the first refinement, and a
-// faithful q refined with RN(1/b) is RN(a/b).  Five dependent operations
-// instead of the eleven of a division; used where several quotients share
-// a divisor or the divisor is a constant.
-__device__ __forceinline__ double div_rcp(double a, double b, double y) {
-  double q = a * y;
-  double r = __builtin_fma(-b, q, a);
-  q = __builtin_fma(r, y, q);
-  r = __builtin_fma(-b, q, a);
-  return __builtin_fma(r, y, q);
-}
-
 // RN(1/b) for a normal b away from the ends of the exponent range: the steps
 // of a correctly rounded division of 1 by b (two Newton steps on the hardware's
 // estimate, then the residual step) without its operand scaling, which only
@@ -397,17 +384,17 @@ __device__ __forceinline__ void face_flux(int iflux, const double* QL, const dou
 
 // comput_DFn (sub_LU_SGS.f90:111-138), F(U+dU).n - F(U).n of the Euler normal
 // flux, in pieces that two faces of a cell share: pressure_y gives the
-// cell's p from y = RN(1/density), flux_n F(U).n, dfn the difference for
+// cell's p from y = rcp_n(density), flux_n F(U).n, dfn the difference for
 // U2 = U + dU.  Every expression is the reference's, so the difference is
 // bit-identical to the undivided routine's; U(4) - 0.5*K/U(1) is one fma of
 // K/U(1), whose product with 0.5 is exact.
 __device__ __forceinline__ double pressure_y(const double* U, double y, double g) {
-  return (g - 1.0) * __builtin_fma(-0.5, div_rcp(U[1] * U[1] + U[2] * U[2], U[0], y), U[3]);
+  return (g - 1.0) * __builtin_fma(-0.5, div_y(U[1] * U[1] + U[2] * U[2], U[0], y), U[3]);
 }
 
 template <int NV>
 __device__ __forceinline__ void flux_n(double* F, const double* U, double y, double p, double n1, double n2) {
-  const double un = div_rcp(U[1] * n1 + U[2] * n2, U[0], y);
+  const double un = div_y(U[1] * n1 + U[2] * n2, U[0], y);
   F[0] = U[0] * un;
   F[1] = U[1] * un + p * n1;
   F[2] = U[2] * un + p * n2;
