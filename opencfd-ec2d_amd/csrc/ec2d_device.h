@@ -38,6 +38,7 @@ struct BlockDesc {
   int64_t plane;       // doubles per plane = (ny+3)*P
   int fdm;             // 1: finite-difference interior (LFDM = 4 edge layers stay FVM)
   int bc_off, nsub;    // subfaces in the level's subface table
+  int gph, nph;        // ghost fill: phases, their first points at gph .. gph + nph in the level's table
   int sk_S, sk_R;      // LU-SGS records: steps (ncol + nrow - 1), rows (whole sweep waves; the fused launch: nrow)
   int64_t sk_base;     // first double of the block's LU-SGS records in the level's record arena
   int64_t sk_n;        // stride of a record field in doubles: sk_S * sk_R positions + 64 trash slots
@@ -58,7 +59,18 @@ struct SubfaceDesc {
   int nb_block;        // neighbour block index in the level (0-based), or -1
   int nb_face, nb_ist, nb_iend, nb_jst, nb_jend;
   int norm_off;        // offset of per-point outward normals (farfield / symmetry), -1 if none
-  int sync;            // ghost fill: 1 = a barrier before this subface (it depends on the ones since the last)
+};
+
+// One point of a ghost fill (k_ghost): a boundary point with its two layers, or
+// one cell of a 1:1 interface.  Places are offsets in a plane.
+struct GhostPoint {
+  int type;        // SubfaceDesc::neighb; 0: interface
+  int norm;        // boundary: index of the point's normal; interface: doubles of the neighbour's plane
+  int src, dst;    // interface: the neighbour's cell and the ghost cell; boundary: of layer 1
+  union {
+    struct { int src2, dst2; };  // boundary: of layer 2
+    int64_t nb_base;             // interface: first double of the neighbour's planes
+  };
 };
 
 struct TileDesc {

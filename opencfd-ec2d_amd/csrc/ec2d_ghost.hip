@@ -9,12 +9,18 @@
 // loops include the subface end points, :325-327, :478-479), and interfaces
 // overwrite what boundary conditions wrote.  One workgroup per block keeps
 // that order with a barrier before every subface that depends on the ones
-// since the last barrier (SubfaceDesc::sync, from the host's analysis of the
-// cells each subface reads and writes), and before the corners; between
-// barriers the points of all subfaces form one index space over the
-// workgroup's threads; blocks run in parallel
-// because every stage reads only the own block's cells, except the interface
-// copy, which reads neighbour INTERIOR cells that this kernel never writes.
+// since the last barrier (from the host's analysis of the cells each subface
+// reads and writes), and before the corners; between barriers, in a phase, the
+// points of all subfaces are one index space over the workgroup's threads;
+// blocks run in parallel because every stage reads only the own block's
+// cells, except the interface copy, which reads neighbour INTERIOR cells that
+// this kernel never writes.
+//
+// Memory latency bounds it (257 x 65 cells: 640 points in two phases and the
+// corners).  The host writes every point out (GhostPoint), so that a phase is a point's
+// record, the cells it reads, its stores: 12.5 -> 7.0 us (walking the subface table,
+// a chain of dependent loads per subface and thread); 64 blocks of up to 257 x
+// 129 cells 14.6 -> 10.4 us, 256 SA blocks 23.5 -> 18.0 us.
 #include "ec2d_device.h"
 #include "ec2d_physics.h"
 
@@ -22,9 +28,8 @@ namespace ec2d {
 
 struct GhostArgs {
   const BlockDesc* blocks;
-  const int* block_list;
-  const SubfaceDesc* subs;
-  const int* units;       // per block (at bc_off): its subfaces in fill order, boundary conditions first
+  const GhostPoint* points;
+  const int* phases;      // per block (at gph): the first points of its phases, boundary conditions before interfaces
   const double* normals;  // per boundary point (n1, n2)
   const CaseParams* cps;
   double* arena;
@@ -40,27 +45,19 @@ struct GhostArgs {
 // round trip per variable and layer.  Each branch therefore loads all it
 // reads first, then computes and stores.
 template <int NV>
-__device__ void bc_point(const GhostArgs& a, const BlockDesc& B, const CaseParams& cp, const SubfaceDesc& sf, int i,
-                         int j, int pt, double* const* U) {
+__device__ void bc_point(const GhostArgs& a, const BlockDesc& B, const CaseParams& cp, const GhostPoint& gp,
+                         double* const* U) {
   const double g = cp.gamma;
-  const int face = sf.face;
-  const int type = sf.neighb;
+  const int type = gp.type;
+  const int q1[EC2D_LAP] = {gp.src, gp.src2}, q2[EC2D_LAP] = {gp.dst, gp.dst2};
   if (type == -10 || type == -30) {  // wall (sub_boundary.f90:306-386), symmetry / slip wall (:391-451)
-    int64_t q1[EC2D_LAP], q2[EC2D_LAP];
     double v[EC2D_LAP][NV], dwv[EC2D_LAP];
 #pragma unroll
-    for (int k = 1; k <= EC2D_LAP; k++) {
-      int i1, j1, i2, j2;
-      if (face == 1) { i1 = i + k - 1; j1 = j; i2 = i - k; j2 = j; }
-      else if (face == 2) { i1 = i; j1 = j + k - 1; i2 = i; j2 = j - k; }
-      else if (face == 3) { i1 = i - k; j1 = j; i2 = i + k - 1; j2 = j; }
-      else { i1 = i; j1 = j - k; i2 = i; j2 = j + k - 1; }
-      q1[k - 1] = pidx(B, i1, j1);
-      q2[k - 1] = pidx(B, i2, j2);
+    for (int k = 0; k < EC2D_LAP; k++) {
 #pragma unroll
-      for (int m = 0; m < NV; m++) v[k - 1][m] = U[m][q1[k - 1]];
+      for (int m = 0; m < NV; m++) v[k][m] = U[m][q1[k]];
       if constexpr (NV == 6) {
-        if (type == -10) dwv[k - 1] = (a.arena + B.base + (int64_t)a.pm.dw * B.plane)[q1[k - 1]];
+        if (type == -10) dwv[k] = (a.arena + B.base + (int64_t)a.pm.dw * B.plane)[q1[k]];
       }
     }
     if (type == -10) {
@@ -101,7 +98,7 @@ __device__ void bc_point(const GhostArgs& a, const BlockDesc& B, const CaseParam
         }
       }
     } else {
-      double n1 = a.normals[2 * (sf.norm_off + pt)], n2 = a.normals[2 * (sf.norm_off + pt) + 1];
+      double n1 = a.normals[2 * gp.norm], n2 = a.normals[2 * gp.norm + 1];
 #pragma unroll
       for (int k = 0; k < EC2D_LAP; k++) {
         const double* w = v[k];
@@ -115,64 +112,55 @@ __device__ void bc_point(const GhostArgs& a, const BlockDesc& B, const CaseParam
       }
     }
   } else {  // far field / inlet / outlet, sub_boundary.f90:457-581
-    int i1 = i, j1 = j;
-    if (face == 3) i1 = i - 1;
-    else if (face == 4) j1 = j - 1;
-    int64_t q1 = pidx(B, i1, j1);
     double w[NV];
 #pragma unroll
-    for (int m = 0; m < NV; m++) w[m] = U[m][q1];
-    double n1 = a.normals[2 * (sf.norm_off + pt)], n2 = a.normals[2 * (sf.norm_off + pt) + 1];
+    for (int m = 0; m < NV; m++) w[m] = U[m][q1[0]];
+    double n1 = a.normals[2 * gp.norm], n2 = a.normals[2 * gp.norm + 1];
     double d1 = w[0], u1 = w[1] / d1, v1 = w[2] / d1;
     double p1 = (w[3] - 0.5 * d1 * (u1 * u1 + v1 * v1)) * (g - 1.0);
     double c1 = sqrt(g * p1 / d1);
     double Ma_n = (u1 * n1 + v1 * n2) / c1;
     const double d_inf = 1.0;
-    for (int k = 1; k <= EC2D_LAP; k++) {
-      int i2 = i, j2 = j;
-      if (face == 1) i2 = i - k;
-      else if (face == 2) j2 = j - k;
-      else if (face == 3) i2 = i + k - 1;
-      else j2 = j + k - 1;
-      int64_t q2 = pidx(B, i2, j2);
+#pragma unroll
+    for (int k = 0; k < EC2D_LAP; k++) {
       if (type == -50 || (type == -20 && Ma_n >= 0.0)) {
         if (Ma_n > 1.0 || cp.P_outlet < 0 || type == -20) {
 #pragma unroll
-          for (int m = 0; m < NV; m++) U[m][q2] = w[m];
+          for (int m = 0; m < NV; m++) U[m][q2[k]] = w[m];
         } else {
           double pb = cp.P_outlet;
           double db = d1 + (cp.P_outlet - p1) / (c1 * c1);
           double ub = u1 + (p1 - cp.P_outlet) / (d1 * c1) * n1;
           double vb = v1 + (p1 - cp.P_outlet) / (d1 * c1) * n2;
           double p2 = 2.0 * pb - p1, d2 = 2.0 * db - d1, u2 = 2.0 * ub - u1, v2 = 2.0 * vb - v1;
-          U[0][q2] = d2;
-          U[1][q2] = d2 * u2;
-          U[2][q2] = d2 * v2;
-          U[3][q2] = p2 / (g - 1.0) + 0.5 * d2 * (u2 * u2 + v2 * v2);
+          U[0][q2[k]] = d2;
+          U[1][q2[k]] = d2 * u2;
+          U[2][q2[k]] = d2 * v2;
+          U[3][q2[k]] = p2 / (g - 1.0) + 0.5 * d2 * (u2 * u2 + v2 * v2);
 #pragma unroll
-          for (int m = 4; m < NV; m++) U[m][q2] = w[m];
+          for (int m = 4; m < NV; m++) U[m][q2[k]] = w[m];
         }
       } else {
         if (cp.P_outlet < 0 || Ma_n <= -1.0) {
-          U[0][q2] = d_inf;
-          U[1][q2] = d_inf * cp.u_inf;
-          U[2][q2] = d_inf * cp.v_inf;
-          U[3][q2] = cp.p_inf / (g - 1.0) + 0.5 * d_inf * (cp.u_inf * cp.u_inf + cp.v_inf * cp.v_inf);
+          U[0][q2[k]] = d_inf;
+          U[1][q2[k]] = d_inf * cp.u_inf;
+          U[2][q2[k]] = d_inf * cp.v_inf;
+          U[3][q2[k]] = cp.p_inf / (g - 1.0) + 0.5 * d_inf * (cp.u_inf * cp.u_inf + cp.v_inf * cp.v_inf);
         } else {
           double pb = 0.5 * (p1 + cp.p_inf - d1 * c1 * ((cp.u_inf - u1) * n1 + (cp.v_inf - v1) * n2));
           double db = d_inf + (pb - cp.p_inf) / (c1 * c1);
           double ub = cp.u_inf - (cp.p_inf - pb) / (d1 * c1) * n1;
           double vb = cp.v_inf - (cp.p_inf - pb) / (d1 * c1) * n2;
           double p2 = 2.0 * pb - p1, d2 = 2.0 * db - d1, u2 = 2.0 * ub - u1, v2 = 2.0 * vb - v1;
-          U[0][q2] = d2;
-          U[1][q2] = d2 * u2;
-          U[2][q2] = d2 * v2;
-          U[3][q2] = p2 / (g - 1.0) + 0.5 * d2 * (u2 * u2 + v2 * v2);
+          U[0][q2[k]] = d2;
+          U[1][q2[k]] = d2 * u2;
+          U[2][q2[k]] = d2 * v2;
+          U[3][q2[k]] = p2 / (g - 1.0) + 0.5 * d2 * (u2 * u2 + v2 * v2);
         }
-        if constexpr (NV == 5) U[4][q2] = cp.vt_inf / cp.Re;
+        if constexpr (NV == 5) U[4][q2[k]] = cp.vt_inf / cp.Re;
         if constexpr (NV == 6) {
-          U[4][q2] = d_inf * cp.Kt_inf;
-          U[5][q2] = d_inf * cp.Wt_inf;
+          U[4][q2[k]] = d_inf * cp.Kt_inf;
+          U[5][q2[k]] = d_inf * cp.Wt_inf;
         }
       }
     }
@@ -198,71 +186,30 @@ __device__ __forceinline__ void corner(double* const* U, int64_t q1, int64_t q2,
 
 template <int NV>
 __global__ __launch_bounds__(1024) void k_ghost(GhostArgs a) {
-  const int bidx = a.block_list[blockIdx.x];
-  const BlockDesc B = a.blocks[bidx];
+  const BlockDesc B = a.blocks[blockIdx.x];
   if (case_frozen(B.case_id)) return;
   const CaseParams cp = a.cps[B.case_id];
   double* U[NV];
 #pragma unroll
   for (int m = 0; m < NV; m++) U[m] = a.arena + B.base + (int64_t)(a.pm.U + m) * B.plane;
   const int tid = threadIdx.x;
-  // Phases: a unit with sync = 1 starts a new one.  The points of all units
-  // of a phase are independent of each other, so the threads take them as
-  // one index space (one memory round trip per phase, not per subface).
-  auto on = [&](const SubfaceDesc& sf) { return sf.neighb < 0 ? a.do_bc != 0 : a.do_exchange != 0; };
-  auto npoints = [&](const SubfaceDesc& sf) {
-    if (!on(sf)) return 0;
-    if (sf.neighb < 0) return (sf.iend - sf.ist + 1) * (sf.jend - sf.jst + 1);
-    return (sf.iend - sf.ist + sf.jend - sf.jst) * EC2D_LAP;
-  };
-  const int* un = a.units + B.bc_off;
-  for (int u0 = 0; u0 < B.nsub;) {
-    int u1 = u0 + 1;
-    while (u1 < B.nsub && !a.subs[un[u1]].sync) u1++;
-    int total = 0;
-    for (int u = u0; u < u1; u++) total += npoints(a.subs[un[u]]);
-    for (int p = tid; p < total; p += blockDim.x) {
-      int u = u0, lp = p;
-      for (;;) {
-        const int np = npoints(a.subs[un[u]]);
-        if (lp < np) break;
-        lp -= np;
-        u++;
-      }
-      const SubfaceDesc sf = a.subs[un[u]];
-      if (sf.neighb < 0) {
-        const int ni = sf.iend - sf.ist + 1;
-        bc_point<NV>(a, B, cp, sf, sf.ist + lp % ni, sf.jst + lp / ni, lp, U);
-      } else {
-        const BlockDesc B1 = a.blocks[sf.nb_block];
-        const double* U1[NV];
-#pragma unroll
-        for (int m = 0; m < NV; m++) U1[m] = a.arena + B1.base + (int64_t)(a.pm.U + m) * B1.plane;
-        const int n1 = sf.iend - sf.ist + sf.jend - sf.jst;
-        const int kk = lp % n1 + 1, l = lp / n1 + 1;  // cell along the face (1..n1), layer (1..LAP)
-        const int k1 = (sf.orient == 2) ? kk : n1 + 1 - kk;
-        // source cell: slot (k1, l) of the neighbour's buffer (sub_boundary.f90:76-108)
-        int si_, sj_;
-        if (sf.nb_face == 1) { si_ = sf.nb_ist + l - 1; sj_ = sf.nb_jst + k1 - 1; }
-        else if (sf.nb_face == 2) { si_ = sf.nb_ist + k1 - 1; sj_ = sf.nb_jst + l - 1; }
-        else if (sf.nb_face == 3) { si_ = sf.nb_iend - EC2D_LAP - 1 + l; sj_ = sf.nb_jst + k1 - 1; }
-        else { si_ = sf.nb_ist + k1 - 1; sj_ = sf.nb_jend - EC2D_LAP - 1 + l; }
-        // destination ghost cell (:118-135)
-        int di, dj;
-        if (sf.face == 1) { di = sf.ist - EC2D_LAP - 1 + l; dj = sf.jst + kk - 1; }
-        else if (sf.face == 2) { di = sf.ist + kk - 1; dj = sf.jst - EC2D_LAP - 1 + l; }
-        else if (sf.face == 3) { di = sf.iend + l - 1; dj = sf.jst + kk - 1; }
-        else { di = sf.ist + kk - 1; dj = sf.jend + l - 1; }
-        const int64_t qs = pidx(B1, si_, sj_), qd = pidx(B, di, dj);
+  for (int f = 0; f < B.nph; f++) {
+    const int p1 = a.phases[B.gph + f + 1];
+    for (int p = a.phases[B.gph + f] + tid; p < p1; p += 1024) {
+      const GhostPoint gp = a.points[p];
+      if (gp.type < 0) {
+        if (a.do_bc) bc_point<NV>(a, B, cp, gp, U);
+      } else if (a.do_exchange) {
+        // the source cell is slot (k1, l) of the neighbour's buffer (sub_boundary.f90:76-108)
+        const double* U1 = a.arena + gp.nb_base + (int64_t)a.pm.U * gp.norm;
         double w[NV];
 #pragma unroll
-        for (int m = 0; m < NV; m++) w[m] = U1[m][qs];
+        for (int m = 0; m < NV; m++) w[m] = U1[(int64_t)m * gp.norm + gp.src];
 #pragma unroll
-        for (int m = 0; m < NV; m++) U[m][qd] = w[m];
+        for (int m = 0; m < NV; m++) U[m][gp.dst] = w[m];
       }
     }
-    u0 = u1;
-    if (u0 < B.nsub) __syncthreads();
+    if (f + 1 < B.nph) __syncthreads();
   }
   if (a.do_exchange) {
     __syncthreads();

@@ -58,7 +58,8 @@ struct DLevel {
   std::vector<int> blk_case, blk_local;
   BlockDesc* db = nullptr;
   SubfaceDesc* ds = nullptr;
-  int* dunits = nullptr;  // ghost fill order per block: subface indices, boundary conditions first
+  GhostPoint* dgpts = nullptr;  // ghost fill: points and phases (ghost_phases)
+  int* dgph = nullptr;
   int bl_walls = 0, bl_lines = 0;  // Baldwin-Lomax: most wall subfaces of a block, most lines of one
   int64_t max_plane = 0;           // largest block plane (doubles)
   double* dnorm = nullptr;
@@ -186,72 +187,97 @@ int fail(const std::string& m) {
   } while (0)
 
 // Ghost-fill phases of one block (k_ghost): the fill runs the boundary
-// subfaces in file order, then the interfaces, then the corners; units gets
-// that order (level subface indices).  A subface
+// subfaces in file order, then the interfaces, then the corners.  A subface
 // joins the running phase (no barrier) when it writes no cell that the phase
 // read or wrote and reads no cell that the phase wrote; otherwise it starts a
-// new phase (sync = 1).  The cell sets follow bc_point and the interface copy
-// in ec2d_ghost.hip exactly; interfaces read neighbour interior cells, which
-// no fill writes, so only their writes count.  The corners always follow a
-// barrier.
-void ghost_phases(const BlockDesc& B, SubfaceDesc* s, int* units) {
+// new phase.  Interfaces read neighbour interior cells, which no fill writes,
+// so only their writes count.  The corners always follow a barrier.  Appends the
+// points to pts and the phases' first points, and the end, to ph.
+void ghost_phases(BlockDesc& B, const std::vector<BlockDesc>& hb, const SubfaceDesc* s, std::vector<GhostPoint>& pts,
+                  std::vector<int>& ph) {
   std::vector<int> wph((size_t)B.plane, 0), rph((size_t)B.plane, 0);
-  int ph = 1;
-  std::vector<int64_t> rd, wr;
-  auto q = [&](int i, int j) { return pidx(B, i, j); };
-  int nu = 0;
-  auto join = [&](SubfaceDesc& sf) {
-    units[nu++] = B.bc_off + (int)(&sf - s);
+  int cur = 1;
+  B.gph = (int)ph.size();
+  ph.push_back((int)pts.size());
+  auto q = [&](int i, int j) { return (int)pidx(B, i, j); };
+  // the subface whose points begin at pts[p0]
+  auto join = [&](size_t p0) {
     bool dep = false;
-    for (int64_t c : wr) dep = dep || c < 0 || c >= B.plane || wph[c] == ph || rph[c] == ph;
-    for (int64_t c : rd) dep = dep || c < 0 || c >= B.plane || wph[c] == ph;
-    sf.sync = dep ? 1 : 0;
-    if (dep) ph++;
-    for (int64_t c : wr) if (c >= 0 && c < B.plane) wph[c] = ph;
-    for (int64_t c : rd) if (c >= 0 && c < B.plane) rph[c] = ph;
+    auto each = [&](auto&& read, auto&& write) {
+      for (size_t k = p0; k < pts.size(); k++) {
+        const GhostPoint& p = pts[k];
+        write(p.dst);
+        if (p.type < 0) {
+          read(p.src);
+          write(p.dst2);
+          if (p.type == -10 || p.type == -30) read(p.src2);
+        }
+      }
+    };
+    auto out = [&](int c) { return c < 0 || c >= B.plane; };
+    each([&](int c) { dep = dep || out(c) || wph[c] == cur; },
+         [&](int c) { dep = dep || out(c) || wph[c] == cur || rph[c] == cur; });
+    if (dep) {
+      cur++;
+      if (p0 > (size_t)ph.back()) ph.push_back((int)p0);
+    }
+    each([&](int c) { if (!out(c)) rph[c] = cur; }, [&](int c) { if (!out(c)) wph[c] = cur; });
   };
   for (int k = 0; k < B.nsub; k++) {
-    SubfaceDesc& sf = s[k];
+    const SubfaceDesc& sf = s[k];
     if (sf.neighb >= 0) continue;
-    rd.clear();
-    wr.clear();
+    const size_t p0 = pts.size();
+    int pt = 0;
     for (int j = sf.jst; j <= sf.jend; j++)
       for (int i = sf.ist; i <= sf.iend; i++) {
         const int f = sf.face;
+        GhostPoint p{};
+        p.type = sf.neighb;
+        p.norm = sf.norm_off + pt++;
         if (sf.neighb == -10 || sf.neighb == -30) {
-          for (int l = 1; l <= EC2D_LAP; l++) {
-            if (f == 1) { rd.push_back(q(i + l - 1, j)); wr.push_back(q(i - l, j)); }
-            else if (f == 2) { rd.push_back(q(i, j + l - 1)); wr.push_back(q(i, j - l)); }
-            else if (f == 3) { rd.push_back(q(i - l, j)); wr.push_back(q(i + l - 1, j)); }
-            else { rd.push_back(q(i, j - l)); wr.push_back(q(i, j + l - 1)); }
-          }
+          int* qs[EC2D_LAP] = {&p.src, &p.src2};
+          for (int l = 1; l <= EC2D_LAP; l++)
+            *qs[l - 1] = f == 1 ? q(i + l - 1, j) : f == 2 ? q(i, j + l - 1) : f == 3 ? q(i - l, j) : q(i, j - l);
         } else {
-          rd.push_back(q(f == 3 ? i - 1 : i, f == 4 ? j - 1 : j));
-          for (int l = 1; l <= EC2D_LAP; l++) {
-            if (f == 1) wr.push_back(q(i - l, j));
-            else if (f == 2) wr.push_back(q(i, j - l));
-            else if (f == 3) wr.push_back(q(i + l - 1, j));
-            else wr.push_back(q(i, j + l - 1));
-          }
+          p.src = q(f == 3 ? i - 1 : i, f == 4 ? j - 1 : j);
         }
+        int* qd[EC2D_LAP] = {&p.dst, &p.dst2};
+        for (int l = 1; l <= EC2D_LAP; l++)
+          *qd[l - 1] = f == 1 ? q(i - l, j) : f == 2 ? q(i, j - l) : f == 3 ? q(i + l - 1, j) : q(i, j + l - 1);
+        pts.push_back(p);
       }
-    join(sf);
+    join(p0);
   }
   for (int k = 0; k < B.nsub; k++) {
-    SubfaceDesc& sf = s[k];
+    const SubfaceDesc& sf = s[k];
     if (sf.neighb < 0) continue;
-    rd.clear();
-    wr.clear();
+    const size_t p0 = pts.size();
+    const BlockDesc& N = hb[sf.nb_block];
     const int n1 = sf.iend - sf.ist + sf.jend - sf.jst;
     for (int l = 1; l <= EC2D_LAP; l++)
-      for (int kk = 1; kk <= n1; kk++) {
-        if (sf.face == 1) wr.push_back(q(sf.ist - EC2D_LAP - 1 + l, sf.jst + kk - 1));
-        else if (sf.face == 2) wr.push_back(q(sf.ist + kk - 1, sf.jst - EC2D_LAP - 1 + l));
-        else if (sf.face == 3) wr.push_back(q(sf.iend + l - 1, sf.jst + kk - 1));
-        else wr.push_back(q(sf.ist + kk - 1, sf.jend + l - 1));
+      for (int kk = 1; kk <= n1; kk++) {  // cell along the face (1..n1), layer (1..LAP)
+        GhostPoint p{};
+        p.norm = (int)N.plane;
+        p.nb_base = N.base;
+        const int k1 = sf.orient == 2 ? kk : n1 + 1 - kk;
+        // source cell: slot (k1, l) of the neighbour's buffer (sub_boundary.f90:76-108)
+        int si, sj;
+        if (sf.nb_face == 1) { si = sf.nb_ist + l - 1; sj = sf.nb_jst + k1 - 1; }
+        else if (sf.nb_face == 2) { si = sf.nb_ist + k1 - 1; sj = sf.nb_jst + l - 1; }
+        else if (sf.nb_face == 3) { si = sf.nb_iend - EC2D_LAP - 1 + l; sj = sf.nb_jst + k1 - 1; }
+        else { si = sf.nb_ist + k1 - 1; sj = sf.nb_jend - EC2D_LAP - 1 + l; }
+        p.src = (int)pidx(N, si, sj);
+        // destination ghost cell (:118-135)
+        if (sf.face == 1) p.dst = q(sf.ist - EC2D_LAP - 1 + l, sf.jst + kk - 1);
+        else if (sf.face == 2) p.dst = q(sf.ist + kk - 1, sf.jst - EC2D_LAP - 1 + l);
+        else if (sf.face == 3) p.dst = q(sf.iend + l - 1, sf.jst + kk - 1);
+        else p.dst = q(sf.ist + kk - 1, sf.jend + l - 1);
+        pts.push_back(p);
       }
-    join(sf);
+    join(p0);
   }
+  B.nph = (int)ph.size() - B.gph;
+  ph.push_back((int)pts.size());
 }
 
 // k_lusgs_parts waits between the workgroups of a block: all of them must be
@@ -849,9 +875,8 @@ int launch_ghost(int level, int do_bc, int do_exchange) {
   DLevel& L = R.lv[level];
   GhostArgs a;
   a.blocks = L.db;
-  a.block_list = L.dblocks_all;
-  a.subs = L.ds;
-  a.units = L.dunits;
+  a.points = L.dgpts;
+  a.phases = L.dgph;
   a.normals = L.dnorm;
   a.cps = R.dcps;
   a.arena = L.arena;
@@ -1421,7 +1446,7 @@ int ec2d_finalize(void) {
   hipStreamSynchronize(R.s);
   if (R.graph) hipGraphExecDestroy(R.graph);
   for (auto& L : R.lv) {
-    hipFree(L.arena); hipFree(L.db); hipFree(L.ds); hipFree(L.dunits); hipFree(L.dnorm); hipFree(L.dt); hipFree(L.dperm);
+    hipFree(L.arena); hipFree(L.db); hipFree(L.ds); hipFree(L.dgpts); hipFree(L.dgph); hipFree(L.dnorm); hipFree(L.dt); hipFree(L.dperm);
     hipFree(L.dcase_tile0); hipFree(L.dncell); hipFree(L.dpartials); hipFree(L.dnorms); hipFree(L.drows);
     hipFree(L.dblocks_all); hipFree(L.sk); hipFree(L.dwall); hipFree(L.dcase_wall0);
     hipFree(L.dgring);
@@ -1920,6 +1945,13 @@ int ec2d_commit(void) {
     }
     HIPCHK(hipMalloc(&L.arena, sizeof(double) * (size_t)std::max<int64_t>(off, 1)));
     HIPCHK(hipMemcpy(L.arena, img.data(), sizeof(double) * (size_t)off, hipMemcpyHostToDevice));
+    std::vector<GhostPoint> gpts;
+    std::vector<int> gph;
+    for (auto& b : L.hb) ghost_phases(b, L.hb, subs.data() + b.bc_off, gpts, gph);
+    HIPCHK(hipMalloc(&L.dgpts, sizeof(GhostPoint) * std::max<size_t>(gpts.size(), 1)));
+    HIPCHK(hipMemcpy(L.dgpts, gpts.data(), sizeof(GhostPoint) * gpts.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMalloc(&L.dgph, sizeof(int) * gph.size()));
+    HIPCHK(hipMemcpy(L.dgph, gph.data(), sizeof(int) * gph.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&L.db, sizeof(BlockDesc) * L.hb.size()));
     HIPCHK(hipMemcpy(L.db, L.hb.data(), sizeof(BlockDesc) * L.hb.size(), hipMemcpyHostToDevice));
     // after the block table: the wall-distance kernels read it
@@ -1937,10 +1969,6 @@ int ec2d_commit(void) {
       }
       L.bl_walls = std::max(L.bl_walls, nw);
     }
-    std::vector<int> units(std::max<size_t>(subs.size(), 1), 0);
-    for (auto& b : L.hb) ghost_phases(b, subs.data() + b.bc_off, units.data() + b.bc_off);
-    HIPCHK(hipMalloc(&L.dunits, sizeof(int) * units.size()));
-    HIPCHK(hipMemcpy(L.dunits, units.data(), sizeof(int) * units.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&L.ds, sizeof(SubfaceDesc) * std::max<size_t>(subs.size(), 1)));
     HIPCHK(hipMemcpy(L.ds, subs.data(), sizeof(SubfaceDesc) * subs.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&L.dnorm, sizeof(double) * std::max<size_t>(norms.size(), 2)));
