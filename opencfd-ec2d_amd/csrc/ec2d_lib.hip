@@ -658,17 +658,20 @@ int launch_residual(int level, int clip, int force = 0, int set_un = 0, double* 
     hipLaunchKernelGGL(k_sst_cell, dim3(L.nrows), dim3(256), 0, R.s, sa);
     hipLaunchKernelGGL(k_sst_res, dim3(L.nrows), dim3(256), 0, R.s, sa);
   }
-  // MUSCL3 / van Albada on both face directions and the original
-  // reconstruction, with Roe's flux (1) or, for the Euler equations, AUSM (2), as
-  // compile-time constants: 64 Euler blocks of up to 257 x 129 cells with AUSM
-  // 90 -> 50 us a residual, one SST case of 257 x 65 28 -> 16 us (with the kernel's
-  // other changes, which take the general instance of the same size from 16 to 14)
+  // Options that an instance has as compile-time constants (see k_residual; FIX 0:
+  // any).  Against the general instance: 64 Euler blocks of up to 257 x 129 cells
+  // with AUSM 90 -> 50 us a residual, one SST case of 257 x 65 28 -> 16 us, the coarse
+  // levels of a 257 x 65 Euler V-cycle 14.5 -> 9 us (the general instance itself 16
+  // -> 14 us by the kernel's other changes).
   const bool fix = L.o.scheme == 5 && L.o.global_scheme == 5 && L.o.recon == 0;
-  const int fx = !fix ? 0 : L.o.flux == 4 ? 1 : L.o.flux == 6 && nv == 4 && !visc ? 2 : 0;
+  const bool fix3 = L.o.scheme == 0 && L.o.global_scheme == 5 && L.o.recon == 0 && L.o.flux == 4 && nv == 4;
+  const int fx = fix3 ? 3 : !fix ? 0 : L.o.flux == 4 ? 1 : L.o.flux == 6 && nv == 4 && !visc ? 2 : 0;
 #define RLAUNCH(TX, TY, NV, V, S)                                                                            \
   do {                                                                                                      \
     if (fx == 1) hipLaunchKernelGGL((k_residual<TX, TY, NV, V, S, 1>), grid, dim3(TX * TY), 0, R.s, a);     \
     else if (fx == 2) hipLaunchKernelGGL((k_residual<TX, TY, NV, V, S, NV == 4 && !V ? 2 : 0>), grid,       \
+                                         dim3(TX * TY), 0, R.s, a);                                         \
+    else if (fx == 3) hipLaunchKernelGGL((k_residual<TX, TY, NV, V, S, NV == 4 ? 3 : 0>), grid,             \
                                          dim3(TX * TY), 0, R.s, a);                                         \
     else hipLaunchKernelGGL((k_residual<TX, TY, NV, V, S, 0>), grid, dim3(TX * TY), 0, R.s, a);             \
   } while (0)

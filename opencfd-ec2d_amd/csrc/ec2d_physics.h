@@ -165,9 +165,11 @@ __device__ __forceinline__ void cons_to_prim(const double Q[4], double W[4], dou
   W[3] = (Q[3] - (W[1] * Q[1] + W[2] * Q[2]) * 0.5) * (g - 1.0);
 }
 
-// characteristic reconstruction: sub_Residual.f90:531-586.  U0[k][m]: k = i-2..i+1
-__device__ __forceinline__ void recon_characteristic(const double U0[4][4], double UL[4], double UR[4], double g,
-                                                     int flag) {
+// characteristic reconstruction: sub_Residual.f90:531-586.  The left
+// eigenvectors of the mean state of cells 1 and 2 take the conservative
+// variables U0[k][m] (k = i-2..i+1) to V0; S1, the right ones, take the
+// reconstructed V back (char_to_prim).
+__device__ __forceinline__ void to_char(const double U0[4][4], double V0[4][4], double S1[4][4], double g) {
   double Uh[4];
   for (int m = 0; m < 4; m++) Uh[m] = 0.5 * (U0[1][m] + U0[2][m]);
   double d1 = Uh[0], u1 = Uh[1] / d1, v1 = Uh[2] / d1;
@@ -178,7 +180,7 @@ __device__ __forceinline__ void recon_characteristic(const double U0[4][4], doub
   double tmp3 = (g - 1.0) / (c1 * c1);
   double tmp5 = 1.0 / (2.0 * c1);
   double tmp0 = 1.0 / tmp3;
-  double S[4][4], S1[4][4];
+  double S[4][4];
   S[0][0] = V2 - tmp0; S[0][1] = -u1; S[0][2] = -v1; S[0][3] = 1.0;
   S[1][0] = -v1; S[1][1] = 0.0; S[1][2] = 1.0; S[1][3] = 0.0;
   S[2][0] = -u1 - V2 * tmp1; S[2][1] = 1.0 + tmp1 * u1; S[2][2] = tmp1 * v1; S[2][3] = -tmp1;
@@ -187,28 +189,21 @@ __device__ __forceinline__ void recon_characteristic(const double U0[4][4], doub
   S1[1][0] = -tmp3 * u1; S1[1][1] = 0.0; S1[1][2] = 0.5 - u1 * tmp5; S1[1][3] = 0.5 + u1 * tmp5;
   S1[2][0] = -tmp3 * v1; S1[2][1] = 1.0; S1[2][2] = -v1 * tmp5; S1[2][3] = v1 * tmp5;
   S1[3][0] = -tmp3 * V2; S1[3][1] = v1; S1[3][2] = (c1 * u1 - V2 - tmp0) * tmp5; S1[3][3] = (c1 * u1 + V2 + tmp0) * tmp5;
-  double V0[4][4], VL[4], VR[4], QL[4], QR[4];
   for (int k = 0; k < 4; k++)
     for (int m = 0; m < 4; m++) {
       double s = 0.0;
       for (int j = 0; j < 4; j++) s = s + S[m][j] * U0[k][j];
       V0[k][m] = s;
     }
+}
+__device__ __forceinline__ void char_to_prim(const double V[4], const double S1[4][4], double W[4], double g) {
+  double Q[4];
   for (int m = 0; m < 4; m++) {
-    VL[m] = scheme_fP(V0[0][m], V0[1][m], V0[2][m], V0[3][m], flag);
-    VR[m] = scheme_fm(V0[0][m], V0[1][m], V0[2][m], V0[3][m], flag);
+    double a = 0.0;
+    for (int j = 0; j < 4; j++) a = a + S1[m][j] * V[j];
+    Q[m] = a;
   }
-  for (int m = 0; m < 4; m++) {
-    double a = 0.0, b = 0.0;
-    for (int j = 0; j < 4; j++) {
-      a = a + S1[m][j] * VL[j];
-      b = b + S1[m][j] * VR[j];
-    }
-    QL[m] = a;
-    QR[m] = b;
-  }
-  cons_to_prim(QL, UL, g);
-  cons_to_prim(QR, UR, g);
+  cons_to_prim(Q, W, g);
 }
 
 // ---- interface fluxes, Q = (rho, u_n, u_t, p): sub_flux_split.f90 -----------

@@ -110,17 +110,22 @@ __device__ __forceinline__ void wave_fold(double (&v)[N], OP op) {
 //   waves_per_eu: 128 registers, so that the four workgroups that a CU's LDS
 // holds do run.
 //
-// FIX: the level's scheme and reconstruction are MUSCL3 with the van Albada
-// limiter on both face directions and the original (primitive) reconstruction,
-// and the flux is Roe's (1) or AUSM (2), as compile-time constants, so that the
-// compiler drops the other branches of every face; the launch picks it when
-// the options match.
+// FIX: scheme, reconstruction and flux as compile-time constants, so that the
+// compiler drops the other branches of every face; the launch picks it when the
+// options match.  All with the original (primitive) reconstruction: MUSCL3 with the van
+// Albada limiter in both directions and Roe's flux (1) or AUSM (2), and what a coarse
+// level of a V-cycle makes of (1): first order over the i-faces (3).
+//   FIX 0, any options: with every loop and reconstruction holding its own copy of
+// all schemes and fluxes the code is 108 KB, more than the instruction cache.  Here
+// one loop takes both directions in turn and the three reconstructions share the
+// schemes (32 KB): 129 x 49 laminar cells with WENO3, HLLC and characteristic
+// variables 34 -> 30 us.
 template <int TX, int TY, int NV, bool VISC, bool SA, int FIX>
-__global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) void k_residual(ResArgs a) {
+__global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 : 3))) void k_residual(ResArgs a) {
   constexpr int RW = TX + 4, RH = TY + 4, NT = TX * TY;
   constexpr int CW = TX + 2, CH = TY + 2;  // the viscous quantities are used one cell out
-  const int o_scheme = FIX ? 5 : a.o.scheme, o_gscheme = FIX ? 5 : a.o.global_scheme;
-  const int o_flux = FIX == 1 ? 4 : FIX == 2 ? 6 : a.o.flux, o_recon = FIX ? 0 : a.o.recon;
+  const int o_scheme = FIX == 3 ? 0 : FIX ? 5 : a.o.scheme, o_gscheme = FIX ? 5 : a.o.global_scheme;
+  const int o_flux = FIX == 2 ? 6 : FIX ? 4 : a.o.flux, o_recon = FIX ? 0 : a.o.recon;
   // reciprocals of the constant divisors; div_y with them gives the
   // reference's quotients (x / Pr, x / Pr_t, x / sigma, x / k^2, x / Ma)
   constexpr double yPrt = 1.0 / EC2D_PRT, ySig = 1.0 / (2.0 / 3.0), yK2 = 1.0 / (0.41 * 0.41);
@@ -315,24 +320,16 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) voi
     double UL[4], UR[4];
     double F1 = 0.0, F2 = 0.0, F3 = 0.0, F4 = 0.0;
     if (!skip_fvm) {
-      // the j-direction original-variable reconstruction uses the global
-      // scheme option, not the mesh's own (sub_Residual.f90:367)
+      double W[4][4], S1[4][4];  // cells -2 back .. back: the variables to reconstruct
       if (o_recon == 0) {
-        const int sch = J ? o_gscheme : o_scheme;
-        auto recon = [&](int m, double w0, double w1, double w2, double w3) {
-          UL[m] = scheme_fP(w0, w1, w2, w3, sch);
-          UR[m] = scheme_fm(w0, w1, w2, w3, sch);
-        };
-        recon(0, d_[-2 * back], d_[-back], d_[0], d_[back]);
-        recon(1, u_[-2 * back], u_[-back], u_[0], u_[back]);
-        recon(2, v_[-2 * back], v_[-back], v_[0], v_[back]);
-        if constexpr (VISC) {
-          const double* T_ = &sT[0][0] + o;
-          auto p = [&](int k) { return cp.p00 * d_[k] * T_[k]; };
-          recon(3, p(-2 * back), p(-back), p(0), p(back));
-        } else {
-          const double* p_ = &sp[0][0] + o;
-          recon(3, p_[-2 * back], p_[-back], p_[0], p_[back]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int at_ = (k - 2) * back;
+          W[k][0] = d_[at_];
+          W[k][1] = u_[at_];
+          W[k][2] = v_[at_];
+          if constexpr (VISC) W[k][3] = cp.p00 * d_[at_] * (&sT[0][0] + o)[at_];
+          else W[k][3] = (&sp[0][0] + o)[at_];
         }
       } else {
         double U0[4][4];
@@ -341,16 +338,29 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) voi
           for (int m = 0; m < 4; m++) U0[k][m] = at(PL(pm.U + m), qk);
         }
         if (o_recon == 1) {
-          double QL[4], QR[4];
-          for (int m = 0; m < 4; m++) {
-            QL[m] = scheme_fP(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
-            QR[m] = scheme_fm(U0[0][m], U0[1][m], U0[2][m], U0[3][m], o_scheme);
-          }
-          cons_to_prim(QL, UL, g);
-          cons_to_prim(QR, UR, g);
+          for (int k = 0; k < 4; k++)
+            for (int m = 0; m < 4; m++) W[k][m] = U0[k][m];
         } else {
-          recon_characteristic(U0, UL, UR, g, o_scheme);
+          to_char(U0, W, S1, g);
         }
+      }
+      // the j-direction original-variable reconstruction uses the global
+      // scheme option, not the mesh's own (sub_Residual.f90:367)
+      const int sch = J && o_recon == 0 ? o_gscheme : o_scheme;
+      double VL[4], VR[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        VL[m] = scheme_fP(W[0][m], W[1][m], W[2][m], W[3][m], sch);
+        VR[m] = scheme_fm(W[0][m], W[1][m], W[2][m], W[3][m], sch);
+      }
+      if (o_recon == 0) {
+        for (int m = 0; m < 4; m++) UL[m] = VL[m], UR[m] = VR[m];
+      } else if (o_recon == 1) {
+        cons_to_prim(VL, UL, g);
+        cons_to_prim(VR, UR, g);
+      } else {
+        char_to_prim(VL, S1, UL, g);
+        char_to_prim(VR, S1, UR, g);
       }
       double QL[4], QR[4], F0[4];
       QL[0] = UL[0]; QL[1] = UL[1] * n1 + UL[2] * n2; QL[2] = -UL[1] * n2 + UL[2] * n1; QL[3] = UL[3];
@@ -424,28 +434,6 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) voi
 #pragma unroll
     for (int m = 0; m < NC; m++) sFj[fj][m][fi] = F[m];
   };
-  // ---- 2a. i-faces, one per thread; then the TY of the last column and, where
-  // one wave takes both in one pass (FIX: the same code for either direction),
-  // the TX j-faces of the last row
-  constexpr bool JOIN = FIX != 0;
-  constexpr int NX = JOIN ? TY + TX : TY;
-  for (int f = tid; f < NT + NX; f += NT) {
-    double F[6] = {};
-    const int x = f - NT;
-    if constexpr (JOIN) {
-      const bool J = x >= TY;
-      const int fi = x < 0 ? f % TX : J ? x - TY : TX, fj = x < 0 ? f / TX : J ? TY : x;
-      if (!face(J, fi, fj, F)) continue;
-      if (J) put_j(fi, fj, F);
-      else put_i(fi, fj, F);
-    } else {
-      const int fi = x < 0 ? f % TX : TX, fj = x < 0 ? f / TX : x;
-      if (face(std::false_type{}, fi, fj, F)) put_i(fi, fj, F);
-    }
-  }
-  __syncthreads();
-
-  fresh();
   // The cell of this thread in phases 3a and 3: row-major, or, when the
   // epilogue also writes the hyperplane-order copy (sk_out), along the
   // tile's hyperplanes: TY consecutive lanes take the TY rows of one
@@ -461,25 +449,58 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(4))) voi
   // reference's order), before the j-faces take over the LDS --------------
   double R[NV];
   double r5 = 0.0, v0c = 0.0;  // SA: the cell's v0 of sub_turbulence_SA.f90, kept for phase 3
-  if (mine) {
-    if (!fdm_cell) {
-#pragma unroll
-      for (int m = 0; m < 4; m++) R[m] = sFi[m][cj][ci + 1] - sFi[m][cj][ci];
+  auto i_diff = [&] {
+    if (mine) {
+      if (!fdm_cell) {
+  #pragma unroll
+        for (int m = 0; m < 4; m++) R[m] = sFi[m][cj][ci + 1] - sFi[m][cj][ci];
+      }
+      if constexpr (SA) {
+        const double SA_sigma = 2.0 / 3.0, Cb2 = 0.622;
+        v0c = div_y((svt[cj + 1][ci + 1] + snu[cj + 1][ci + 1]) * Cb2, SA_sigma, ySig);
+        r5 = sFi[NC - 2][cj][ci + 1] - sFi[NC - 2][cj][ci] - v0c * (sFi[NC - 1][cj][ci + 1] - sFi[NC - 1][cj][ci]);
+      }
     }
-    if constexpr (SA) {
-      const double SA_sigma = 2.0 / 3.0, Cb2 = 0.622;
-      v0c = div_y((svt[cj + 1][ci + 1] + snu[cj + 1][ci + 1]) * Cb2, SA_sigma, ySig);
-      r5 = sFi[NC - 2][cj][ci + 1] - sFi[NC - 2][cj][ci] - v0c * (sFi[NC - 1][cj][ci + 1] - sFi[NC - 1][cj][ci]);
+  };
+  // ---- 2a. i-faces, one per thread, and the TY of the last column; 2b. j-faces
+  // and the TX of the last row
+  if constexpr (FIX != 0) {
+    // one wave takes both remainders in one pass
+    for (int f = tid; f < NT + TY + TX; f += NT) {
+      double F[6] = {};
+      const int x = f - NT;
+      const bool J = x >= TY;
+      const int fi = x < 0 ? f % TX : J ? x - TY : TX, fj = x < 0 ? f / TX : J ? TY : x;
+      if (!face(J, fi, fj, F)) continue;
+      if (J) put_j(fi, fj, F);
+      else put_i(fi, fj, F);
     }
-  }
-  __syncthreads();
-  // ---- 2b. j-faces, one per thread (and the last row, without JOIN) ---------
-  for (int f = tid; f < (JOIN ? NT : NT + TX); f += NT) {
+    __syncthreads();
+    fresh();
+    i_diff();
+    __syncthreads();
     double F[6] = {};
-    if (face(std::true_type{}, f % TX, f / TX, F)) put_j(f % TX, f / TX, F);
+    if (face(std::true_type{}, tid % TX, tid / TX, F)) put_j(tid % TX, tid / TX, F);
+    __syncthreads();
+  } else {
+#pragma unroll 1
+    for (int dir = 0; dir < 2; dir++) {
+      const bool J = dir != 0;
+      for (int f = tid; f < NT + (J ? TX : TY); f += NT) {
+        double F[6] = {};
+        const int x = f - NT;
+        const int fi = x < 0 ? f % TX : J ? x : TX, fj = x < 0 ? f / TX : J ? TY : x;
+        if (!face(J, fi, fj, F)) continue;
+        if (J) put_j(fi, fj, F);
+        else put_i(fi, fj, F);
+      }
+      __syncthreads();
+      if (!J) {
+        i_diff();
+        __syncthreads();
+      }
+    }
   }
-  __syncthreads();
-
   fresh();
   // ---- 3. cells ------------------------------------------------------------
   double rmax[NV], rsum[NV];
