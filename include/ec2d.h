@@ -317,7 +317,7 @@ int ec2d_set_wait_budget(int polls);
  * CUs, for levels of at most 256/split blocks taller than split/2 waves), or
  * 0 with one lane per cell, for blocks of at most 64 rows: the fused launches,
  * whose workgroups make each block's records themselves, so that they never go
- * through device memory - in parts of 32 rows where every part finds a CU of
+ * through device memory - in parts of 16 or 32 rows where every part finds a CU of
  * its own, one workgroup per block otherwise (-3: one workgroup per block in
  * any case).  Results do not depend on it. */
 int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block);

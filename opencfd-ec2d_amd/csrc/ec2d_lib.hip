@@ -83,7 +83,8 @@ struct DLevel {
   int lusgs_lpc = 1;          // LU-SGS lanes per cell: 2 when every block has at most 32 rows
   int lusgs_split = 1;        // LU-SGS sweep workgroups per block (2 or 4: a block's rows split between CUs)
   bool lusgs_fused = false;   // LU-SGS records made inside the sweep workgroup (k_lusgs_fused, k_lusgs_parts)
-  bool lusgs_parts = false;   // with lusgs_fused: workgroups of 32 rows (k_lusgs_parts), lusgs_split per block
+  bool lusgs_parts = false;   // with lusgs_fused: workgroups of part_rows rows (k_lusgs_parts), lusgs_split per block
+  int part_rows = 0;
   bool planar_stale = false;  // Res, dt, Lc, Lv are current only in the hyperplane copy (planar_refresh)
   bool skew_static = false;   // the record arena holds the skewed copy of the mesh planes
   unsigned long long* dgring = nullptr;  // split sweeps: one ring per boundary between workgroups and direction
@@ -280,13 +281,20 @@ void ghost_phases(BlockDesc& B, const std::vector<BlockDesc>& hb, const SubfaceD
   ph.push_back((int)pts.size());
 }
 
-// k_lusgs_parts waits between the workgroups of a block: all of them must be
-// resident at once, one per CU.  A block of one part has nothing to wait for.
-bool parts_fit(const DLevel& L) {
+// Rows of a part of k_lusgs_parts for a level, 0 if it does not fit.  A block's
+// parts wait for each other: all of them must be resident at once, one per CU.  A
+// part alone waits for nothing.  Parts of 16 rows (four lanes per cell) have the
+// shorter step, parts of 32 (two lanes) half the links: per pass, 513 x 129 SA cells
+// (8 blocks) 640 against 670 us, 257 x 65 Euler 221 against 241, SST 313 against
+// 365.  Blocks of 17 .. 32 rows stay one part of 32, whose sweeps share a launch
+// (129 x 33 SA cells 131 us an update, 141 as two parts of 16).
+int parts_rows(const DLevel& L) {
   int max_rows = 1;
   for (auto& d : L.hb) max_rows = std::max(max_rows, d.ny - 1);
-  const int G = (max_rows + PART_ROWS - 1) / PART_ROWS;
-  return G == 1 || (int64_t)G * (int64_t)L.hb.size() <= R.ncu;
+  if (max_rows <= 32) return max_rows <= 16 ? 16 : 32;
+  for (int rows : {16, 32})
+    if ((int64_t)((max_rows + rows - 1) / rows) * (int64_t)L.hb.size() <= R.ncu) return rows;
+  return 0;
 }
 
 // LU-SGS record layout of a level for lpc lanes per cell (see ec2d_lusgs.hip);
@@ -295,7 +303,7 @@ bool parts_fit(const DLevel& L) {
 // of rows, so a step holds exactly the block's rows (R = nrow): the rows of
 // consecutive steps share cache lines instead of padding each step to 64.
 // parts: that of k_lusgs_parts (also R = nrow), with `split` set here to the
-// parts of 32 rows of the tallest block.
+// parts of the tallest block.
 int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false, bool parts = false) {
   L.skew_static = false;  // the arena is cleared below
   int max_rows = 1;
@@ -303,8 +311,9 @@ int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false,
   const int rq = 64 / lpc;  // rows per wave
   if (parts) {
     fused = true;
-    split = (max_rows + PART_ROWS - 1) / PART_ROWS;
-    if (!parts_fit(L)) return fail("too many blocks for an LU-SGS launch in parts of 32 rows");
+    L.part_rows = parts_rows(L);
+    if (!L.part_rows) return fail("too many blocks for an LU-SGS launch in parts");
+    split = (max_rows + L.part_rows - 1) / L.part_rows;
     if (max_rows > 1024) return fail("blocks with more than 1024 rows of cells are not supported by the LU-SGS kernel");
   } else if (split != 1 && split != 2 && split != 4) {
     return fail("LU-SGS split must be 1, 2 or 4");
@@ -807,7 +816,10 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
     if (L.lusgs_parts) {                                                                    \
       for (int d = (a.split > 1 ? 1 : 0); d <= (a.split > 1 ? 2 : 0); d++) {                \
         a.dir = d;                                                                          \
-        hipLaunchKernelGGL((k_lusgs_parts<NV, V>), dim3(nblk * a.split), dim3(PART_THREADS), 0, R.s, a); \
+        if (L.part_rows == 16)                                                              \
+          hipLaunchKernelGGL((k_lusgs_parts<NV, V, 4>), dim3(nblk * a.split), dim3(PART_THREADS), 0, R.s, a); \
+        else                                                                                \
+          hipLaunchKernelGGL((k_lusgs_parts<NV, V, 2>), dim3(nblk * a.split), dim3(PART_THREADS), 0, R.s, a); \
       }                                                                                     \
     } else                                                                                  \
       hipLaunchKernelGGL((k_lusgs_fused<NV, V>), dim3(nblk), dim3(FUSED_THREADS), 0, R.s, a); \
@@ -1402,7 +1414,7 @@ struct Lcg {
 // autotune report text of an LU-SGS shape (0, -1: the fused launches)
 std::string shape_text(int sp) {
   if (sp == 0) return "fused preparation and sweeps";
-  if (sp == -1) return "fused preparation and sweeps in parts of 32 rows";
+  if (sp == -1) return "fused preparation and sweeps in parts";
   return "workgroups per block " + std::to_string(sp);
 }
 
@@ -1894,17 +1906,16 @@ int ec2d_commit(void) {
     for (auto& d : L.hb)
       if (d.plane >= ((int64_t)1 << 29)) return fail("a block's plane must be smaller than 4 GiB");
     L.arena_n = off;
-    // The LU-SGS shape until ec2d_autotune times them.  In parts of 32 rows
-    // where all parts fit the device: 257 x 65 cells of six equations 0.31 ms an
-    // update (0.38 with one lane per row and the records in memory), 64 blocks
-    // of up to 257 x 129 cells 0.28 ms (0.40).  Blocks of one part have no chain
-    // between workgroups to shorten: the records in memory are as fast up to
-    // about 16 blocks of 129 x 33 cells (0.148 against 0.146 ms a pass; one
-    // block 0.136 against 0.144, 64 blocks 0.183 against 0.168).  Else the fused
-    // launch for blocks of at most 64 rows (256 SA blocks: 0.36 against 1.35 ms);
-    // else the records in memory.
-    L.lusgs_parts = parts_fit(L) && (max_rows > PART_ROWS || L.hb.size() >= 16);
-    L.lusgs_fused = L.lusgs_parts || (max_rows > PART_ROWS && max_rows <= 64);
+    // The LU-SGS shape until ec2d_autotune times them.  In parts where all of them
+    // fit the device: an update of 257 x 65 cells of six equations 0.27 ms (0.38 with
+    // one lane per row and the records in memory), of 64 blocks of up to 257 x 129
+    // cells 0.26 ms (0.40).  Blocks of one part have no chain between workgroups to
+    // shorten: the records in memory are as fast up to about 16 blocks of 129 x 33
+    // cells (0.148 against 0.146 ms a pass; one block 0.136 against 0.144, 64 blocks
+    // 0.183 against 0.168).  Else the fused launch for blocks of at most 64 rows (256
+    // SA blocks: 0.36 against 1.35 ms); else the records in memory.
+    L.lusgs_parts = parts_rows(L) && (max_rows > 32 || L.hb.size() >= 16);
+    L.lusgs_fused = L.lusgs_parts || (max_rows > 32 && max_rows <= 64);
     if (lusgs_layout(L, !L.lusgs_fused && max_rows <= 32 ? 2 : 1, 1, false, L.lusgs_fused, L.lusgs_parts)) return 1;
     // host image of the arena
     std::vector<double> img((size_t)off, 0.0);
@@ -2468,7 +2479,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
   if (lanes_per_cell != 1 && lanes_per_cell != 2) return fail("lanes per cell must be 1 or 2");
   HIPCHK(hipStreamSynchronize(R.s));
   DLevel& L = R.lv[nMesh - 1];
-  // 0: fused, in parts of 32 rows where they fit; -3: fused, a workgroup per block
+  // 0: fused, in parts where they fit; -3: fused, a workgroup per block
   const bool fused = workgroups_per_block == 0 || workgroups_per_block == -3;
   if (workgroups_per_block < 0 && !fused) return fail("workgroups per block 1, 2, 4, or 0 / -3 (fused)");
   if (fused) {
@@ -2476,7 +2487,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
     for (auto& b : L.hb)
       if (b.ny - 1 > 64) return fail("the fused LU-SGS launch needs blocks of at most 64 rows of cells");
   }
-  const bool parts = workgroups_per_block == 0 && parts_fit(L);
+  const bool parts = workgroups_per_block == 0 && parts_rows(L) != 0;
   if (lusgs_layout(L, lanes_per_cell, fused ? 1 : workgroups_per_block, true, fused, parts)) return 1;
   L.lusgs_fused = fused;
   L.lusgs_parts = parts;
@@ -2574,14 +2585,14 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
           if (ms < best) { best = ms; best_lp = lp; best_sp = sp; }
         }
       // the fused variants: records made in the sweep workgroup, a workgroup
-      // per block (0; rows <= 64) or per part of 32 rows (-1).  Timed with the
+      // per block (0; rows <= 64) or per part (-1).  Timed with the
       // residual before them, which writes their inputs in a main-loop pass
       // (advance_lusgs), less the plain residual: the copy kernel that a lone
       // update needs is no part of a pass.
       bool fits = true;
       for (auto& b : L.hb) fits = fits && b.ny - 1 <= 64;
       for (int sp : {0, -1}) {
-        if (!(sp == 0 ? fits : parts_fit(L)) || lusgs_layout(L, 1, 1, true, true, sp == -1)) continue;
+        if (!(sp == 0 ? fits : parts_rows(L)) || lusgs_layout(L, 1, 1, true, true, sp == -1)) continue;
         L.lusgs_fused = true;
         L.lusgs_parts = sp == -1;
         const bool rskew = !L.fdm;
@@ -2615,7 +2626,7 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
     L.tile_cols = best_tr >= 100 ? 32 : 64;
     L.tile_rows = best_tr % 100;
     if (build_tiles(L)) return 1;
-    if (best_sp == -1 && !parts_fit(L)) best_sp = 1;  // a cache file of a device with more compute units
+    if (best_sp == -1 && !parts_rows(L)) best_sp = 1;  // a cache file of a device with more compute units
     if (lusgs_layout(L, best_lp, best_sp <= 0 ? 1 : best_sp, true, best_sp <= 0, best_sp == -1)) return 1;
     L.lusgs_fused = best_sp <= 0;
     L.lusgs_parts = best_sp == -1;

@@ -9,8 +9,8 @@
 //           k_lusgs_scatter puts dU into the block planes (and U = U + dU);
 //   fused   k_lusgs_fused makes the records in the sweep's own workgroup and
 //           writes the planes itself (blocks of at most 64 rows);
-//   parts   k_lusgs_parts does the same by workgroups of 32 rows, linked as
-//           the split sweeps are (few blocks, any number of rows).
+//   parts   k_lusgs_parts does the same by workgroups of 16 or 32 rows, linked
+//           as the split sweeps are (few blocks, any number of rows).
 //
 // Sweep order.  The forward sweep needs dU(i-1,j) and dU(i,j-1), the backward
 // sweep dU(i+1,j) and dU(i,j+1).  Any order that respects these dependencies
@@ -43,7 +43,8 @@
 // terms move one lane up (DPP wave shift): lane 2t then holds its own term
 // and row t-1's, forms the sum and hands it to lane 2t+1 (DPP quad permute),
 // and both finish the cell with the same bits; with one lane per row, lane t
-// receives row t-1's.  The first lane of a wave gets row t-1 through LDS.
+// receives row t-1's.  The first lane of a wave gets row t-1 through LDS.  Four
+// (QuadSlot): each half of the wave has half of the equations.
 //
 // Divisions.  Every quotient of a sweep has a divisor known before its
 // numerator (the diagonal) or shared by three quotients (rho of U + dU).
@@ -1042,7 +1043,7 @@ __device__ __forceinline__ bool wait_bounded(const int* p, int v, int* err, int 
 // one: positions without a cell (about (nrow-1)/ncol of the field) are
 // never written, and a wave reading them would fetch lines nobody needs;
 // such a lane's value never reaches a cell.
-template <int NV, bool VISC>
+template <int NV, bool VISC, int LPC = 1>
 __device__ __forceinline__ void load_x(double* x, __amdgpu_buffer_rsrc_t rs, uint32_t bw, uint32_t n16, int st, int r,
                                        int S, int R, int ncol, int nrow) {
   const int sc = min(st, S - 1);
@@ -1057,6 +1058,11 @@ __device__ __forceinline__ void load_x(double* x, __amdgpu_buffer_rsrc_t rs, uin
       x[2 * j] = v.x;
       x[2 * j + 1] = v.y;
     }
+  }
+  if constexpr (LPC == 4) {  // the sweep wave stores momentum first
+    const double t = x[0];
+    x[0] = x[1];
+    x[1] = t;
   }
 }
 
@@ -1339,17 +1345,20 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_lusgs_fused(LusgsArgs a) {
   run_dir(std::false_type{});
 }
 
-// ------------------------------------- the same, in parts of 32 rows of a block
+// ------------------------------------------- the same, in parts of a block's rows
 // For levels of few blocks (k parts each, at most one workgroup per CU): each
-// part of 32 rows is a workgroup of its own, linked to the next through
+// part of 16 or 32 rows is a workgroup of its own, linked to the next through
 // global memory as the split sweeps' workgroups are, and makes its records in
-// LDS as k_lusgs_fused does.  The sweep wave has two lanes per cell: its step
-// is a quarter shorter than with one, and what bounds a single block is the
-// chain of steps (the split sweeps' wave reads its records by 13 memory loads a
-// step, which take it about 7 ns each to issue; the LDS reads here 3).
-//   A producer's 64 lanes make the records of two steps at a time.  LDS
-// records come in pairs of doubles: the cell's part by row, the sides' by lane,
-// so that the sweep wave's reads are 16 bytes a lane without bank conflicts.
+// LDS as k_lusgs_fused does.  What bounds a single block is the chain of steps,
+// so a cell of the sweep wave has two lanes (32 rows) or four (16): of a step of
+// four equations' 130 instructions 70 are FP64 with two, of 107 42 with four, in
+// which each half of the wave takes half of the equations.  (The split sweeps'
+// wave reads its records by 13 memory loads a step, which take it about 7 ns each
+// to issue; the LDS reads here 3.)  An update of 257 x 65 cells, four equations,
+// 0.19 ms with four lanes, 0.22 with two and with the split sweeps.
+//   A producer's 64 lanes make the records of two (four) steps at a time.  LDS
+// records come in pairs of doubles, the cell's part by row, the sides' by
+// lane, so that the sweep wave's reads are 16 bytes a lane without bank conflicts.
 //   A block of one part runs both sweeps in one launch; with several the
 // sweeps are separate launches (a.dir), as in k_lusgs_sweep.
 template <int NV, bool VISC>
@@ -1365,25 +1374,247 @@ struct PartSlot {
   __device__ static constexpr int cell(int d, int row) { return d / 2 * 64 + 2 * row + (d & 1); }
   __device__ static constexpr int side(int k, int e, int row) { return SIDE + e / 2 * 128 + 2 * (2 * row + k) + (e & 1); }
 };
+// Four lanes per cell (parts of 16 rows): lane 32 h + 2 t + k of row t has side k and
+// half h of the equations, NP of them: one of the momentum equations, then mass or
+// energy, then what the turbulence model adds (one equation: h = 0 only, and half
+// 1 computes with whatever is in its place).
 template <int NV, bool VISC>
+struct QuadSlot {
+  using F = RecF<NV, VISC>;
+  static constexpr int U = NV, YH0 = 2 * NV, YL0 = YH0 + 1, YH4 = YH0 + 2, YL4 = YH0 + 3;
+  static constexpr int NP = NV == 4 ? 2 : 3;
+  static constexpr int CY = NP * 64, SIDE = CY + (NV == 5 ? 64 : 32), LANE = SIDE + (VISC ? 192 : 128);
+  static constexpr int N = LANE + (NP + 1) / 2 * 128;  // doubles of a slot
+  static constexpr int XD = 4;
+  static constexpr int NRING = 16;
+  static constexpr int NGRP = NRING / XD;
+  // half and place of equation m
+  __device__ static constexpr int half(int m) { return m == 2 || m == 3 || m == 5; }
+  __device__ static constexpr int place(int m) { return m == 1 || m == 2 ? 0 : m < 4 ? 1 : 2; }
+  // X and U by (half, row): pairs X0 X1, U0 U1 or X0 X1, X2 U2, U0 U1
+  __device__ static constexpr int xu(bool u, int h, int p, int row) {
+    const int d = p == 2 ? 2 + u : NP == 2 ? 2 * u + p : 4 * u + p;
+    return d / 2 * 64 + 2 * (16 * h + row) + (d & 1);
+  }
+  __device__ static constexpr int cell(int d, int row) {
+    if (d < 2 * NV) return xu(d >= NV, half(d % NV), place(d % NV), row);
+    return CY + (d - YH0) / 2 * 32 + 2 * row + ((d - YH0) & 1);
+  }
+  // F by lane; n1 n2, a Lc, Lv by (row, side)
+  __device__ static constexpr int side(int k, int e, int row) {
+    if (e < NV) return LANE + place(e) / 2 * 128 + 2 * (32 * half(e) + 2 * row + k) + (place(e) & 1);
+    const int d = e == F::N1 ? 0 : e == F::N2 ? 1 : e == F::A ? 2 : e == F::LC ? 3 : 4;
+    return SIDE + d / 2 * 64 + 2 * (2 * row + k) + (d & 1);
+  }
+};
+template <int NV, bool VISC, int LPC>
+using PartSlotOf = std::conditional_t<LPC == 4, QuadSlot<NV, VISC>, PartSlot<NV, VISC>>;
+template <int NV, bool VISC, int LPC>
 struct PartLds {
-  using F = PartSlot<NV, VISC>;
+  using F = PartSlotOf<NV, VISC, LPC>;
   alignas(16) double rec[F::NRING][F::N];
-  double ob[8][NV][32];  // the backward U + dU (update) or dU of eight steps
+  double ob[8][NV][64 / LPC];  // the backward U + dU (update) or dU of eight steps
   Chain<NV, 2> ch[2];    // one per sweep
   int filled[F::NGRP];
   int consumed, turned, ob_ready, ob_taken;
 };
-constexpr int PART_ROWS = 32;
 constexpr int PART_PROD = 3;       // producers: waves 1 .. 3 (wave 4 ends at once, see FUSED_THREADS)
 constexpr int PART_THREADS = 512;  // then the writer, the receiving and the sending wave
 
+// the value of lane l and of lane l ^ 32: x in the lower lanes, y in the upper
+__device__ __forceinline__ void both_halves(double v, double& x, double& y) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+  x = __hiloint2double(hi[0], lo[0]);
+  y = __hiloint2double(hi[1], lo[1]);
+}
+
+// The sweep wave of a part of 16 rows (lanes: QuadSlot).  A step is a sum, a
+// quotient and U + dU per equation of the lane's half, the halves' exchange by
+// lane moves, p and F(U).n once per side, and the lane's terms.
 template <int NV, bool VISC>
+__device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC, 4>& L, __amdgpu_buffer_rsrc_t rs,
+                                            uint32_t bw, uint32_t n16, int S, int R, int ncol, int nrow, int row0,
+                                            int lane, int npad, double g, bool do_f, bool do_b) {
+  using PS = QuadSlot<NV, VISC>;
+  constexpr int NP = PS::NP, NRING = PS::NRING, XD = PS::XD, NGRP = PS::NGRP;
+  const int h = lane >> 5, row = lane >> 1 & 15, k = lane & 1, t = row0 + row;
+  struct R4 {
+    double X[NP], U[NP], F[NP], yh, yl, yh4, yl4, n1, n2, a, Lc, Lv;
+  };
+  const int o_xu = 2 * (16 * h + row), o_cy = PS::CY + 2 * row, o_sd = PS::SIDE + 2 * (lane & 31),
+            o_ln = PS::LANE + 2 * lane;
+  auto load_lds = [&](R4& r, const double* rec) {
+    auto pair = [&](int at) { return *reinterpret_cast<const D2a*>(rec + at); };
+    D2a v = pair(o_xu);
+    r.X[0] = v.x;
+    r.X[1] = v.y;
+    if constexpr (NP == 3) {
+      v = pair(o_xu + 64);
+      r.X[NP - 1] = v.x;
+      r.U[NP - 1] = v.y;
+    }
+    v = pair(o_xu + (NP - 1) * 64);
+    r.U[0] = v.x;
+    r.U[1] = v.y;
+    v = pair(o_cy);
+    r.yh = v.x;
+    r.yl = v.y;
+    if constexpr (NV == 5) v = pair(o_cy + 32);
+    r.yh4 = v.x;
+    r.yl4 = v.y;
+    v = pair(o_sd);
+    r.n1 = v.x;
+    r.n2 = v.y;
+    v = pair(o_sd + 64);
+    r.a = v.x;
+    r.Lc = v.y;
+    r.Lv = VISC ? rec[o_sd + (VISC ? 128 : 0)] : 0.0;
+    v = pair(o_ln);
+    r.F[0] = v.x;
+    r.F[1] = v.y;
+    if constexpr (NP == 3) r.F[NP - 1] = rec[o_ln + 128];
+  };
+  constexpr int NREAD = NP + 1 + (NV == 5) + 2 + VISC + NP - 1;
+  // this lane's equations, for the planes' chunk buffer
+  const int eq[3] = {h ? 2 : 1, h ? 3 : 0, NV == 6 && h ? 5 : 4};
+  // in a ring slot: momentum, mass or energy of half 0, of half 1, then the rest
+  const int rg = 2 * h, rg2 = NV == 6 ? 4 + h : 4;
+  bool ok = true;
+  int grp = 0, round = 1;  // the group slot of the turn and its use
+  auto run_dir = [&](auto fwd_c, int gs0) {
+    constexpr bool fwd = decltype(fwd_c)::value;
+    Chain<NV, 2>& ch = L.ch[fwd ? 0 : 1];
+    double tm[NP] = {};
+    constexpr uint32_t NOWHERE = 0x80000000u;  // out of the buffer's range: the store is dropped
+    const int ts = t < nrow && k == 0 ? t : 0x40000000;
+    uint32_t w8 = (uint32_t)((S - 1) * R + (nrow - 1 - t)) * 8u;
+    double in[NP];
+    // the last row's terms go to the next part, the others' nowhere (half 1 of five
+    // equations has no third)
+    const bool out = row == 15 && k == 1;
+    double(*rout)[NV] = out ? ch.ring[1] : ch.dump;
+    double(*rout2)[NV] = out && !(NV == 5 && h) ? ch.ring[1] : ch.dump;
+    auto read_in = [&](int slot) {
+      in[0] = ch.ring[0][slot][rg];
+      in[1] = ch.ring[0][slot][rg + 1];
+      if constexpr (NP == 3) in[NP - 1] = ch.ring[0][slot][rg2];
+    };
+    int prog = 0, cons = 0, pv = 0;
+    auto look = [&] {
+      prog = lds_get(&ch.prog[0]);
+      cons = lds_get(&ch.cons[1]);
+    };
+    look();
+    R4 rn;
+    if (ok) ok = wait_bounded(&L.filled[grp], XD * round, a.err, a.spin_max);
+    load_lds(rn, L.rec[grp * XD]);
+    for (int st = 0; st < npad; st += XD) {
+      const double* rec = L.rec[grp * XD];
+      const int grp1 = grp + 1 == NGRP ? 0 : grp + 1, round1 = grp + 1 == NGRP ? round + 1 : round;
+      const int slot0 = st & (RING - 1);
+      if (prog < st + XD - 1) wait_at_least(&ch.prog[0], st + XD - 1);
+      if (cons < st + XD - RING) wait_at_least(&ch.cons[1], st + XD - RING);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      read_in((st - 1) & (RING - 1));
+#pragma unroll
+      for (int u = 0; u < XD; u++) {
+        const int s = st + u;
+        const R4 r = rn;
+        if (u == XD - 1) {
+          if (s + 1 < npad && ok && pv < XD * round1)
+            ok = wait_bounded(&L.filled[grp1], XD * round1, a.err, a.spin_max);
+          __atomic_signal_fence(__ATOMIC_SEQ_CST);
+          load_lds(rn, L.rec[grp1 * XD]);
+        } else {
+          load_lds(rn, rec + (u + 1) * PS::N);
+        }
+        double jin[NP];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          const double x = shr1_in(in[p], tm[p]);
+          jin[p] = lane == 32 ? in[p] : x;
+        }
+        if (u + 1 < XD) read_in(slot0 + u);
+        // the reference's order per equation: (Res + dui) + duj forward, X + (dui +
+        // duj) / alfa backward (cell_step)
+        double du[NP], W[NP];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          const double sum = even_lane(fwd ? (r.X[p] + tm[p]) + jin[p] : tm[p] + jin[p]);
+          const bool sa = NV == 5 && p == 2;
+          const double q = div_hl(sum, sa ? r.yh4 : r.yh, sa ? r.yl4 : r.yl);
+          du[p] = fwd ? q : r.X[p] + q;
+          W[p] = r.U[p] + du[p];
+        }
+        double C[4];
+        both_halves(W[1], C[0], C[3]);
+        both_halves(W[0], C[1], C[2]);
+        const double y = rcp_n(C[0]);
+        const double pr = pressure_y(C, y, g);
+        const double un = div_y(C[1] * r.n1 + C[2] * r.n2, C[0], y);
+        const double nA = h ? r.n2 : r.n1, pB = h ? pr : 0.0;
+        double Fn[NP];
+        Fn[0] = W[0] * un + pr * nA;
+        Fn[1] = (W[1] + pB) * un;
+        if constexpr (NP == 3) Fn[NP - 1] = W[NP - 1] * un;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+          tm[p] = (Fn[p] - r.F[p]) * r.a + r.Lc * du[p];
+          if constexpr (VISC) tm[p] = tm[p] + r.Lv * du[p];
+        }
+        rout[slot0 + u][rg] = tm[0];
+        rout[slot0 + u][rg + 1] = tm[1];
+        if constexpr (NP == 3) rout2[slot0 + u][rg2] = tm[NP - 1];
+        interleave<0x100, NREAD, 1>();
+        if constexpr (fwd) {
+          const bool act = (uint32_t)(s - ts) < (uint32_t)ncol;
+          bstore2(du[0], du[1], rs, act ? 2 * w8 + (h ? n16 : 0u) : NOWHERE, bw);
+          if constexpr (NV == 5) bstore1(du[NP - 1], rs, act && !h ? w8 : NOWHERE, bw + 2 * n16);
+          if constexpr (NV == 6) bstore1(du[NP - 1], rs, act ? 2 * w8 + 8u * h : NOWHERE, bw + 2 * n16);
+          w8 -= (uint32_t)R * 8u;
+        } else {
+          const int b8 = s & 7, ck = s >> 3;
+          if (u == 0 && b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
+#pragma unroll
+          for (int p = 0; p < NP; p++)
+            if (!(NV == 5 && p == 2 && h)) L.ob[b8][eq[p]][row] = a.update ? W[p] : du[p];
+          if (u == XD - 1 && (b8 == 7 || s == npad - 1)) {
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // the chunk's writes done before it is handed over
+            lds_put(&L.ob_ready, ck + 1);
+          }
+        }
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        lds_put(&ch.prog[1], s + 1);
+        if (u == XD - 2) {
+          look();
+          pv = lds_get(&L.filled[grp1]);
+        }
+      }
+      lds_put(&ch.cons[0], st + XD - 1);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      lds_put(&L.consumed, gs0 + st + XD);
+      grp = grp1;
+      round = round1;
+    }
+  };
+  if (do_f) run_dir(std::true_type{}, 0);
+  if (do_f && do_b) {
+    // the forward sweep's stores before the producers' loads (see k_lusgs_fused)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    lds_put(&L.turned, 1);
+  }
+  if (do_b) run_dir(std::false_type{}, do_f ? npad : 0);
+}
+
+template <int NV, bool VISC, int LPC>
 __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
   using F = RecF<NV, VISC>;
-  using PS = PartSlot<NV, VISC>;
+  using PS = PartSlotOf<NV, VISC, LPC>;
   constexpr int NRING = PS::NRING, XD = PS::XD, NGRP = PS::NGRP;
-  __shared__ PartLds<NV, VISC> L;
+  constexpr int PART_ROWS = 64 / LPC;
+  __shared__ PartLds<NV, VISC, LPC> L;
   const int G = a.split, bi = blockIdx.x / G, part = blockIdx.x % G;
   const BlockDesc B = a.blocks[a.block_list[bi]];
   if (case_frozen(B.case_id)) return;  // every part of the block returns: no part waits on another
@@ -1432,17 +1663,17 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
     return;
   }
   if (wave > 0) {
-    // ---- producer: steps 2q (lanes 0-31) and 2q + 1 (lanes 32-63) of every
-    // PART_PROD-th q
+    // ---- producer: steps LPC q, .., LPC q + LPC - 1 (of PART_ROWS lanes each) of
+    // every PART_PROD-th q
     const double* skin = a.sk + B.sk_base;
-    const int row = lane & 31, half = lane >> 5, r = row0 + row;
+    const int row = lane % PART_ROWS, half = lane / PART_ROWS, r = row0 + row;
     auto produce = [&](auto fwd_c, int q0) {
       constexpr bool fwd = decltype(fwd_c)::value;
       RecSrc<NV> nx[2];
       auto fetch = [&](RecSrc<NV>& n, int q, bool x) {
-        const int sn = min(2 * q + half, npad - 1);  // past the last step: clamped to it
+        const int sn = min(LPC * q + half, npad - 1);  // past the last step: clamped to it
         load_src_sk<NV, VISC, fwd>(n, B, skin, sn - r, r);
-        if (!fwd && x) load_x<NV, VISC>(n.Res, rs, bw, n16, sn, r, S, R, ncol, nrow);
+        if (!fwd && x) load_x<NV, VISC, LPC>(n.Res, rs, bw, n16, sn, r, S, R, ncol, nrow);
       };
       int q = wave - 1;
       fetch(nx[0], q, false);
@@ -1451,13 +1682,13 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
         // the forward dU, from here on in memory
         ok = wait_bounded(&L.turned, 1, a.err, a.spin_max);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        load_x<NV, VISC>(nx[0].Res, rs, bw, n16, min(2 * q + half, npad - 1), r, S, R, ncol, nrow);
-        load_x<NV, VISC>(nx[1].Res, rs, bw, n16, min(2 * (q + PART_PROD) + half, npad - 1), r, S, R, ncol, nrow);
+        load_x<NV, VISC, LPC>(nx[0].Res, rs, bw, n16, min(LPC * q + half, npad - 1), r, S, R, ncol, nrow);
+        load_x<NV, VISC, LPC>(nx[1].Res, rs, bw, n16, min(LPC * (q + PART_PROD) + half, npad - 1), r, S, R, ncol, nrow);
       }
       auto record = [&](RecSrc<NV>& n, int q) {
         const RecSrc<NV> in = n;
         fetch(n, q + 2 * PART_PROD, true);
-        const int gs = q0 + 2 * q;  // the first of the two steps in the sequence of both sweeps
+        const int gs = q0 + LPC * q;  // the first of the steps in the sequence of both sweeps
         ok = wait_bounded(&L.consumed, (gs / XD + 1) * XD - NRING, a.err, a.spin_max);
         double* rec = L.rec[(gs + half) % NRING];
         auto SH = [&](int d) -> double& { return rec[PS::cell(d, row)]; };
@@ -1466,12 +1697,12 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_s_waitcnt(0xc07f);  // the slots' LDS writes done (lgkmcnt 0) before counting them
         if (lane == 0)
-          __hip_atomic_fetch_add(&L.filled[(gs / XD) % NGRP], 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add(&L.filled[(gs / XD) % NGRP], LPC, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       };
-      while (2 * q < npad && ok) {
+      while (LPC * q < npad && ok) {
         record(nx[0], q);
         q += PART_PROD;
-        if (2 * q >= npad || !ok) break;
+        if (LPC * q >= npad || !ok) break;
         record(nx[1], q);
         q += PART_PROD;
       }
@@ -1482,6 +1713,10 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
   }
   // ---- the sweep wave: lanes 2t, 2t+1 = row row0 + t; it issues first on its SIMD
   __builtin_amdgcn_s_setprio(3);
+  if constexpr (LPC == 4) {
+    quad_sweeps<NV, VISC>(a, L, rs, bw, n16, S, R, ncol, nrow, row0, lane, npad, g, do_f, do_b);
+    return;
+  } else {
   const int row = lane >> 1, t = row0 + row, k = lane & 1;
   auto load_lds = [&](Rec<NV, 1>& r, const double* rec) {
     const double* cp = rec + 2 * row;
@@ -1609,6 +1844,7 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
     lds_put(&L.turned, 1);
   }
   if (do_b) run_dir(std::false_type{}, do_f ? npad : 0);
+  }
 }
 
 // ----------------------------------------------------------------- scatter

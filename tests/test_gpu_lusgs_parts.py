@@ -1,4 +1,4 @@
-"""The LU-SGS launch in parts of 32 rows (GPU).
+"""The LU-SGS launch in parts of 16 or 32 rows (GPU).
 
 Blocks whose rows end one short of, at and one past a part, blocks narrower
 than a turn of the sweep wave, and blocks of different heights in one launch:
@@ -12,6 +12,7 @@ import pytest
 
 import oracle as O
 from ec2d import cases
+from ec2d import formats as F
 from ec2d import solver
 from helpers import first_diff, naca_case, vortex_case
 
@@ -31,8 +32,8 @@ def _passes(b, ref, nb, exact):
     b.res_norms()  # reports a wait that ran out of its budget, if any
 
 
-@pytest.mark.parametrize("rows,cols", [(3, 3), (31, 40), (32, 3), (32, 40), (33, 3), (33, 40), (63, 5), (64, 40),
-                                       (65, 7), (97, 3), (97, 40), ((4, 80), 16)])
+@pytest.mark.parametrize("rows,cols", [(3, 3), (15, 40), (16, 5), (17, 3), (31, 40), (32, 3), (32, 40), (33, 3), (33, 40),
+                                       (48, 7), (49, 3), (63, 5), (64, 40), (65, 7), (97, 3), (97, 40), ((4, 80), 16)])
 def test_parts_at_their_edges(rows, cols):
     lo, hi = rows if isinstance(rows, tuple) else (rows, rows)
     d = vortex_case(f"parts_{hi}_{cols}", cases.control_vortex(iters=10), nbx=1, nby=3, wmin=cols + 1, wmax=cols + 1,
@@ -58,9 +59,33 @@ def test_parts_at_their_edges(rows, cols):
 
 
 @pytest.mark.parametrize("ny", [66, 98])
-def test_parts_of_six_equations(ny):
+def test_parts_of_five_equations(ny):
     c = cases.control_sa_naca(iters=10, Re=1e6, Ma=0.6)
     d = naca_case(f"parts_sa_{ny}", c, nx=129, ny=ny, ds1=1e-5)
+    ref = O.OracleCase(d)
+    ref.init_flow()
+    with solver.Batch([solver.Case.from_dir(d)]) as b:
+        b.init_flow()
+        _passes(b, ref, 1, False)
+
+
+@pytest.mark.parametrize("rows", [33, 40])
+def test_parts_of_many_blocks(rows):
+    """More parts of 16 rows than compute units: parts of 32 (100 blocks)."""
+    d = vortex_case(f"parts_many_{rows}", cases.control_vortex(iters=10), nbx=10, nby=10, wmin=4, wmax=7,
+                    hmin=rows - 5, hmax=rows + 1)
+    ref = O.OracleCase(d)
+    ref.init_flow()
+    with solver.Batch([solver.Case.from_dir(d)]) as b:
+        b.init_flow()
+        _passes(b, ref, 100, True)
+
+
+def test_parts_of_six_equations():
+    c = cases.control_sa_naca(iters=10, Re=1e5, Ma=0.5)
+    c.Iflag_turbulence_model = F.TURB_SST
+    c.Twall = 300.0
+    d = naca_case("parts_sst", c, nx=97, ny=50, ds1=1e-4)
     ref = O.OracleCase(d)
     ref.init_flow()
     with solver.Batch([solver.Case.from_dir(d)]) as b:
