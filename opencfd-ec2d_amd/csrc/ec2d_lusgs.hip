@@ -854,8 +854,11 @@ __global__ void k_fill_u64(unsigned long long* p, int64_t n, unsigned long long 
   if (i < n) p[i] = v;
 }
 
-// The communication waves move CK steps at a time (64 / NV, at most half the
-// LDS ring), one double per lane, so that one round trip to global memory covers CK steps.
+// The communication waves have a lane for every double of CK steps (64 / NV, at
+// most half the LDS ring).  They move what has arrived, up to CK steps a round trip:
+// a row's terms reach the next part a step and a trip later.  (Whole batches of CK:
+// 7 links of 513 x 129 SA cells 0.64 -> 0.66 ms a pass, 3 of 257 x 65 Euler 221 -> 226
+// us.)
 template <int NV>
 struct CommLane {
   static constexpr int CK = 64 / NV < RING / 2 ? 64 / NV : RING / 2;
@@ -868,43 +871,51 @@ struct CommLane {
 template <int NV, int NW>
 __device__ void comm_forward(Chain<NV, NW>& ch, int nw, unsigned long long* gr, int npad) {
   const CommLane<NV> c;
-  for (int s0 = 0; s0 < npad - 1; s0 += c.CK) {
-    const int nst = min(c.CK, npad - 1 - s0);
-    wait_at_least(&ch.prog[nw], s0 + nst);
+  for (int s0 = 0; s0 < npad - 1;) {
+    int done;
+    while ((done = lds_get(&ch.prog[nw])) <= s0) __builtin_amdgcn_s_sleep(1);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const int nst = min(min(done, npad - 1) - s0, c.CK);
     const bool on = c.on && c.kk < nst;
     const double v = on ? ch.ring[nw][(s0 + c.kk) & (RING - 1)][c.f] : 0.0;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.cons[nw], s0 + nst);
     if (on) gstore(gr + (s0 + c.kk) * NV + c.f, __builtin_bit_cast(unsigned long long, v));
+    s0 += nst;
   }
 }
 
-// receiving side: take each batch of rows and feed ring[0]; then reset
+// receiving side: poll the next CK steps at once, feed those that have arrived to
+// ring[0]; then reset
 template <int NV, int NW>
 __device__ void comm_receive(Chain<NV, NW>& ch, unsigned long long* gr, int npad, int* err, int spin_max) {
   const CommLane<NV> c;
   static_assert(CommLane<NV>::CK <= RING, "a batch must fit the LDS ring");
   bool gone = false;  // the other workgroup stopped answering: wait no more
-  for (int s0 = 0; s0 < npad - 1; s0 += c.CK) {
-    const int nst = min(c.CK, npad - 1 - s0);
-    const bool on = c.on && c.kk < nst;
-    double v = 0.0;
-    if (on && !gone) {
-      unsigned long long* slot = gr + (s0 + c.kk) * NV + c.f;
-      unsigned long long x;
-      int n = 0;
-      while ((x = gload(slot)) == GSENT && ++n < spin_max) __builtin_amdgcn_s_sleep(1);
-      if (n >= spin_max) {
-        atomicOr(err, 1);
-        gone = true;
-      }
-      v = __builtin_bit_cast(double, x);
+  int tries = 0;
+  for (int s0 = 0; s0 < npad - 1;) {
+    const int rest = min(c.CK, npad - 1 - s0);
+    const bool in = c.on && c.kk < rest;
+    unsigned long long x = 0;
+    if (in && !gone) x = gload(gr + (s0 + c.kk) * NV + c.f);
+    const unsigned long long missing = __ballot(x == GSENT);
+    const int nst = missing ? min(rest, (int)__builtin_ctzll(missing) / NV) : rest;
+    if (!gone && (nst == 0 ? ++tries >= spin_max : spin_max == 0)) {
+      if (c.kk == 0 && c.f == 0) atomicOr(err, 1);
+      gone = true;
+      continue;
     }
+    if (nst == 0) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
+    tries = 0;
     // the slots of steps s0 .. s0+nst-1 are free once wave 0 read step s0+nst-1-RING
     wait_at_least(&ch.cons[0], s0 + nst - RING);
-    if (on) ch.ring[0][(s0 + c.kk) & (RING - 1)][c.f] = v;
+    if (in && c.kk < nst) ch.ring[0][(s0 + c.kk) & (RING - 1)][c.f] = __builtin_bit_cast(double, x);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.prog[0], s0 + nst);
+    s0 += nst;
   }
   // every value of this launch has been read: back to the sentinel
   for (int i = (int)(threadIdx.x & 63); i < (npad - 1) * NV; i += 64) gstore(gr + i, GSENT);
