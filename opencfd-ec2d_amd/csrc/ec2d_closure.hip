@@ -91,7 +91,7 @@ __device__ __forceinline__ void store_act(unsigned short* S, const f32x4 (&H)[4]
 
 // features of interior cell (i, j), raw (not normalised); false if undefined
 __device__ __forceinline__ bool closure_features(float* f, const BlockDesc& B, const double* base, const PlaneMap& pm,
-                                                 const CaseParams& cp, int i, int j) {
+                                                 const CaseParams& cp, int i, int j, double& mu) {
   auto PL = [&](int slot) { return base + (int64_t)slot * B.plane; };
   const double *U0 = PL(pm.U), *U1 = PL(pm.U + 1), *U2 = PL(pm.U + 2), *U3 = PL(pm.U + 3), *x1 = PL(pm.x1),
                *y1 = PL(pm.y1);
@@ -118,7 +118,7 @@ __device__ __forceinline__ bool closure_features(float* f, const BlockDesc& B, c
   grad(pr(qe), pr(qw), pr(qn), pr(qs), px, py);
   const double d = U0[q], u = uu(q), v = vv(q), p = pr(q);
   const double T = (U3[q] - 0.5 * d * (u * u + v * v)) / (cp.Cv * d);
-  const double mu = 1.0 / cp.Re * (1.0 + cp.Tsb) * sqrt(T * T * T) / (cp.Tsb + T);
+  mu = 1.0 / cp.Re * (1.0 + cp.Tsb) * sqrt(T * T * T) / (cp.Tsb + T);
   const double nu = mu / d;
   const double dw = PL(pm.dw)[q];
   const double om = fabs(vx - uy);
@@ -195,12 +195,12 @@ __device__ __forceinline__ void closure_forward(Fwd& F, const ClosureNet& N, con
 
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
-// load the network into LDS (cooperatively, the whole workgroup)
+// load the network into LDS (cooperatively, the whole workgroup; the caller's
+// barrier follows)
 __device__ __forceinline__ void load_net(ClosureNet& S, const ClosureNet* G) {
   const unsigned* src = reinterpret_cast<const unsigned*>(G);
   unsigned* dst = reinterpret_cast<unsigned*>(&S);
   for (int k = threadIdx.x; k < (int)(sizeof(ClosureNet) / 4); k += blockDim.x) dst[k] = src[k];
-  __syncthreads();
 }
 
 struct ClosureArgs {
@@ -234,12 +234,11 @@ __global__ __launch_bounds__(256) void k_closure_collect(ClosureArgs a) {
   const CaseParams cp = a.cps[B.case_id];
   const double* base = a.arena + B.base;
   float f[CL_NF];
-  const bool ok = closure_features(f, B, base, a.pm, cp, i, j);
+  double mu;
+  const bool ok = closure_features(f, B, base, a.pm, cp, i, j, mu);
   const int64_t q = pidx(B, i, j);
   auto PL = [&](int slot) { return base + (int64_t)slot * B.plane; };
-  const double d = PL(a.pm.U)[q], u = PL(a.pm.U + 1)[q] / d, v = PL(a.pm.U + 2)[q] / d;
-  const double T = (PL(a.pm.U + 3)[q] - 0.5 * d * (u * u + v * v)) / (cp.Cv * d);
-  const double mu = 1.0 / cp.Re * (1.0 + cp.Tsb) * sqrt(T * T * T) / (cp.Tsb + T);
+  const double d = PL(a.pm.U)[q];
   const double vt = PL(a.pm.U + 4)[q];
   const double X = d * vt / mu, X3 = X * X * X;
   const double fv1 = X3 / (X3 + 7.1 * 7.1 * 7.1);
@@ -251,68 +250,56 @@ __global__ __launch_bounds__(256) void k_closure_collect(ClosureArgs a) {
   o[7] = (ok && isfinite(target) && target >= 0.0) ? 1.f : 0.f;
 }
 
-// Inference over the listed cells: 64 cells per workgroup (16 per wave).
+// Inference over the listed cells: 64 cells per workgroup (16 per wave).  A chain
+// of latencies: 257 x 65 cells are one round of workgroups.  The features (FP64
+// divisions and logarithms on 16 lanes) run while the network's loads are in flight,
+// and their lanes keep the cell's mu and place for the result: 34 -> 24 us.
 __global__ __launch_bounds__(256) void k_closure_infer(ClosureArgs a) {
   __shared__ ClosureNet N;
-  __shared__ unsigned short sX[4][16 * 16], s1[4][16 * 64], s2[4][16 * 64], s3[4][16 * 64];
-  __shared__ int sok[4][16];
-  load_net(N, a.net);
+  __shared__ alignas(8) unsigned short sX[4][16 * 16], s1[4][16 * 64], s2[4][16 * 64], s3[4][16 * 64];
+  __shared__ float sz[4][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c0 = blockIdx.x * 64 + wave * 16;
-  // features: lanes 0..15 one cell each
+  const int c = blockIdx.x * 64 + wave * 16 + lane;
+  const bool mine = lane < 16 && c < a.ncell;  // one cell each
+  float f[CL_NF] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  bool ok = false, frozen = false;
+  double mu = 0.0;
+  double* out = nullptr;
+  int64_t plane = 0;
+  load_net(N, a.net);
+  if (mine) {
+    int b, i, j;
+    unpack_cell(a.cells[c], b, i, j);
+    const BlockDesc B = a.blocks[b];
+    ok = closure_features(f, B, a.arena + B.base, a.pm, a.cps[B.case_id], i, j, mu);
+    frozen = case_frozen(B.case_id);
+    plane = B.plane;
+    out = a.arena + B.base + (int64_t)a.pm.clo * plane + pidx(B, i, j);
+  }
+  __syncthreads();
   if (lane < 16) {
-    const int c = c0 + lane;
-    float f[CL_NF] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    bool ok = false;
-    if (c < a.ncell) {
-      int b, i, j;
-      unpack_cell(a.cells[c], b, i, j);
-      const BlockDesc B = a.blocks[b];
-      ok = closure_features(f, B, a.arena + B.base, a.pm, a.cps[B.case_id], i, j);
-    }
     const bool finite = ok;
-    float xs[CL_NF];
 #pragma unroll
     for (int k = 0; k < CL_NF; k++) {
-      const float x = (f[k] - N.mean[k]) * N.inv_std[k];
-      ok = ok && x >= N.lo[k] && x <= N.hi[k];
-      xs[k] = finite ? fminf(fmaxf(x, N.lo[k]), N.hi[k]) : 0.f;  // stand-in: clamped into the range
+      const float v = (f[k] - N.mean[k]) * N.inv_std[k];
+      ok = ok && v >= N.lo[k] && v <= N.hi[k];
+      f[k] = finite ? fminf(fmaxf(v, N.lo[k]), N.hi[k]) : 0.f;  // stand-in: clamped into the range
     }
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-      float x = 0.f;
-      if (k < CL_NF) x = a.standin ? xs[k] : (ok ? xs[k] : 0.f);
-      sX[wave][lane * 16 + k] = f2bf(x);
-    }
-    sok[wave][lane] = ok ? 1 : 0;
+    for (int k = 0; k < 16; k++) sX[wave][lane * 16 + k] = f2bf(k < CL_NF && (a.standin || ok) ? f[k < CL_NF ? k : 0] : 0.f);
   }
   __builtin_amdgcn_wave_barrier();
   Fwd F;
   closure_forward(F, N, sX[wave], s1[wave], s2[wave], s3[wave], lane);
-  const int r = lane & 15, q = lane >> 4;
-  if (r == 0) {
+  if ((lane & 15) == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int m = 4 * q + i, c = c0 + m;
-      if (c >= a.ncell) continue;
-      int b, ii, jj;
-      unpack_cell(a.cells[c], b, ii, jj);
-      const BlockDesc B = a.blocks[b];
-      if (case_frozen(B.case_id)) continue;
-      const CaseParams cp = a.cps[B.case_id];
-      double* base = a.arena + B.base;
-      const int64_t qq = pidx(B, ii, jj);
-      auto PL = [&](int slot) { return base + (int64_t)slot * B.plane; };
-      const double d = PL(a.pm.U)[qq], u = PL(a.pm.U + 1)[qq] / d, v = PL(a.pm.U + 2)[qq] / d;
-      const double T = (PL(a.pm.U + 3)[qq] - 0.5 * d * (u * u + v * v)) / (cp.Cv * d);
-      const double mu = 1.0 / cp.Re * (1.0 + cp.Tsb) * sqrt(T * T * T) / (cp.Tsb + T);
-      const bool ok = sok[wave][m] != 0;
-      const double mt = (ok || a.standin) ? mu * (double)softplus(F.Z4[i]) : 0.0;
-      double* out = PL(a.pm.clo) + qq;
-      *out = (a.standin && a.relax < 1.0) ? *out + a.relax * (mt - *out) : mt;
-      PL(a.pm.clo + 1)[qq] = ok ? 1.0 : 0.0;
-    }
+    for (int i = 0; i < 4; i++) sz[wave][4 * (lane >> 4) + i] = F.Z4[i];
   }
+  __builtin_amdgcn_wave_barrier();
+  if (!mine || frozen) return;
+  const double mt = (ok || a.standin) ? mu * (double)softplus(sz[wave][lane]) : 0.0;
+  *out = (a.standin && a.relax < 1.0) ? *out + a.relax * (mt - *out) : mt;
+  out[plane] = ok ? 1.0 : 0.0;
 }
 
 // Training: forward + backward over a mini-batch of samples (rows of
@@ -333,6 +320,7 @@ __global__ __launch_bounds__(256) void k_closure_train(TrainArgs a) {
   __shared__ float sdel4[4][16];
   __shared__ float sred[1][CL_NPARAM + 1];
   load_net(N, a.net);
+  __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
   const int c0 = blockIdx.x * 64 + wave * 16;
   const float inv_n = 1.f / (float)a.nbatch;
