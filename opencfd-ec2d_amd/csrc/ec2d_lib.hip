@@ -1066,9 +1066,11 @@ int advance_euler1(int level) {
 
 int advance_rk3(int level) {
   if (flush_clip(level)) return 1;
-  if (launch_pw(level, PW_COPY_UN)) return 1;
+  // Un = U: with four equations by the first residual (Set_Un's cells and variables)
+  const bool in_res = R.lv[level].o.nvar == 4;
+  if (!in_res && launch_pw(level, PW_COPY_UN)) return 1;
   for (int k = 1; k <= 3; k++) {
-    if (residual(level, level != 0 ? 2 : 0)) return 1;
+    if (residual(level, level != 0 ? 2 : 0, in_res && k == 1)) return 1;
     if (launch_pw(level, PW_RK3, k)) return 1;
     if (launch_ghost(level, 1, 1)) return 1;
   }
