@@ -1543,8 +1543,8 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
         double jin[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-          const double x = shr1_in(in[p], tm[p]);
-          jin[p] = lane == 32 ? in[p] : x;
+          const double x = shr1(tm[p]);
+          jin[p] = row == 0 ? in[p] : x;
         }
         if (u + 1 < XD) read_in(slot0 + u);
         // the reference's order per equation: (Res + dui) + duj forward, X + (dui +
