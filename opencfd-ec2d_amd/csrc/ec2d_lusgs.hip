@@ -1060,6 +1060,18 @@ __device__ __forceinline__ void load_x(double* x, __amdgpu_buffer_rsrc_t rs, uin
   const int sc = min(st, S - 1);
   const int tr = min(max(r, sc - (ncol - 1)), min(sc, nrow - 1));
   const uint32_t pos = (uint32_t)(sc * R + tr);
+  if constexpr (LPC == 4) {
+    // as the sweep wave stores them: pairs (1, 0), (2, 3), then single doubles
+    D2 v = bload2(rs, pos * 16u, bw);
+    x[1] = v.x;
+    x[0] = v.y;
+    v = bload2(rs, pos * 16u, bw + n16);
+    x[2] = v.x;
+    x[3] = v.y;
+#pragma unroll
+    for (int m = 4; m < NV; m++) x[m] = bload1(rs, pos * 16u, bw + (uint32_t)(m - 2) * n16);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < (NV + 1) / 2; j++) {
     if (2 * j + 1 == NV) {
@@ -1069,11 +1081,6 @@ __device__ __forceinline__ void load_x(double* x, __amdgpu_buffer_rsrc_t rs, uin
       x[2 * j] = v.x;
       x[2 * j + 1] = v.y;
     }
-  }
-  if constexpr (LPC == 4) {  // the sweep wave stores momentum first
-    const double t = x[0];
-    x[0] = x[1];
-    x[1] = t;
   }
 }
 
@@ -1411,7 +1418,8 @@ struct QuadSlot {
     if (d < 2 * NV) return xu(d >= NV, half(d % NV), place(d % NV), row);
     return CY + (d - YH0) / 2 * 32 + 2 * row + ((d - YH0) & 1);
   }
-  // F by lane; n1 n2, a Lc, Lv by (row, side)
+  // F by lane (of three, then the normal's component of the momentum equation);
+  // n1 n2, a Lc, Lv by (row, side)
   __device__ static constexpr int side(int k, int e, int row) {
     if (e < NV) return LANE + place(e) / 2 * 128 + 2 * (32 * half(e) + 2 * row + k) + (place(e) & 1);
     const int d = e == F::N1 ? 0 : e == F::N2 ? 1 : e == F::A ? 2 : e == F::LC ? 3 : 4;
@@ -1451,7 +1459,7 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
   constexpr int NP = PS::NP, NRING = PS::NRING, XD = PS::XD, NGRP = PS::NGRP;
   const int h = lane >> 5, row = lane >> 1 & 15, k = lane & 1, t = row0 + row;
   struct R4 {
-    double X[NP], U[NP], F[NP], yh, yl, yh4, yl4, n1, n2, a, Lc, Lv;
+    double X[NP], U[NP], F[NP], yh, yl, yh4, yl4, n1, n2, nA, a, Lc, Lv;
   };
   const int o_xu = 2 * (16 * h + row), o_cy = PS::CY + 2 * row, o_sd = PS::SIDE + 2 * (lane & 31),
             o_ln = PS::LANE + 2 * lane;
@@ -1484,7 +1492,13 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
     v = pair(o_ln);
     r.F[0] = v.x;
     r.F[1] = v.y;
-    if constexpr (NP == 3) r.F[NP - 1] = rec[o_ln + 128];
+    if constexpr (NP == 3) {
+      v = pair(o_ln + 128);
+      r.F[NP - 1] = v.x;
+      r.nA = v.y;
+    } else {
+      r.nA = h ? r.n2 : r.n1;
+    }
   };
   constexpr int NREAD = NP + 1 + (NV == 5) + 2 + VISC + NP - 1;
   // this lane's equations, for the planes' chunk buffer
@@ -1492,14 +1506,15 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
   // in a ring slot: momentum, mass or energy of half 0, of half 1, then the rest
   const int rg = 2 * h, rg2 = NV == 6 ? 4 + h : 4;
   bool ok = true;
-  int grp = 0, round = 1;  // the group slot of the turn and its use
+  int grp = 0, need = XD;  // the group slot of the turn, its steps when it is full
+  const double* rec = L.rec[0];
   auto run_dir = [&](auto fwd_c, int gs0) {
     constexpr bool fwd = decltype(fwd_c)::value;
     Chain<NV, 2>& ch = L.ch[fwd ? 0 : 1];
     double tm[NP] = {};
     constexpr uint32_t NOWHERE = 0x80000000u;  // out of the buffer's range: the store is dropped
     const int ts = t < nrow && k == 0 ? t : 0x40000000;
-    uint32_t w8 = (uint32_t)((S - 1) * R + (nrow - 1 - t)) * 8u;
+    uint32_t w16 = (uint32_t)((S - 1) * R + (nrow - 1 - t)) * 16u + (h ? n16 : 0u);
     double in[NP];
     // the last row's terms go to the next part, the others' nowhere (half 1 of five
     // equations has no third)
@@ -1518,11 +1533,12 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
     };
     look();
     R4 rn;
-    if (ok) ok = wait_bounded(&L.filled[grp], XD * round, a.err, a.spin_max);
-    load_lds(rn, L.rec[grp * XD]);
+    if (ok) ok = wait_bounded(&L.filled[grp], need, a.err, a.spin_max);
+    load_lds(rn, rec);
     for (int st = 0; st < npad; st += XD) {
-      const double* rec = L.rec[grp * XD];
-      const int grp1 = grp + 1 == NGRP ? 0 : grp + 1, round1 = grp + 1 == NGRP ? round + 1 : round;
+      const bool wrap = grp == NGRP - 1;
+      const int grp1 = wrap ? 0 : grp + 1, need1 = wrap ? need + XD : need;
+      const double* rec1 = wrap ? L.rec[0] : rec + XD * PS::N;
       const int slot0 = st & (RING - 1);
       if (prog < st + XD - 1) wait_at_least(&ch.prog[0], st + XD - 1);
       if (cons < st + XD - RING) wait_at_least(&ch.cons[1], st + XD - RING);
@@ -1533,10 +1549,10 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
         const int s = st + u;
         const R4 r = rn;
         if (u == XD - 1) {
-          if (s + 1 < npad && ok && pv < XD * round1)
-            ok = wait_bounded(&L.filled[grp1], XD * round1, a.err, a.spin_max);
+          if (s + 1 < npad && ok && pv < need1)
+            ok = wait_bounded(&L.filled[grp1], need1, a.err, a.spin_max);
           __atomic_signal_fence(__ATOMIC_SEQ_CST);
-          load_lds(rn, L.rec[grp1 * XD]);
+          load_lds(rn, rec1);
         } else {
           load_lds(rn, rec + (u + 1) * PS::N);
         }
@@ -1564,9 +1580,9 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
         const double y = rcp_n(C[0]);
         const double pr = pressure_y(C, y, g);
         const double un = div_y(C[1] * r.n1 + C[2] * r.n2, C[0], y);
-        const double nA = h ? r.n2 : r.n1, pB = h ? pr : 0.0;
+        const double pB = h ? pr : 0.0;
         double Fn[NP];
-        Fn[0] = W[0] * un + pr * nA;
+        Fn[0] = W[0] * un + pr * r.nA;
         Fn[1] = (W[1] + pB) * un;
         if constexpr (NP == 3) Fn[NP - 1] = W[NP - 1] * un;
 #pragma unroll
@@ -1579,11 +1595,12 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
         if constexpr (NP == 3) rout2[slot0 + u][rg2] = tm[NP - 1];
         interleave<0x100, NREAD, 1>();
         if constexpr (fwd) {
-          const bool act = (uint32_t)(s - ts) < (uint32_t)ncol;
-          bstore2(du[0], du[1], rs, act ? 2 * w8 + (h ? n16 : 0u) : NOWHERE, bw);
-          if constexpr (NV == 5) bstore1(du[NP - 1], rs, act && !h ? w8 : NOWHERE, bw + 2 * n16);
-          if constexpr (NV == 6) bstore1(du[NP - 1], rs, act ? 2 * w8 + 8u * h : NOWHERE, bw + 2 * n16);
-          w8 -= (uint32_t)R * 8u;
+          // (load_x reads them; the third of half 1 lands in a field that only the split
+          // sweeps' records have, with five equations unused)
+          const uint32_t w = (uint32_t)(s - ts) < (uint32_t)ncol ? w16 : NOWHERE;
+          bstore2(du[0], du[1], rs, w, bw);
+          if constexpr (NP == 3) bstore1(du[NP - 1], rs, w, bw + 2 * n16);
+          w16 -= (uint32_t)R * 16u;
         } else {
           const int b8 = s & 7, ck = s >> 3;
           if (u == 0 && b8 == 0 && ck > 0 && ok) ok = wait_bounded(&L.ob_taken, ck, a.err, a.spin_max);
@@ -1607,7 +1624,8 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       lds_put(&L.consumed, gs0 + st + XD);
       grp = grp1;
-      round = round1;
+      need = need1;
+      rec = rec1;
     }
   };
   if (do_f) run_dir(std::true_type{}, 0);
@@ -1705,6 +1723,13 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
         auto SH = [&](int d) -> double& { return rec[PS::cell(d, row)]; };
         auto SD = [&](int k, int e) -> double& { return rec[PS::side(k, e, row)]; };
         rec_body<NV, VISC, fwd, true, PS>(SH, SD, in, g, a.alfa1);
+        if constexpr (LPC == 4 && NV > 4) {
+#pragma unroll
+          for (int k = 0; k < 2; k++) {
+            rec[PS::LANE + 128 + 2 * (2 * row + k) + 1] = in.n1[k];
+            rec[PS::LANE + 128 + 2 * (32 + 2 * row + k) + 1] = in.n2[k];
+          }
+        }
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_s_waitcnt(0xc07f);  // the slots' LDS writes done (lgkmcnt 0) before counting them
         if (lane == 0)
