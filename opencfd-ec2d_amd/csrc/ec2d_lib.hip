@@ -281,9 +281,10 @@ void ghost_phases(BlockDesc& B, const std::vector<BlockDesc>& hb, const SubfaceD
   ph.push_back((int)pts.size());
 }
 
-// Rows of a part of k_lusgs_parts for a level, 0 if it does not fit.  A block's
-// parts wait for each other: all of them must be resident at once, one per CU.  A
-// part alone waits for nothing.  Parts of 16 rows (four lanes per cell) have the
+// Rows of a part of k_lusgs_parts for a level, 0 if it does not fit.  A part waits
+// for the one before it, which is dispatched before it, so a launch always ends; but
+// all of them should be resident at once, one per CU.  A part alone waits for
+// nothing.  Parts of 16 rows (four lanes per cell) have the
 // shorter step, parts of 32 (two lanes) half the links: per pass, 513 x 129 SA cells
 // (8 blocks) 640 against 670 us, 257 x 65 Euler 221 against 241, SST 313 against
 // 365.  Blocks of 17 .. 32 rows stay one part of 32, whose sweeps share a launch
@@ -2188,7 +2189,8 @@ int ec2d_du_lu_sgs_2d_noalloc(int nMesh, int mBlock, double alfa1) {
   }
   const size_t rec_bytes = ((size_t)L.sk_total * 8 + 255) / 256 * 256;
   const int64_t nring = L.dgring ? (int64_t)L.hb.size() * (L.lusgs_split - 1) * 2 * L.gstride : 0;
-  const size_t need = rec_bytes + (size_t)nring * 8;
+  const size_t need = rec_bytes;
+  const bool rings_fit = rec_bytes + (size_t)nring * 8 <= SCRATCH_BYTES;  // else the level's own
   if (need > SCRATCH_BYTES) {
     char msg[200];
     std::snprintf(msg, sizeof(msg),
@@ -2197,12 +2199,13 @@ int ec2d_du_lu_sgs_2d_noalloc(int nMesh, int mBlock, double alfa1) {
     return fail(msg);
   }
   double* sk = static_cast<double*>(base);
-  unsigned long long* gr = nring ? reinterpret_cast<unsigned long long*>(static_cast<char*>(base) + rec_bytes) : nullptr;
+  unsigned long long* gr =
+      nring && rings_fit ? reinterpret_cast<unsigned long long*>(static_cast<char*>(base) + rec_bytes) : nullptr;
   // the array keeps the last call's contents: records start at zero (padding
   // positions are read, never written), ring slots at the sentinel
   hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((L.sk_total + 255) / 256)), dim3(256), 0, R.s,
                      reinterpret_cast<unsigned long long*>(sk), L.sk_total, 0ull);
-  if (nring)
+  if (gr)
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nring + 255) / 256)), dim3(256), 0, R.s, gr, nring, GSENT);
   HIPCHK(hipGetLastError());
   if (flush_clip(nMesh - 1)) return 1;

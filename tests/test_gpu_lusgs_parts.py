@@ -91,3 +91,22 @@ def test_parts_of_six_equations():
     with solver.Batch([solver.Case.from_dir(d)]) as b:
         b.init_flow()
         _passes(b, ref, 1, False)
+
+
+def test_noalloc_at_the_scratch_limit():
+    """Euler, 1042 x 128 cells: the records fill the 64 MiB scratch but for 45 KB, the
+    links' slots (eight parts of 16 rows, 0.5 MB) stay the level's own."""
+    d = vortex_case("parts_limit", cases.control_vortex(iters=10), nbx=1, nby=1, wmin=1043, wmax=1043, hmin=129,
+                    hmax=129)
+    with solver.Batch([solver.Case.from_dir(d)]) as b:
+        b.init_flow()
+        b.run(1)
+        b.comput_residual_one_mesh(1)
+        b.du_lu_sgs_2d(1, 0, 0.0)
+        ref = b.get("dU")
+        for _ in range(2):
+            w = ref.copy()
+            w[:-1, :-1] = np.nan
+            b.put("dU", w)
+            b.du_lu_sgs_2d_noalloc(1, 0, 0.0)
+            assert first_diff(b.get("dU"), ref) is None
