@@ -234,11 +234,16 @@ __global__ __launch_bounds__(256) void k_fdm_res(FdmArgs a) {
   }
 }
 
-// Res_max / sum Res^2 of every tile from the Res planes (used when FDM blocks
-// exist, because their interior residual is only known after k_fdm_res)
+// Res_max / sum Res^2 of every tile from the Res planes: when FDM blocks
+// exist, because their interior residual is only known after k_fdm_res, and in
+// dual time, whose source (sfac not 0) follows the whole residual:
+// Res - (3 U - 4 Un + Un1) vol Sfac (sub_Residual.f90:55-64), evaluated left to
+// right.  (The source as a launch of its own: 129 x 33 cells 4.2 us of 172 an inner
+// iteration.)
 template <int NV>
 __global__ __launch_bounds__(256) void k_tile_norms(const TileDesc* tiles, const BlockDesc* blocks, double* arena,
-                                                    PlaneMap pm, double* partials, int tile_cols, int tile_rows) {
+                                                    PlaneMap pm, double* partials, int tile_cols, int tile_rows,
+                                                    double sfac) {
   const int lt = blockIdx.x;
   const TileDesc t = tiles[lt];
   const BlockDesc B = blocks[t.block];
@@ -254,7 +259,13 @@ __global__ __launch_bounds__(256) void k_tile_norms(const TileDesc* tiles, const
     if (i > B.nx - 1 || j > B.ny - 1) continue;
     int64_t q = pidx(B, i, j);
     for (int m = 0; m < NV; m++) {
-      double r = base[(int64_t)(pm.Res + m) * B.plane + q];
+      auto at = [&](int slot) -> double& { return base[(int64_t)slot * B.plane + q]; };
+      double r = at(pm.Res + m);
+      if (sfac != 0.0) {
+        const double t = (3.0 * at(pm.U + m) - 4.0 * at(pm.Un + m)) + at(pm.Un1 + m);
+        r = r - (t * at(pm.vol)) * sfac;
+        at(pm.Res + m) = r;
+      }
       mx[m] = fmax(mx[m], fabs(r));
       sm[m] = sm[m] + r * r;
     }

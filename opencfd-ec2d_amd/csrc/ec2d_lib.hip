@@ -604,6 +604,16 @@ int closure_infer() {
   return 0;
 }
 
+void launch_tile_norms(DLevel& L, double sfac) {
+#define TILE_NORMS(NV)                                                                                              \
+  hipLaunchKernelGGL(k_tile_norms<NV>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials,   \
+                     L.tile_cols, L.tile_rows, sfac)
+  if (L.o.nvar == 4) TILE_NORMS(4);
+  else if (L.o.nvar == 5) TILE_NORMS(5);
+  else TILE_NORMS(6);
+#undef TILE_NORMS
+}
+
 int launch_residual(int level, int clip, int force = 0, int set_un = 0, double* sk_out = nullptr,
                     bool sk_only = false) {
   DLevel& L = R.lv[level];
@@ -732,9 +742,7 @@ int launch_residual(int level, int clip, int force = 0, int set_un = 0, double* 
     // k_residual has just written) in one launch
     hipLaunchKernelGGL(k_fdm_lines, dim3(f.n_lines + (visc ? L.n_frows : 0)), dim3(256), 0, R.s, f);
     hipLaunchKernelGGL(k_fdm_res, dim3(L.n_frows), dim3(256), 0, R.s, f);
-    if (nv == 4) hipLaunchKernelGGL(k_tile_norms<4>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
-    else if (nv == 5) hipLaunchKernelGGL(k_tile_norms<5>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
-    else hipLaunchKernelGGL(k_tile_norms<6>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
+    launch_tile_norms(L, 0.0);
     HIPCHK(hipGetLastError());
   }
   // the per-tile partials hold this residual's norms; they are reduced when
@@ -921,7 +929,6 @@ int launch_pw(int level, int op, int krk) {
   a.nvar = L.o.nvar;
   a.op = op;
   a.krk = krk;
-  a.sfac = 0.0;
   const double Ra[3] = {1.0, 3.0 / 4.0, 1.0 / 3.0}, Rb[3] = {1.0, 1.0 / 4.0, 2.0 / 3.0}, Rg[3] = {0.0, 1.0 / 4.0, 2.0 / 3.0};
   if (krk >= 1) {
     a.ra = Ra[krk - 1];
@@ -989,21 +996,7 @@ int residual(int level, int force = 0, int set_un = 0, double* sk_out = nullptr,
     // Sfac = 1/(3 dt) on the first residual call, 1/(2 dt) afterwards
     DLevel& L = R.lv[level];
     const double dtg = R.cases[0].ctl.dt_global;
-    PwArgs a;
-    a.blocks = L.db;
-    a.rows = L.drows;
-    a.arena = L.arena;
-    a.pm = L.pm;
-    a.nvar = L.o.nvar;
-    a.op = PW_DUAL_SRC;
-    a.krk = 0;
-    a.ra = a.rb = a.rg = 0.0;
-    a.sfac = R.residual_calls == 0 ? 1.0 / (3.0 * dtg) : 1.0 / (2.0 * dtg);
-    hipLaunchKernelGGL(k_pointwise, dim3(L.nrows), dim3(256), 0, R.s, a);
-    const int nv = L.o.nvar;
-    if (nv == 4) hipLaunchKernelGGL(k_tile_norms<4>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
-    else if (nv == 5) hipLaunchKernelGGL(k_tile_norms<5>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
-    else hipLaunchKernelGGL(k_tile_norms<6>, dim3(L.ntiles), dim3(256), 0, R.s, L.dt, L.db, L.arena, L.pm, L.dpartials, L.tile_cols, L.tile_rows);
+    launch_tile_norms(L, R.residual_calls == 0 ? 1.0 / (3.0 * dtg) : 1.0 / (2.0 * dtg));
     rc = hipGetLastError() == hipSuccess ? 0 : fail("dual-time source launch failed");
   }
   R.residual_calls++;
