@@ -631,17 +631,19 @@ __device__ __forceinline__ void side_term(double* v, const Rec<NV, NS>& p, int h
 // of the last row of wave w-1 at step s-1 and nothing else from other waves,
 // so waves do not meet at a barrier per step: wave w-1 puts its last row's
 // terms of step s into slot s % RING of an LDS ring and then publishes
-// prog = s + 1; wave w reads slot (s-1) % RING.  A sweep wave runs turns of
+// prog = s + 1; wave w reads slot (s-1) % RING.  Its step 0 has no input below it: it
+// reads slot RING-1 of the cleared ring, so cons counts that read too and step
+// RING-1 is not written before it.  A sweep wave runs turns of
 // D steps and looks at the other waves' counters
 // once a turn: before a turn that starts at s0 it waits for prog >= s0+D-1
-// (its inputs) and for cons >= s0+D-RING (the slots it will write), and
-// after the turn it publishes cons = s0+D-1 (the inputs of these steps
+// (its inputs) and for cons >= s0+D+1-RING (the slots it will write), and
+// after the turn it publishes cons = s0+D (the inputs of these steps
 // taken).  Checked at every step, the counters, the branches around them and
 // the selects of the first lane cost each linked wave about 50 instructions a
 // step, a quarter of the step.
-//   Neither wait can block forever: a wave at s0 has published s0-1, the wave
+//   Neither wait can block forever: a wave at s0 has published s0, the wave
 // below stops at a turn of at most s0+D-2 when that turn needs more than
-// s0-1, that is when 2D > RING+1; D <= 4 and RING = 16.  The communication
+// s0, that is when 2D > RING+1; D <= 4 and RING = 16.  The communication
 // waves move at most RING/2 steps at a time, under the same rules.  Wave 0
 // without an input below it reads a ring of zeros whose prog is at its end,
 // the last wave without a consumer writes a ring whose cons is, so that no
@@ -663,7 +665,7 @@ struct Chain {
   double dump[RING][NV];      // where the lanes below a wave's last one write
   double ring[NW][RING][NV];  // input of wave w: the terms of the row below it
   int prog[NW];               // steps finished by the producer of ring[w]
-  int cons[NW];               // steps whose input wave w has read
+  int cons[NW];               // inputs that wave w has read, from that of step 0 on
 };
 
 __device__ __forceinline__ int lds_get(const int* p) {
@@ -782,7 +784,7 @@ __device__ __forceinline__ void sweep(__amdgpu_buffer_rsrc_t rs, uint32_t rec, u
     const int slot0 = s0 & (RING - 1);
     if constexpr (LINK) {
       if (prog < s0 + D - 1) wait_at_least(&ch.prog[wave], s0 + D - 1);
-      if (cons < s0 + D - RING) wait_at_least(&ch.cons[wave + 1], s0 + D - RING);
+      if (cons < s0 + D + 1 - RING) wait_at_least(&ch.cons[wave + 1], s0 + D + 1 - RING);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       read_in((s0 - 1) & (RING - 1));
     }
@@ -815,7 +817,7 @@ __device__ __forceinline__ void sweep(__amdgpu_buffer_rsrc_t rs, uint32_t rec, u
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (LINK) lds_put(&ch.cons[wave], s0 + D - 1);
+    if constexpr (LINK) lds_put(&ch.cons[wave], s0 + D);
   }
 }
 
@@ -879,7 +881,7 @@ __device__ void comm_forward(Chain<NV, NW>& ch, int nw, unsigned long long* gr, 
     const bool on = c.on && c.kk < nst;
     const double v = on ? ch.ring[nw][(s0 + c.kk) & (RING - 1)][c.f] : 0.0;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    lds_put(&ch.cons[nw], s0 + nst);
+    lds_put(&ch.cons[nw], s0 + nst + 1);
     if (on) gstore(gr + (s0 + c.kk) * NV + c.f, __builtin_bit_cast(unsigned long long, v));
     s0 += nst;
   }
@@ -911,7 +913,7 @@ __device__ void comm_receive(Chain<NV, NW>& ch, unsigned long long* gr, int npad
     }
     tries = 0;
     // the slots of steps s0 .. s0+nst-1 are free once wave 0 read step s0+nst-1-RING
-    wait_at_least(&ch.cons[0], s0 + nst - RING);
+    wait_at_least(&ch.cons[0], s0 + nst + 1 - RING);
     if (in && c.kk < nst) ch.ring[0][(s0 + c.kk) & (RING - 1)][c.f] = __builtin_bit_cast(double, x);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     lds_put(&ch.prog[0], s0 + nst);
@@ -1541,7 +1543,7 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
       const double* rec1 = wrap ? L.rec[0] : rec + XD * PS::N;
       const int slot0 = st & (RING - 1);
       if (prog < st + XD - 1) wait_at_least(&ch.prog[0], st + XD - 1);
-      if (cons < st + XD - RING) wait_at_least(&ch.cons[1], st + XD - RING);
+      if (cons < st + XD + 1 - RING) wait_at_least(&ch.cons[1], st + XD + 1 - RING);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       read_in((st - 1) & (RING - 1));
 #pragma unroll
@@ -1620,7 +1622,7 @@ __device__ __forceinline__ void quad_sweeps(const LusgsArgs& a, PartLds<NV, VISC
           pv = lds_get(&L.filled[grp1]);
         }
       }
-      lds_put(&ch.cons[0], st + XD - 1);
+      lds_put(&ch.cons[0], st + XD);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       lds_put(&L.consumed, gs0 + st + XD);
       grp = grp1;
@@ -1814,7 +1816,7 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
       const int grp1 = grp + 1 == NGRP ? 0 : grp + 1, round1 = grp + 1 == NGRP ? round + 1 : round;
       const int slot0 = st & (RING - 1);
       if (prog < st + XD - 1) wait_at_least(&ch.prog[0], st + XD - 1);
-      if (cons < st + XD - RING) wait_at_least(&ch.cons[1], st + XD - RING);
+      if (cons < st + XD + 1 - RING) wait_at_least(&ch.cons[1], st + XD + 1 - RING);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       read_in((st - 1) & (RING - 1));
 #pragma unroll
@@ -1866,7 +1868,7 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
           pv = lds_get(&L.filled[grp1]);
         }
       }
-      lds_put(&ch.cons[0], st + XD - 1);
+      lds_put(&ch.cons[0], st + XD);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       lds_put(&L.consumed, gs0 + st + XD);
       grp = grp1;
