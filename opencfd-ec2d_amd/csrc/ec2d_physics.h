@@ -33,8 +33,10 @@ __device__ __forceinline__ double rcp_rn(double b) {
 // residual).  Together they are the compiler's own a / b without the
 // operand scaling and the fix-up of zeros, infinities and extreme exponents:
 // the same bits for normal operands, and about 45 cycles of issue
-// instead of 65 (12 for each further quotient).  An operand outside the range
-// (a flow that has blown up) gives NaN.
+// instead of 65 (12 for each further quotient).  An operand or a quotient outside
+// the range (zero density, a flow that has blown up) gives NaN; where the reference's
+// value matters there (the cold-cell stop, the time step), the caller tests for it
+// and divides.
 __device__ __forceinline__ double rcp_n(double b) {
   double y = __builtin_amdgcn_rcp(b);
 #pragma unroll
@@ -52,7 +54,8 @@ __device__ __forceinline__ double div_n(double a, double b) { return div_y(a, b,
 
 // sqrt(x) of a normal x > 0 likewise: Goldschmidt's iteration on the
 // hardware's 1/sqrt(x), then two steps with the exact residual x - g^2, the
-// compiler's own steps without scaling and the cases 0 and infinity.
+// compiler's own steps without scaling and the cases 0 and infinity, which give
+// NaN (callers test for it, as above).
 __device__ __forceinline__ double sqrt_n(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;

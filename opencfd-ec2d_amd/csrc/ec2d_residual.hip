@@ -196,6 +196,11 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
     double uu = div_y(u1, d, yd);
     double vv = div_y(u2, d, yd);
     double T = div_n(u3 - 0.5 * d * (uu * uu + vv * vv), cp.Cv * d);
+    if (T != T) {  // out of div_n's range: an energy of minus infinity is a cold cell, as for the reference
+      uu = u1 / d;
+      vv = u2 / d;
+      T = (u3 - 0.5 * d * (uu * uu + vv * vv)) / (cp.Cv * d);
+    }
     sd[lj][li] = d;
     su[lj][li] = uu;
     sv[lj][li] = vv;
@@ -215,7 +220,10 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
       const int lc = lj - 1, lr = li - 1;
       bool ring = (i >= 0 && i <= nx && j >= 0 && j <= ny);
       double am = 0.0;
-      if (ring) am = div_n(cp.c_am * sqrt_n(T * T * T), cp.Tsb + T);
+      if (ring) {
+        am = div_n(cp.c_am * sqrt_n(T * T * T), cp.Tsb + T);
+        if (am != am) am = cp.c_am * sqrt(T * T * T) / (cp.Tsb + T);
+      }
       // SST: the model scaled interior Amu by Re and back (sub_turbulence_SST.f90:85, 259)
       if constexpr (NV == 6) {
         if (interior) am = (am * cp.Re) / cp.Re;
@@ -589,9 +597,15 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
     double uni = su[lj][li] * ni1 + sv[lj][li] * ni2;
     double unj = su[lj][li] * nj1 + sv[lj][li] * nj2;
     double T;
-    if constexpr (VISC) T = sT[lj][li];
-    else T = div_n(at(PL(pm.U + 3), q8) - 0.5 * d * (su[lj][li] * su[lj][li] + sv[lj][li] * sv[lj][li]), cp.Cv * d);
+    if constexpr (VISC) {
+      T = sT[lj][li];
+    } else {
+      const double e = at(PL(pm.U + 3), q8) - 0.5 * d * (su[lj][li] * su[lj][li] + sv[lj][li] * sv[lj][li]);
+      T = div_n(e, cp.Cv * d);
+      if (T != T) T = e / (cp.Cv * d);
+    }
     double cc = div_y(sqrt_n(T), cp.Ma, cp.yMa);
+    if (cc != cc) cc = sqrt(T) / cp.Ma;
     double Lci = (fabs(uni) + cc) * si;
     double Lcj = (fabs(unj) + cc) * sj;
     double Lvi = 0.0, Lvj = 0.0;
@@ -600,6 +614,11 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
       const double y0 = rcp_n(s0);
       Lvi = div_y(tmp1 * si * si, s0, y0);
       Lvj = div_y(tmp1 * sj * sj, s0, y0);
+      if (Lvi + Lvj != Lvi + Lvj) {
+        tmp1 = g / d * (sAm[cc_][cr] / cp.Pr + sAt[cc_][cr] / EC2D_PRT);
+        Lvi = tmp1 * si * si / s0;
+        Lvj = tmp1 * sj * sj / s0;
+      }
     }
     if (!a.sk_only) {
       if constexpr (VISC) {
@@ -614,6 +633,7 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
       dt = cp.dt_global;
     } else {
       dt = div_n(cp.CFL * s0, Lci + Lcj + 1.0 * (Lvi + Lvj));
+      if (dt != dt) dt = cp.CFL * s0 / (Lci + Lcj + 1.0 * (Lvi + Lvj));
       if (dt > cp.dtmax) dt = cp.dtmax;
       if (dt < cp.dtmin) dt = cp.dtmin;
     }
