@@ -253,6 +253,11 @@ __device__ __forceinline__ void flux_ausm(const double* QL, const double* QR, do
   double hr = div_n(g * pr, (g - 1.0) * dr) + 0.5 * (uur * uur + vvr * vvr);
   double al = sqrt_n(div_n(g * pl, dl)), ar = sqrt_n(div_n(g * pr, dr));
   double a = 0.5 * (al + ar);
+  if (a != a) {  // a pressure of zero
+    al = sqrt(g * pl / dl);
+    ar = sqrt(g * pr / dr);
+    a = 0.5 * (al + ar);
+  }
   const double ya = rcp_n(a);
   double Ml = div_y(uul, a, ya), Mr = div_y(uur, a, ya);
   double Mp4, Mm4, Pp5, Pm5;

@@ -97,3 +97,22 @@ def test_time_step_of_a_hot_cell(kind, e):
             if a != "dt":
                 g, r = g[:-1, :-1], r[:-1, :-1]
             assert first_diff(g, r) is None, a
+
+
+@pytest.mark.parametrize("kind", ["euler", "laminar"])
+def test_ausm_with_zero_pressure(kind):
+    """A ghost cell of zero pressure and temperature, first-order AUSM: the sound
+    speed on its side of the face is zero."""
+    d = _case(kind, F.SCHEME_UD1, F.FLUX_AUSM)
+    ref = O.OracleCase(d)
+    ref.init_flow()
+    with solver.Batch([solver.Case.from_dir(d)]) as b:
+        b.init_flow()
+        U = b.get("U")
+        _spoil(U[7, 1], m=0.0, e=0.0)
+        b.put("U", U)
+        ref.block().U[...] = U
+        ref.residual()
+        assert np.isfinite(ref.block().Res).all()
+        b.comput_residual_one_mesh(1)
+        assert first_diff(b.get("Res"), ref.block().Res) is None
