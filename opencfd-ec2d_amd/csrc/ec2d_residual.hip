@@ -548,7 +548,9 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
       double fv1 = div_n(X3, X3 + Cv1_3);
       double fv2 = 1.0 - div_n(X, 1.0 + X * fv1);
       double kd_ = SA_k * dwc;
-      double S1 = fmax(S + div_n(fv2 * vtc, kd_ * kd_), EC2D_SP(0.3) * S);
+      double Sd = div_n(fv2 * vtc, kd_ * kd_);
+      if (Sd != Sd) Sd = fv2 * vtc / (kd_ * kd_);  // (fmax would drop a NaN: a wall distance whose square overflows)
+      double S1 = fmax(S + Sd, EC2D_SP(0.3) * S);
       // S1 is zero in a uniform stream: the full division, whose infinity becomes 10
       double r = fmin(vtc / (S1 * SA_k * SA_k * dwc * dwc), 10.0);
       double gg = r + Cw2 * (r * r * r * r * r * r - r);

@@ -116,3 +116,27 @@ def test_ausm_with_zero_pressure(kind):
         assert np.isfinite(ref.block().Res).all()
         b.comput_residual_one_mesh(1)
         assert first_diff(b.get("Res"), ref.block().Res) is None
+
+
+@pytest.mark.parametrize("dw", [1e154, 1e200, 1.7e308])
+def test_sa_source_far_from_any_wall(dw):
+    """A wall distance whose square overflows (a caller's own dw where there is no
+    wall): the source keeps its production by the vorticity.  exp is the device's
+    own: 1e-11 of the largest value, as everywhere with this model."""
+    d = _case("sa")
+    ref = O.OracleCase(d)
+    ref.init_flow()
+    with solver.Batch([solver.Case.from_dir(d)]) as b:
+        b.init_flow()
+        U = b.get("U")
+        rng = np.random.default_rng(3)
+        U[..., 1:3] += 0.1 * rng.standard_normal(U[..., 1:3].shape)
+        b.put("U", U)
+        ref.block().U[...] = U
+        ref.block().dw[:] = dw
+        b.put("dw", ref.block().dw)
+        ref.residual()
+        b.comput_residual_one_mesh(1)
+        g, r = b.get("Res")[..., 4], ref.block().Res[..., 4]
+        assert np.isfinite(r).all()
+        np.testing.assert_allclose(g, r, rtol=0, atol=1e-11 * np.abs(r).max())
