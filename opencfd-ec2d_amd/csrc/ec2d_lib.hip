@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -162,6 +163,12 @@ struct Runtime {
 };
 
 Runtime R;
+
+// Held by an entry point from its first use of the staging buffers or the mailbox to
+// its last, so that host threads may read and write arrays, norms and forces at the
+// same time (dual-time stepping reads norms inside ec2d_run: recursive).
+std::recursive_mutex io_mutex;
+typedef std::lock_guard<std::recursive_mutex> IoLock;
 
 constexpr int STAGE_N = 1 << 17;  // 1 MiB: a 257 x 65 block of six components in one chunk
 
@@ -515,6 +522,7 @@ int check_ready(bool refresh = true) {
 int mailed_errors(bool cold);
 
 int device_errors(bool cold) {
+  IoLock lock(io_mutex);
   hipLaunchKernelGGL(k_mail, dim3(1), dim3(64), 0, R.s, R.mail, (const double*)nullptr, R.derr, R.dsweep_err);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(R.s));
@@ -2056,6 +2064,7 @@ int ec2d_commit(void) {
 }
 
 int ec2d_put_array(int case_id, int nMesh, int mBlock, int which, const double* src) {
+  IoLock lock(io_mutex);
   if (check_ready()) return 1;
   if (case_id < 0 || case_id >= (int)R.cases.size() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad case / mesh");
   int gb = global_block(case_id, nMesh - 1, mBlock);
@@ -2072,6 +2081,7 @@ int ec2d_put_array(int case_id, int nMesh, int mBlock, int which, const double* 
 }
 
 int ec2d_get_array(int case_id, int nMesh, int mBlock, int which, double* dst) {
+  IoLock lock(io_mutex);
   if (check_ready(which != EC2D_U)) return 1;
   if (case_id < 0 || case_id >= (int)R.cases.size() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad case / mesh");
   int gb = global_block(case_id, nMesh - 1, mBlock);
@@ -2887,6 +2897,7 @@ int ec2d_closure_monitor(double growth, int* active) {
 }
 
 int ec2d_force_coefficients(int case_id, double* cl, double* cd, double* forces) {
+  IoLock lock(io_mutex);
   if (check_ready()) return 1;
   if (case_id < 0 || case_id >= (int)R.cases.size()) return fail("bad case id");
   DLevel& L = R.lv[0];
@@ -2943,6 +2954,7 @@ int ec2d_synchronize(void) {
 }
 
 int ec2d_res_norms(int case_id, int nMesh, double* res_max, double* res_rms) {
+  IoLock lock(io_mutex);
   if (check_ready(false)) return 1;
   if (case_id < 0 || case_id >= (int)R.cases.size() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad case / mesh");
   DLevel& L = R.lv[nMesh - 1];
