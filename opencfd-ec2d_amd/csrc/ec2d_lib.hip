@@ -234,6 +234,8 @@ void ghost_phases(BlockDesc& B, const std::vector<BlockDesc>& hb, const SubfaceD
   for (int k = 0; k < B.nsub; k++) {
     const SubfaceDesc& sf = s[k];
     if (sf.neighb >= 0) continue;
+    // other types are no boundary condition (sub_boundary.f90:20-32): their ghost cells stay
+    if (sf.neighb != -10 && sf.norm_off < 0) continue;
     const size_t p0 = pts.size();
     int pt = 0;
     for (int j = sf.jst; j <= sf.jend; j++)
@@ -1855,6 +1857,7 @@ int ec2d_commit(void) {
           sf.neighb = s[6]; sf.nsub_nb = s[7]; sf.orient = s[8];
           sf.nb_block = -1;
           sf.norm_off = -1;
+          if (sf.neighb == 0) return fail("subface without a boundary condition or a neighbour block");
           if (sf.neighb > 0) {
             if (sf.neighb > (int)c.levels[l].size()) return fail("interface to a missing block");
             auto& nb = c.levels[l][sf.neighb - 1];
