@@ -88,6 +88,8 @@ struct DLevel {
   int part_rows = 0;
   bool planar_stale = false;  // Res, dt, Lc, Lv are current only in the hyperplane copy (planar_refresh)
   bool skew_static = false;   // the record arena holds the skewed copy of the mesh planes
+  bool du_stale = false;      // the last update wrote U alone: dU from its inputs (du_refresh)
+  double du_alfa1 = 0.0;      // that update's alfa1
   unsigned long long* dgring = nullptr;  // split sweeps: one ring per boundary between workgroups and direction
   int64_t gstride = 0;                   // slots of one ring
   int4* dwall = nullptr;      // wall faces (block, face, i, j), cases in order
@@ -315,7 +317,7 @@ int parts_rows(const DLevel& L) {
 // parts: that of k_lusgs_parts (also R = nrow), with `split` set here to the
 // parts of the tallest block.
 int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false, bool parts = false) {
-  L.skew_static = false;  // the arena is cleared below
+  L.skew_static = L.du_stale = false;  // the arena is cleared below
   int max_rows = 1;
   for (auto& d : L.hb) max_rows = std::max(max_rows, d.ny - 1);
   const int rq = 64 / lpc;  // rows per wave
@@ -822,7 +824,10 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
   // the level's own record arena (when a launch covers every block), on
   // every launch into a caller's arena
   const bool static_skew = L.lusgs_fused && (sk != nullptr || !L.skew_static);
-  if (L.lusgs_fused && sk == nullptr && dlist == L.dblocks_all && nblk == (int)L.hb.size()) L.skew_static = true;
+  const bool all = dlist == L.dblocks_all && nblk == (int)L.hb.size();
+  if (L.lusgs_fused && sk == nullptr && all) L.skew_static = true;
+  if (all) L.du_stale = L.lusgs_fused && update;
+  if (L.du_stale) L.du_alfa1 = alfa1;
 #define LLAUNCH(NV, V)                                                                      \
   if (L.lusgs_fused) {                                                                      \
     prof_mark(4 + pk);                                                                      \
@@ -903,6 +908,15 @@ int planar_refresh() {
     HIPCHK(hipGetLastError());
   }
   return 0;
+}
+
+// dU of a level's last main-loop update on the fused path, which writes U alone: the
+// same sweeps once more, from the inputs that it left in hyperplane order, into the dU
+// planes.  Called where dU is read, replaced in part, or its inputs go.
+int du_refresh(int level) {
+  DLevel& L = R.lv[level];
+  if (!L.du_stale) return 0;
+  return launch_lusgs(level, L.dblocks_all, (int)L.hb.size(), L.du_alfa1, 0, nullptr, nullptr, true);
 }
 
 int launch_ghost(int level, int do_bc, int do_exchange) {
@@ -2077,6 +2091,7 @@ int ec2d_put_array(int case_id, int nMesh, int mBlock, int which, const double* 
   DLevel& L = R.lv[nMesh - 1];
   int slot, nc, kind;
   if (array_map(L, which, &slot, &nc, &kind)) return fail("bad array selector");
+  if (which == EC2D_DU && du_refresh(nMesh - 1)) return 1;
   const BlockDesc& bd = L.hb[gb];
   if (move_array<true>(bd, L.arena + bd.base + (int64_t)slot * bd.plane, const_cast<double*>(src), kind, nc)) return 1;
   if (which == EC2D_U) R.clip_pending[nMesh - 1] = false;
@@ -2093,6 +2108,7 @@ int ec2d_get_array(int case_id, int nMesh, int mBlock, int which, double* dst) {
   DLevel& L = R.lv[nMesh - 1];
   int slot, nc, kind;
   if (array_map(L, which, &slot, &nc, &kind)) return fail("bad array selector");
+  if (which == EC2D_DU && du_refresh(nMesh - 1)) return 1;
   const BlockDesc& bd = L.hb[gb];
   if (move_array<false>(bd, L.arena + bd.base + (int64_t)slot * bd.plane, dst, kind, nc)) return 1;
   // the arrays of a run stopped by T < 1e-5 stay readable; a timed-out sweep fails
@@ -2178,6 +2194,7 @@ int ec2d_du_lu_sgs_2d(int nMesh, int mBlock, double alfa1) {
   if (mBlock == 0) return launch_lusgs(nMesh - 1, L.dblocks_all, (int)L.hb.size(), alfa1, 0);
   if (R.cases.size() != 1) return fail("a single block can only be selected in a one-case batch");
   if (mBlock < 1 || mBlock > (int)L.hb.size()) return fail("bad block");
+  if (du_refresh(nMesh - 1)) return 1;  // the other blocks' dU, before the launch's copy replaces this block's inputs
   return launch_lusgs(nMesh - 1, L.dblocks_all + (mBlock - 1), 1, alfa1, 0);
 }
 
@@ -2216,12 +2233,13 @@ int ec2d_du_lu_sgs_2d_noalloc(int nMesh, int mBlock, double alfa1) {
   HIPCHK(hipGetLastError());
   if (flush_clip(nMesh - 1)) return 1;
   if (mBlock == 0) return launch_lusgs(nMesh - 1, L.dblocks_all, (int)L.hb.size(), alfa1, 0, sk, gr);
+  if (du_refresh(nMesh - 1)) return 1;  // the other blocks' dU
   return launch_lusgs(nMesh - 1, L.dblocks_all + (mBlock - 1), 1, alfa1, 0, sk, gr);
 }
 
 int ec2d_update_u(int nMesh) {
   if (check_ready() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad mesh level");
-  if (flush_clip(nMesh - 1)) return 1;
+  if (flush_clip(nMesh - 1) || du_refresh(nMesh - 1)) return 1;
   return launch_pw(nMesh - 1, PW_UPDATE);
 }
 
@@ -2310,6 +2328,9 @@ int ec2d_run(int n_iter) {
       for (int l = 0; l < 3; l++)
         for (int t = 0; t < R.graph_ticks[l]; t++) tick(l);
     if (R.graph_sko) R.lv[0].planar_stale = true;  // as advance_lusgs marks it in an eager pass
+    if (R.cases[0].ctl.Time_Method == 0)            // and launch_lusgs
+      for (auto& L : R.lv)
+        if (L.lusgs_fused) L.du_stale = true, L.du_alfa1 = 0.0;
   } else {
     // capture one pass of the loop body; the clip flag must be in a steady
     // state (the body leaves it as it found it from the second pass on)
@@ -2446,8 +2467,10 @@ int ec2d_run_to_drop(double drop, int max_iter, int check_every, int* iters, int
       last_print = el;
     }
   }
-  // leave the mode: every case runs again in later calls
+  // leave the mode: every case runs again in later calls.  Where a case stopped, the
+  // residual of that check has replaced the inputs of its last update: no dU from them.
   R.conv_on = false;
+  for (auto& L : R.lv) L.du_stale = false;
   mask = nullptr;
   if (hipMemcpyToSymbol(HIP_SYMBOL(g_case_active), &mask, sizeof(mask)) != hipSuccess && !rc)
     rc = fail("ec2d_run_to_drop: clearing the case mask failed");
@@ -2488,6 +2511,7 @@ int ec2d_timing(double* run_ms, double* residual_ms, double* lusgs_ms, double* g
 int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block) {
   if (check_ready() || nMesh < 1 || nMesh > R.num_mesh) return fail("bad mesh level");
   if (lanes_per_cell != 1 && lanes_per_cell != 2) return fail("lanes per cell must be 1 or 2");
+  if (du_refresh(nMesh - 1)) return 1;  // the arena that holds its inputs goes
   HIPCHK(hipStreamSynchronize(R.s));
   DLevel& L = R.lv[nMesh - 1];
   // 0: fused, in parts where they fit; -3: fused, a workgroup per block
@@ -2513,6 +2537,8 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
   if (check_ready()) return 1;
   if (R.profile) return fail("autotune needs the profile mode off");
   if (reps < 1) reps = 5;
+  for (int l = 0; l < R.num_mesh; l++)
+    if (du_refresh(l)) return 1;
   HIPCHK(hipStreamSynchronize(R.s));  // the layouts below are rewritten with null-stream copies
   // cache: one line per level configuration, "key tile_rows lpc split u"; the
   // last field held a launch option that no longer exists (kept, so that older files still load)
