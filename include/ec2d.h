@@ -328,8 +328,10 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block);
  * workgroups per block (1, 2 or 4, see ec2d_lusgs_shape) and the fused LU-SGS
  * launches, each timed with HIP events over `reps` launches on the current
  * state; the fastest is kept.  Results are cached per level configuration
- * (equations, scheme, flux, reconstruction, turbulence model, viscosity,
- * block shapes) in the text file cache_path (NULL or "": no cache).  report
+ * (time method, one level or several, equations, scheme, flux, reconstruction,
+ * turbulence model, viscosity, block shapes) in the text file cache_path (NULL
+ * or "": no cache); lines of earlier versions of the library, which chose among other
+ * launches, are left in the file and not used.  report
  * receives one line per level.  Changes no result bit: the level's planes are
  * copied before the timed launches and put back after them (a learned
  * closure's under-relaxed mu_t included).  No reference counterpart. */

@@ -2541,7 +2541,8 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
     if (du_refresh(l)) return 1;
   HIPCHK(hipStreamSynchronize(R.s));  // the layouts below are rewritten with null-stream copies
   // cache: one line per level configuration, "key tile_rows lpc split u"; the
-  // last field held a launch option that no longer exists (kept, so that older files still load)
+  // last field held a launch option that no longer exists.  A file may hold lines of
+  // older keys, whose choices were made among other launches: no key finds them.
   struct Choice { int tr, lp, sp, u; };
   std::vector<std::pair<std::string, Choice>> cache;
   if (cache_path && cache_path[0]) {
@@ -2556,8 +2557,10 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
   std::vector<std::pair<std::string, Choice>> added;
   for (int l = 0; l < R.num_mesh; l++) {
     DLevel& L = R.lv[l];
-    // key: the level's block shapes, equations and discretisation
-    std::string key = "nv" + std::to_string(L.o.nvar) + "_s" + std::to_string(L.o.scheme) + "_f" +
+    // key: a format number (raised with the launches to choose from), the level's
+    // block shapes, equations and discretisation, and what decides what a pass's update
+    // costs (below): the time method, and whether the level is the only one
+    std::string key = "2_m" + std::to_string(R.cases[0].ctl.Time_Method) + (R.num_mesh > 1 ? "_mg" : "") + "_nv" + std::to_string(L.o.nvar) + "_s" + std::to_string(L.o.scheme) + "_f" +
                       std::to_string(L.o.flux) + "_r" + std::to_string(L.o.recon) + "_t" + std::to_string(L.o.turb) +
                       "_v" + std::to_string(R.cases[0].cp.If_viscous) + (L.fdm ? "_fdm" : "");
     // the block shapes in order, as a count and a 64-bit FNV-1a hash (a key
@@ -2622,24 +2625,24 @@ int ec2d_autotune(const char* cache_path, int reps, char* report, int report_len
           if (ms < best) { best = ms; best_lp = lp; best_sp = sp; }
         }
       // the fused variants: records made in the sweep workgroup, a workgroup
-      // per block (0; rows <= 64) or per part (-1).  Timed with the
-      // residual before them, which writes their inputs in a main-loop pass
-      // (advance_lusgs), less the plain residual: the copy kernel that a lone
-      // update needs is no part of a pass.
+      // per block (0; rows <= 64) or per part (-1).  Where the residual of a
+      // main-loop pass writes their inputs (advance_lusgs: steady LU-SGS), timed with it,
+      // less the plain residual; in other time methods and on finite-difference
+      // levels alone, with the copy of the inputs that they make themselves there.
       bool fits = true;
       for (auto& b : L.hb) fits = fits && b.ny - 1 <= 64;
       for (int sp : {0, -1}) {
         if (!(sp == 0 ? fits : parts_rows(L)) || lusgs_layout(L, 1, 1, true, true, sp == -1)) continue;
         L.lusgs_fused = true;
         L.lusgs_parts = sp == -1;
-        const bool rskew = !L.fdm;
+        const bool rskew = !L.fdm && R.cases[0].ctl.Time_Method == 0;
         double ms;
         if (time_launches(reps, [&] {
-              return launch_residual(l, 0, 0, 0, rskew ? L.sk : nullptr, rskew && R.num_mesh == 1) ||
+              return (rskew && launch_residual(l, 0, 0, 0, L.sk, R.num_mesh == 1)) ||
                      launch_lusgs(l, L.dblocks_all, (int)L.hb.size(), 0.0, 0, nullptr, nullptr, rskew);
             }, &ms))
           return 1;
-        ms -= res_ms;
+        if (rskew) ms -= res_ms;
         note(sp == 0 ? "fused" : "parts", ms);
         if (ms < best) { best = ms; best_lp = 1; best_sp = sp; }
       }
