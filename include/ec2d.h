@@ -304,11 +304,13 @@ int ec2d_kernel_time(int nMesh, int kind, double *ms, int *launches);
  * No reference counterpart: measurement support. */
 int ec2d_set_profile(int on);
 
-/* The budget of the LU-SGS sweeps' bounded waits between waves and between
+/* The budget of the LU-SGS launches' bounded waits between waves and between
  * workgroups, in polls (default 2^20, about a second); past it the wave gives
- * up and the device error word is set (see ec2d_synchronize).  With 0 every
- * receiving wave of a split sweep gives up at its first slot: a host-forced
- * way to exercise the error path.  No reference counterpart. */
+ * up and the device error word is set (see ec2d_synchronize).  It bounds the waits
+ * between workgroups (split sweeps, parts) and, in the fused launches, those between
+ * the waves that make, use and store a block's records.  With 0 every
+ * receiving wave gives up at its first slot, every other at its first poll that
+ * fails: a host-forced way to exercise the error path.  No reference counterpart. */
 int ec2d_set_wait_budget(int polls);
 
 /* No reference counterpart: the LU-SGS launch shape of one level, chosen by
@@ -320,11 +322,14 @@ int ec2d_set_wait_budget(int polls);
  * whose workgroups make each block's records themselves, so that they never go
  * through device memory - in parts of 16 or 32 rows where every part finds a CU of
  * its own, one workgroup per block otherwise (-3: one workgroup per block in
- * any case).  Results do not depend on it. */
+ * any case).  Levels of taller blocks get the launch in parts from the rule or from
+ * ec2d_autotune, not by hand.  The flow does not depend on the shape; of the residual
+ * norms the last places do, since before a fused launch the residual walks its tiles in
+ * another order. */
 int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block);
 
 /* Autotune the launch shapes of every mesh level on the committed batch:
- * residual tile rows (1, 2, 4, 8 x 64 cells), LU-SGS lanes per cell (1 or 2),
+ * residual tiles (1, 2, 4 or 8 rows of 64 cells, 8 or 16 of 32), LU-SGS lanes per cell (1 or 2),
  * workgroups per block (1, 2 or 4, see ec2d_lusgs_shape) and the fused LU-SGS
  * launches, each timed with HIP events over `reps` launches on the current
  * state; the fastest is kept.  Results are cached per level configuration
@@ -332,7 +337,7 @@ int ec2d_lusgs_shape(int nMesh, int lanes_per_cell, int workgroups_per_block);
  * turbulence model, viscosity, block shapes) in the text file cache_path (NULL
  * or "": no cache); lines of earlier versions of the library, which chose among other
  * launches, are left in the file and not used.  report
- * receives one line per level.  Changes no result bit: the level's planes are
+ * receives one line per level.  Changes no bit of the flow: the level's planes are
  * copied before the timed launches and put back after them (a learned
  * closure's under-relaxed mu_t included).  No reference counterpart. */
 int ec2d_autotune(const char *cache_path, int reps, char *report, int report_len);

@@ -212,7 +212,8 @@ __device__ __forceinline__ void char_to_prim(const double V[4], const double S1[
 // ---- interface fluxes, Q = (rho, u_n, u_t, p): sub_flux_split.f90 -----------
 // The quotients keep the reference's operands; those that share a divisor
 // (1 + tmpp three times, ava*ava and 2*ava*ava = 2 RN(ava*ava) exactly) share
-// its reciprocal, those by a constant (2 delt) take it from the compiler.
+// its reciprocal, those by a constant (2 delt) take it from the compiler (div_y's one
+// step for both: see the constant divisors of k_residual).
 __device__ __forceinline__ void flux_roe(const double* QL, const double* QR, double* Fx, double g) {
   constexpr double delt = 0.1;  // :271
   constexpr double y2d = 1.0 / (2.0 * delt);

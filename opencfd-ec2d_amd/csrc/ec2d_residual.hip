@@ -99,7 +99,7 @@ __device__ __forceinline__ void wave_fold(double (&v)[N], OP op) {
 
 // One workgroup per tile of TX x TY cells, one thread per cell.  Instruction
 // issue bounds large batches: of 256 SA blocks (3.1e6 cells, 32 x 8 tiles) a
-// cell takes 2510 vector instructions, which keep the units busy 71% of 0.35
+// cell takes 2480 vector instructions, which keep the units busy 69% of 0.35
 // ms; its loads and stores alone would take 0.17 ms.  (3284 instructions and
 // 0.45 ms with the general divisions, square roots and pow, 64-bit addresses per
 // access, a division of each thread index by the halo's width, LDS
@@ -126,8 +126,10 @@ __global__ __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(FIX ? 4 
   constexpr int CW = TX + 2, CH = TY + 2;  // the viscous quantities are used one cell out
   const int o_scheme = FIX == 3 ? 0 : FIX ? 5 : a.o.scheme, o_gscheme = FIX ? 5 : a.o.global_scheme;
   const int o_flux = FIX == 2 ? 6 : FIX ? 4 : a.o.flux, o_recon = FIX ? 0 : a.o.recon;
-  // reciprocals of the constant divisors; div_y with them gives the
-  // reference's quotients (x / Pr, x / Pr_t, x / sigma, x / k^2, x / Ma)
+  // reciprocals of the constant divisors for div_y (x / Pr, x / Pr_t, x / sigma,
+  // x / k^2, x / Ma): the reference's quotients in every comparison, but by trial and
+  // not by a theorem, since a y need not be within an ulp of the quotient (1.2e9
+  // numerators over 16 such divisors and random ones on the CPU: all correctly rounded)
   constexpr double yPrt = 1.0 / EC2D_PRT, ySig = 1.0 / (2.0 / 3.0), yK2 = 1.0 / (0.41 * 0.41);
   // viscous cases stage T and rebuild p = p00 d T from it (the staging's own
   // expression, so the same value); the cell centres of the viscous
