@@ -92,6 +92,7 @@ struct DLevel {
   double du_alfa1 = 0.0;      // that update's alfa1
   unsigned long long* dgring = nullptr;  // split sweeps: one ring per boundary between workgroups and direction
   int64_t gstride = 0;                   // slots of one ring
+  unsigned* dtickets = nullptr;          // launch in parts: one count per block, 0 between launches
   int4* dwall = nullptr;      // wall faces (block, face, i, j), cases in order
   int* dcase_wall0 = nullptr;
   double* sk = nullptr;       // LU-SGS records (skewed, see ec2d_lusgs.hip)
@@ -293,8 +294,8 @@ void ghost_phases(BlockDesc& B, const std::vector<BlockDesc>& hb, const SubfaceD
 }
 
 // Rows of a part of k_lusgs_parts for a level, 0 if it does not fit.  A part waits
-// for the one before it, which is dispatched before it, so a launch always ends; but
-// all of them should be resident at once, one per CU.  A part alone waits for
+// for the one before it, which has started before it (its tickets), so a launch always
+// ends; but all of them should be resident at once, one per CU.  A part alone waits for
 // nothing.  Parts of 16 rows (four lanes per cell) have the
 // shorter step, parts of 32 (two lanes) half the links: per pass, 513 x 129 SA cells
 // (8 blocks) 640 against 670 us, 257 x 65 Euler 221 against 241, SST 313 against
@@ -369,6 +370,8 @@ int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false,
   L.lusgs_threads = threads;
   if (L.dgring) HIPCHK(hipFree(L.dgring));
   L.dgring = nullptr;
+  if (L.dtickets) HIPCHK(hipFree(L.dtickets));
+  L.dtickets = nullptr;
   L.gstride = 0;
   if (split > 1) {
     // one ring per boundary between parts of a block and sweep direction, a
@@ -379,6 +382,12 @@ int lusgs_layout(DLevel& L, int lpc, int split, bool upload, bool fused = false,
     const int64_t n = (int64_t)L.hb.size() * (split - 1) * 2 * L.gstride;
     HIPCHK(hipMalloc(&L.dgring, sizeof(unsigned long long) * n));
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, R.s, L.dgring, n, GSENT);
+    if (parts) {
+      const int64_t nt = ((int64_t)L.hb.size() + 1) / 2;
+      HIPCHK(hipMalloc(&L.dtickets, sizeof(unsigned long long) * nt));
+      hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, R.s,
+                         reinterpret_cast<unsigned long long*>(L.dtickets), nt, 0ull);
+    }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(R.s));
   }
@@ -800,6 +809,7 @@ int launch_lusgs(int level, const int* dlist, int nblk, double alfa1, int update
   a.dir = 0;
   a.gring = gring ? gring : L.dgring;
   a.gstride = L.gstride;
+  a.tickets = L.dtickets;
   a.err = R.dsweep_err;
   a.spin_max = R.wait_budget;
   a.nblk = nblk;
@@ -1484,7 +1494,7 @@ int ec2d_finalize(void) {
     hipFree(L.arena); hipFree(L.db); hipFree(L.ds); hipFree(L.dgpts); hipFree(L.dgph); hipFree(L.dnorm); hipFree(L.dt); hipFree(L.dperm);
     hipFree(L.dcase_tile0); hipFree(L.dncell); hipFree(L.dpartials); hipFree(L.dnorms); hipFree(L.drows);
     hipFree(L.dblocks_all); hipFree(L.sk); hipFree(L.dwall); hipFree(L.dcase_wall0);
-    hipFree(L.dgring);
+    hipFree(L.dgring); hipFree(L.dtickets);
     hipFree(L.d_ilines); hipFree(L.d_frows);
   }
   hipFree(R.clo.dnet); hipFree(R.clo.theta); hipFree(R.clo.m1); hipFree(R.clo.m2); hipFree(R.clo.part);

@@ -102,6 +102,7 @@ struct LusgsArgs {
   int dir;                // sweep: 0 both sweeps, 1 forward only, 2 backward only (split launches)
   unsigned long long* gring;  // sweep, split: one ring per boundary between workgroups and direction
   int64_t gstride;        // sweep, split: slots of one ring (at least npad * NV)
+  unsigned* tickets;      // parts: per block of the launch, the workgroups that have started (0 between launches)
   int* err;               // sweep, split: set when a cross-workgroup wait ran out of its budget
   int spin_max;           // the budget of a bounded wait, in polls
   int nblk;               // skew: blocks of this launch
@@ -1438,6 +1439,7 @@ struct PartLds {
   Chain<NV, 2> ch[2];    // one per sweep
   int filled[F::NGRP];
   int consumed, turned, ob_ready, ob_taken;
+  int part;
 };
 constexpr int PART_PROD = 3;       // producers: waves 1 .. 3 (wave 4 ends at once, see FUSED_THREADS)
 constexpr int PART_THREADS = 512;  // then the writer, the receiving and the sending wave
@@ -1646,16 +1648,19 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
   constexpr int NRING = PS::NRING, XD = PS::XD, NGRP = PS::NGRP;
   constexpr int PART_ROWS = 64 / LPC;
   __shared__ PartLds<NV, VISC, LPC> L;
-  const int G = a.split, bi = blockIdx.x / G, part = blockIdx.x % G;
+  const int G = a.split, bi = blockIdx.x / G;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // A block's workgroups take its parts in the order in which they start, so that the
+  // part below has always started before one that waits for it, however another
+  // process's kernels share the device (by block index alone each could hold the CUs that
+  // the other's lower parts need).  The count wraps to 0 with the last of them.
+  if (tid == 0) L.part = G > 1 ? (int)atomicInc(a.tickets + bi, (unsigned)(G - 1)) : 0;
   const BlockDesc B = a.blocks[a.block_list[bi]];
   if (case_frozen(B.case_id)) return;  // every part of the block returns: no part waits on another
   const double g = a.cps[B.case_id].gamma;
   const int ncol = B.nx - 1, nrow = B.ny - 1;
   const int nparts = (nrow + PART_ROWS - 1) / PART_ROWS;
-  if (part >= nparts) return;  // the launch fits the level's tallest block
-  const bool has_in = part > 0, has_out = part < nparts - 1;
-  const int S = B.sk_S, R = B.sk_R, row0 = part * PART_ROWS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int S = B.sk_S, R = B.sk_R;
   for (int q = tid; q < 2 * (int)(sizeof(Chain<NV, 2>) / 8); q += PART_THREADS) reinterpret_cast<double*>(L.ch)[q] = 0.0;
   if (tid < NGRP) L.filled[tid] = 0;
   if (tid == 0) {
@@ -1663,6 +1668,10 @@ __global__ __launch_bounds__(PART_THREADS) void k_lusgs_parts(LusgsArgs a) {
     L.turned = a.dir == 2 ? 1 : 0;  // a backward launch finds the forward dU in memory
   }
   __syncthreads();
+  const int part = __builtin_amdgcn_readfirstlane(L.part);
+  if (part >= nparts) return;  // the launch fits the level's tallest block
+  const bool has_in = part > 0, has_out = part < nparts - 1;
+  const int row0 = part * PART_ROWS;
   if (tid < 2) {
     if (!has_in) L.ch[tid].prog[0] = CHAIN_END;
     if (!has_out) L.ch[tid].cons[1] = CHAIN_END;
